@@ -15,6 +15,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <new>
+#include <type_traits>
 #include <vector>
 
 #include "pf_common.hpp"
@@ -1404,6 +1405,182 @@ __global__ __launch_bounds__(kSmallThreads) void k_small_vcycle(SmallArgs a) {
     }
 }
 
+// ================================================================ a coarsest level too large for the V-cycle above
+// The coarsest level's `sweeps` red-black sweeps from zero and its mean
+// removal in one workgroup, for a level that does not fit k_small_vcycle
+// (a grid whose extents stop halving early: 104 x 76 x 52 ends at 26 x 19 x
+// 13, 200^3 at 25^3).  One launch per half-sweep costs about 3 us of launch
+// and memory latency for a few thousand cells, 120 times per V-cycle; here a
+// half-sweep is LDS reads and a barrier.  Each thread keeps the faces, b and
+// omega / diag of its cells in registers (KP pairs along k, one cell of each
+// colour per pair) and only the iterate is in LDS, since 5 n floats would
+// not fit.  The cells of even and of odd k are kept in two arrays, indexed by
+// pair: the cells of one colour in a row then lie next to each other, and a
+// wave's reads fall on all LDS banks (in cell order one colour uses every
+// other bank: 108 us instead of 69 at 26 x 19 x 13).  Faces on a wall are
+// given weight 0 in the sum (their neighbour is the cell itself, so their
+// flux is 0; they stay in the diagonal), so the neighbour addresses need no
+// clamps: zeros on either side of the arrays keep them inside.  ZL: the z
+// faces are in LDS too, which holds 8 pairs per thread without spilling in
+// the sweeps (a cell's high z face is the next cell's low one).
+// FP32 faces and iterate in every precision, like k_small_vcycle; p is
+// rounded to ST once, when stored.
+// What is left is VALU issue and LDS bandwidth of one CU, 0.6 us per
+// half-sweep.  A V-cycle on the grid of twice the extents, launched
+// half-sweeps -> this: 26 x 19 x 13 365 -> 113 us, 33 x 25 x 11 371 -> 157,
+// 27 x 27 x 15 472 -> 188, 25^3 384 -> 297 (beyond 8 pairs per thread one CU
+// would be slower than the launches).
+constexpr int kCoarsestPairs = 8;        // largest KP
+constexpr int kCoarsestPairsRegs = 5;    // largest KP with the z faces in registers
+constexpr int kCoarsestBytes = 156 * 1024;
+
+// floats from k_coarsest's even-k array to its odd-k one: the pairs, with
+// room on both sides, in whole rounds of the LDS banks
+__host__ __device__ inline int coarsest_stride(const Dims& d) {
+    const int nkp = (d.nz + 1) >> 1;
+    return (d.nx * d.ny * nkp + 2 * d.ny * nkp + 63) & ~63;
+}
+
+template <typename ST, int KP, bool ZL>
+__global__ __launch_bounds__(kSmallThreads) void k_coarsest(Dims d, const float* __restrict__ bx,
+                                                            const float* __restrict__ by,
+                                                            const float* __restrict__ bz,
+                                                            const float* __restrict__ b, ST* __restrict__ pout,
+                                                            int sweeps, float omega, const int* __restrict__ done) {
+    extern __shared__ float lds[];
+    __shared__ double sh[16];
+    __shared__ float shift;
+    constexpr int NF = ZL ? 4 : 6;
+    const int tid = threadIdx.x;
+    const int SJ = d.nz, SI = d.ny * d.nz, n = d.nx * SI;
+    const int nkp = (d.nz + 1) >> 1, npair = d.nx * d.ny * nkp, SP = d.ny * nkp;
+    const int OFF = coarsest_stride(d);  // the odd array behind the even one
+    float* P = lds + SP;                 // pair t: even k at P[t], odd k at P[OFF + t]
+    float* Z = lds + 2 * OFF;            // low z faces, the same layout
+    if (done && *done) return;  // uniform: no barrier has been reached yet
+    for (int e = tid; e < 2 * OFF; e += kSmallThreads) lds[e] = 0.0f;
+    if (ZL && tid == 0) Z[npair] = Z[OFF + npair] = 0.0f;
+    int own0[KP];  // index of the pair's colour-0 cell; -1: no pair
+    float f[2][KP][NF], rb[2][KP], w[2][KP];
+#pragma unroll
+    for (int q = 0; q < KP; ++q) {
+        const int t = tid + q * kSmallThreads, tc = min(t, npair - 1);
+        const int row = tc / nkp, kp = tc - row * nkp;
+        const int i = row / d.ny, j = row - i * d.ny;
+        const int par = (i + j) & 1;  // k = 2 kp + par has colour 0
+        own0[q] = t < npair ? t + (par ? OFF : 0) : -1;
+#pragma unroll
+        for (int col = 0; col < 2; ++col) {
+            const int kk = 2 * kp + (par ^ col), k = min(kk, d.nz - 1);
+            const int c = row * d.nz + k;
+            const int fy = c + i * d.nz, fz = c + row;
+            float v[6] = {bx[c], bx[c + SI], by[fy], by[fy + SJ], bz[fz], bz[fz + 1]};
+            const float dg = v[0] + v[1] + v[2] + v[3] + v[4] + v[5];
+            const bool own = t < npair && kk < d.nz;
+            if (i == 0) v[0] = 0.0f;
+            if (i == d.nx - 1) v[1] = 0.0f;
+            if (j == 0) v[2] = 0.0f;
+            if (j == d.ny - 1) v[3] = 0.0f;
+            if (k == 0) v[4] = 0.0f;
+            if (k == d.nz - 1) v[5] = 0.0f;
+#pragma unroll
+            for (int m = 0; m < NF; ++m) f[col][q][m] = v[m];
+            if (ZL && t < npair) Z[t + ((par ^ col) ? OFF : 0)] = own ? v[4] : 0.0f;
+            rb[col][q] = b[c];
+            // 0: a cell that is never updated (none there, or no faces)
+            w[col][q] = own && dg > 0.0f ? omega / dg : 0.0f;
+        }
+    }
+    __syncthreads();
+    auto half = [&](auto colour) {
+        constexpr int col = decltype(colour)::value;
+#pragma unroll
+        for (int q = 0; q < KP; ++q) {
+#pragma clang fp contract(off)
+            // many pairs: form the addresses anew each time (kept across the
+            // loop they spill)
+            if constexpr (KP >= 5) asm volatile("" : "+v"(own0[q]));
+            if (own0[q] < 0 || w[col][q] == 0.0f) continue;
+            const int t = tid + q * kSmallThreads;
+            const int c = col == 0 ? own0[q] : 2 * t + OFF - own0[q];  // this cell
+            const int o = 2 * t + OFF - c;                            // the pair's other cell
+            const int hi = c == t ? o : o + 1;                        // the cells above and below along k
+            const float* p = P + c;
+            const float pc = p[0];
+            float s = f[col][q][0] * (pc - p[-SP]);
+            s = fmaf(f[col][q][1], pc - p[SP], s);
+            s = fmaf(f[col][q][2], pc - p[-nkp], s);
+            s = fmaf(f[col][q][3], pc - p[nkp], s);
+            s = fmaf(ZL ? Z[c] : f[col][q][NF - 2], pc - P[hi - 1], s);
+            s = fmaf(ZL ? Z[hi] : f[col][q][NF - 1], pc - P[hi], s);
+            P[c] = fmaf(rb[col][q] - s, w[col][q], pc);
+        }
+        __syncthreads();
+    };
+    for (int sw = 0; sw < sweeps; ++sw) {
+        half(std::integral_constant<int, 0>{});
+        half(std::integral_constant<int, 1>{});
+    }
+    // everything outside the cells is still 0
+    double sm[1] = {0.0};
+    for (int e = tid; e < 2 * OFF; e += kSmallThreads) sm[0] += (double)lds[e];
+    block_sum<1>(sm, sh);
+    if (tid == 0) shift = (float)(-(sm[0] / (double)n));
+    __syncthreads();
+    for (int e = tid; e < n; e += kSmallThreads) {
+        const int row = e / d.nz, k = e - row * d.nz;
+        pout[e] = from_f32<ST>(P[row * nkp + (k >> 1) + ((k & 1) ? OFF : 0)] + shift);
+    }
+}
+
+static int64_t coarsest_lds_bytes(const Dims& d, int kp) {
+    const int64_t npair = (int64_t)d.nx * d.ny * ((d.nz + 1) / 2), off = coarsest_stride(d);
+    return (2 * off + (kp > kCoarsestPairsRegs ? off + npair + 1 : 0)) * (int64_t)sizeof(float);
+}
+
+// pairs per thread of k_coarsest on a level, 0 if it does not take it
+static int coarsest_pairs(const Dims& d) {
+    const int64_t npair = (int64_t)d.nx * d.ny * ((d.nz + 1) / 2);
+    const int64_t kp = cdiv(npair, kSmallThreads);
+    if (kp > kCoarsestPairs) return 0;
+    return coarsest_lds_bytes(d, (int)kp) <= kCoarsestBytes ? (int)kp : 0;
+}
+
+template <typename ST, int KP>
+static int launch_coarsest_kp(const Dims& d, const pf_mg_level& lv, ST* p, int sweeps, float omega, const int* done,
+                              hipStream_t s) {
+    constexpr bool ZL = KP > kCoarsestPairsRegs;
+    static std::atomic<uint64_t> done_mask{0};  // devices whose LDS limit has been raised
+    int dev = 0;
+    PF_CHECK_HIP(hipGetDevice(&dev));
+    const uint64_t bit = 1ull << (dev & 63);
+    if (!(done_mask.load() & bit)) {
+        PF_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_coarsest<ST, KP, ZL>),
+                                         hipFuncAttributeMaxDynamicSharedMemorySize, kCoarsestBytes));
+        done_mask.fetch_or(bit);
+    }
+    k_coarsest<ST, KP, ZL><<<1, kSmallThreads, (size_t)coarsest_lds_bytes(d, KP), s>>>(d, lv.bx, lv.by, lv.bz, lv.b, p, sweeps, omega, done);
+    PF_CHECK_LAUNCH();
+    return PF_OK;
+}
+
+template <typename ST>
+static int launch_coarsest(int kp, const Dims& d, const pf_mg_level& lv, ST* p, int sweeps, float omega,
+                           const int* done, hipStream_t s) {
+    switch (kp) {
+    case 1:
+    case 2:  // levels this small are k_small_vcycle's
+    case 3: return launch_coarsest_kp<ST, 3>(d, lv, p, sweeps, omega, done, s);
+    case 4: return launch_coarsest_kp<ST, 4>(d, lv, p, sweeps, omega, done, s);
+    case 5: return launch_coarsest_kp<ST, 5>(d, lv, p, sweeps, omega, done, s);
+    case 6: return launch_coarsest_kp<ST, 6>(d, lv, p, sweeps, omega, done, s);
+    case 7: return launch_coarsest_kp<ST, 7>(d, lv, p, sweeps, omega, done, s);
+    case 8: return launch_coarsest_kp<ST, 8>(d, lv, p, sweeps, omega, done, s);
+    }
+    PF_REQUIRE(false, "launch_coarsest: at most 8 pairs per thread");
+    return PF_OK;
+}
+
 // Column j of the coarsest level's smoother map: `sweeps` red-black sweeps
 // (colours (0,1)) from p = 0 with b = e_j, then mean removal, as the
 // single-workgroup V-cycle runs them, in FP64.  One workgroup per column,
@@ -2108,19 +2285,28 @@ static int vcycle(const pf_mg& mg, const float* r0, ST* z0, const int* done, con
         }
         PF_CHECK_LAUNCH();
     } else {
-        // coarsest level out of HBM: sweeps, then mean removal
+        // coarsest level out of HBM: sweeps, then mean removal (in one
+        // workgroup where it fits; a one-level hierarchy's level 0 has its
+        // own right-hand side scale and residual test and stays launched)
         const int l = L - 1;
-        int rc = smooth(l, mg.coarsest, false, true);
-        if (rc) return rc;
-        CGState* st = static_cast<CGState*>(mg.scalars);
-        const int64_t n = ncell(mg.lev[l]);
-        // p is ST; the mean is taken in FP64 and the shifted value stored back
-        k_part_sum<ST><<<red_blocks(n), RT, 0, s>>>(cur[l], n, st->part);
-        PF_CHECK_LAUNCH();
-        k_comb<<<1, RT, 0, s>>>(st, C_MEAN, (int)red_blocks(n), n, &st->mu_x, 0.0);
-        PF_CHECK_LAUNCH();
-        k_shift<ST, ST><<<red_blocks(n), RT, 0, s>>>(cur[l], cur[l], n, &st->mu_x);
-        PF_CHECK_LAUNCH();
+        const int kp = L > 1 ? coarsest_pairs(ldims(mg.lev[l])) : 0;
+        if (kp) {
+            cur[l] = P(l);
+            const int rc = launch_coarsest<ST>(kp, ldims(mg.lev[l]), mg.lev[l], cur[l], mg.coarsest, mg.omega, done, s);
+            if (rc) return rc;
+        } else {
+            int rc = smooth(l, mg.coarsest, false, true);
+            if (rc) return rc;
+            CGState* st = static_cast<CGState*>(mg.scalars);
+            const int64_t n = ncell(mg.lev[l]);
+            // p is ST; the mean is taken in FP64 and the shifted value stored back
+            k_part_sum<ST><<<red_blocks(n), RT, 0, s>>>(cur[l], n, st->part);
+            PF_CHECK_LAUNCH();
+            k_comb<<<1, RT, 0, s>>>(st, C_MEAN, (int)red_blocks(n), n, &st->mu_x, 0.0);
+            PF_CHECK_LAUNCH();
+            k_shift<ST, ST><<<red_blocks(n), RT, 0, s>>>(cur[l], cur[l], n, &st->mu_x);
+            PF_CHECK_LAUNCH();
+        }
     }
     for (int l = G - 1; l >= 0; --l) {
         const pf_mg_level& lv = mg.lev[l];
