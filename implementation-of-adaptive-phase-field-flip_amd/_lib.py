@@ -216,6 +216,7 @@ SIGNATURES = {
     "pf_rasterize_spray": (ctypes.c_int, [P, P, P, I64, P, ctypes.c_int, ctypes.c_int, ctypes.c_int,
                                           F32, P]),
     "pf_adj_g2p_advect": (ctypes.c_int, [ctypes.POINTER(G2PArgs), P, P, P, P, PP, PP, PP, P]),
+    "pf_adj_g2p_advect_binned": (ctypes.c_int, [ctypes.POINTER(G2PArgs), P, P, P, P, P, P, P, PP, PP, PP, P]),
     "pf_adj_extrapolate": (ctypes.c_int, [P, PP, PP, PP, ctypes.c_int, ctypes.c_int, ctypes.c_int,
                                           ctypes.c_int, P]),
     "pf_adj_project": (ctypes.c_int, [P, PP, PP, PP, PP, P, ctypes.c_int, ctypes.c_int, ctypes.c_int,

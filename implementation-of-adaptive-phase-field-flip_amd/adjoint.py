@@ -9,7 +9,7 @@ the steps in reverse, rebuilds each step's grid fields from its checkpoint
 extrapolation: the same kernels as the forward step, so the same bits) and
 applies the transposed stages in libpfflip_hip.so:
 
-    G2P + RK3 + reflect   pf_adj_g2p_advect   (per particle; scatter to the grid)
+    G2P + RK3 + reflect   pf_adj_g2p_advect_binned (per tile; scatter to the grid)
     extrapolation         pf_adj_extrapolate  (transposed Jacobi sweeps)
     projection            pf_adj_project
     pressure solve        MG-PCG on p-bar (the operator is symmetric), then
@@ -89,7 +89,9 @@ class StepAdjoint:
         gx_in = torch.empty_like(x)
         gv_in = torch.empty_like(v)
         a = sim._g2p_args(_lib.GA_G2P | _lib.GA_ADVECT | _lib.GA_REFLECT, dt)
-        _lib.call("pf_adj_g2p_advect", ctypes.byref(a), _lib.ptr(gx_out.contiguous()),
+        # rebuild() has binned the particles at x
+        _lib.call("pf_adj_g2p_advect_binned", ctypes.byref(a), _lib.ptr(sim.perm), _lib.ptr(sim.cell_start),
+                  _lib.ptr(sim._n_active), _lib.ptr(gx_out.contiguous()),
                   _lib.ptr(gv_out.contiguous()), _lib.ptr(gx_in), _lib.ptr(gv_in),
                   _lib.ptr3(self.g_vel), _lib.ptr3(self.g_dvel), _lib.ptr3(self.g_vel_liq), _lib.stream())
         _lib.call("pf_adj_extrapolate", _lib.ptr(sim.is_liquid), _lib.ptr3(self.g_vel_liq),

@@ -7,7 +7,8 @@
 // forward stage, evaluated at the forward state that the caller rebuilds
 // from a per-step checkpoint:
 //   G2P + RK3 + reflect  -> per-particle recompute, then a P2G-shaped scatter
-//                           of the grid adjoints (pf_adj_g2p_advect)
+//                           of the grid adjoints (pf_adj_g2p_advect, or over
+//                           binned particles pf_adj_g2p_advect_binned)
 //   extrapolation        -> transposed Jacobi sweeps (pf_adj_extrapolate)
 //   projection           -> cell gather of p-bar, face beta-bar (pf_adj_project)
 //   pressure solve       -> the same symmetric MG-PCG on p-bar (caller), then
@@ -148,68 +149,13 @@ struct AdjG2PArgs {
     float* g_vel_liq[3];
 };
 
-__global__ __launch_bounds__(256) void k_adj_g2p_advect(AdjG2PArgs a) {
-    const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= a.n) return;
-    const int st = a.pstate[p];
-    const bool liquid = a.ptype[p] == 1, active = st == 0, dead = st == 2;
-    float gx[3] = {0.f, 0.f, 0.f}, gv[3] = {0.f, 0.f, 0.f};
-    if (dead) {
-        // dead particles are not touched by the forward pass
-        for (int q = 0; q < 3; ++q) {
-            a.gx_in[3 * p + q] = a.gx_out[3 * p + q];
-            a.gv_in[3 * p + q] = a.gv_out[3 * p + q];
-        }
-        return;
-    }
+// Transpose of the wall reflection and the solid push-out, which follow the
+// advection: xb, vb (adjoints of x', v') lose the components that the forward
+// pass fixed.  xc: the advected, clamped position, v1: the G2P velocity.
+__device__ inline void adj_walls_solids(const AdjG2PArgs& a, const float (&xc)[3], const float (&v1)[3],
+                                        float (&xb)[3], float (&vb)[3]) {
     const Dims d = a.d;
-    const float dx = a.dx, dt = a.dt;
-    const float x0[3] = {a.px[3 * p], a.px[3 * p + 1], a.px[3 * p + 2]};
-    const float v0[3] = {a.pv[3 * p], a.pv[3 * p + 1], a.pv[3 * p + 2]};
-
-    // ---- forward recompute
-    VelSample sx;  // samples at x: vel and dvel share the taps
-    float pic[3] = {0.f, 0.f, 0.f}, dux[3] = {0.f, 0.f, 0.f};
-    const bool do_g2p = active && (a.flags & PF_GA_G2P);
-    const bool do_adv = active && (a.flags & PF_GA_ADVECT);
-    const float al = liquid ? a.alpha_l : a.alpha_a;
-    float v1[3] = {v0[0], v0[1], v0[2]};
-    if (do_g2p || do_adv) vel_sample(sx, a.vel, x0[0], x0[1], x0[2], dx, d, pic);
-    if (do_g2p) {
-        dux[0] = interp(sx.t0, a.dvel[0]);
-        dux[1] = interp(sx.t1, a.dvel[1]);
-        dux[2] = interp(sx.t2, a.dvel[2]);
-        for (int q = 0; q < 3; ++q) v1[q] = al * (v0[q] + dux[q]) + (1.0f - al) * pic[q];
-    }
-    const float* const* f = liquid ? a.vel_liq : a.vel;
-    float* const* fbar = liquid ? a.g_vel_liq : a.g_vel;
-    VelSample s1, s2, s3;
-    float k1[3], k2[3], k3[3], xc[3] = {x0[0], x0[1], x0[2]}, y2[3], y3[3];
-    bool clamped[3] = {false, false, false};
-    const float h1 = 0.5f * dt, h2 = 0.75f * dt;
-    const float c1 = 2.0f / 9.0f, c2 = 3.0f / 9.0f, c3 = 4.0f / 9.0f;
-    if (do_adv) {
-        if (liquid)
-            vel_sample(s1, f, x0[0], x0[1], x0[2], dx, d, k1);
-        else
-            for (int q = 0; q < 3; ++q) k1[q] = pic[q];
-        for (int q = 0; q < 3; ++q) y2[q] = x0[q] + h1 * k1[q];
-        vel_sample(s2, f, y2[0], y2[1], y2[2], dx, d, k2);
-        for (int q = 0; q < 3; ++q) y3[q] = x0[q] + h2 * k2[q];
-        vel_sample(s3, f, y3[0], y3[1], y3[2], dx, d, k3);
-        for (int q = 0; q < 3; ++q) {
-            const float xn = x0[q] + dt * (c1 * k1[q] + c2 * k2[q] + c3 * k3[q]);
-            xc[q] = fminf(fmaxf(xn, a.lo[q]), a.hi[q]);
-            clamped[q] = xc[q] != xn;
-        }
-    }
-
-    // ---- backward
-    float xb[3], vb[3];
-    for (int q = 0; q < 3; ++q) {
-        xb[q] = a.gx_out[3 * p + q];
-        vb[q] = a.gv_out[3 * p + q];
-    }
+    const float dx = a.dx;
     if ((a.flags & PF_GA_SOLIDS) && a.solid) {
         // push_out_of_solids (kernels.py:630-679) after the reflection: the
         // position moves by a constant, and an inward velocity component is
@@ -267,6 +213,76 @@ __global__ __launch_bounds__(256) void k_adj_g2p_advect(AdjG2PArgs a) {
             }
         }
     }
+}
+
+// OUTSIDE: only the particles outside the bins (pstate != 0), which the tiled
+// kernel does not visit; they scatter nothing.
+template <bool OUTSIDE>
+__global__ __launch_bounds__(256) void k_adj_g2p_advect(AdjG2PArgs a, const int* __restrict__ n_binned) {
+    if (OUTSIDE && *n_binned == a.n) return;
+    const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (p >= a.n) return;
+    const int st = a.pstate[p];
+    if (OUTSIDE && st == 0) return;
+    const bool liquid = a.ptype[p] == 1, active = !OUTSIDE && st == 0, dead = st == 2;
+    float gx[3] = {0.f, 0.f, 0.f}, gv[3] = {0.f, 0.f, 0.f};
+    if (dead) {
+        // dead particles are not touched by the forward pass
+        for (int q = 0; q < 3; ++q) {
+            a.gx_in[3 * p + q] = a.gx_out[3 * p + q];
+            a.gv_in[3 * p + q] = a.gv_out[3 * p + q];
+        }
+        return;
+    }
+    const Dims d = a.d;
+    const float dx = a.dx, dt = a.dt;
+    const float x0[3] = {a.px[3 * p], a.px[3 * p + 1], a.px[3 * p + 2]};
+    const float v0[3] = {a.pv[3 * p], a.pv[3 * p + 1], a.pv[3 * p + 2]};
+
+    // ---- forward recompute
+    VelSample sx;  // samples at x: vel and dvel share the taps
+    float pic[3] = {0.f, 0.f, 0.f}, dux[3] = {0.f, 0.f, 0.f};
+    const bool do_g2p = active && (a.flags & PF_GA_G2P);
+    const bool do_adv = active && (a.flags & PF_GA_ADVECT);
+    const float al = liquid ? a.alpha_l : a.alpha_a;
+    float v1[3] = {v0[0], v0[1], v0[2]};
+    if (do_g2p || do_adv) vel_sample(sx, a.vel, x0[0], x0[1], x0[2], dx, d, pic);
+    if (do_g2p) {
+        dux[0] = interp(sx.t0, a.dvel[0]);
+        dux[1] = interp(sx.t1, a.dvel[1]);
+        dux[2] = interp(sx.t2, a.dvel[2]);
+        for (int q = 0; q < 3; ++q) v1[q] = al * (v0[q] + dux[q]) + (1.0f - al) * pic[q];
+    }
+    const float* const* f = liquid ? a.vel_liq : a.vel;
+    float* const* fbar = liquid ? a.g_vel_liq : a.g_vel;
+    VelSample s1, s2, s3;
+    float k1[3], k2[3], k3[3], xc[3] = {x0[0], x0[1], x0[2]}, y2[3], y3[3];
+    bool clamped[3] = {false, false, false};
+    const float h1 = 0.5f * dt, h2 = 0.75f * dt;
+    const float c1 = 2.0f / 9.0f, c2 = 3.0f / 9.0f, c3 = 4.0f / 9.0f;
+    if (do_adv) {
+        if (liquid)
+            vel_sample(s1, f, x0[0], x0[1], x0[2], dx, d, k1);
+        else
+            for (int q = 0; q < 3; ++q) k1[q] = pic[q];
+        for (int q = 0; q < 3; ++q) y2[q] = x0[q] + h1 * k1[q];
+        vel_sample(s2, f, y2[0], y2[1], y2[2], dx, d, k2);
+        for (int q = 0; q < 3; ++q) y3[q] = x0[q] + h2 * k2[q];
+        vel_sample(s3, f, y3[0], y3[1], y3[2], dx, d, k3);
+        for (int q = 0; q < 3; ++q) {
+            const float xn = x0[q] + dt * (c1 * k1[q] + c2 * k2[q] + c3 * k3[q]);
+            xc[q] = fminf(fmaxf(xn, a.lo[q]), a.hi[q]);
+            clamped[q] = xc[q] != xn;
+        }
+    }
+
+    // ---- backward
+    float xb[3], vb[3];
+    for (int q = 0; q < 3; ++q) {
+        xb[q] = a.gx_out[3 * p + q];
+        vb[q] = a.gv_out[3 * p + q];
+    }
+    adj_walls_solids(a, xc, v1, xb, vb);
     for (int q = 0; q < 3; ++q) gx[q] = xb[q];
     if (do_adv) {
         float kb1[3], kb2[3], kb3[3];
@@ -315,6 +331,349 @@ __global__ __launch_bounds__(256) void k_adj_g2p_advect(AdjG2PArgs a) {
         a.gx_in[3 * p + q] = gx[q];
         a.gv_in[3 * p + q] = gv[q];
     }
+}
+
+// ------------------------------------------------------------------ tiled G2P + RK3 + reflect
+// The same transpose over the binned particles.  The per-particle kernel's
+// 96 to 120 global float atomics per particle bound it (1.8 ms for 2.1M
+// particles, about 1.2e11 atomics/s).  Here one workgroup owns a tile of T^3
+// cells: it stages the sampled fields of the tile plus a 2-cell halo in LDS
+// (as k_g2p_tiled does) and adds the grid adjoints into LDS, in FP64, since
+// ds_add_f64 runs at 2.4e12/s where ds_add_f32 reaches 2.0e11 (512
+// workgroups, one cell per lane).  One global float atomic per box entry and
+// field flushes them: about 30 times fewer at 8 particles per cell.
+// The particles of one phase share their blend factor and RK3 field, so a
+// pass per phase needs six accumulated fields instead of nine (83 KB next to
+// 62 KB of samples): I^T of v-bar, which the flush splits between dvel and
+// vel, and I^T of the RK3 stages' adjoints.  Most tiles hold one phase and
+// run one pass.  Each lane takes one cell (two lanes share its particles), so
+// the lanes of a wave add to different addresses.
+// 64^3 x 8 ppc (2.1M particles): 1.80 -> 0.24 ms; 128 x 96 x 64 x 8 ppc with a
+// solid column (6.2M): 5.71 -> 0.52 ms.
+constexpr int AT = PF_TILE;
+constexpr int AB = AT + 4, AB2 = AB * AB, AB3 = AB * AB * AB;
+constexpr int kAdjThreads = 1024;
+
+// A sample point: per axis the cell and fraction on the face-normal grid (n)
+// and on the half-cell shifted one (t); in: every tap lies in the tile's box.
+struct AdjPoint {
+    int n[3], t[3];
+    float fn[3], ft[3];
+    bool in;
+};
+
+__device__ inline AdjPoint adj_point(const float (&x)[3], float inv_dx, const int (&o)[3]) {
+    AdjPoint q;
+    q.in = true;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        const float g = x[a] * inv_dx, h = g - 0.5f;
+        q.n[a] = (int)floorf(g);
+        q.fn[a] = g - (float)q.n[a];
+        q.t[a] = (int)floorf(h);
+        q.ft[a] = h - (float)q.t[a];
+        q.in = q.in && q.t[a] >= o[a] && q.n[a] <= o[a] + AB - 2;
+    }
+    return q;
+}
+
+template <int A>
+__device__ inline int adj_cell(const AdjPoint& q, int ax) { return ax == A ? q.n[ax] : q.t[ax]; }
+template <int A>
+__device__ inline float adj_frac(const AdjPoint& q, int ax) { return ax == A ? q.fn[ax] : q.ft[ax]; }
+
+template <int A>
+__device__ inline int adj_box(const AdjPoint& q, const int (&o)[3]) {
+    return ((adj_cell<A>(q, 0) - o[0]) * AB + adj_cell<A>(q, 1) - o[1]) * AB + adj_cell<A>(q, 2) - o[2];
+}
+
+// index of tap (di, dj, dk) on the face grid of axis A, clamped per axis
+template <int A>
+__device__ inline int adj_tap(const AdjPoint& q, int di, int dj, int dk, const Dims& d) {
+    const int n0 = d.nx + (A == 0), n1 = d.ny + (A == 1), n2 = d.nz + (A == 2);
+    const int i = min(max(adj_cell<A>(q, 0) + di, 0), n0 - 1), j = min(max(adj_cell<A>(q, 1) + dj, 0), n1 - 1),
+              k = min(max(adj_cell<A>(q, 2) + dk, 0), n2 - 1);
+    return (i * n1 + j) * n2 + k;
+}
+
+// value and gradient (per unit length) of one component at a point
+template <int A>
+__device__ inline void adj_sample1(const AdjPoint& q, const float* L, const float* __restrict__ G, const Dims& d,
+                                   const int (&o)[3], float inv_dx, float& val, float (&g)[3]) {
+    float v[8];
+    if (q.in) {
+        const float* l = L + adj_box<A>(q, o);
+#pragma unroll
+        for (int m = 0; m < 8; ++m) v[m] = l[(m >> 2) * AB2 + ((m >> 1) & 1) * AB + (m & 1)];
+    } else {
+#pragma unroll
+        for (int m = 0; m < 8; ++m) v[m] = G[adj_tap<A>(q, m >> 2, (m >> 1) & 1, m & 1, d)];
+    }
+    const float fx = adj_frac<A>(q, 0), fy = adj_frac<A>(q, 1), fz = adj_frac<A>(q, 2);
+    const float d00 = v[1] - v[0], d01 = v[3] - v[2], d10 = v[5] - v[4], d11 = v[7] - v[6];
+    const float c00 = v[0] + fz * d00, c01 = v[2] + fz * d01, c10 = v[4] + fz * d10, c11 = v[6] + fz * d11;
+    const float e0 = c01 - c00, e1 = c11 - c10;
+    const float b0 = c00 + fy * e0, b1 = c10 + fy * e1;
+    val = b0 + fx * (b1 - b0);
+    const float z0 = d00 + fy * (d01 - d00), z1 = d10 + fy * (d11 - d10);
+    g[0] = (b1 - b0) * inv_dx;
+    g[1] = (e0 + fx * (e1 - e0)) * inv_dx;
+    g[2] = (z0 + fx * (z1 - z0)) * inv_dx;
+}
+
+struct AdjSample {
+    float u[3];     // the three components
+    float J[3][3];  // J[c][a] = d u_c / d x_a
+};
+
+__device__ inline void adj_sample(const AdjPoint& q, const float* L, const float* const* G, const Dims& d,
+                                  const int (&o)[3], float inv_dx, AdjSample& s) {
+    adj_sample1<0>(q, L, G[0], d, o, inv_dx, s.u[0], s.J[0]);
+    adj_sample1<1>(q, L + AB3, G[1], d, o, inv_dx, s.u[1], s.J[1]);
+    adj_sample1<2>(q, L + 2 * AB3, G[2], d, o, inv_dx, s.u[2], s.J[2]);
+}
+
+__device__ inline void adj_add_JT(const AdjSample& s, const float (&k)[3], float (&y)[3]) {
+#pragma unroll
+    for (int a = 0; a < 3; ++a) y[a] += s.J[0][a] * k[0] + s.J[1][a] * k[1] + s.J[2][a] * k[2];
+}
+
+// field-bar += I^T s: into the box, or for a point outside it straight into
+// the global fields G0 (times c0) and, if non-NULL, G1 (times c1)
+template <int A>
+__device__ inline void adj_scatter1(const AdjPoint& q, double* L, const Dims& d, const int (&o)[3], float s,
+                                    float* G0, float c0, float* G1, float c1) {
+    if (s == 0.0f) return;
+    const float fx = adj_frac<A>(q, 0), fy = adj_frac<A>(q, 1), fz = adj_frac<A>(q, 2);
+    const float wx[2] = {(1.0f - fx) * s, fx * s}, wy[2] = {1.0f - fy, fy}, wz[2] = {1.0f - fz, fz};
+    if (q.in) {
+        double* l = L + adj_box<A>(q, o);
+#pragma unroll
+        for (int m = 0; m < 8; ++m)
+            unsafeAtomicAdd(l + (m >> 2) * AB2 + ((m >> 1) & 1) * AB + (m & 1),
+                            (double)(wx[m >> 2] * wy[(m >> 1) & 1] * wz[m & 1]));
+    } else {
+#pragma unroll
+        for (int m = 0; m < 8; ++m) {
+            const float w = wx[m >> 2] * wy[(m >> 1) & 1] * wz[m & 1];
+            const int f = adj_tap<A>(q, m >> 2, (m >> 1) & 1, m & 1, d);
+            unsafeAtomicAdd(G0 + f, c0 * w);
+            if (G1) unsafeAtomicAdd(G1 + f, c1 * w);
+        }
+    }
+}
+
+// the adjoint of one component of a stage sample, to the RK3 field's box
+__device__ inline void adj_scatter_stage(const AdjPoint& q, double* L, const Dims& d, const int (&o)[3],
+                                         const float (&k)[3], float* const* G) {
+    adj_scatter1<0>(q, L, d, o, k[0], G[0], 1.0f, nullptr, 0.0f);
+    adj_scatter1<1>(q, L + AB3, d, o, k[1], G[1], 1.0f, nullptr, 0.0f);
+    adj_scatter1<2>(q, L + 2 * AB3, d, o, k[2], G[2], 1.0f, nullptr, 0.0f);
+}
+
+// the same position through an opaque copy, so that what depends on it is
+// computed anew instead of being kept in registers
+struct Pos {
+    float v[3];
+};
+__device__ inline Pos fresh(const float (&x)[3]) {
+    Pos c{{x[0], x[1], x[2]}};
+    asm volatile("" : "+v"(c.v[0]), "+v"(c.v[1]), "+v"(c.v[2]));
+    return c;
+}
+
+// One particle of phase LIQ.  F: staged vel, dvel, vel_liq; AV, AK: the
+// accumulators of v-bar and of the RK3 stages.
+template <bool LIQ>
+__device__ inline void adj_particle(const AdjG2PArgs& a, int64_t p, const float* F, double* AV, double* AK,
+                                    const int (&o)[3]) {
+    const Dims d = a.d;
+    const float dt = a.dt, inv_dx = 1.0f / a.dx, al = LIQ ? a.alpha_l : a.alpha_a;
+    const bool do_g2p = a.flags & PF_GA_G2P, do_adv = a.flags & PF_GA_ADVECT;
+    const float* fk = LIQ ? F + 6 * AB3 : F;
+    const float* const* gk = LIQ ? a.vel_liq : a.vel;
+    float* const* kbar = LIQ ? a.g_vel_liq : a.g_vel;
+    const float x0[3] = {a.px[3 * p], a.px[3 * p + 1], a.px[3 * p + 2]};
+    float v1[3] = {a.pv[3 * p], a.pv[3 * p + 1], a.pv[3 * p + 2]};
+    float xb[3], vb[3];
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+        xb[q] = a.gx_out[3 * p + q];
+        vb[q] = a.gv_out[3 * p + q];
+    }
+    // ---- forward recompute.  Sample points and the gradients of the G2P
+    // samples are formed again where the backward part needs them: held, they
+    // spill (AdjPoint is 13 registers, a gradient 9).
+    AdjSample s1, s2, s3;
+    {
+        const AdjPoint q1 = adj_point(x0, inv_dx, o);
+        if (do_g2p || !LIQ) adj_sample(q1, F, a.vel, d, o, inv_dx, s1);
+        if (do_g2p) {
+            AdjSample sd;
+            adj_sample(q1, F + 3 * AB3, a.dvel, d, o, inv_dx, sd);
+#pragma unroll
+            for (int q = 0; q < 3; ++q) v1[q] = al * (v1[q] + sd.u[q]) + (1.0f - al) * s1.u[q];
+        }
+        // the first stage: vel_liq, or for air the PIC sample
+        if (LIQ && do_adv) adj_sample(q1, fk, gk, d, o, inv_dx, s1);
+    }
+    float y2[3], y3[3], xc[3] = {x0[0], x0[1], x0[2]};
+    bool clamped[3] = {false, false, false};
+    const float h1 = 0.5f * dt, h2 = 0.75f * dt;
+    const float c1 = 2.0f / 9.0f, c2 = 3.0f / 9.0f, c3 = 4.0f / 9.0f;
+    if (do_adv) {
+#pragma unroll
+        for (int q = 0; q < 3; ++q) y2[q] = x0[q] + h1 * s1.u[q];
+        adj_sample(adj_point(y2, inv_dx, o), fk, gk, d, o, inv_dx, s2);
+#pragma unroll
+        for (int q = 0; q < 3; ++q) y3[q] = x0[q] + h2 * s2.u[q];
+        adj_sample(adj_point(y3, inv_dx, o), fk, gk, d, o, inv_dx, s3);
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            const float xn = x0[q] + dt * (c1 * s1.u[q] + c2 * s2.u[q] + c3 * s3.u[q]);
+            xc[q] = fminf(fmaxf(xn, a.lo[q]), a.hi[q]);
+            clamped[q] = xc[q] != xn;
+        }
+    }
+    // ---- backward
+    adj_walls_solids(a, xc, v1, xb, vb);
+    float gx[3] = {xb[0], xb[1], xb[2]};
+    if (do_adv) {
+        float k1[3], k2[3], k3[3], yb[3] = {0.f, 0.f, 0.f};
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            if (clamped[q]) xb[q] = 0.0f;  // clamp into [lo, hi]
+            gx[q] = xb[q];
+            k1[q] = dt * c1 * xb[q];
+            k2[q] = dt * c2 * xb[q];
+            k3[q] = dt * c3 * xb[q];
+        }
+        adj_add_JT(s3, k3, yb);  // k3 = U(y3), y3 = x + h2 k2
+        adj_scatter_stage(adj_point(fresh(y3).v, inv_dx, o), AK, d, o, k3, kbar);
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            gx[q] += yb[q];
+            k2[q] += h2 * yb[q];
+            yb[q] = 0.f;
+        }
+        adj_add_JT(s2, k2, yb);  // k2 = U(y2), y2 = x + h1 k1
+        adj_scatter_stage(adj_point(fresh(y2).v, inv_dx, o), AK, d, o, k2, kbar);
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            gx[q] += yb[q];
+            k1[q] += h1 * yb[q];
+        }
+        adj_add_JT(s1, k1, gx);  // k1 = U(x)
+        adj_scatter_stage(adj_point(fresh(x0).v, inv_dx, o), AK, d, o, k1, kbar);
+    }
+    if (do_g2p) {
+        // v1 = al (v0 + I(dvel)) + (1 - al) I(vel)
+        const float kd[3] = {al * vb[0], al * vb[1], al * vb[2]};
+        const float kp[3] = {(1.0f - al) * vb[0], (1.0f - al) * vb[1], (1.0f - al) * vb[2]};
+        const AdjPoint q1 = adj_point(fresh(x0).v, inv_dx, o);
+        AdjSample s;
+        adj_sample(q1, F + 3 * AB3, a.dvel, d, o, inv_dx, s);
+        adj_add_JT(s, kd, gx);
+        adj_sample(q1, F, a.vel, d, o, inv_dx, s);
+        adj_add_JT(s, kp, gx);
+        adj_scatter1<0>(q1, AV, d, o, vb[0], a.g_dvel[0], al, a.g_vel[0], 1.0f - al);
+        adj_scatter1<1>(q1, AV + AB3, d, o, vb[1], a.g_dvel[1], al, a.g_vel[1], 1.0f - al);
+        adj_scatter1<2>(q1, AV + 2 * AB3, d, o, vb[2], a.g_dvel[2], al, a.g_vel[2], 1.0f - al);
+#pragma unroll
+        for (int q = 0; q < 3; ++q) vb[q] = kd[q];
+    }
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+        a.gx_in[3 * p + q] = gx[q];
+        a.gv_in[3 * p + q] = vb[q];
+    }
+}
+
+// box entry e of the face grid of axis AX, clamped into the grid
+template <int AX>
+__device__ inline int adj_box_src(int e, const Dims& d, const int (&o)[3]) {
+    const int n0 = d.nx + (AX == 0), n1 = d.ny + (AX == 1), n2 = d.nz + (AX == 2);
+    const int gi = min(max(o[0] + e / AB2, 0), n0 - 1), gj = min(max(o[1] + (e / AB) % AB, 0), n1 - 1),
+              gk = min(max(o[2] + e % AB, 0), n2 - 1);
+    return (gi * n1 + gj) * n2 + gk;
+}
+
+template <int AX>
+__device__ inline void adj_stage_axis(const AdjG2PArgs& a, float* F, const int (&o)[3]) {
+    const bool g2p = a.flags & PF_GA_G2P, adv = a.flags & PF_GA_ADVECT;
+    constexpr int N = (AB3 + kAdjThreads - 1) / kAdjThreads;
+    float v[3][N];
+#pragma unroll
+    for (int m = 0; m < N; ++m) {
+        const int f = adj_box_src<AX>(min((int)threadIdx.x + m * kAdjThreads, AB3 - 1), a.d, o);
+        v[0][m] = a.vel[AX][f];
+        v[1][m] = g2p ? a.dvel[AX][f] : 0.0f;
+        v[2][m] = adv ? a.vel_liq[AX][f] : 0.0f;
+    }
+#pragma unroll
+    for (int m = 0; m < N; ++m) {
+        const int e = (int)threadIdx.x + m * kAdjThreads;
+        if (e < AB3)
+#pragma unroll
+            for (int q = 0; q < 3; ++q) F[(3 * q + AX) * AB3 + e] = v[q][m];
+    }
+}
+
+template <int AX, bool LIQ>
+__device__ inline void adj_flush_axis(const AdjG2PArgs& a, const double* AV, const double* AK, const int (&o)[3]) {
+    const float al = LIQ ? a.alpha_l : a.alpha_a;
+    for (int e = threadIdx.x; e < AB3; e += kAdjThreads) {
+        const double v = AV[AX * AB3 + e], k = AK[AX * AB3 + e];
+        if (v == 0.0 && k == 0.0) continue;
+        const int f = adj_box_src<AX>(e, a.d, o);
+        if (v != 0.0) unsafeAtomicAdd(a.g_dvel[AX] + f, (float)((double)al * v));
+        if (LIQ) {
+            if (v != 0.0) unsafeAtomicAdd(a.g_vel[AX] + f, (float)((double)(1.0f - al) * v));
+            if (k != 0.0) unsafeAtomicAdd(a.g_vel_liq[AX] + f, (float)k);
+        } else {
+            unsafeAtomicAdd(a.g_vel[AX] + f, (float)((double)(1.0f - al) * v + k));
+        }
+    }
+}
+
+template <bool LIQ>
+__device__ inline bool adj_pass(const AdjG2PArgs& a, const int* __restrict__ perm, const int* __restrict__ start,
+                                int key0, const float* F, double* acc, const int (&o)[3]) {
+    for (int e = threadIdx.x; e < 6 * AB3; e += kAdjThreads) acc[e] = 0.0;
+    __syncthreads();
+    const int cell = threadIdx.x & (AT * AT * AT - 1), part = threadIdx.x / (AT * AT * AT);
+    const int e0 = start[key0 + cell + 1];
+    bool other = false;
+    for (int s = start[key0 + cell] + part; s < e0; s += kAdjThreads / (AT * AT * AT)) {
+        const int64_t p = perm[s];
+        if ((a.ptype[p] == 1) != LIQ) {
+            other = true;
+            continue;
+        }
+        adj_particle<LIQ>(a, p, F, acc, acc + 3 * AB3, o);
+    }
+    const bool more = __syncthreads_or(other);
+    adj_flush_axis<0, LIQ>(a, acc, acc + 3 * AB3, o);
+    adj_flush_axis<1, LIQ>(a, acc, acc + 3 * AB3, o);
+    adj_flush_axis<2, LIQ>(a, acc, acc + 3 * AB3, o);
+    __syncthreads();
+    return more;
+}
+
+__global__ __launch_bounds__(kAdjThreads) void k_adj_g2p_tiled(AdjG2PArgs a, const int* __restrict__ perm,
+                                                               const int* __restrict__ start, int ntx, int nty,
+                                                               int ntz) {
+    __shared__ float F[9 * AB3];
+    __shared__ double acc[6 * AB3];
+    const int t = xcd_block(blockIdx.x, ntx * nty * ntz);
+    const int tz = t % ntz, ty = (t / ntz) % nty, tx = t / (ntz * nty);
+    const int o[3] = {tx * AT - 2, ty * AT - 2, tz * AT - 2};
+    const int key0 = t * AT * AT * AT;
+    if (start[key0] == start[key0 + AT * AT * AT]) return;
+    adj_stage_axis<0>(a, F, o);
+    adj_stage_axis<1>(a, F, o);
+    adj_stage_axis<2>(a, F, o);
+    if (adj_pass<true>(a, perm, start, key0, F, acc, o)) adj_pass<false>(a, perm, start, key0, F, acc, o);
 }
 
 // ------------------------------------------------------------------ extrapolation
@@ -675,9 +1034,8 @@ __global__ __launch_bounds__(256) void k_adj_p2g(AdjP2GK a) {
 
 using namespace pf;
 
-PF_API int pf_adj_g2p_advect(const pf_g2p_args* fwd, const float* gx_out, const float* gv_out, float* gx_in,
-                             float* gv_in, float* const g_vel[3], float* const g_dvel[3],
-                             float* const g_vel_liq[3], pf_stream_t stream) {
+static int adj_g2p_args(const pf_g2p_args* fwd, const float* gx_out, const float* gv_out, float* gx_in, float* gv_in,
+                        float* const g_vel[3], float* const g_dvel[3], float* const g_vel_liq[3], AdjG2PArgs& a) {
     PF_REQUIRE(fwd, "pf_adj_g2p_advect: null args");
     const pf_g2p_args& in = *fwd;
     PF_REQUIRE(in.px && in.pv && in.ptype && in.pstate, "pf_adj_g2p_advect: need px, pv, ptype, pstate");
@@ -685,7 +1043,6 @@ PF_API int pf_adj_g2p_advect(const pf_g2p_args* fwd, const float* gx_out, const 
     PF_REQUIRE(!(in.flags & PF_GA_SOLIDS) || in.solid, "pf_adj_g2p_advect: solids flag without mask");
     PF_REQUIRE(gx_out && gv_out && gx_in && gv_in && g_vel && g_dvel && g_vel_liq, "pf_adj_g2p_advect: null adjoint");
     PF_REQUIRE(in.nx > 0 && in.ny > 0 && in.nz > 0 && in.n >= 0 && in.dx > 0.0f, "pf_adj_g2p_advect: bad sizes");
-    AdjG2PArgs a;
     a.px = in.px;
     a.pv = in.pv;
     a.ptype = in.ptype;
@@ -715,8 +1072,38 @@ PF_API int pf_adj_g2p_advect(const pf_g2p_args* fwd, const float* gx_out, const 
     a.gv_out = gv_out;
     a.gx_in = gx_in;
     a.gv_in = gv_in;
-    if (in.n == 0) return PF_OK;
-    k_adj_g2p_advect<<<cdiv(in.n, 256), 256, 0, S(stream)>>>(a);
+    return PF_OK;
+}
+
+PF_API int pf_adj_g2p_advect(const pf_g2p_args* fwd, const float* gx_out, const float* gv_out, float* gx_in,
+                             float* gv_in, float* const g_vel[3], float* const g_dvel[3],
+                             float* const g_vel_liq[3], pf_stream_t stream) {
+    AdjG2PArgs a;
+    const int rc = adj_g2p_args(fwd, gx_out, gv_out, gx_in, gv_in, g_vel, g_dvel, g_vel_liq, a);
+    if (rc) return rc;
+    if (a.n == 0) return PF_OK;
+    k_adj_g2p_advect<false><<<cdiv(a.n, 256), 256, 0, S(stream)>>>(a, nullptr);
+    PF_CHECK_LAUNCH();
+    return PF_OK;
+}
+
+PF_API int pf_adj_g2p_advect_binned(const pf_g2p_args* fwd, const int32_t* perm, const int32_t* cell_start,
+                                    const int32_t* n_active, const float* gx_out, const float* gv_out, float* gx_in,
+                                    float* gv_in, float* const g_vel[3], float* const g_dvel[3],
+                                    float* const g_vel_liq[3], pf_stream_t stream) {
+    AdjG2PArgs a;
+    const int rc = adj_g2p_args(fwd, gx_out, gv_out, gx_in, gv_in, g_vel, g_dvel, g_vel_liq, a);
+    if (rc) return rc;
+    PF_REQUIRE(perm && cell_start && n_active, "pf_adj_g2p_advect_binned: needs perm, cell_start and n_active");
+    const int ntx = (a.d.nx + AT - 1) / AT, nty = (a.d.ny + AT - 1) / AT, ntz = (a.d.nz + AT - 1) / AT;
+    // faces and binning keys are indexed with 32-bit ints
+    PF_REQUIRE((int64_t)(a.d.nx + 1) * (a.d.ny + 1) * (a.d.nz + 1) < ((int64_t)1 << 31) &&
+                   (int64_t)ntx * nty * ntz * AT * AT * AT < ((int64_t)1 << 31) - 1,
+               "pf_adj_g2p_advect_binned: grid too large");
+    if (a.n == 0) return PF_OK;
+    k_adj_g2p_tiled<<<(unsigned)(ntx * nty * ntz), kAdjThreads, 0, S(stream)>>>(a, perm, cell_start, ntx, nty, ntz);
+    PF_CHECK_LAUNCH();
+    k_adj_g2p_advect<true><<<cdiv(a.n, 256), 256, 0, S(stream)>>>(a, n_active);
     PF_CHECK_LAUNCH();
     return PF_OK;
 }

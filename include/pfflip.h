@@ -625,7 +625,7 @@ int pf_mr_emit(const pf_mr_particles* in, const int32_t* lnew, const int32_t* no
  * counterpart: the reference has no adjoint).  Each entry point transposes
  * one forward stage at the forward state, which the caller rebuilds from a
  * checkpoint of (x, v).  Order of a backward step:
- *   pf_adj_g2p_advect -> pf_adj_extrapolate -> pf_adj_project ->
+ *   pf_adj_g2p_advect (or _binned) -> pf_adj_extrapolate -> pf_adj_project ->
  *   pf_mgpcg_solve(lam = A^+ p-bar) -> pf_adj_solve_beta -> pf_adj_phase ->
  *   pf_adj_p2g.
  * Liquid tags, wall/solid masks and extrapolation masks are held at their
@@ -640,6 +640,15 @@ int pf_mr_emit(const pf_mr_particles* in, const int32_t* lnew, const int32_t* no
 int pf_adj_g2p_advect(const pf_g2p_args* fwd, const float* gx_out, const float* gv_out, float* gx_in,
                       float* gv_in, float* const g_vel[3], float* const g_dvel[3],
                       float* const g_vel_liq[3], pf_stream_t stream);
+/* The same transpose for particles binned by pf_bin_sort at px (perm,
+ * cell_start and n_active from that call, pstate unchanged since), as
+ * pf_g2p_advect_binned is the binned pf_g2p_advect: the grid adjoints are
+ * summed per 8^3 tile in LDS (FP64) before they are added with float
+ * atomics.  Results equal pf_adj_g2p_advect's up to rounding. */
+int pf_adj_g2p_advect_binned(const pf_g2p_args* fwd, const int32_t* perm, const int32_t* cell_start,
+                             const int32_t* n_active, const float* gx_out, const float* gv_out, float* gx_in,
+                             float* gv_in, float* const g_vel[3], float* const g_dvel[3],
+                             float* const g_vel_liq[3], pf_stream_t stream);
 /* Transpose of pf_extrapolate: adds E^T g_vel_liq into g_vel; g_vel_liq is
  * used as scratch; level (3 uint8 face arrays) is scratch. */
 int pf_adj_extrapolate(const int32_t* is_liquid, float* const g_vel_liq[3], float* const g_vel[3],
