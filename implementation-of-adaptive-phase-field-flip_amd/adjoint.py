@@ -3,9 +3,9 @@
 The reference has no adjoint (its Warp kernels are never recorded on a
 tape).  ``rollout`` runs ``Simulator.step`` ``n`` times inside a
 ``torch.autograd.Function``: the forward pass keeps one checkpoint of the
-particle state (x, v) and the time step per step; the backward pass walks
-the steps in reverse, rebuilds each step's grid fields from its checkpoint
-(binning, P2G, eq. (7) / beta / forces / RHS, MG-PCG, projection,
+particle state (x, v), the pressure and the time step per step; the backward
+pass walks the steps in reverse, rebuilds each step's grid fields from its
+checkpoint (binning, P2G, eq. (7) / beta / forces / RHS, projection,
 extrapolation: the same kernels as the forward step, so the same bits) and
 applies the transposed stages in libpfflip_hip.so:
 
@@ -58,8 +58,11 @@ class StepAdjoint:
         self.last_solve = (0, 0.0)
 
     # ------------------------------------------------------------------ forward rebuild
-    def rebuild(self, x: torch.Tensor, v: torch.Tensor, dt: float) -> None:
-        """Grid fields of the step that starts at (x, v); particles stay put."""
+    def rebuild(self, x: torch.Tensor, v: torch.Tensor, dt: float, pressure: torch.Tensor | None = None) -> None:
+        """Grid fields of the step that starts at (x, v); particles stay put.
+        ``pressure`` is that step's pressure where the caller has kept it: the
+        solve, most of a rebuild (3.4 of 3.9 ms at 64^3 to 1e-8), is then a
+        copy of one cell field."""
         sim = self.sim
         cfg = sim.cfg
         sim.px.copy_(x)
@@ -69,7 +72,10 @@ class StepAdjoint:
         sim._splat()
         sim._phase(_ALL_PHASE, dt)
         sim.solver.build_hierarchy(*sim.beta)
-        sim.solver.solve(sim.rhs, sim.pressure, tol=cfg.pcg_tol, max_iter=cfg.pcg_max_iter)
+        if pressure is None:
+            sim.solver.solve(sim.rhs, sim.pressure, tol=cfg.pcg_tol, max_iter=cfg.pcg_max_iter)
+        else:
+            sim.pressure.copy_(pressure)
         nx, ny, nz = sim.res
         _lib.call("pf_project", _lib.ptr(sim.pressure), _lib.ptr3(sim.beta), _lib.ptr3(sim.vel),
                   _lib.ptr3(sim.vel_star), _lib.ptr3(sim.dvel), nx, ny, nz, cfg.dx, float(dt),
@@ -77,13 +83,13 @@ class StepAdjoint:
         sim._extrapolate_liquid_velocity()
 
     # ------------------------------------------------------------------ backward
-    def backward(self, x, v, dt, gx_out, gv_out):
+    def backward(self, x, v, dt, gx_out, gv_out, pressure=None):
         """(x, v)-bar of the step from (x, v) with time step dt, given the
-        adjoints of its output (x', v')."""
+        adjoints of its output (x', v').  ``pressure``: as in ``rebuild``."""
         sim = self.sim
         cfg = sim.cfg
         nx, ny, nz = sim.res
-        self.rebuild(x, v, dt)
+        self.rebuild(x, v, dt, pressure)
         for t in self.g_vel + self.g_dvel + self.g_vel_liq:
             t.zero_()
         gx_in = torch.empty_like(x)
@@ -121,8 +127,9 @@ class _Rollout(torch.autograd.Function):
         sim.pv.copy_(v0.detach())
         ckpt, used = [], []
         for k in range(n_steps):
-            ckpt.append((sim.px.clone(), sim.pv.clone()))
+            x, v = sim.px.clone(), sim.pv.clone()
             rec = sim.step(None if dts is None else float(dts[k]))
+            ckpt.append((x, v, sim.pressure.clone()))
             used.append(rec["dt"])
         ctx.sim, ctx.ckpt, ctx.dts, ctx.adj = sim, ckpt, used, adj
         return sim.px.clone(), sim.pv.clone()
@@ -134,8 +141,8 @@ class _Rollout(torch.autograd.Function):
         gv = torch.zeros_like(sim.pv) if gv is None else gv.contiguous().float()
         adj = ctx.adj if ctx.adj is not None else StepAdjoint(sim)
         for k in reversed(range(len(ctx.ckpt))):
-            x, v = ctx.ckpt[k]
-            gx, gv = adj.backward(x, v, ctx.dts[k], gx, gv)
+            x, v, pressure = ctx.ckpt[k]
+            gx, gv = adj.backward(x, v, ctx.dts[k], gx, gv, pressure)
         return gx, gv, None, None, None, None
 
 
