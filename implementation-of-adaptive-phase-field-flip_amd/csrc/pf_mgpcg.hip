@@ -5,7 +5,7 @@
 // faces), red-black weighted Gauss-Seidel (omega = 6/7), V-cycle with
 // pre (0,1) / post (1,0) colour orders.  Large levels run one kernel per
 // red-black sweep out of HBM (one per half-sweep on request), levels of up
-// to 32^3 cells below level 0 one kernel per smoothing phase; every level
+// to about 64^3 cells one kernel per smoothing phase; every level
 // from `small_from` down is solved inside one workgroup with all its data
 // in LDS.  The FPCG scalars live on the
 // device; dot products are deterministic FP64 block reductions, and the
@@ -832,198 +832,361 @@ __global__ __launch_bounds__(RT) void k_prolong(Dims d, Dims dc, const ST* pin, 
     if (!skip) pout[t] = from_f32<ST>(v);
 }
 
-// ================================================================ fused small levels
-// A small HBM level's whole pre-smoothing phase (sweeps from zero, colour
-// order (0,1), then the residual restricted to the coarse level) or whole
-// post-smoothing phase (input pin plus the prolongation of the coarse
-// iterate, colour order (1,0)) in one launch: on a level of a few ten
-// thousand cells each per-sweep launch is bound by launch latency, not by
-// its bytes.  A workgroup owns a TI x TJ x TK tile and holds the tile plus
-// an H-cell halo (two cells per sweep) of faces, right-hand side and
-// iterate in LDS.  Each half-sweep runs on the region the tile's result
-// still depends on (margin m of the box; it shrinks by one cell per
-// half-sweep), so the halo updates duplicate the neighbouring tiles' work
-// and no workgroup waits for another.  Every update goes through the
-// helpers of the per-sweep kernels in their operation order, so the
-// results are bitwise those of the per-sweep path.  A neighbour outside the
-// grid is the cell itself (the reference's clamped indices).
-template <int TI, int TJ, int TK, int NSW>
-struct LvBox {
+// ================================================================ one launch per smoothing phase
+// A level's whole pre-smoothing phase (sweeps from zero, colour order (0,1),
+// then the residual restricted to the coarse level) or whole post-smoothing
+// phase (input pin plus the prolongation of the coarse iterate, colour order
+// (1,0)) in one launch: a level of up to about 64^3 cells is bound by its
+// launches' latency (about 5 us per sweep for 64^3 and for 32^3 alike), not
+// by its bytes.  A workgroup owns a T x T x TK tile.  It holds the faces, b
+// and diagonals of the tile plus an H-cell halo (two cells per sweep) in
+// registers and their iterate in LDS, so no workgroup waits for another: each
+// half-sweep runs on the region the tile's result still depends on (margin M
+// of the box, one cell more per half-sweep) and repeats the neighbouring
+// tiles' work there.
+//  - The box's columns (x, y) are numbered from the tile outwards in rings,
+//    so the columns at margin >= M are a prefix, and a thread's slots (pairs
+//    of cells along k, one of each colour) drop out from the last one on.
+//    Along k the whole column is updated; its ends beyond the margin are not
+//    read again.
+//  - The cells of even and odd k are in two arrays indexed by pair: one
+//    colour's cells then cover all LDS banks, and every neighbour is at a
+//    compile-time offset from one of two addresses.
+//  - A face on a wall has weight 0 in the sum (its neighbour is the cell
+//    itself, so its flux is 0) but counts in the diagonal; cells outside the
+//    grid have diagonal 0 and keep their value.
+// Every update has the operations of the per-sweep kernels in their order,
+// so the results are bitwise those of the per-sweep path.
+// VALU issue bounds it (the repeated updates are 4.7 times the tile's own at
+// 64^3, 16.5 at 32^3), so the columns' indices and walls are worked out once
+// per column, in LDS, and b is in LDS, which leaves the rest in registers.
+// One phase of 3 sweeps with its restriction / prolongation, in the solve's
+// graph: 64^3 15 / 15 us (one launch per sweep: 20 / 17), 32^3 8.6 / 7.8 us
+// (faces and b in LDS instead of registers: 10 / 10).  FPCG iteration at
+// 128^3 216 -> 207 us (BF16 212 -> 199), at 64^3 106 -> 99, at 32^3 78 -> 67.
+template <int T, int TK, int NSW>
+struct PhBox {
     static constexpr int NT = 1024;
     static constexpr int H = 2 * NSW;
-    static constexpr int BI = TI + 2 * H, BJ = TJ + 2 * H, BK = TK + 2 * H;
-    // one extra layer per axis holds the high faces of the outermost cells;
-    // rows of BK + 2 (even) entries: with odd strides every cell of one
-    // colour would sit at an address of one parity, so a half-sweep's
-    // accesses would use half the LDS banks
-    static constexpr int SJ = BK + 2, SI = (BJ + 1) * SJ, N = (BI + 1) * SI;
-    static constexpr int NPT = (N + NT - 1) / NT;
-    static_assert(TI % 2 == 0 && TJ % 2 == 0 && TK % 2 == 0, "tiles restrict to whole coarse cells");
+    static constexpr int B = T + 2 * H, BM = (TK + 2 * H) / 2;  // box: B x B columns of BM pairs
+    static constexpr int SY = BM, SX = B * BM, N = B * SX;      // LDS strides, pairs
+    static constexpr int OFF = (N + 63) & ~63;                  // odd-k array behind the even one
+    static constexpr int pairs(int M) { return (T + 2 * (H - M)) * (T + 2 * (H - M)) * BM; }  // at margin >= M
+    static constexpr int slots(int M) { return (pairs(M) + NT - 1) / NT; }
+    static_assert(T % 2 == 0 && TK % 2 == 0, "tiles restrict to whole coarse cells");
+    static_assert((T & (T - 1)) == 0, "column numbering");
 };
 
-// One half-sweep of colour col on the cells at margin >= M of the box
-// (origin o, which is even on every axis).  ZI: the iterate is zero.
-// A neighbour outside the grid is read from its ghost entry, the box entry
-// beyond the wall, which every update of the cell sets to the cell's value
-// (the reference's clamped index is the cell itself), so the six
-// neighbour reads take no branches.
-template <typename ST, typename BX, int M, bool ZI>
-__device__ inline void lv_half_sweep(float* P, const float* B, const float* FX, const float* FY,
-                                     const float* FZ, const Dims& d, int ox, int oy, int oz, int col,
-                                     float omega) {
-    constexpr int RJ = BX::BJ - 2 * M, RK2 = (BX::BK - 2 * M) / 2;
-    constexpr int NPAIR = (BX::BI - 2 * M) * RJ * RK2;
-    constexpr int SI = BX::SI, SJ = BX::SJ;
-    for (int e = threadIdx.x; e < NPAIR; e += BX::NT) {
-        const int kp = e % RK2, y = M + (e / RK2) % RJ, x = M + e / (RK2 * RJ);
-        const int z = M + 2 * kp + ((col - (x + y + M)) & 1);
-        const int gi = ox + x, gj = oy + y, gk = oz + z;
-        if (gi < 0 || gj < 0 || gk < 0 || gi >= d.nx || gj >= d.ny || gk >= d.nz) continue;
-        const int c = x * SI + y * SJ + z;
-        const float fc[6] = {FX[c], FX[c + SI], FY[c], FY[c + SJ], FZ[c], FZ[c + 1]};
-        float v;
-        if (ZI) {
-            const float dg = fc[0] + fc[1] + fc[2] + fc[3] + fc[4] + fc[5];
-            v = dg > 0.0f ? rb_first(B[c], dg, omega) : 0.0f;
-        } else {
-            const float pc = P[c], bc = B[c];
-            const float pn[6] = {P[c - SI], P[c + SI], P[c - SJ], P[c + SJ], P[c - 1], P[c + 1]};
-            float dg, Ap;
-            stencil_vals(pc, fc, pn, dg, Ap);
-            // (formed unconditionally: every read is issued at once)
-            const float vr = rb_relax(pc, bc, Ap, dg, omega);
-            v = dg > 0.0f ? vr : pc;
-        }
-        v = round_st<ST>(v);
-        P[c] = v;
-        // the ghosts (only the cell itself reads them; a low ghost of a cell
-        // on the box's first layer lies outside the box, and that cell is
-        // not updated again)
-        if (gi == 0 && (M > 0 || x > 0)) P[c - SI] = v;
-        if (gi == d.nx - 1) P[c + SI] = v;
-        if (gj == 0 && (M > 0 || y > 0)) P[c - SJ] = v;
-        if (gj == d.ny - 1) P[c + SJ] = v;
-        if (gk == 0 && (M > 0 || z > 0)) P[c - 1] = v;
-        if (gk == d.nz - 1) P[c + 1] = v;
+// column c of the ring numbering -> (x, y) in the box
+template <typename BX, int T>
+__device__ inline void ph_column(int c, int& x, int& y) {
+    int s = 0;
+#pragma unroll
+    for (int r = 0; r < BX::H; ++r) s += c >= (T + 2 * r) * (T + 2 * r);
+    const int in = T + 2 * (s - 1), e = T + 2 * s - 1;  // inner square's side, this ring's side - 1
+    int r = c - in * in;
+    const int lo = BX::H - s, hi = BX::H + T - 1 + s;
+    const int w = (r >= e) + (r >= 2 * e) + (r >= 3 * e);
+    r -= w * e;
+    x = w == 0 ? lo : (w == 1 ? lo + r : (w == 2 ? hi : hi - r));
+    y = w == 0 ? lo + r : (w == 1 ? hi : (w == 2 ? hi - r : lo));
+    if (s == 0) {
+        x = BX::H + c / T;
+        y = BX::H + c % T;
     }
 }
 
-// half-sweeps h .. 2*NSW-1 at margins M0 + h, colours c1, 1 - c1, ...
-template <typename ST, typename BX, int M0, int h, bool ZFIRST>
-__device__ inline void lv_sweeps(float* P, const float* B, const float* FX, const float* FY, const float* FZ,
-                                 const Dims& d, int ox, int oy, int oz, int c1, float omega) {
-    if constexpr (h < 2 * (BX::H / 2)) {
-        lv_half_sweep<ST, BX, M0 + h, ZFIRST && h == 0>(P, B, FX, FY, FZ, d, ox, oy, oz, (c1 + h) & 1, omega);
+// two adjacent values as stored
+template <typename ST>
+struct RawPair {
+    ST v[2];
+    __device__ float get(bool second) const { return to_f32(second ? v[1] : v[0]); }
+};
+
+// a T at byte offset o of a uniform base (4-byte aligned; 2-byte for one
+// 16-bit value)
+template <typename T, typename B>
+__device__ inline T at_byte(const B* base, unsigned o) {
+    T v;
+    __builtin_memcpy(&v, reinterpret_cast<const char*>(base) + o, sizeof(T));
+    return v;
+}
+
+// One pair's data in registers, by colour: faces x-low, x-high, y-low,
+// y-high of each cell; the z face between the cells and each cell's other
+// one; b; the diagonal; the pair's LDS index * 2 + (x + y) & 1 (the k parity
+// of its colour-0 cell).
+struct PhSlot {
+    float f[2][4], zm, zo[2], dg[2];
+    int pk;
+};
+
+template <typename BX>
+__device__ inline void ph_addr(int pk, int col, int& own, int& hi, bool& odd) {
+    const int h = (pk ^ col) & 1, base = pk >> 1;
+    odd = h != 0;
+    own = base + h * BX::OFF;
+    hi = base + BX::OFF + h * (1 - BX::OFF);  // the cell above along k; below: one entry before
+}
+
+template <typename BX>
+__device__ inline void ph_stencil(const float* P, const PhSlot& S, int col, int own, int hi, bool odd, float pc,
+                                  float& Ap) {
+    const float f[6] = {S.f[col][0], S.f[col][1], S.f[col][2],
+                        S.f[col][3], odd ? S.zm : S.zo[col], odd ? S.zo[col] : S.zm};
+    const float pn[6] = {P[own - BX::SX], P[own + BX::SX], P[own - BX::SY],
+                         P[own + BX::SY], P[hi - 1],       P[hi]};
+    float dg;
+    stencil_vals(pc, f, pn, dg, Ap);
+}
+
+// half-sweeps h .. 2*NSW-1 at margins M0 + h, colours c1, 1 - c1, ...; ZI: the
+// first one starts from zero everywhere
+template <typename ST, typename BX, int M0, int h, bool ZI, int NS>
+__device__ inline void ph_sweeps(float* P, const float* B, PhSlot (&S)[NS], float omega) {
+    if constexpr (h < BX::H) {
+        constexpr int M = M0 + h;
+#pragma unroll
+        for (int q = 0; q < BX::slots(M); ++q) {
+            // (the addresses are formed anew in every half-sweep: held, they spill)
+            asm volatile("" : "+v"(S[q].pk));
+            if ((q + 1) * BX::NT > BX::pairs(M) && (int)threadIdx.x + q * BX::NT >= BX::pairs(M)) continue;
+            const int col = h & 1;  // slots are ordered by colour: first colour at [0]
+            int own, hi;
+            bool odd;
+            ph_addr<BX>(S[q].pk, col, own, hi, odd);
+            const float dg = S[q].dg[col];
+            if constexpr (ZI && h == 0) {
+                const float v = dg > 0.0f ? rb_first(B[own], dg, omega) : 0.0f;
+                P[own] = round_st<ST>(v);
+                P[odd ? hi - 1 : hi] = 0.0f;  // the pair's other cell
+            } else {
+                const float pc = P[own], bc = B[own];
+                float Ap;
+                ph_stencil<BX>(P, S[q], col, own, hi, odd, pc, Ap);
+                // (formed unconditionally: every read is issued at once)
+                const float v = rb_relax(pc, bc, Ap, dg, omega);
+                P[own] = round_st<ST>(dg > 0.0f ? v : pc);
+            }
+        }
         __syncthreads();
-        lv_sweeps<ST, BX, M0, h + 1, ZFIRST>(P, B, FX, FY, FZ, d, ox, oy, oz, c1, omega);
+        ph_sweeps<ST, BX, M0, h + 1, ZI, NS>(P, B, S, omega);
     }
 }
 
 // PRE: pin is unused (the level starts from zero), pout gets the smoothed
-// iterate and bc the restricted residual (k_resid_restrict's order).
-// !PRE: pout gets the post-smoothed iterate of pin + P pcoarse.
-template <typename ST, bool PRE, int TI, int TJ, int TK, int NSW, typename CT = float>
-__global__ __launch_bounds__(1024) void k_level(Dims d, Dims dc, const ST* __restrict__ bx,
+// iterate and bc the restricted residual (k_resid_restrict's order); uf: the
+// residual test rides along (level 0).  !PRE: pout gets the post-smoothed
+// iterate of pin + P pcoarse; df: with the CG's inner products (level 0).
+template <typename ST, bool PRE, int T, int TK, int NSW, typename CT = float>
+__global__ __launch_bounds__(1024) void k_phase(Dims d, Dims dc, const ST* __restrict__ bx,
                                                 const ST* __restrict__ by, const ST* __restrict__ bz,
                                                 const float* __restrict__ b, const ST* __restrict__ pin,
                                                 const CT* __restrict__ pcoarse, ST* __restrict__ pout,
                                                 float* __restrict__ bc, float omega,
-                                                const int* __restrict__ done) {
-    using BX = LvBox<TI, TJ, TK, NSW>;
-    __shared__ float P[BX::N], B[BX::N], FX[BX::N], FY[BX::N], FZ[BX::N];
+                                                const int* __restrict__ done, const float* __restrict__ bscale,
+                                                UpdateFold uf, DotFold df) {
+    using BX = PhBox<T, TK, NSW>;
+    constexpr int M0 = PRE ? 0 : 1, NS = BX::slots(M0), H = BX::H, NT = BX::NT;
+    constexpr int c1 = PRE ? 0 : 1;
+    __shared__ float P[2 * BX::OFF], B[2 * BX::OFF];
     const int tid = threadIdx.x;
-    const int ntk = (d.nz + TK - 1) / TK, ntj = (d.ny + TJ - 1) / TJ;
+    const bool fold = PRE && uf.st != nullptr;
+    int was_done = 0;
+    float fm = 0.0f;
+    if (fold) {
+        was_done = uf.st->done;
+        for (int e = tid; e < uf.nparts; e += NT) fm = fmaxf(fm, uf.st->fpart[e]);
+    }
+    const int ntk = (d.nz + TK - 1) / TK, ntj = (d.ny + T - 1) / T;
     const int tile = xcd_block(blockIdx.x, gridDim.x);
-    const int i0 = (tile / (ntk * ntj)) * TI, j0 = ((tile / ntk) % ntj) * TJ, k0 = (tile % ntk) * TK;
-    const int ox = i0 - BX::H, oy = j0 - BX::H, oz = k0 - BX::H;
+    const int i0 = (tile / (ntk * ntj)) * T, j0 = ((tile / ntk) % ntj) * T, k0 = (tile % ntk) * TK;
+    const int ox = i0 - H, oy = j0 - H, oz = k0 - H;  // even
 
-    // staging: every load of the box issued before the first wait, all from
-    // coordinates clamped into their array (no branches), the entries
-    // outside it zeroed afterwards
-    // (array indices by 32-bit 24x24-bit multiply-adds: the level's face
-    // arrays hold fewer than 2^24 entries.  Left to itself the compiler
-    // forms a*n + b as a 64-bit multiply-add whose unused upper addend half
-    // may be the register of a load in flight, and each address then waits
-    // for the previous load.)
-    auto mad24 = [](unsigned a, unsigned n, unsigned b) {
-        unsigned r;
-        asm("v_mad_u32_u24 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(n), "v"(b));
-        return r;
-    };
-    auto ix = [&](unsigned a, unsigned n1, unsigned b, unsigned n2, unsigned c) {
-        return mad24(mad24(a, n1, b), n2, c);
-    };
-    ST lf[BX::NPT][3], lp[BX::NPT];
-    CT lc[BX::NPT];
-    float lb[BX::NPT];
-    unsigned m[BX::NPT];
+    // staging of the iterate (every pair of the box, from clamped coordinates)
+    constexpr int NST = PRE ? 1 : (BX::N + NT - 1) / NT;
+    RawPair<ST> lp[NST];
+    CT lc[NST];
+    if constexpr (!PRE) {
 #pragma unroll
-    for (int q = 0; q < BX::NPT; ++q) {
-        const int e = min(tid + q * BX::NT, BX::N - 1);
-        const int z = e % BX::SJ, y = (e / BX::SJ) % (BX::BJ + 1), x = e / BX::SI;
-        const int gi = ox + x, gj = oy + y, gk = oz + z;
-        const int ci = min(max(gi, 0), d.nx - 1), cj = min(max(gj, 0), d.ny - 1), ck = min(max(gk, 0), d.nz - 1);
-        const bool ii = gi == ci, jj = gj == cj, kk = gk == ck;
-        // bit 0-2: the face of axis 0-2 exists, bit 3: the cell is in the grid
-        m[q] = (tid + q * BX::NT < BX::N)
-                   ? ((gi >= 0 && gi <= d.nx && jj && kk) | (ii && gj >= 0 && gj <= d.ny && kk) << 1 |
-                      (ii && jj && gk >= 0 && gk <= d.nz) << 2 | (ii && jj && kk) << 3)
-                   : 0u;
-        const int fi = min(max(gi, 0), d.nx), fj = min(max(gj, 0), d.ny), fk = min(max(gk, 0), d.nz);
-        lf[q][0] = bx[ix(fi, d.ny, cj, d.nz, ck)];
-        lf[q][1] = by[ix(ci, d.ny + 1, fj, d.nz, ck)];
-        lf[q][2] = bz[ix(ci, d.ny, cj, d.nz + 1, fk)];
-        const unsigned cc = ix(ci, d.ny, cj, d.nz, ck);
-        lb[q] = b[cc];
-        if constexpr (!PRE) {
-            lp[q] = pin[cc];
-            lc[q] = pcoarse[ix(ci >> 1, dc.ny, cj >> 1, dc.nz, ck >> 1)];
+        for (int q = 0; q < NST; ++q) {
+            const int e = min(tid + q * NT, BX::N - 1);
+            const int m = e % BX::BM, y = (e / BX::BM) % BX::B, x = e / BX::SX;
+            const int gi = min(max(ox + x, 0), d.nx - 1), gj = min(max(oy + y, 0), d.ny - 1),
+                      gk = min(max(oz + 2 * m, 0), d.nz - 2);
+            lp[q] = at_byte<RawPair<ST>>(pin, (unsigned)cell_index(d, gi, gj, gk) * sizeof(ST));
+            lc[q] = at_byte<CT>(pcoarse, (unsigned)cell_index(dc, gi >> 1, gj >> 1, gk >> 1) * sizeof(CT));
         }
     }
-    const bool skip = done && *done;
-#pragma unroll
-    for (int q = 0; q < BX::NPT; ++q) {
-        const int e = tid + q * BX::NT;
-        if (e < BX::N) {
-            const unsigned mq = m[q];
-            FX[e] = (mq & 1u) ? to_f32(lf[q][0]) : 0.0f;
-            FY[e] = (mq & 2u) ? to_f32(lf[q][1]) : 0.0f;
-            FZ[e] = (mq & 4u) ? to_f32(lf[q][2]) : 0.0f;
-            B[e] = (mq & 8u) ? lb[q] : 0.0f;
-            // (every entry from clamped coordinates: the ghosts hold their
-            // cell's value)
-            P[e] = PRE ? 0.0f : round_st<ST>(to_f32(lp[q]) + to_f32(lc[q]));
-        }
+    // the box's columns: their first cell's index, what leads from a cell to
+    // its y and z faces, and the column's LDS index * 2 + the k parity of the
+    // first colour's cells, with the walls in bits 20-23 (low x, high x, low
+    // y, high y) and bit 26: outside the grid
+    constexpr int NC = BX::pairs(M0) / BX::BM;
+    __shared__ uint4 col[NC];
+    static_assert(2 * BX::N < 1 << 20 && NC <= NT, "column word");
+    if (tid < NC) {
+        int x, y;
+        ph_column<BX, T>(tid, x, y);
+        const int i = min(max(ox + x, 0), d.nx - 1), j = min(max(oy + y, 0), d.ny - 1);
+        const unsigned walls = (i == 0) | (i == d.nx - 1) << 1 | (j == 0) << 2 | (j == d.ny - 1) << 3 |
+                               (unsigned)(i != ox + x || j != oy + y) << 6;
+        col[tid] = make_uint4((i * d.ny + j) * d.nz, i * d.nz, i * d.ny + j,
+                              (2 * (x * BX::SX + y * BX::SY) + ((x + y + c1) & 1)) | walls << 20);
     }
     __syncthreads();
-    if (skip) return;  // a finished solve's queued iteration: no sweeps (uniform)
+    // the slots: every load from clamped coordinates (byte offsets of 32 bits
+    // from uniform bases), all issued before the first use
+    PhSlot S[NS];
+    RawPair<ST> rx[NS][2], ry[NS][2];
+    ST rz[NS][3];
+    float2 rb[NS];
+    unsigned wall[NS];
+    float2 ap = make_float2(0.0f, 0.0f);
+#pragma unroll
+    for (int q = 0; q < NS; ++q) {
+        const int t = min(tid + q * NT, BX::pairs(M0) - 1);
+        const int c = t / BX::BM, m = t - c * BX::BM;
+        const uint4 cl = col[c];
+        const int kb = oz + 2 * m, k = min(max(kb, 0), d.nz - 2);
+        const unsigned cell = cl.x + k, fy = cell + cl.y, fz = cell + cl.z;
+        rx[q][0] = at_byte<RawPair<ST>>(bx, cell * sizeof(ST));
+        rx[q][1] = at_byte<RawPair<ST>>(bx, (cell + d.ny * d.nz) * sizeof(ST));
+        ry[q][0] = at_byte<RawPair<ST>>(by, fy * sizeof(ST));
+        ry[q][1] = at_byte<RawPair<ST>>(by, (fy + d.nz) * sizeof(ST));
+#pragma unroll
+        for (int e = 0; e < 3; ++e) rz[q][e] = at_byte<ST>(bz, (fz + e) * sizeof(ST));
+        rb[q] = at_byte<float2>(b, cell * 4u);
+        if (!PRE && q == 0 && df.Ap) ap = at_byte<float2>(df.Ap, cell * 4u);
+        S[q].pk = (int)(cl.w & 0xFFFFFu) + 2 * m;
+        wall[q] = (cl.w >> 20) | (k == 0) << 4 | (k == d.nz - 2) << 5 | (k != kb) << 6;
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (!PRE) {
+#pragma unroll
+        for (int q = 0; q < NST; ++q) {
+            const int e = tid + q * NT;
+            if (e < BX::N) {
+                P[e] = round_st<ST>(lp[q].get(false) + to_f32(lc[q]));
+                P[e + BX::OFF] = round_st<ST>(lp[q].get(true) + to_f32(lc[q]));
+            }
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int q = 0; q < NS; ++q) {
+        const int par = S[q].pk & 1;
+        const unsigned wl = wall[q];
+        const float z[3] = {to_f32(rz[q][0]), to_f32(rz[q][1]), to_f32(rz[q][2])};
+#pragma unroll
+        for (int col = 0; col < 2; ++col) {
+            const bool odd = (par ^ col) != 0;
+            const float fc[6] = {rx[q][0].get(odd), rx[q][1].get(odd), ry[q][0].get(odd),
+                                 ry[q][1].get(odd), odd ? z[1] : z[0], odd ? z[2] : z[1]};
+            const float dg = fc[0] + fc[1] + fc[2] + fc[3] + fc[4] + fc[5];
+            S[q].dg[col] = dg;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) S[q].f[col][e] = fc[e];
+            S[q].zo[col] = odd ? z[2] : z[0];
+        }
+        // bits 0-5: the pair has a wall on the low / high side of an axis;
+        // 6: it lies outside the grid
+        if (__any(wl)) {
+#pragma unroll
+            for (int col = 0; col < 2; ++col) {
+                const bool odd = (par ^ col) != 0;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) S[q].f[col][e] = (wl >> e & 1u) ? 0.0f : S[q].f[col][e];
+                S[q].zo[col] = (wl & (odd ? 32u : 16u)) ? 0.0f : S[q].zo[col];
+                S[q].dg[col] = (wl & 64u) ? 0.0f : S[q].dg[col];
+            }
+        }
+        S[q].zm = z[1];
+        // (b: written and read by this thread alone, unscaled until bs is known)
+        if (tid + q * NT < BX::pairs(M0)) {
+            B[S[q].pk >> 1] = rb[q].x;
+            B[(S[q].pk >> 1) + BX::OFF] = rb[q].y;
+        }
+#pragma unroll
+        for (int col = 0; col < 2; ++col)  // formed here and now, not at every use
+            asm volatile("" : "+v"(S[q].f[col][0]), "+v"(S[q].f[col][1]), "+v"(S[q].f[col][2]), "+v"(S[q].f[col][3]),
+                              "+v"(S[q].zo[col]), "+v"(S[q].dg[col]));
+    }
+    bool skip = !fold && done && *done;
+    __shared__ float s_fm[NT / 64];
+    if (fold) {
+        fm = wave_max(fm);
+        if ((tid & 63) == 0) s_fm[tid >> 6] = fm;
+        __syncthreads();
+    }
+    float bs = 1.0f;
+    if (fold) {
+        float mm = s_fm[0];
+#pragma unroll
+        for (int w = 1; w < NT / 64; ++w) mm = fmaxf(mm, s_fm[w]);
+        const bool conv = (double)mm / uf.st->b_norm < uf.st->tol;
+        skip = was_done || conv;
+        bs = ldexpf(1.0f, -vscale_exponent(mm));
+        if (blockIdx.x == 0 && tid == 0) residual_test_record(uf.st, mm, uf.host_flag);
+    } else if (bscale) {
+        bs = *bscale;
+    }
+    if (skip) return;  // a finished solve's queued iteration (uniform)
+    if (bscale) {
+#pragma unroll
+        for (int q = 0; q < NS; ++q) {
+            if (tid + q * NT < BX::pairs(M0)) {
+                B[S[q].pk >> 1] *= bs;
+                B[(S[q].pk >> 1) + BX::OFF] *= bs;
+            }
+        }
+    }
+    if (!PRE) __syncthreads();
     // PRE: the first half-sweep from zero runs on the whole box (it reads no
     // neighbour), the last at margin H - 1; !PRE: margins 1 .. H
-    lv_sweeps<ST, BX, PRE ? 0 : 1, 0, PRE>(P, B, FX, FY, FZ, d, ox, oy, oz, PRE ? 0 : 1, omega);
+    ph_sweeps<ST, BX, M0, 0, PRE, NS>(P, B, S, omega);
 
-    // the tile goes out; PRE: each cell's residual (k_resid_restrict's
-    // stencil with bscale 1) into LDS, then the sums of 2x2x2 children
-    constexpr int TC = TI * TJ * TK;
-    __shared__ float Rs[PRE ? TC : 1];
-    for (int e = tid; e < TC; e += BX::NT) {
-        const int kl = e % TK, jl = (e / TK) % TJ, il = e / (TK * TJ);
-        const int gi = i0 + il, gj = j0 + jl, gk = k0 + kl;
-        if (gi >= d.nx || gj >= d.ny || gk >= d.nz) continue;
-        const int c = (il + BX::H) * BX::SI + (jl + BX::H) * BX::SJ + (kl + BX::H);
-        const float pc = P[c];
-        if (!skip) pout[cell_index(d, gi, gj, gk)] = from_f32<ST>(pc);
+    // the tile goes out: its pairs are all in slot 0
+    static_assert(T * T * BX::BM <= NT, "the tile's columns fit slot 0");
+    const int col0 = tid / BX::BM, m = tid - col0 * BX::BM;
+    const int il = col0 / T, jl = col0 % T, kl = 2 * m - H;
+    const bool mine = tid < T * T * BX::BM && kl >= 0 && kl < TK && i0 + il < d.nx && j0 + jl < d.ny && k0 + kl < d.nz;
+    __shared__ float Rs[PRE ? T * T * TK : 1];
+    double dsum[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+    if (mine) {
+        const int base = S[0].pk >> 1;
+        const float p0 = P[base], p1 = P[base + BX::OFF];
+        st_pair(pout, cell_index(d, i0 + il, j0 + jl, k0 + kl), p0, p1);
         if constexpr (PRE) {
-            const float fc[6] = {FX[c], FX[c + BX::SI], FY[c], FY[c + BX::SJ], FZ[c], FZ[c + 1]};
-            const float pn[6] = {P[c - BX::SI], P[c + BX::SI], P[c - BX::SJ], P[c + BX::SJ], P[c - 1], P[c + 1]};
-            float dg, Ap;
-            stencil_vals(pc, fc, pn, dg, Ap);
-            Rs[e] = B[c] - Ap;
+#pragma unroll
+            for (int col = 0; col < 2; ++col) {
+                int own, hi;
+                bool odd;
+                ph_addr<BX>(S[0].pk, col, own, hi, odd);
+                float Ap;
+                ph_stencil<BX>(P, S[0], col, own, hi, odd, odd ? p1 : p0, Ap);
+                Rs[(il * T + jl) * TK + kl + (odd ? 1 : 0)] = B[own] - Ap;
+            }
+        } else if (df.Ap) {
+            // k_cg_beta's sums: z as stored times zscale, r = b unscaled, Ap
+            const float zsc = df.zscale ? *df.zscale : 1.0f;
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                const double zz = (double)((e ? p1 : p0) * zsc);
+                const double rr = (double)(B[base + e * BX::OFF] * zsc);
+                const double aa = (double)(e ? ap.y : ap.x);
+                dsum[0] += zz;
+                dsum[1] += rr;
+                dsum[2] += aa;
+                dsum[3] += rr * zz;
+                dsum[4] += aa * zz;
+            }
         }
     }
     if constexpr (PRE) {
         __syncthreads();
-        constexpr int CJ = TJ / 2, CK = TK / 2;
-        for (int e = tid; e < TC / 8; e += BX::NT) {
+        constexpr int CJ = T / 2, CK = TK / 2;
+        for (int e = tid; e < T * T * TK / 8; e += NT) {
             const int K = e % CK, J = (e / CK) % CJ, I = e / (CK * CJ);
             const int gI = i0 / 2 + I, gJ = j0 / 2 + J, gK = k0 / 2 + K;
             if (gI >= dc.nx || gJ >= dc.ny || gK >= dc.nz) continue;
@@ -1033,8 +1196,16 @@ __global__ __launch_bounds__(1024) void k_level(Dims d, Dims dc, const ST* __res
 #pragma unroll
                 for (int bb = 0; bb < 2; ++bb)
 #pragma unroll
-                    for (int c = 0; c < 2; ++c) acc += Rs[((2 * I + a) * TJ + 2 * J + bb) * TK + 2 * K + c];
-            if (!skip) bc[cell_index(dc, gI, gJ, gK)] = acc;
+                    for (int c = 0; c < 2; ++c) acc += Rs[((2 * I + a) * T + 2 * J + bb) * TK + 2 * K + c];
+            bc[cell_index(dc, gI, gJ, gK)] = acc;
+        }
+    } else if (df.Ap) {
+        __shared__ double s_dot[5 * 16];
+        block_sum<5>(dsum, s_dot);
+        if (tid == 0) {
+#pragma unroll
+            for (int q = 0; q < 5; ++q) df.st->part[q * MAXB + blockIdx.x] = dsum[q];
+            if (blockIdx.x == 0) df.st->beta_parts = 1;  // read by the next k_cg_apply
         }
     }
 }
@@ -2083,40 +2254,61 @@ static int launch_full_sweep(const Dims& d, const ST* fx, const ST* fy, const ST
     return PF_OK;
 }
 
-// Largest level whose pre and post phases run as one k_level launch each
-// (32^3: 256 tiles of 4 x 4 x 8 cells, one workgroup per CU).
-constexpr int64_t kLevelFusedMaxCells = 32768;
+// Levels whose pre and post phases run as one k_phase launch each: those of
+// at most one workgroup per CU, with 4 x 4 x 8 tiles (up to 32^3), else with
+// 8 x 8 x 16 ones (up to 64^3).  A second round of workgroups costs more than
+// the per-sweep launches: a V-cycle of 80^3 (500 tiles) took 121 us with its
+// level 0 in phases, 111 without; 64^3 (256 tiles) 82 and 90.
+constexpr unsigned kPhaseTiles = 256;
 
-// One k_level launch: PRE (the pre-smoothing phase from zero and the
-// restricted residual into bc) or the post phase (pin plus the
-// prolongation of pcoarse, dims dc, into pout); nsw sweeps, 1..3.
-template <typename ST, bool PRE, typename CT = float>
-static int launch_level(const Dims& d, const Dims& dc, int nsw, const ST* fx, const ST* fy, const ST* fz,
-                        const float* b, const ST* pin, const CT* pcoarse, ST* pout, float* bc, float omega,
-                        const int* done, hipStream_t s) {
-    constexpr int TI = 4, TJ = 4, TK = 8;
-    PF_REQUIRE(d.nx == 2 * dc.nx && d.ny == 2 * dc.ny && d.nz == 2 * dc.nz, "launch_level: fine dims must be 2x coarse");
-    // the kernel forms indices with 24-bit multiplies
-    PF_REQUIRE((int64_t)(d.nx + 1) * (d.ny + 1) * (d.nz + 1) < ((int64_t)1 << 24), "launch_level: level too large");
-    const unsigned grid = cdiv(d.nx, TI) * cdiv(d.ny, TJ) * cdiv(d.nz, TK);
+static unsigned phase_tiles(const Dims& d, int t) {
+    return (unsigned)(cdiv(d.nx, t) * cdiv(d.ny, t) * cdiv(d.nz, 2 * t));
+}
+// tile edge of a level's k_phase launches, 0: too large for them
+static int phase_tile(const Dims& d) {
+    for (int t = 4; t <= 8; t *= 2)
+        if (phase_tiles(d, t) <= kPhaseTiles) return t;
+    return 0;
+}
+
+template <typename ST, bool PRE, int T, typename CT>
+static int launch_phase_tile(const Dims& d, const Dims& dc, int nsw, const ST* fx, const ST* fy, const ST* fz,
+                             const float* b, const ST* pin, const CT* pcoarse, ST* pout, float* bc, float omega,
+                             const int* done, const float* bscale, UpdateFold uf, DotFold df, hipStream_t s) {
+    const unsigned grid = phase_tiles(d, T);
     switch (nsw) {
     case 1:
-        k_level<ST, PRE, TI, TJ, TK, 1, CT><<<grid, 1024, 0, s>>>(d, dc, fx, fy, fz, b, pin, pcoarse, pout, bc,
-                                                                  omega, done);
+        k_phase<ST, PRE, T, 2 * T, 1, CT><<<grid, 1024, 0, s>>>(d, dc, fx, fy, fz, b, pin, pcoarse, pout, bc, omega,
+                                                               done, bscale, uf, df);
         break;
     case 2:
-        k_level<ST, PRE, TI, TJ, TK, 2, CT><<<grid, 1024, 0, s>>>(d, dc, fx, fy, fz, b, pin, pcoarse, pout, bc,
-                                                                  omega, done);
+        k_phase<ST, PRE, T, 2 * T, 2, CT><<<grid, 1024, 0, s>>>(d, dc, fx, fy, fz, b, pin, pcoarse, pout, bc, omega,
+                                                               done, bscale, uf, df);
         break;
     case 3:
-        k_level<ST, PRE, TI, TJ, TK, 3, CT><<<grid, 1024, 0, s>>>(d, dc, fx, fy, fz, b, pin, pcoarse, pout, bc,
-                                                                  omega, done);
+        k_phase<ST, PRE, T, 2 * T, 3, CT><<<grid, 1024, 0, s>>>(d, dc, fx, fy, fz, b, pin, pcoarse, pout, bc, omega,
+                                                               done, bscale, uf, df);
         break;
     default:
-        PF_REQUIRE(false, "launch_level: 1 to 3 sweeps");
+        PF_REQUIRE(false, "launch_phase: 1 to 3 sweeps");
     }
     PF_CHECK_LAUNCH();
     return PF_OK;
+}
+
+// One k_phase launch: PRE (the pre-smoothing phase from zero and the
+// restricted residual into bc) or the post phase (pin plus the prolongation
+// of pcoarse, dims dc, into pout); nsw sweeps, 1..3.
+template <typename ST, bool PRE, typename CT = float>
+static int launch_phase(const Dims& d, const Dims& dc, int nsw, const ST* fx, const ST* fy, const ST* fz,
+                        const float* b, const ST* pin, const CT* pcoarse, ST* pout, float* bc, float omega,
+                        const int* done, const float* bscale, UpdateFold uf, DotFold df, hipStream_t s) {
+    PF_REQUIRE(d.nx == 2 * dc.nx && d.ny == 2 * dc.ny && d.nz == 2 * dc.nz, "launch_phase: fine dims must be 2x coarse");
+    return phase_tile(d) == 4
+               ? launch_phase_tile<ST, PRE, 4, CT>(d, dc, nsw, fx, fy, fz, b, pin, pcoarse, pout, bc, omega, done,
+                                                   bscale, uf, df, s)
+               : launch_phase_tile<ST, PRE, 8, CT>(d, dc, nsw, fx, fy, fz, b, pin, pcoarse, pout, bc, omega, done,
+                                                   bscale, uf, df, s);
 }
 
 // workgroups of launch_full_sweep on a level of dims d (one per tile)
@@ -2139,12 +2331,12 @@ static bool fused_smoother(const pf_mg& mg, int l) {
     return !(mg.options & PF_MG_UNFUSED_SMOOTHER) && (mg.lev[l].nz % 2) == 0;
 }
 
-// level l (restricted to l + 1, below level 0) runs each smoothing phase
-// as one k_level launch
-static bool level_fused(const pf_mg& mg, int l, int G) {
-    return l >= 1 && l < G && !(mg.options & (PF_MG_UNFUSED_SMOOTHER | PF_MG_SPLIT_LEVELS)) &&
-           ncell(mg.lev[l]) <= kLevelFusedMaxCells && mg.pre >= 1 && mg.pre <= 3 && mg.post >= 1 &&
-           mg.post <= 3;
+// level l (restricted to l + 1) runs each smoothing phase as one k_phase
+// launch
+static bool level_fused(const pf_mg& mg, int l) {
+    const int G = mg.small_from < mg.nlev ? mg.small_from : mg.nlev - 1;
+    return l < G && !(mg.options & PF_MG_SPLIT_LEVELS) && fused_smoother(mg, l) && phase_tile(ldims(mg.lev[l])) &&
+           mg.pre >= 1 && mg.pre <= 3 && mg.post >= 1 && mg.post <= 3;
 }
 
 // One V-cycle: z0 = M^{-1} r0 (no mean removal at level 0).
@@ -2214,12 +2406,15 @@ static int vcycle(const pf_mg& mg, const float* r0, ST* z0, const int* done, con
     for (int l = 0; l < G; ++l) {
         const pf_mg_level& lv = mg.lev[l];
         const pf_mg_level& cv = mg.lev[l + 1];
-        if (level_fused(mg, l, G)) {
-            cur[l] = P(l);
-            const int rc = launch_level<ST, true>(ldims(lv), ldims(cv), mg.pre, Lv<ST>::fx(lv), Lv<ST>::fy(lv),
+        if (level_fused(mg, l)) {
+            // (level 0: the post phase then lands in z0)
+            cur[l] = l == 0 ? second_buffer<ST>(mg, 0) : P(l);
+            const int rc = launch_phase<ST, true>(ldims(lv), ldims(cv), mg.pre, Lv<ST>::fx(lv), Lv<ST>::fy(lv),
                                                   Lv<ST>::fz(lv), B(l), static_cast<const ST*>(nullptr),
                                                   static_cast<const float*>(nullptr), cur[l], mg.lev[l + 1].b,
-                                                  mg.omega, done, s);
+                                                  mg.omega, done, l == 0 ? bscale : nullptr,
+                                                  uf && l == 0 ? *uf : UpdateFold{nullptr, 0, nullptr},
+                                                  DotFold{nullptr, nullptr, nullptr}, s);
             if (rc) return rc;
             continue;
         }
@@ -2311,16 +2506,21 @@ static int vcycle(const pf_mg& mg, const float* r0, ST* z0, const int* done, con
     for (int l = G - 1; l >= 0; --l) {
         const pf_mg_level& lv = mg.lev[l];
         const pf_mg_level& cv = mg.lev[l + 1];
-        if (level_fused(mg, l, G)) {
+        if (level_fused(mg, l)) {
             ST* out = other(l, cur[l]);
+            const float* bsc = l == 0 ? bscale : nullptr;
+            const UpdateFold nf{nullptr, 0, nullptr};
+            const bool dots = dfold && l == 0;
+            const DotFold df = dots ? *dfold : DotFold{nullptr, nullptr, nullptr};
             const int rc =
                 (l + 1 == sm)
-                    ? launch_level<ST, false, float>(ldims(lv), ldims(cv), mg.post, Lv<ST>::fx(lv), Lv<ST>::fy(lv),
+                    ? launch_phase<ST, false, float>(ldims(lv), ldims(cv), mg.post, Lv<ST>::fx(lv), Lv<ST>::fy(lv),
                                                      Lv<ST>::fz(lv), B(l), cur[l], cv.p, out, nullptr, mg.omega,
-                                                     done, s)
-                    : launch_level<ST, false, ST>(ldims(lv), ldims(cv), mg.post, Lv<ST>::fx(lv), Lv<ST>::fy(lv),
+                                                     done, bsc, nf, df, s)
+                    : launch_phase<ST, false, ST>(ldims(lv), ldims(cv), mg.post, Lv<ST>::fx(lv), Lv<ST>::fy(lv),
                                                   Lv<ST>::fz(lv), B(l), cur[l], cur[l + 1], out, nullptr,
-                                                  mg.omega, done, s);
+                                                  mg.omega, done, bsc, nf, df, s);
+            if (dots && dot_done) *dot_done = true;
             if (rc) return rc;
             cur[l] = out;
             continue;
@@ -2399,17 +2599,21 @@ static const float* vcycle_scale(const CGK<ST>& a) {
 // Every kernel returns at once when the flag is set, so an iteration
 // enqueued past convergence does nothing.
 // The residual test rides in the V-cycle's first kernel when that is the
-// fused zero-start sweep of an HBM level 0.
+// fused zero-start sweep or pre phase of an HBM level 0.
 static bool fold_residual_test(const pf_mg& mg) {
     return mg.small_from > 0 && mg.pre > 0 && fused_smoother(mg, 0);
 }
 
-// The inner products after the V-cycle ride on its last level-0 sweep when
-// that is a plain fused sweep (at least two post-sweeps on an HBM level 0)
-// whose workgroups fit the partials array.
+// The inner products after the V-cycle ride on its last level-0 kernel when
+// that is the post phase or a plain fused sweep (at least two post-sweeps on
+// an HBM level 0) whose workgroups fit the partials array.
+static int64_t dot_blocks(const pf_mg& mg) {
+    const Dims d = ldims(mg.lev[0]);
+    return level_fused(mg, 0) ? (int64_t)phase_tiles(d, phase_tile(d)) : full_sweep_blocks(d);
+}
 static bool fold_dots(const pf_mg& mg) {
-    return !(mg.options & PF_MG_SEPARATE_DOTS) && mg.small_from > 0 && mg.post >= 2 && fused_smoother(mg, 0) &&
-           full_sweep_blocks(ldims(mg.lev[0])) <= MAXB;
+    return !(mg.options & PF_MG_SEPARATE_DOTS) && mg.small_from > 0 && (mg.post >= 2 || level_fused(mg, 0)) &&
+           fused_smoother(mg, 0) && dot_blocks(mg) <= MAXB;
 }
 
 template <typename ST>
@@ -2692,7 +2896,7 @@ static int solve_impl(const pf_mg& mg, const float* b, float* x, double tol, int
     const unsigned nb = red_blocks(n);
     a.slot = 1;
     a.np_apply = a.np_beta = (int)std::min<int64_t>(WB, (n + WT - 1) / WT);
-    if (fold_dots(mg)) a.np_beta = (int)full_sweep_blocks(d);  // one partial per level-0 tile
+    if (fold_dots(mg)) a.np_beta = (int)dot_blocks(mg);  // one partial per level-0 tile
     const int* done = &st->done;
 
     k_part_sum<float><<<nb, RT, 0, s>>>(b, n, st->part);

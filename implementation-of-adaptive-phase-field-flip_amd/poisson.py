@@ -22,10 +22,10 @@ Differences from the reference that do not change the algorithm:
   buffer and writes it to a second one (``levels[l].r``, and ``levels[0].p``
   in FP32); ``fused_smoother=False`` runs the two half-sweeps in place, with
   the same result bit for bit;
-* on the small levels below level 0 (up to 32^3 cells) the pre-sweeps with
-  the restriction, and the prolongation with the post-sweeps, are one kernel
-  each over LDS-resident tiles with redundant halos; ``split_levels=True``
-  runs them one kernel per sweep (the same result bit for bit);
+* on the levels of up to about 64^3 cells the pre-sweeps with the
+  restriction, and the prolongation with the post-sweeps, are one kernel
+  each over tiles with redundant halos; ``split_levels=True`` runs them one
+  kernel per sweep (the same result bit for bit);
 * the CG's inner products after the preconditioner (sum z, sum r, sum Ap,
   <r, z>, <Ap, z>) are formed by the V-cycle's last level-0 sweep from the
   values it holds, one FP64 partial per tile; ``fold_dots=False`` forms
