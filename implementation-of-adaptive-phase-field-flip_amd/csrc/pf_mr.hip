@@ -149,6 +149,29 @@ __device__ inline long long fixed(float v, float scale) {
     return __double_as_longlong(d) - 0x4338000000000000LL;
 }
 
+// Distance of a cell centre (axis index i of a block with low corner o) from
+// a particle, squared distances and eq. (6) weights, written without
+// contraction: the compiler would otherwise fuse different products in
+// different kernels, and the P2G kernels are to agree bit for bit.
+__device__ inline float centre_dist(float o, int i, float h, float x) {
+#pragma clang fp contract(off)
+    return o + ((float)i + 0.5f) * h - x;
+}
+__device__ inline float square(float d) {
+#pragma clang fp contract(off)
+    return d * d;
+}
+__device__ inline float eq6_weight(float x2, float y2, float z2, float inv_r2) {
+#pragma clang fp contract(off)
+    const float t = fmaxf(1.0f - (x2 + y2 + z2) * inv_r2, 0.0f);
+    return t * t * t;
+}
+
+// The blocks an axis of a particle's support touches, clamped to the grid.
+__device__ inline int2 touched_blocks(float x, float r, float bext, int nb) {
+    return make_int2(max((int)floorf((x - r) / bext), 0), min((int)floorf((x + r) / bext), nb - 1));
+}
+
 template <class Add>
 __device__ inline void splat_particle(const MGrid& g, const float* __restrict__ x, const float* __restrict__ v,
                                       const int* __restrict__ type, const int* __restrict__ lev, int64_t p,
@@ -160,12 +183,11 @@ __device__ inline void splat_particle(const MGrid& g, const float* __restrict__ 
     const float rp = c.r0 * (float)(1 << lp);
     const float r2 = rp * rp, inv_r2 = 1.0f / r2;
     const float bext = (float)g.n0 * g.h0;
-    const int bi0 = max((int)floorf((px - rp) / bext), 0), bi1 = min((int)floorf((px + rp) / bext), g.nbx - 1);
-    const int bj0 = max((int)floorf((py - rp) / bext), 0), bj1 = min((int)floorf((py + rp) / bext), g.nby - 1);
-    const int bk0 = max((int)floorf((pz - rp) / bext), 0), bk1 = min((int)floorf((pz + rp) / bext), g.nbz - 1);
-    for (int bi = bi0; bi <= bi1; ++bi)
-        for (int bj = bj0; bj <= bj1; ++bj)
-            for (int bk = bk0; bk <= bk1; ++bk) {
+    const int2 bi_ = touched_blocks(px, rp, bext, g.nbx), bj_ = touched_blocks(py, rp, bext, g.nby),
+               bk_ = touched_blocks(pz, rp, bext, g.nbz);
+    for (int bi = bi_.x; bi <= bi_.y; ++bi)
+        for (int bj = bj_.x; bj <= bj_.y; ++bj)
+            for (int bk = bk_.x; bk <= bk_.y; ++bk) {
                 const int s = g.slot[(bi * g.nby + bj) * g.nbz + bk];
                 if (s < 0) continue;
                 const int l = g.blev[s];
@@ -186,24 +208,24 @@ __device__ inline void splat_particle(const MGrid& g, const float* __restrict__ 
                 const int k1 = min((int)floorf((pz + rp - oz) / h), nn - 1);
                 const int base = g.coff[s];
                 for (int i = i0; i <= i1; ++i) {
-                    const float dxc = ox + ((float)i + 0.5f) * h - px, dxf = dxc - half;
-                    const float xc2 = dxc * dxc, xf2 = dxf * dxf;
+                    const float dxc = centre_dist(ox, i, h, px), dxf = dxc - half;
+                    const float xc2 = square(dxc), xf2 = square(dxf);
                     if (fminf(xc2, xf2) >= r2) continue;
                     for (int j = j0; j <= j1; ++j) {
-                        const float dyc = oy + ((float)j + 0.5f) * h - py, dyf = dyc - half;
-                        const float yc2 = dyc * dyc, yf2 = dyf * dyf;
+                        const float dyc = centre_dist(oy, j, h, py), dyf = dyc - half;
+                        const float yc2 = square(dyc), yf2 = square(dyf);
                         if (fminf(xc2, xf2) + fminf(yc2, yf2) >= r2) continue;
                         for (int k = k0; k <= k1; ++k) {
-                            const float dzc = oz + ((float)k + 0.5f) * h - pz, dzf = dzc - half;
-                            const float zc2 = dzc * dzc, zf2 = dzf * dzf;
+                            const float dzc = centre_dist(oz, k, h, pz), dzf = dzc - half;
+                            const float zc2 = square(dzc), zf2 = square(dzf);
                             const int addr = base + (i * nn + j) * nn + k;
-                            const float d2[4] = {xc2 + yc2 + zc2, xf2 + yc2 + zc2, xc2 + yf2 + zc2, xc2 + yc2 + zf2};
+                            const float wt[4] = {eq6_weight(xc2, yc2, zc2, inv_r2), eq6_weight(xf2, yc2, zc2, inv_r2),
+                                                 eq6_weight(xc2, yf2, zc2, inv_r2), eq6_weight(xc2, yc2, zf2, inv_r2)};
                             long long val[kAcc];
                             unsigned mask = 0u;
 #pragma unroll
                             for (int q = 0; q < 4; ++q) {
-                                const float t = fmaxf(1.0f - d2[q] * inv_r2, 0.0f);
-                                const float w = t * t * t;
+                                const float w = wt[q];
                                 if (!(w > 0.0f)) continue;
                                 const float wm = w * mp;
                                 if (q == 0) {
@@ -254,66 +276,324 @@ __global__ __launch_bounds__(256) void k_mr_cell_key(MGrid g, const float* __res
 
 __global__ __launch_bounds__(256) void k_mr_cell_scatter(const int* __restrict__ key, const int* __restrict__ rank,
                                                          const int* __restrict__ start, int64_t n,
-                                                         int* __restrict__ perm) {
+                                                         int* __restrict__ perm, int* __restrict__ nlist) {
     const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (p == 0) *nlist = 0;  // the particles k_mr_p2g_tile leaves to the cached walk
     if (p >= n) return;
     perm[start[key[p]] + rank[p]] = (int)p;
 }
 
-// P2G over the cell-sorted order.  A workgroup's particles are neighbours,
-// so their contributions land on a few hundred cells: each workgroup keeps
-// a hash of kP2GSlots cells in LDS (tag + the 8 fixed-point channels), adds
-// there with LDS atomics, and flushes every cached cell with one global
-// atomic per non-zero channel at the end.  A contribution whose slot holds
-// another cell goes to global memory directly.  Integer sums, so the result
-// equals the uncached kernel's bit for bit.
-// 512 slots (34 KB of LDS) let four workgroups share a CU; 1024 slots with
-// 512 particles per workgroup ran 6 % slower at two workgroups per CU
-constexpr int kP2GSlots = 512;
-constexpr int kP2GPerBlock = 256;  // particles per workgroup (1 per thread)
-static_assert(kP2GSlots == 1 << 9, "the slot hash keeps 9 bits");
+// P2G by tiles of 8^3 cells of a block (a coarser block's whole cell range if
+// it has fewer).  A workgroup adds its cells' particles into LDS, at plain
+// tile coordinates: the tile plus R cells on every side, 8 fixed-point
+// channels, then one global atomic per non-zero entry.  This is the uniform
+// splat where it applies: R = 1 takes the particles of the block's own level
+// (2 candidates per axis and stagger), R = 2 those one level coarser (5 cells
+// per axis), which fill a ring of blocks that a neighbouring finer level has
+// refined; in both every block the support touches must have this block's
+// level.  What remains (about 0.5 % of the particles of a settled dam break,
+// along the 2:1 jumps, and those outside the grid) is left to k_mr_p2g_list.  The sums are those of
+// the per-particle walk bit for bit: the same cells, weights and fixed-point
+// roundings, and integer adds.
+// A hash of cells in LDS for every particle (what k_mr_p2g_list does) was
+// bound by its lookups, one per touched cell.
+// 128^3 grid, 9.2M particles (6 % one level coarser than their block):
+// 4.95 -> 1.15 ms (0.47 own level, 0.33 one coarser, 0.35 the walk).
+template <int R>
+struct P2GTile {
+    static constexpr int E = 8 + 2 * R, E3 = E * E * E;
+    static constexpr int NT = R == 1 ? 512 : 1024;
+};
 
-__global__ __launch_bounds__(256) void k_mr_p2g_cached(MGrid g, const float* __restrict__ x,
-                                                       const float* __restrict__ v, const int* __restrict__ type,
-                                                       const int* __restrict__ lev, const int* __restrict__ perm,
-                                                       int64_t n, MRConst c, unsigned long long* __restrict__ acc) {
-    __shared__ int tag[kP2GSlots];
-    __shared__ unsigned long long lacc[kP2GSlots * kAcc];
-    for (int s = threadIdx.x; s < kP2GSlots; s += blockDim.x) tag[s] = -1;
-    for (int s = threadIdx.x; s < kP2GSlots * kAcc; s += blockDim.x) lacc[s] = 0ull;
-    __syncthreads();
-    const int64_t nc = g.ncells;
-    const int64_t p0 = (int64_t)blockIdx.x * kP2GPerBlock;
-    for (int q = threadIdx.x; q < kP2GPerBlock; q += blockDim.x) {
-        if (p0 + q >= n) break;
-        const int64_t p = perm[p0 + q];
-        splat_particle(g, x, v, type, lev, p, c, [&](int addr, const long long* val, unsigned mask) {
-            const int s = (int)(((unsigned)addr * 2654435761u) >> 23);  // 9-bit multiplicative hash
-            int t = tag[s];
-            if (t != addr && t == -1) {
-                t = atomicCAS(tag + s, -1, addr);
-                if (t == -1) t = addr;
-            }
-            if (t == addr) {
+// The block of a tile and the tile in it.
+struct TileRef {
+    int level, nn, base;   // cells per axis of the block, first cell address
+    int b[3], t0[3], tn;   // block coordinates, first local cell, cells per axis
+    float h, bext;
+};
+
+// How a particle whose centre lies in the tile is splatted: 0, 1: by the
+// R = 1, 2 tile kernel, 2: by the walk.  ok: which of the 27 blocks around
+// exist at the tile's level.
+__device__ inline int p2g_class(const MGrid& g, const TileRef& t, unsigned ok, const float (&x)[3], float r0,
+                                float rp, int lp, int2 (&blk)[3], int (&ic)[3]) {
+    const int nb[3] = {g.nbx, g.nby, g.nbz};
+    bool in = true;
 #pragma unroll
-                for (int ch = 0; ch < kAcc; ++ch)
-                    if (mask & (1u << ch)) atomicAdd(lacc + s * kAcc + ch, (unsigned long long)val[ch]);
-            } else {
-#pragma unroll
-                for (int ch = 0; ch < kAcc; ++ch)
-                    if (mask & (1u << ch)) atomicAdd(acc + ch * nc + addr, (unsigned long long)val[ch]);
+    for (int a = 0; a < 3; ++a) {
+        blk[a] = touched_blocks(x[a], rp, t.bext, nb[a]);
+        ic[a] = (int)floorf((x[a] - (float)t.b[a] * t.bext) / t.h);
+        in = in && (unsigned)(ic[a] - t.t0[a]) < (unsigned)t.tn && blk[a].x >= t.b[a] - 1 && blk[a].y <= t.b[a] + 1;
+    }
+    const int d = lp - t.level;
+    if (!in || d < 0 || d > 1 || r0 > g.h0) return 2;  // (candidates sized for radii of at most a cell per level)
+    for (int i = blk[0].x; i <= blk[0].y; ++i)
+        for (int j = blk[1].x; j <= blk[1].y; ++j)
+            for (int k = blk[2].x; k <= blk[2].y; ++k)
+                if (!(ok >> (((i - t.b[0] + 1) * 3 + j - t.b[1] + 1) * 3 + k - t.b[2] + 1) & 1u)) return 2;
+    return d;
+}
+
+// squared distances of cell i's centre and low face along axis a, from the
+// block that holds it; a cell of a block the support does not touch gets a
+// distance that makes its weight zero
+__device__ inline void cell_dist2(const TileRef& t, int a, int i, const int2& blk, float x, float& c2, float& f2) {
+    const int side = i < 0 ? -1 : (i >= t.nn ? 1 : 0), b = t.b[a] + side;
+    const float d = centre_dist((float)b * t.bext, i - side * t.nn, t.h, x);
+    const bool touched = b >= blk.x && b <= blk.y;
+    c2 = touched ? square(d) : 1e30f;
+    f2 = touched ? square(d - 0.5f * t.h) : 1e30f;
+}
+
+template <int R>
+__global__ __launch_bounds__(P2GTile<R>::NT) void k_mr_p2g_tile(MGrid g, int subs, const float* __restrict__ x,
+                                                                const float* __restrict__ v,
+                                                                const int* __restrict__ type,
+                                                                const int* __restrict__ lev,
+                                                                const int* __restrict__ perm,
+                                                                const int* __restrict__ start, MRConst c,
+                                                                int* __restrict__ coarse_tile, int* __restrict__ list,
+                                                                int* __restrict__ nlist,
+                                                                unsigned long long* __restrict__ acc) {
+    using PT = P2GTile<R>;
+    constexpr int E = PT::E, E3 = PT::E3, NT = PT::NT;
+    __shared__ unsigned long long L[kAcc * E3];
+    __shared__ int s_ok;
+    const int wg = xcd_block(blockIdx.x, gridDim.x), slot = wg / subs, sub = wg - slot * subs;
+    TileRef t;
+    t.level = g.blev[slot];
+    t.nn = g.n0 >> t.level;
+    t.base = g.coff[slot];
+    t.tn = min(t.nn, 8);
+    const int ns = t.nn / t.tn;  // tiles per axis
+    if (sub >= ns * ns * ns) return;
+    int* flag = coarse_tile + t.base + sub;  // (a block has at least as many cells as tiles)
+    if (R == 2 && *flag == 0) return;
+    const int blk = g.blk[slot];
+    t.b[2] = blk % g.nbz;
+    t.b[1] = (blk / g.nbz) % g.nby;
+    t.b[0] = blk / (g.nbz * g.nby);
+    t.t0[0] = sub / (ns * ns) * t.tn;
+    t.t0[1] = sub / ns % ns * t.tn;
+    t.t0[2] = sub % ns * t.tn;
+    t.h = cell_size(g, t.level);
+    t.bext = (float)g.n0 * g.h0;
+    const int tid = threadIdx.x;
+    for (int e = tid; e < kAcc * E3; e += NT) L[e] = 0ull;
+    if (tid < 64) {
+        bool same = false;
+        if (tid < 27) {
+            const int i = t.b[0] + tid / 9 - 1, j = t.b[1] + tid / 3 % 3 - 1, k = t.b[2] + tid % 3 - 1;
+            if (i >= 0 && j >= 0 && k >= 0 && i < g.nbx && j < g.nby && k < g.nbz) {
+                const int s = g.slot[(i * g.nby + j) * g.nbz + k];
+                same = s >= 0 && g.blev[s] == t.level;
             }
-        });
+        }
+        const unsigned long long m = __ballot(same);
+        if (tid == 0) s_ok = (int)(unsigned)m;
     }
     __syncthreads();
-    for (int s = threadIdx.x; s < kP2GSlots; s += blockDim.x) {
-        const int a = tag[s];
-        if (a < 0) continue;
+    const unsigned ok = (unsigned)s_ok;
+    const int tn3 = t.tn * t.tn * t.tn;
+    bool coarse = false;
+    // lanes of a wave take different cells; the threads beyond one per cell
+    // share its particles
+    const int parts = tn3 <= NT ? NT / tn3 : 1;
+    const int cell0 = tid % tn3, part = min(tid / tn3, parts);
+    if (part < parts) {
+        const int li = cell0 / (t.tn * t.tn), lj = cell0 / t.tn % t.tn, lk = cell0 % t.tn;
+        const int addr = t.base + ((t.t0[0] + li) * t.nn + t.t0[1] + lj) * t.nn + t.t0[2] + lk;
+        const int e0 = start[addr + 1];
+        for (int q = start[addr] + part; q < e0; q += parts) {
+            const int p = perm[q];
+            const float px[3] = {x[3 * (int64_t)p], x[3 * (int64_t)p + 1], x[3 * (int64_t)p + 2]};
+            const float vel[3] = {v[3 * (int64_t)p], v[3 * (int64_t)p + 1], v[3 * (int64_t)p + 2]};
+            const int lp = lev[p];
+            const float mp = (type[p] == 1 ? c.rho_l : c.rho_g) * (float)(1 << (3 * lp));
+            const float rp = c.r0 * (float)(1 << lp);
+            const float inv_r2 = 1.0f / (rp * rp);
+            int2 tb[3];
+            int ic[3];
+            const int cls = p2g_class(g, t, ok, px, c.r0, rp, lp, tb, ic);
+            if (R == 1) {
+                if (cls == 1) coarse = true;
+                if (cls == 2) {  // one atomic for the lanes that are here
+                    const unsigned long long m = __ballot(1);
+                    const int lane = tid & 63, first = __ffsll((long long)m) - 1;
+                    int at = 0;
+                    if (lane == first) at = atomicAdd(nlist, __popcll(m));
+                    at = __shfl(at, first, 64);
+                    list[at + __popcll(m & ((1ull << lane) - 1))] = p;
+                }
+            }
+            if (cls != R - 1) continue;
+            auto add = [&](int ch, int at, float value, float scale) {
+                atomicAdd(L + ch * E3 + at, (unsigned long long)fixed(value, scale));
+            };
+            if constexpr (R == 1) {
+                // per axis: the two centres (first index it) and the two low
+                // faces (first index ic) within the radius
+                float c2[3][2], f2[3][2];
+                int lc[3], lf[3];
+#pragma unroll
+                for (int a = 0; a < 3; ++a) {
+                    const float gx = (px[a] - (float)t.b[a] * t.bext) / t.h;
+                    const int it = gx - (float)ic[a] < 0.5f ? ic[a] - 1 : ic[a];
+                    float unused;
+                    cell_dist2(t, a, it, tb[a], px[a], c2[a][0], unused);
+                    cell_dist2(t, a, it + 1, tb[a], px[a], c2[a][1], unused);
+                    cell_dist2(t, a, ic[a], tb[a], px[a], unused, f2[a][0]);
+                    cell_dist2(t, a, ic[a] + 1, tb[a], px[a], unused, f2[a][1]);
+                    lc[a] = it - t.t0[a] + R;
+                    lf[a] = ic[a] - t.t0[a] + R;
+                }
+#pragma unroll
+                for (int q4 = 0; q4 < 4; ++q4) {
+                    // q4 = 0: centres, 1-3: low faces of axis q4 - 1
+                    const int at0 = ((q4 == 1 ? lf[0] : lc[0]) * E + (q4 == 2 ? lf[1] : lc[1])) * E +
+                                    (q4 == 3 ? lf[2] : lc[2]);
+#pragma unroll
+                    for (int m = 0; m < 8; ++m) {
+                        const int i = m >> 2, j = (m >> 1) & 1, k = m & 1;
+                        const float w = eq6_weight(q4 == 1 ? f2[0][i] : c2[0][i], q4 == 2 ? f2[1][j] : c2[1][j],
+                                                   q4 == 3 ? f2[2][k] : c2[2][k], inv_r2);
+                        if (!(w > 0.0f)) continue;
+                        const int at = at0 + (i * E + j) * E + k;
+                        const float wm = w * mp;
+                        if (q4 == 0) {
+                            add(0, at, wm, c.mass_scale);
+                            add(1, at, w, c.w_scale);
+                        } else {
+                            add(1 + q4, at, wm, c.mass_scale);
+                            add(4 + q4, at, wm * vel[q4 - 1], c.mom_scale);
+                        }
+                    }
+                }
+            } else {
+                float zc[5], zf[5];
+#pragma unroll
+                for (int k = 0; k < 5; ++k) cell_dist2(t, 2, ic[2] - 2 + k, tb[2], px[2], zc[k], zf[k]);
+                const float r2 = rp * rp;
+                for (int i = 0; i < 5; ++i) {
+                    float xc, xf;
+                    cell_dist2(t, 0, ic[0] - 2 + i, tb[0], px[0], xc, xf);
+                    if (fminf(xc, xf) >= r2) continue;
+                    for (int j = 0; j < 5; ++j) {
+                        float yc, yf;
+                        cell_dist2(t, 1, ic[1] - 2 + j, tb[1], px[1], yc, yf);
+                        if (fminf(xc, xf) + fminf(yc, yf) >= r2) continue;
+                        const int row = ((ic[0] - 2 + i - t.t0[0] + R) * E + ic[1] - 2 + j - t.t0[1] + R) * E +
+                                        ic[2] - 2 - t.t0[2] + R;
+#pragma unroll
+                        for (int k = 0; k < 5; ++k) {
+                            const float wt[4] = {eq6_weight(xc, yc, zc[k], inv_r2), eq6_weight(xf, yc, zc[k], inv_r2),
+                                                 eq6_weight(xc, yf, zc[k], inv_r2), eq6_weight(xc, yc, zf[k], inv_r2)};
+#pragma unroll
+                            for (int q4 = 0; q4 < 4; ++q4) {
+                                if (!(wt[q4] > 0.0f)) continue;
+                                const float wm = wt[q4] * mp;
+                                if (q4 == 0) {
+                                    add(0, row + k, wm, c.mass_scale);
+                                    add(1, row + k, wt[0], c.w_scale);
+                                } else {
+                                    add(1 + q4, row + k, wm, c.mass_scale);
+                                    add(4 + q4, row + k, wm * vel[q4 - 1], c.mom_scale);
+                                }
+                            }
+                        }
+                    }
+                }
+            }
+        }
+    }
+    if (R == 1) {
+        const bool any = __syncthreads_or(coarse);
+        if (tid == 0) *flag = any ? 1 : 0;
+    } else {
+        __syncthreads();
+    }
+    // flush: an entry beyond the block belongs to the neighbouring block
+    const int64_t nc = g.ncells;
+    const int ext = t.tn + 2 * R;
+    for (int e = tid; e < E3; e += NT) {
+        const int ek = e % E, ej = e / E % E, ei = e / (E * E);
+        if (ei >= ext || ej >= ext || ek >= ext) continue;
+        bool any = false;
+#pragma unroll
+        for (int ch = 0; ch < kAcc; ++ch) any = any || L[ch * E3 + e] != 0ull;
+        if (!any) continue;
+        const int i = t.t0[0] + ei - R, j = t.t0[1] + ej - R, k = t.t0[2] + ek - R;
+        const int di = i < 0 ? -1 : (i >= t.nn ? 1 : 0), dj = j < 0 ? -1 : (j >= t.nn ? 1 : 0),
+                  dk = k < 0 ? -1 : (k >= t.nn ? 1 : 0);
+        int base = t.base;
+        if (di | dj | dk)  // (non-zero entries only lie in blocks of this level)
+            base = g.coff[g.slot[((t.b[0] + di) * g.nby + t.b[1] + dj) * g.nbz + t.b[2] + dk]];
+        const int64_t a = base + ((i - di * t.nn) * t.nn + j - dj * t.nn) * t.nn + k - dk * t.nn;
 #pragma unroll
         for (int ch = 0; ch < kAcc; ++ch) {
-            const unsigned long long val = lacc[s * kAcc + ch];
+            const unsigned long long val = L[ch * E3 + e];
             if (val != 0ull) atomicAdd(acc + ch * nc + a, val);
         }
+    }
+}
+
+// The listed particles, by the walk: a workgroup keeps a hash of kP2GSlots
+// cells in LDS (tag + the 8 fixed-point channels), adds there with LDS
+// atomics, and flushes every cached cell with one global atomic per non-zero
+// channel.  A contribution whose slot holds another cell goes to global
+// memory directly.  Integer sums, so the result equals the uncached kernel's
+// bit for bit.
+constexpr int kP2GSlots = 512;
+constexpr int kP2GPerBlock = 256;  // particles per chunk (1 per thread)
+constexpr unsigned kP2GListBlocks = 1024;
+static_assert(kP2GSlots == 1 << 9, "the slot hash keeps 9 bits");
+
+__global__ __launch_bounds__(256) void k_mr_p2g_list(MGrid g, const float* __restrict__ x, const float* __restrict__ v,
+                                                     const int* __restrict__ type, const int* __restrict__ lev,
+                                                     const int* __restrict__ list, const int* __restrict__ nlist,
+                                                     const int* __restrict__ perm, const int* __restrict__ outside,
+                                                     int np, MRConst c, unsigned long long* __restrict__ acc) {
+    __shared__ int tag[kP2GSlots];
+    __shared__ unsigned long long lacc[kP2GSlots * kAcc];
+    const int64_t nc = g.ncells;
+    // the listed ones, then those outside every block (the last of the order)
+    const int nl = *nlist, out0 = *outside, n = nl + np - out0;
+    for (int p0 = blockIdx.x * kP2GPerBlock; p0 < n; p0 += gridDim.x * kP2GPerBlock) {
+        for (int s = threadIdx.x; s < kP2GSlots; s += blockDim.x) tag[s] = -1;
+        for (int s = threadIdx.x; s < kP2GSlots * kAcc; s += blockDim.x) lacc[s] = 0ull;
+        __syncthreads();
+        if (p0 + (int)threadIdx.x < n) {
+            const int q = p0 + (int)threadIdx.x;
+            const int64_t p = q < nl ? list[q] : perm[out0 + q - nl];
+            splat_particle(g, x, v, type, lev, p, c, [&](int addr, const long long* val, unsigned mask) {
+                const int s = (int)(((unsigned)addr * 2654435761u) >> 23);  // 9-bit multiplicative hash
+                int t = tag[s];
+                if (t != addr && t == -1) {
+                    t = atomicCAS(tag + s, -1, addr);
+                    if (t == -1) t = addr;
+                }
+                if (t == addr) {
+#pragma unroll
+                    for (int ch = 0; ch < kAcc; ++ch)
+                        if (mask & (1u << ch)) atomicAdd(lacc + s * kAcc + ch, (unsigned long long)val[ch]);
+                } else {
+#pragma unroll
+                    for (int ch = 0; ch < kAcc; ++ch)
+                        if (mask & (1u << ch)) atomicAdd(acc + ch * nc + addr, (unsigned long long)val[ch]);
+                }
+            });
+        }
+        __syncthreads();
+        for (int s = threadIdx.x; s < kP2GSlots; s += blockDim.x) {
+            const int a = tag[s];
+            if (a < 0) continue;
+#pragma unroll
+            for (int ch = 0; ch < kAcc; ++ch) {
+                const unsigned long long val = lacc[s * kAcc + ch];
+                if (val != 0ull) atomicAdd(acc + ch * nc + a, val);
+            }
+        }
+        __syncthreads();
     }
 }
 
@@ -921,10 +1201,25 @@ PF_API int pf_mr_p2g_sorted(const pf_msbg_grid* g, const pf_mr_particles* ps, co
     PF_CHECK_LAUNCH();
     rc = exclusive_scan(count, nk, start, tmp, s);
     if (rc) return rc;
-    k_mr_cell_scatter<<<pgrid(n), 256, 0, s>>>(key, rank, start, n, perm);
+    // the scan's scratch and the counts are free now: the walk list's length,
+    // and a flag per tile (at the block's first cell + tile); the list takes
+    // the keys' place once the scatter has read them
+    int* nlist = tmp;
+    k_mr_cell_scatter<<<pgrid(n), 256, 0, s>>>(key, rank, start, n, perm, nlist);
     PF_CHECK_LAUNCH();
-    k_mr_p2g_cached<<<cdiv(n, kP2GPerBlock), 256, 0, s>>>(m, ps->x, ps->v, ps->type, ps->level, perm, n,
-                                                           mrconst(*prm), reinterpret_cast<unsigned long long*>(f->acc));
+    const MRConst c = mrconst(*prm);
+    unsigned long long* acc = reinterpret_cast<unsigned long long*>(f->acc);
+    const int sa = m.n0 > 8 ? m.n0 / 8 : 1, subs = sa * sa * sa;
+    PF_REQUIRE((int64_t)m.nslots * subs < (int64_t)1 << 31, "pf_mr_p2g_sorted: too many tiles");
+    const unsigned tiles = (unsigned)(m.nslots * subs);
+    k_mr_p2g_tile<1><<<tiles, P2GTile<1>::NT, 0, s>>>(m, subs, ps->x, ps->v, ps->type, ps->level, perm, start, c, count,
+                                                      key, nlist, acc);
+    PF_CHECK_LAUNCH();
+    k_mr_p2g_tile<2><<<tiles, P2GTile<2>::NT, 0, s>>>(m, subs, ps->x, ps->v, ps->type, ps->level, perm, start, c, count,
+                                                      key, nlist, acc);
+    PF_CHECK_LAUNCH();
+    k_mr_p2g_list<<<kP2GListBlocks, 256, 0, s>>>(m, ps->x, ps->v, ps->type, ps->level, key, nlist, perm, start + g->ncells,
+                                                (int)n, c, acc);
     PF_CHECK_LAUNCH();
     return PF_OK;
 }

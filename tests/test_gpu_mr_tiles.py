@@ -1,0 +1,50 @@
+"""The tiled adaptive P2G against the per-particle kernel, bit for bit: every
+class of particle (own level, one level coarser, two coarser, finer, across
+2:1 jumps, outside the grid) on blocks of one cell per axis up to several
+tiles per block."""
+
+import numpy as np
+import pytest
+
+from conftest import load_pkg
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("nb,n0,max_level,seed", [
+    ((3, 2, 2), 16, 2, 1),   # 16^3, 8^3 and 4^3 cells per block: 8 tiles, 1 tile, part of a tile
+    ((2, 3, 2), 32, 1, 2),   # 64 and 8 tiles per block
+    ((4, 3, 5), 8, 3, 3),    # down to one cell per block
+    ((5, 4, 3), 2, 1, 4),    # blocks of 2 and of 1 cells: every support crosses blocks
+    ((1, 1, 1), 8, 0, 5),    # one block: every neighbour is missing
+])
+def test_tiled_p2g_equals_per_particle_atomics(nb, n0, max_level, seed):
+    from importlib import import_module
+    pf = load_pkg()
+    cfgm, mrs = (import_module(pf.__name__ + "." + m) for m in ("config", "mr_sim"))
+    print(f"[gpu] tiled adaptive P2G {nb} n0={n0} max_level={max_level}", flush=True)
+    rng = np.random.default_rng(seed)
+    dx = 0.37 / n0  # no power of two: cell centres round
+    cfg = cfgm.Config(res=tuple(n * n0 for n in nb), dx=dx, ppc=27, droplets=False)
+    levels = rng.integers(0, max_level + 1, size=int(np.prod(nb)))
+    sim = mrs.AdaptiveSimulator(cfg, nb, n0=n0, max_level=max_level, frozen_levels=levels)
+    L = np.array(nb) * n0 * dx
+    n = 40000
+    x = rng.random((n, 3)) * L
+    x[: n // 50] = rng.random((n // 50, 3)) * (1.2 * L) - 0.1 * L       # some outside the box
+    on = rng.integers(0, n, size=n // 20)
+    x[on] = np.round(x[on] / dx) * dx                                   # on faces and corners
+    lev = rng.integers(0, max_level + 1, size=n).astype(np.int32)
+    sim.set_particles(x.astype(np.float32), rng.standard_normal((n, 3)).astype(np.float32),
+                      rng.integers(0, 2, size=n).astype(np.int32), lev)
+    sim._rebuild_grid(1e-3)
+    prm = sim._params(1e-3, sim._max_speed())
+    out = []
+    for sorted_ in (True, False, True):  # the second tiled run: on a used scratch buffer
+        sim.p2g_sorted = sorted_
+        sim.stage_p2g(prm)
+        out.append({k: getattr(sim, k).cpu().numpy().copy() for k in ("cwsum", "phi", "fmass", "fvel", "is_liquid")})
+    for k in out[0]:
+        assert np.array_equal(out[0][k], out[1][k]), k
+        assert np.array_equal(out[2][k], out[1][k]), k
+    assert np.abs(out[0]["fmass"]).max() > 0
