@@ -270,56 +270,78 @@ __global__ __launch_bounds__(kCoarsestThreads) void k_msbg_coarsest(MGrid g, flo
 
 // The coarsest level's smoothing as a matrix: `sweeps` red-black sweeps
 // from zero followed by mean removal are a linear map b -> p, so column j
-// is that map applied to the unit vector e_j.  One workgroup per column,
-// the sweeps in FP64 from LDS (couplings gathered as in k_msbg_coarsest);
-// op[j * n + t] is entry (t, j).  A V-cycle then applies it with one
-// matrix-vector product (k_msbg_coarse_apply) instead of the sweeps.
+// is that map applied to the unit vector e_j.  One workgroup per column and
+// one thread per cell, in FP64; op[j * n + t] is entry (t, j).  A V-cycle then
+// applies it with one matrix-vector product (k_msbg_coarse_apply) instead of
+// the sweeps.
+// A row's first kOpRow couplings are in registers (a cell without finer
+// neighbours has no more; another row walks its rest anew in every sweep) and
+// only the iterate is read from LDS.  That leaves 27 KB of LDS per workgroup,
+// so all 512 columns run at once instead of in two rounds, and a half-sweep
+// is 7 reads: 259 -> 64 us at 512 cells and 80 sweeps, once per solve.
 constexpr int kMsbgCoarseOpMax = 512;
+constexpr int kOpRow = 6;
 
-__host__ __device__ inline size_t coarse_op_lds_bytes(int n) {
-    return (size_t)n * (kRowMax * (sizeof(float) + sizeof(unsigned short)) + 2 * sizeof(double) + sizeof(float) + 2);
+__host__ __device__ constexpr size_t coarse_op_lds_bytes(int n) {
+    return (size_t)n * (2 * sizeof(double) + kOpRow * (sizeof(float) + sizeof(unsigned short)));
 }
 
 __global__ __launch_bounds__(kCoarsestThreads) void k_msbg_coarse_op(MGrid g, const float* __restrict__ bface,
                                                                      const float* __restrict__ diag, int sweeps,
                                                                      double omega, double* __restrict__ op) {
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
-    const int n = g.ncells, j = blockIdx.x;
+    static_assert(kMsbgCoarseOpMax <= kCoarsestThreads, "one cell per thread");
+    const int n = g.ncells, j = blockIdx.x, a = threadIdx.x;
     double* p0 = reinterpret_cast<double*>(lds);
     double* p1 = p0 + n;
     float* coef = reinterpret_cast<float*>(p1 + n);
-    float* dd = coef + (size_t)n * kRowMax;
-    unsigned short* nbr = reinterpret_cast<unsigned short*>(dd + n);
-    unsigned char* cnt = reinterpret_cast<unsigned char*>(nbr + (size_t)n * kRowMax);
-    unsigned char* col = cnt + n;
+    unsigned short* nbr = reinterpret_cast<unsigned short*>(coef + (size_t)kOpRow * n);
     __shared__ double sh[16];
     __shared__ double shift;
-    for (int a = threadIdx.x; a < n; a += blockDim.x) {
-        int k = 0;
-        for_each_coupling(g, bface, a, [&](int nb, float t) {
-            coef[k * n + a] = t;
-            nbr[k * n + a] = (unsigned short)nb;
-            ++k;
+    int cnt = 0, colour = -1;
+    double w = 0.0;
+    float c[kOpRow];
+    int nb[kOpRow];
+    if (a < n) {
+        for_each_coupling(g, bface, a, [&](int b, float t) {
+            if (cnt < kOpRow) {
+                coef[cnt * n + a] = t;
+                nbr[cnt * n + a] = (unsigned short)b;
+            }
+            ++cnt;
         });
-        cnt[a] = (unsigned char)k;
         const int4 o = origin(g, a);
-        col[a] = (unsigned char)(((o.x >> o.w) + (o.y >> o.w) + (o.z >> o.w)) & 1);
-        dd[a] = diag[a];
+        if (diag[a] > 0.0f) {
+            colour = ((o.x >> o.w) + (o.y >> o.w) + (o.z >> o.w)) & 1;
+            w = omega / (double)diag[a];
+        }
         p0[a] = 0.0;
+    }
+#pragma unroll
+    for (int k = 0; k < kOpRow; ++k) {  // (written and read by this thread alone)
+        const bool has = k < cnt;
+        c[k] = has ? coef[k * n + a] : 0.0f;
+        nb[k] = has ? nbr[k * n + a] : min(a, n - 1);
     }
     __syncthreads();
     double* pin = p0;
     double* pout = p1;
     for (int sw = 0; sw < sweeps; ++sw)
-        for (int c = 0; c < 2; ++c) {
-            for (int a = threadIdx.x; a < n; a += blockDim.x) {
+        for (int col = 0; col < 2; ++col) {
+            if (a < n) {
                 double v = pin[a];
-                if (col[a] == c && dd[a] > 0.0f) {
-                    const double pa = pin[a];
+                if (colour == col) {
+                    const double pa = v;
                     double acc = 0.0;
-                    const int m = cnt[a];
-                    for (int k = 0; k < m; ++k) acc += (double)coef[k * n + a] * (pa - pin[nbr[k * n + a]]);
-                    v = pa + omega * ((a == j ? 1.0 : 0.0) - acc) / (double)dd[a];
+#pragma unroll
+                    for (int k = 0; k < kOpRow; ++k) acc += (double)c[k] * (pa - pin[nb[k]]);
+                    if (cnt > kOpRow) {
+                        int k = 0;
+                        for_each_coupling(g, bface, a, [&](int b, float t) {
+                            if (k++ >= kOpRow) acc += (double)t * (pa - pin[b]);
+                        });
+                    }
+                    v = pa + ((a == j ? 1.0 : 0.0) - acc) * w;
                 }
                 pout[a] = v;
             }
@@ -328,35 +350,40 @@ __global__ __launch_bounds__(kCoarsestThreads) void k_msbg_coarse_op(MGrid g, co
             pin = pout;
             pout = t;
         }
-    double sm[1] = {0.0};
-    for (int a = threadIdx.x; a < n; a += blockDim.x) sm[0] += pin[a];
+    double sm[1] = {a < n ? pin[a] : 0.0};
     block_sum<1>(sm, sh);
-    if (threadIdx.x == 0) shift = -(sm[0] / (double)n);
+    if (a == 0) shift = -(sm[0] / (double)n);
     __syncthreads();
-    for (int a = threadIdx.x; a < n; a += blockDim.x) op[(int64_t)j * n + a] = pin[a] + shift;
+    if (a < n) op[(int64_t)j * n + a] = pin[a] + shift;
 }
 
-// p = op b in FP64, rounded to float.  A workgroup takes 64 rows; wave w
-// sums the columns w, w + 8, w + 16, ... of them (a wave reads 64
-// consecutive entries of a column), and the 8 partials of a row are added
-// in wave order.
-__global__ __launch_bounds__(512) void k_msbg_coarse_apply(const double* __restrict__ op,
-                                                           const float* __restrict__ b, float* __restrict__ p,
-                                                           int n) {
-    __shared__ double bs[kMsbgCoarseOpMax];
-    __shared__ double part[8][64];
-    for (int j = threadIdx.x; j < n; j += blockDim.x) bs[j] = (double)b[j];
-    __syncthreads();
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int t = blockIdx.x * 64 + lane;
+// p = op b in FP64, rounded to float.  A workgroup takes kApplyRows rows (128
+// consecutive bytes of a column) and its 1024 threads 64 columns at a time,
+// so 512 cells make 32 workgroups with 8 loads in flight per thread; 64 rows
+// per workgroup of 8 waves left 8 CUs to read the 2 MB (22 -> 4.9 us out of
+// HBM, 11 -> 5.2 out of L2).  Partials are added in a fixed order.
+constexpr int kApplyRows = 16;
+
+__global__ __launch_bounds__(1024) void k_msbg_coarse_apply(const double* __restrict__ op,
+                                                            const float* __restrict__ b, float* __restrict__ p,
+                                                            int n) {
+    __shared__ double part[16][kApplyRows];
+    const int r = threadIdx.x % kApplyRows, w = threadIdx.x >> 6;
+    const int t = blockIdx.x * kApplyRows + r;
+    constexpr int G = 1024 / kApplyRows, M = kMsbgCoarseOpMax / G;
     double acc = 0.0;
-    if (t < n)
-        for (int j = w; j < n; j += 8) acc += op[(int64_t)j * n + t] * bs[j];
-    part[w][lane] = acc;
+#pragma unroll
+    for (int m = 0; m < M; ++m) {
+        const int j = (int)threadIdx.x / kApplyRows + m * G;
+        if (j < n && t < n) acc += op[(int64_t)j * n + t] * (double)b[j];
+    }
+    acc += __shfl_xor(acc, 16, 64);
+    acc += __shfl_xor(acc, 32, 64);
+    if ((threadIdx.x & 63) < kApplyRows) part[w][r] = acc;
     __syncthreads();
-    if (w == 0 && t < n) {
-        double s = part[0][lane];
-        for (int q = 1; q < 8; ++q) s += part[q][lane];
+    if (threadIdx.x < kApplyRows && t < n) {
+        double s = part[0][r];
+        for (int q = 1; q < 16; ++q) s += part[q][r];
         p[t] = (float)s;
     }
 }
@@ -869,13 +896,8 @@ PF_API int pf_msbg_coarse_op(const pf_msbg_grid* g, const float* bface, const fl
     PF_REQUIRE(bface && diag && op && sweeps >= 0, "pf_msbg_coarse_op: bad arguments");
     PF_REQUIRE(g->ncells <= pf_msbg_coarse_op_max_cells(), "pf_msbg_coarse_op: %d cells exceed the limit",
                g->ncells);
-    const size_t bytes = coarse_op_lds_bytes(g->ncells);
-    if (bytes > 65536) {
-        const hipError_t e = hipFuncSetAttribute((const void*)k_msbg_coarse_op,
-                                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
-        PF_REQUIRE(e == hipSuccess, "pf_msbg_coarse_op: cannot raise the LDS limit to %zu bytes", bytes);
-    }
-    k_msbg_coarse_op<<<g->ncells, kCoarsestThreads, bytes, S(stream)>>>(mgrid(*g), bface, diag, sweeps,
+    static_assert(coarse_op_lds_bytes(kMsbgCoarseOpMax) <= 60 * 1024, "the default dynamic LDS limit");
+    k_msbg_coarse_op<<<g->ncells, kCoarsestThreads, coarse_op_lds_bytes(g->ncells), S(stream)>>>(mgrid(*g), bface, diag, sweeps,
                                                                          (double)omega, op);
     PF_CHECK_LAUNCH();
     return PF_OK;
@@ -883,7 +905,7 @@ PF_API int pf_msbg_coarse_op(const pf_msbg_grid* g, const float* bface, const fl
 
 PF_API int pf_msbg_coarse_apply(const double* op, const float* b, float* p, int32_t n, pf_stream_t stream) {
     PF_REQUIRE(op && b && p && n > 0 && n <= kMsbgCoarseOpMax, "pf_msbg_coarse_apply: bad arguments");
-    k_msbg_coarse_apply<<<cdiv(n, 64), 512, 0, S(stream)>>>(op, b, p, n);
+    k_msbg_coarse_apply<<<cdiv(n, kApplyRows), 1024, 0, S(stream)>>>(op, b, p, n);
     PF_CHECK_LAUNCH();
     return PF_OK;
 }

@@ -48,3 +48,38 @@ def test_tiled_p2g_equals_per_particle_atomics(nb, n0, max_level, seed):
         assert np.array_equal(out[0][k], out[1][k]), k
         assert np.array_equal(out[2][k], out[1][k]), k
     assert np.abs(out[0]["fmass"]).max() > 0
+
+
+@pytest.mark.parametrize("nb,n0,levels", [((8, 8, 8), 2, "one"), ((3, 3, 3), 4, "jump"), ((1, 2, 1), 4, "one"),
+                                          ((7, 7, 9), 2, "one")])
+def test_coarse_level_matrix_matches_the_sweeps(nb, n0, levels):
+    """The coarsest level's matrix (rows of 6 couplings, and of up to 24 next
+    to a 2:1 jump; 8 to 512 cells, whole and partial workgroups of its
+    product) against the launched sweeps in FP32: 80 sweeps of FP32 rounding,
+    held to 2e-4 of the solution's size as in the V-cycle tests."""
+    from importlib import import_module
+    import torch
+    pf = load_pkg()
+    lib, msbg, mgm = (import_module(pf.__name__ + "." + m) for m in ("_lib", "msbg", "mr_multigrid"))
+    print(f"[gpu] coarse matrix {nb} n0={n0} {levels}", flush=True)
+    rng = np.random.default_rng(4)
+    top = {2: 1, 4: 2}[n0]
+    lv = np.full(int(np.prod(nb)), top, np.int32)
+    if levels == "jump":
+        lv[len(lv) // 2] = top - 1
+    g = msbg.MSBG(nb, n0=n0, h0=0.1, device="cuda:0", max_level=top)
+    g.build(lv)
+    assert g.ncells <= 512
+    mg = mgm.MRMultigrid(g, min_cells=10 ** 9)
+    bface = torch.from_numpy((0.1 + rng.random(3 * g.ncells)).astype(np.float32)).cuda()
+    mg.build_hierarchy(bface)
+    c = mg.levels[-1]
+    b = torch.from_numpy(rng.standard_normal(c.n).astype(np.float32)).cuda()
+    c.b.copy_(b - b.mean())
+    assert mg.coarsest_mode == "matrix"
+    got = torch.zeros_like(c.p)
+    lib.call("pf_msbg_coarse_apply", lib.ptr(mg._coarse_op), lib.ptr(c.b), lib.ptr(got), c.n, lib.stream())
+    c.p.zero_()
+    mg._smooth(c, mg.coarsest_sweeps)
+    ref = (c.p - c.p.double().mean().float()).double()
+    assert float((got.double() - ref).abs().max()) < 2e-4 * float(ref.abs().max())
