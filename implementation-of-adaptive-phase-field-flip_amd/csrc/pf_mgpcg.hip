@@ -25,6 +25,7 @@ namespace pf {
 int fill_u32(void* dst, int64_t n, uint32_t v, hipStream_t s);
 
 constexpr int MAXB = 1024;  // blocks of a reduction launch
+constexpr int PS = 8192;    // entries per quantity of the partial-sum arrays (the sweeps write one per tile)
 constexpr int RT = 256;     // threads of element-wise / reduction kernels
 // k_cg_apply and k_cg_beta: few, wide blocks, so the kernel that combines
 // their partials itself reads few of them
@@ -47,7 +48,7 @@ struct CGState {
     // vscale_inv, so the FP16 iterates stay in range as r shrinks
     float vscale, vscale_inv;
     unsigned ticket[8];
-    double part[6 * MAXB];  // [0, 5 MAXB): dot-product partials; [5 MAXB, 6 MAXB): <q, Aq> partials
+    double part[6 * PS];  // [0, 5 PS): dot-product partials; [5 PS, 6 PS): <q, Aq> partials
     float fpart[MAXB];
     // the coarsest level's `coarsest` red-black sweeps from zero followed by
     // mean removal, a linear map of its right-hand side: column j (the image
@@ -145,9 +146,10 @@ template <int NV>
 __device__ inline void combine_sums(const double* part, int nparts, double (&v)[NV], double* sh) {
 #pragma unroll
     for (int q = 0; q < NV; ++q) v[q] = 0.0;
+#pragma unroll 4
     for (int b = threadIdx.x; b < nparts; b += blockDim.x)
 #pragma unroll
-        for (int q = 0; q < NV; ++q) v[q] += part[q * MAXB + b];
+        for (int q = 0; q < NV; ++q) v[q] += part[q * PS + b];
     block_sum<NV>(v, sh);
 }
 
@@ -740,7 +742,7 @@ __global__ __launch_bounds__(NTH, 4) void k_rbgs_full(Dims d, const ST* __restri
         block_sum<5>(dsum, s_dot);
         if (tid == 0 && !skip) {
 #pragma unroll
-            for (int q = 0; q < 5; ++q) df.st->part[q * MAXB + blockIdx.x] = dsum[q];
+            for (int q = 0; q < 5; ++q) df.st->part[q * PS + blockIdx.x] = dsum[q];
             if (blockIdx.x == 0) df.st->beta_parts = 1;  // read by the next k_cg_apply
         }
     }
@@ -1204,7 +1206,7 @@ __global__ __launch_bounds__(1024) void k_phase(Dims d, Dims dc, const ST* __res
         block_sum<5>(dsum, s_dot);
         if (tid == 0) {
 #pragma unroll
-            for (int q = 0; q < 5; ++q) df.st->part[q * MAXB + blockIdx.x] = dsum[q];
+            for (int q = 0; q < 5; ++q) df.st->part[q * PS + blockIdx.x] = dsum[q];
             if (blockIdx.x == 0) df.st->beta_parts = 1;  // read by the next k_cg_apply
         }
     }
@@ -1878,7 +1880,7 @@ __global__ __launch_bounds__(RT) void k_cg_first(CGK<ZT> a) {
     }
     block_sum<3>(v, sh);
     if (threadIdx.x == 0)
-        for (int q = 0; q < 3; ++q) a.st->part[q * MAXB + blockIdx.x] = v[q];
+        for (int q = 0; q < 3; ++q) a.st->part[q * PS + blockIdx.x] = v[q];
 }
 
 // q = (z - mu) + beta q_old (the search direction, poisson.py:406; beta = 0
@@ -1985,7 +1987,7 @@ __global__ __launch_bounds__(WT) void k_cg_apply(CGK<ZT> a) {
         i += si;
     }
     block_sum<1>(v, sh);
-    if (threadIdx.x == 0) st->part[5 * MAXB + blockIdx.x] = v[0];
+    if (threadIdx.x == 0) st->part[5 * PS + blockIdx.x] = v[0];
 }
 
 // x += alpha q; r -= alpha Ap; partial max|r| (poisson.py:390-394), after
@@ -2012,7 +2014,7 @@ __global__ __launch_bounds__(RT) void k_cg_update(CGK<ZT> a) {
     }
     if (st->done) return;
     double t[1];
-    combine_sums<1>(st->part + 5 * MAXB, a.np_apply, t, shd);
+    combine_sums<1>(st->part + 5 * PS, a.np_apply, t, shd);
     if (threadIdx.x == 0) {
         const double qAq = t[0];
         const bool ok = qAq > 0.0;
@@ -2065,7 +2067,7 @@ __global__ __launch_bounds__(WT) void k_cg_beta(CGK<ZT> a) {
     }
     block_sum<5>(v, sh);
     if (threadIdx.x == 0) {
-        for (int q = 0; q < 5; ++q) a.st->part[q * MAXB + blockIdx.x] = v[q];
+        for (int q = 0; q < 5; ++q) a.st->part[q * PS + blockIdx.x] = v[q];
         if (blockIdx.x == 0) a.st->beta_parts = 1;  // read by the next k_cg_apply
     }
 }
@@ -2211,8 +2213,33 @@ static int ensure_small_lds() {
     return PF_OK;
 }
 
-// Fused full sweep on one level: tile shape by level size (big tiles cut
-// the redundant halo work, small ones keep enough workgroups in flight).
+// Fused full sweep on one level: tile shape by level size.  Long tiles cut
+// the redundant halo work, small ones keep enough workgroups in flight.
+// us per sweep, FP32 / BF16 (HIP events, 60 sweeps), by tile and threads:
+//                  8x8x64/512    8x8x32/512    8x8x16/256
+//   80^3            8.4 /  8.6    7.6 /  7.8    6.7 /  6.9
+//   128x96x64       8.0 /  8.4    7.4 /  7.5    7.7 /  7.8
+//   96x72x120       8.6 /  8.6    8.1 /  7.8    9.3 /  9.2
+//   128^3          13.2 / 11.9   13.5 / 12.7   16.5 / 14.8
+//   192x128x96     17.3 / 18.2   14.8 / 14.1   17.5 / 15.3
+//   160^3          26.6 / 28.1   24.0 / 21.6   29.4 / 25.3
+//   256^3           112 / 82.4    123 / 73.0    164 / 89.8
+// So 8x8x64 where its tiles are whole along k, in 16 bits only while they are
+// all resident at once (two per CU); otherwise 8x8x32 from 5 x 2^17 cells.
+enum SweepShape { SWEEP_64, SWEEP_32, SWEEP_16, SWEEP_SMALL };
+
+static int64_t sweep_tiles(const Dims& d, SweepShape s) {
+    const int tk = s == SWEEP_64 ? 64 : (s == SWEEP_32 ? 32 : 16);
+    return (int64_t)cdiv(d.nx, s == SWEEP_SMALL ? 4 : 8) * cdiv(d.ny, 8) * cdiv(d.nz, tk);
+}
+
+static SweepShape sweep_shape(const Dims& d, bool half) {
+    const int64_t n = (int64_t)d.nx * d.ny * d.nz;
+    if (n >= (int64_t)1 << 20 && d.nz % 64 == 0 && (!half || sweep_tiles(d, SWEEP_64) <= 512)) return SWEEP_64;
+    if (n >= (int64_t)5 << 17) return SWEEP_32;
+    return n >= (int64_t)1 << 17 ? SWEEP_16 : SWEEP_SMALL;
+}
+
 // PROL (CT = the coarse iterate's type): the input is pin plus the
 // prolongation of pcoarse (dims dc); the fine dims must be twice dc.
 template <typename ST, bool ZINIT, bool PROL = false, typename CT = float>
@@ -2221,35 +2248,51 @@ static int launch_full_sweep(const Dims& d, const ST* fx, const ST* fy, const ST
                              const float* bscale, hipStream_t s, const CT* pcoarse = nullptr,
                              Dims dc = Dims{1, 1, 1}, UpdateFold uf = UpdateFold{nullptr, 0, nullptr},
                              DotFold df = DotFold{nullptr, nullptr, nullptr}) {
-    const int64_t n = (int64_t)d.nx * d.ny * d.nz;
-    auto tiles = [&](int ti, int tj, int tk) {
-        return (unsigned)(cdiv(d.nx, ti) * cdiv(d.ny, tj) * cdiv(d.nz, tk));
-    };
+    const SweepShape shape = sweep_shape(d, sizeof(ST) == 2);
+    const unsigned tiles = (unsigned)sweep_tiles(d, shape);
     if constexpr (!ZINIT && !PROL) {
         if (df.Ap) {  // the plain sweep with the CG's inner products
-            if (n >= (int64_t)1 << 20)
-                k_rbgs_full<ST, false, 8, 8, 64, 512, false, float, true><<<tiles(8, 8, 64), 512, 0, s>>>(
+            switch (shape) {
+            case SWEEP_64:
+                k_rbgs_full<ST, false, 8, 8, 64, 512, false, float, true><<<tiles, 512, 0, s>>>(
                     d, fx, fy, fz, pin, pout, b, c1, omega, done, bscale, nullptr, dc, uf, df);
-            else if (n >= (int64_t)1 << 17)
-                k_rbgs_full<ST, false, 8, 8, 16, 256, false, float, true><<<tiles(8, 8, 16), 256, 0, s>>>(
+                break;
+            case SWEEP_32:
+                k_rbgs_full<ST, false, 8, 8, 32, 512, false, float, true><<<tiles, 512, 0, s>>>(
                     d, fx, fy, fz, pin, pout, b, c1, omega, done, bscale, nullptr, dc, uf, df);
-            else
-                k_rbgs_full<ST, false, 4, 8, 16, 256, false, float, true><<<tiles(4, 8, 16), 256, 0, s>>>(
+                break;
+            case SWEEP_16:
+                k_rbgs_full<ST, false, 8, 8, 16, 256, false, float, true><<<tiles, 256, 0, s>>>(
                     d, fx, fy, fz, pin, pout, b, c1, omega, done, bscale, nullptr, dc, uf, df);
+                break;
+            case SWEEP_SMALL:
+                k_rbgs_full<ST, false, 4, 8, 16, 256, false, float, true><<<tiles, 256, 0, s>>>(
+                    d, fx, fy, fz, pin, pout, b, c1, omega, done, bscale, nullptr, dc, uf, df);
+                break;
+            }
             PF_CHECK_LAUNCH();
             return PF_OK;
         }
     }
     PF_REQUIRE(!df.Ap, "launch_full_sweep: inner products only on a plain sweep");
-    if (n >= (int64_t)1 << 20)
-        k_rbgs_full<ST, ZINIT, 8, 8, 64, 512, PROL, CT><<<tiles(8, 8, 64), 512, 0, s>>>(
+    switch (shape) {
+    case SWEEP_64:
+        k_rbgs_full<ST, ZINIT, 8, 8, 64, 512, PROL, CT><<<tiles, 512, 0, s>>>(
             d, fx, fy, fz, pin, pout, b, c1, omega, done, bscale, pcoarse, dc, uf, df);
-    else if (n >= (int64_t)1 << 17)
-        k_rbgs_full<ST, ZINIT, 8, 8, 16, 256, PROL, CT><<<tiles(8, 8, 16), 256, 0, s>>>(
+        break;
+    case SWEEP_32:
+        k_rbgs_full<ST, ZINIT, 8, 8, 32, 512, PROL, CT><<<tiles, 512, 0, s>>>(
             d, fx, fy, fz, pin, pout, b, c1, omega, done, bscale, pcoarse, dc, uf, df);
-    else
-        k_rbgs_full<ST, ZINIT, 4, 8, 16, 256, PROL, CT><<<tiles(4, 8, 16), 256, 0, s>>>(
+        break;
+    case SWEEP_16:
+        k_rbgs_full<ST, ZINIT, 8, 8, 16, 256, PROL, CT><<<tiles, 256, 0, s>>>(
             d, fx, fy, fz, pin, pout, b, c1, omega, done, bscale, pcoarse, dc, uf, df);
+        break;
+    case SWEEP_SMALL:
+        k_rbgs_full<ST, ZINIT, 4, 8, 16, 256, PROL, CT><<<tiles, 256, 0, s>>>(
+            d, fx, fy, fz, pin, pout, b, c1, omega, done, bscale, pcoarse, dc, uf, df);
+        break;
+    }
     PF_CHECK_LAUNCH();
     return PF_OK;
 }
@@ -2309,14 +2352,6 @@ static int launch_phase(const Dims& d, const Dims& dc, int nsw, const ST* fx, co
                                                    bscale, uf, df, s)
                : launch_phase_tile<ST, PRE, 8, CT>(d, dc, nsw, fx, fy, fz, b, pin, pcoarse, pout, bc, omega, done,
                                                    bscale, uf, df, s);
-}
-
-// workgroups of launch_full_sweep on a level of dims d (one per tile)
-static int64_t full_sweep_blocks(const Dims& d) {
-    const int64_t n = (int64_t)d.nx * d.ny * d.nz;
-    const int ti = n >= (int64_t)1 << 20 ? 8 : (n >= (int64_t)1 << 17 ? 8 : 4);
-    const int tk = n >= (int64_t)1 << 20 ? 64 : 16;
-    return cdiv(d.nx, ti) * cdiv(d.ny, 8) * cdiv(d.nz, tk);
 }
 
 // The two iterate buffers of an HBM level: the level's own (level 0: the
@@ -2609,11 +2644,11 @@ static bool fold_residual_test(const pf_mg& mg) {
 // an HBM level 0) whose workgroups fit the partials array.
 static int64_t dot_blocks(const pf_mg& mg) {
     const Dims d = ldims(mg.lev[0]);
-    return level_fused(mg, 0) ? (int64_t)phase_tiles(d, phase_tile(d)) : full_sweep_blocks(d);
+    return level_fused(mg, 0) ? (int64_t)phase_tiles(d, phase_tile(d)) : sweep_tiles(d, sweep_shape(d, mg.precision != 0));
 }
 static bool fold_dots(const pf_mg& mg) {
     return !(mg.options & PF_MG_SEPARATE_DOTS) && mg.small_from > 0 && (mg.post >= 2 || level_fused(mg, 0)) &&
-           fused_smoother(mg, 0) && dot_blocks(mg) <= MAXB;
+           fused_smoother(mg, 0) && dot_blocks(mg) <= PS;
 }
 
 template <typename ST>
