@@ -1243,33 +1243,173 @@ __global__ __launch_bounds__(RT) void k_zero(T* x, int64_t n, const int* __restr
         x[i] = from_f32<T>(0.0f);
 }
 
+// ================================================================ levels of one workgroup
+constexpr int kSmallThreads = 1024;
+
+// A level (or all of a coarsest one) held by one workgroup: thread t has the
+// pairs of cells along k t, t + 1024, ... (row * nkp + kp), one cell of each
+// colour per pair, with their faces, b and omega / diag in registers.  Only
+// the iterate is in LDS, the cells of even and of odd k in two arrays indexed
+// by pair: one colour's cells of a row then lie next to each other, and a
+// wave's reads fall on all LDS banks (in cell order one colour uses every
+// other bank: 108 us instead of 69 for 60 sweeps of 26 x 19 x 13 cells).
+// Faces on a wall are given weight 0 in the sum (their neighbour is the cell
+// itself, so their flux is 0; they stay in the diagonal), so the neighbour
+// addresses need no clamps: zeros on either side of the arrays keep them
+// inside.  ZL: the low z faces are in LDS too (a cell's high z face is the
+// next cell's low one), which holds 8 pairs per thread without spilling in
+// the sweeps.
+struct PairGeom {
+    Dims d;
+    int nkp, npair, SP, OFF;  // pairs per row / in all; pairs per i; the odd array behind the even one
+};
+
+// floats from the even-k array to the odd-k one: the pairs, with room on both
+// sides, in whole rounds of the LDS banks
+__host__ __device__ inline int pair_stride(const Dims& d) {
+    const int nkp = (d.nz + 1) >> 1;
+    return (d.nx * d.ny * nkp + 2 * d.ny * nkp + 63) & ~63;
+}
+
+__device__ inline PairGeom pair_geom(const Dims& d) {
+    PairGeom g;
+    g.d = d;
+    g.nkp = (d.nz + 1) >> 1;
+    g.npair = d.nx * d.ny * g.nkp;
+    g.SP = d.ny * g.nkp;
+    g.OFF = pair_stride(d);
+    return g;
+}
+
+template <int KP, bool ZL>
+struct RegPairs {
+    static constexpr int NF = ZL ? 4 : 6;
+    int own0[KP];  // index of the pair's colour-0 cell; -1: no pair
+    float f[2][KP][NF], rb[2][KP];
+    float w[2][KP];  // omega / diag; 0: a cell that is never updated (none there, or no faces)
+
+    // cell of colour col of a pair with colour-0 index own0: its index in
+    // the pair arrays, and that of the cell above along k (below: one before)
+    __device__ inline void cell(const PairGeom& g, int q, int col, int& c, int& hi) const {
+        const int t = (int)threadIdx.x + q * kSmallThreads;
+        c = col == 0 ? own0[q] : 2 * t + g.OFF - own0[q];
+        hi = c == t ? t + g.OFF : t + 1;
+    }
+
+    __device__ inline void load(const PairGeom& g, const float* __restrict__ bx, const float* __restrict__ by,
+                                const float* __restrict__ bz, float omega, float* Z) {
+        const Dims& d = g.d;
+        const int SJ = d.nz, SI = d.ny * d.nz;
+#pragma unroll
+        for (int q = 0; q < KP; ++q) {
+            const int t = (int)threadIdx.x + q * kSmallThreads, tc = min(t, g.npair - 1);
+            const int row = tc / g.nkp, kp = tc - row * g.nkp;
+            const int i = row / d.ny, j = row - i * d.ny;
+            const int par = (i + j) & 1;  // k = 2 kp + par has colour 0
+            own0[q] = t < g.npair ? t + (par ? g.OFF : 0) : -1;
+#pragma unroll
+            for (int col = 0; col < 2; ++col) {
+                const int kk = 2 * kp + (par ^ col), k = min(kk, d.nz - 1);
+                const int c = row * d.nz + k;
+                const int fy = c + i * d.nz, fz = c + row;
+                float v[6] = {bx[c], bx[c + SI], by[fy], by[fy + SJ], bz[fz], bz[fz + 1]};
+                const float dg = v[0] + v[1] + v[2] + v[3] + v[4] + v[5];
+                const bool own = t < g.npair && kk < d.nz;
+                if (i == 0) v[0] = 0.0f;
+                if (i == d.nx - 1) v[1] = 0.0f;
+                if (j == 0) v[2] = 0.0f;
+                if (j == d.ny - 1) v[3] = 0.0f;
+                if (k == 0) v[4] = 0.0f;
+                if (k == d.nz - 1) v[5] = 0.0f;
+#pragma unroll
+                for (int m = 0; m < NF; ++m) f[col][q][m] = v[m];
+                if (ZL && t < g.npair) Z[t + ((par ^ col) ? g.OFF : 0)] = own ? v[4] : 0.0f;
+                w[col][q] = own && dg > 0.0f ? omega / dg : 0.0f;
+            }
+        }
+    }
+
+    // cell index (i ny + j) nz + k of a pair's cell of either colour; nz odd:
+    // the last pair of a row has no odd cell (exists = false)
+    __device__ inline int grid_cell(const PairGeom& g, int q, int col, bool& exists) const {
+        const int t = (int)threadIdx.x + q * kSmallThreads;
+        const int row = t / g.nkp, kp = t - row * g.nkp;
+        const bool odd = (own0[q] != t) != (col != 0);
+        const int k = 2 * kp + (odd ? 1 : 0);
+        exists = own0[q] >= 0 && k < g.d.nz;
+        return row * g.d.nz + k;
+    }
+
+    // the right-hand side, in cell order
+    __device__ inline void load_b(const PairGeom& g, const float* b) {
+#pragma unroll
+        for (int q = 0; q < KP; ++q)
+#pragma unroll
+            for (int col = 0; col < 2; ++col) {
+                bool ex;
+                const int c = grid_cell(g, q, col, ex);
+                rb[col][q] = ex ? b[c] : 0.0f;
+            }
+    }
+
+    // A p at a cell (stencil_vals' operations)
+    __device__ inline float Ap(const PairGeom& g, const float* P, const float* Z, int q, int col, int c, int hi,
+                               float pc) const {
+#pragma clang fp contract(off)
+        const float* p = P + c;
+        float s = f[col][q][0] * (pc - p[-g.SP]);
+        s = fmaf(f[col][q][1], pc - p[g.SP], s);
+        s = fmaf(f[col][q][2], pc - p[-g.nkp], s);
+        s = fmaf(f[col][q][3], pc - p[g.nkp], s);
+        s = fmaf(ZL ? Z[c] : f[col][q][NF - 2], pc - P[hi - 1], s);
+        s = fmaf(ZL ? Z[hi] : f[col][q][NF - 1], pc - P[hi], s);
+        return s;
+    }
+
+    __device__ inline void half(const PairGeom& g, float* P, const float* Z, int col) {
+#pragma unroll
+        for (int q = 0; q < KP; ++q) {
+            // many pairs: form the addresses anew each time (kept across the
+            // loop they spill)
+            if constexpr (KP >= 5) asm volatile("" : "+v"(own0[q]));
+            if (own0[q] < 0 || w[col][q] == 0.0f) continue;
+            int c, hi;
+            cell(g, q, col, c, hi);
+            const float pc = P[c];
+            P[c] = fmaf(rb[col][q] - Ap(g, P, Z, q, col, c, hi, pc), w[col][q], pc);
+        }
+    }
+};
+
 // ================================================================ small levels in LDS
 struct SmallArgs {
-    int s, L, pre, post, coarsest;
+    int s, L, pre, post;
+    int nreg;  // levels s .. s + nreg - 1 are held in registers (RegPairs), the rest in LDS
     float omega;
     Dims d[PF_MAX_LEVELS];
-    int off[PF_MAX_LEVELS][5];  // LDS float offsets of bx, by, bz, p, b
-    int scratch;                // LDS float offset of the residual scratch (n(s) floats)
+    int off[PF_MAX_LEVELS][5];  // LDS float offsets of bx, by, bz, p, b (register levels: p and b, not s)
+    int poff[2];                // and of the register levels' pair arrays
+    int scratch;                // LDS float offset of the residual scratch
+    const float* rf[2][3];      // the register levels' faces
+    const float* b_top;
     // global -> LDS copies at entry: segment q copies seg_len[q] floats from
-    // seg_src[q] to LDS offset seg_dst[q] (the top level's faces and b, then
-    // the coarser levels' faces and the coarsest level's matrix)
+    // seg_src[q] to LDS offset seg_dst[q] (the LDS levels' faces, b of a
+    // hierarchy without register levels, the coarsest level's matrix)
     int nseg;
-    int nseg_first;  // segments [0, nseg_first): the top level's; the rest land during its descent
     const float* seg_src[3 * PF_MAX_LEVELS + 2];
     int seg_dst[3 * PF_MAX_LEVELS + 2];
     int seg_len[3 * PF_MAX_LEVELS + 2];
     void* p_top;
     const int* done;
-    const double* cop;  // non-NULL: the coarsest level's smoother as a matrix
+    const double* cop;  // the coarsest level's smoother as a matrix
     int cop_lds;        // >= 0: LDS float offset of a staged copy of that matrix
 };
 
-constexpr int kSmallThreads = 1024;
-constexpr int kSlots = 2;  // cells of one colour per thread and level
+constexpr int kTopPairs = 2;  // pairs of cells per thread on the largest level
 
-// Size of the per-colour enumeration of a level (pairs along k).  A level
-// fits the single-workgroup V-cycle if it is at most kSmallThreads*kSlots;
-// levels of at most 64 are smoothed by one wave.
+// Pairs along k of a level.  The largest level of the single-workgroup V-cycle
+// has at most kSmallThreads * kTopPairs of them (4096 cells), so the third
+// one, the first in LDS, at most 64 cells: 32 pairs, smoothed by one wave.
 __host__ __device__ inline int colour_space(const Dims& d) { return d.nx * d.ny * ((d.nz + 1) >> 1); }
 
 // floor(t / d) for 0 <= t < 2^22 and 1 <= d, with inv = 1.0f / d: t + 1/2
@@ -1352,20 +1492,12 @@ __device__ inline float slot_Ap(const LdsLevel& v, const Slot& S, float pc) {
     return s;
 }
 
-// One half-sweep over a thread's slots: every read first, then every write
-// (cells of one colour never neighbour each other).
-__device__ inline void slots_sweep(const LdsLevel& v, const Slot (&S)[kSlots]) {
-    float nv[kSlots];
-#pragma unroll
-    for (int q = 0; q < kSlots; ++q) {
-        nv[q] = 0.0f;
-        if (S[q].c < 0) continue;
-        const float pc = v.p[S[q].c];
-        nv[q] = pc + (S[q].b - slot_Ap(v, S[q], pc)) * S[q].w;
-    }
-#pragma unroll
-    for (int q = 0; q < kSlots; ++q)
-        if (S[q].c >= 0) v.p[S[q].c] = nv[q];
+// One half-sweep of a wave's slots (cells of one colour never neighbour each
+// other, and a wave's reads are all issued before its writes).
+__device__ inline void slot_sweep(const LdsLevel& v, const Slot& S) {
+    if (S.c < 0) return;
+    const float pc = v.p[S.c];
+    v.p[S.c] = pc + (S.b - slot_Ap(v, S, pc)) * S.w;
 }
 
 __device__ inline void wave_sync() {
@@ -1381,49 +1513,121 @@ __device__ inline void wave_sync() {
 // level's descent.
 __device__ inline void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
-// The slots of both colours of one level for this thread (colour c0 first).
+// The slots of both colours of one LDS level for this thread (colour c0
+// first); the threads beyond the first wave have none.
 struct LevelSlots {
-    Slot s0[kSlots], s1[kSlots];
-    bool wave;  // smoothed by wave 0 alone
+    Slot s0, s1;
 };
 
 __device__ inline void make_level_slots(const LdsLevel& v, int c0, float omega, const Dims* dc, LevelSlots& L) {
-    L.wave = colour_space(v.d) <= 64;
-    const int nth = L.wave ? 64 : kSmallThreads;
-#pragma unroll
-    for (int q = 0; q < kSlots; ++q) {
-        const int t = threadIdx.x + q * nth;
-        const bool mine = !L.wave || threadIdx.x < 64;
-        L.s0[q].c = L.s1[q].c = -1;
-        if (mine) {
-            make_slot(v, c0, t, omega, dc, L.s0[q]);
-            make_slot(v, 1 - c0, t, omega, dc, L.s1[q]);
-        }
+    L.s0.c = L.s1.c = -1;
+    if (threadIdx.x < 64) {
+        make_slot(v, c0, threadIdx.x, omega, dc, L.s0);
+        make_slot(v, 1 - c0, threadIdx.x, omega, dc, L.s1);
     }
 }
 
 // `sweeps` red-black sweeps (colour c0 first); ends with a workgroup barrier
 __device__ inline void small_smooth(const LdsLevel& v, const LevelSlots& L, int sweeps) {
-    if (L.wave) {
-        if (threadIdx.x < 64)
-            for (int sw = 0; sw < sweeps; ++sw) {
-                slots_sweep(v, L.s0);
-                wave_sync();
-                slots_sweep(v, L.s1);
-                wave_sync();
-            }
-    } else {
+    if (threadIdx.x < 64)
         for (int sw = 0; sw < sweeps; ++sw) {
-            slots_sweep(v, L.s0);
-            lds_barrier();
-            slots_sweep(v, L.s1);
-            lds_barrier();
+            slot_sweep(v, L.s0);
+            wave_sync();
+            slot_sweep(v, L.s1);
+            wave_sync();
         }
+    lds_barrier();
+}
+
+// One register level's way down: smooth from zero (pair arrays cleared, b
+// loaded), then the residual restricted into the next level's b (cell order).
+template <int KP>
+__device__ inline void reg_descend(RegPairs<KP, false>& R, const PairGeom& g, float* P, int sweeps, float* scr,
+                                   const Dims& dc, float* bc) {
+    for (int sw = 0; sw < sweeps; ++sw) {
+        R.half(g, P, nullptr, 0);
+        lds_barrier();
+        R.half(g, P, nullptr, 1);
+        lds_barrier();
+    }
+#pragma unroll
+    for (int q = 0; q < KP; ++q)
+#pragma unroll
+        for (int col = 0; col < 2; ++col) {
+            bool ex;
+            const int gc = R.grid_cell(g, q, col, ex);
+            if (!ex) continue;
+            int c, hi;
+            R.cell(g, q, col, c, hi);
+            scr[gc] = R.rb[col][q] - R.Ap(g, P, nullptr, q, col, c, hi, P[c]);
+        }
+    lds_barrier();
+    const int nc = dc.nx * dc.ny * dc.nz;
+    const float inz = 1.0f / (float)dc.nz, iny = 1.0f / (float)dc.ny;
+    for (int t = threadIdx.x; t < nc; t += kSmallThreads) {
+        const int row = fdiv(t, inz), K = t - row * dc.nz;
+        const int I = fdiv(row, iny), J = row - I * dc.ny;
+        float acc = 0.0f;
+#pragma unroll
+        for (int x = 0; x < 2; ++x)
+#pragma unroll
+            for (int y = 0; y < 2; ++y)
+#pragma unroll
+                for (int z = 0; z < 2; ++z) acc += scr[cell_index(g.d, 2 * I + x, 2 * J + y, 2 * K + z)];
+        bc[t] = acc;
     }
     lds_barrier();
 }
 
-// The whole V-cycle below `s` in one workgroup, every level in LDS.
+// and its way up: add the parents (cell order; a pair's two cells share one),
+// smooth with colours (1,0)
+template <int KP>
+__device__ inline void reg_ascend(RegPairs<KP, false>& R, const PairGeom& g, float* P, int sweeps, const Dims& dc,
+                                  const float* pc) {
+#pragma unroll
+    for (int q = 0; q < KP; ++q) {
+        if (R.own0[q] < 0) continue;
+        const int t = (int)threadIdx.x + q * kSmallThreads;
+        const int row = t / g.nkp, kp = t - row * g.nkp;
+        const int i = row / g.d.ny, j = row - i * g.d.ny;
+        const float v = pc[cell_index(dc, i >> 1, j >> 1, kp)];
+        P[t] += v;
+        P[t + g.OFF] += v;
+    }
+    lds_barrier();
+    for (int sw = 0; sw < sweeps; ++sw) {
+        R.half(g, P, nullptr, 1);
+        lds_barrier();
+        R.half(g, P, nullptr, 0);
+        lds_barrier();
+    }
+}
+
+// p of a register level to an array in cell order
+template <int KP, typename OT>
+__device__ inline void reg_store(const RegPairs<KP, false>& R, const PairGeom& g, const float* P, OT* out) {
+#pragma unroll
+    for (int q = 0; q < KP; ++q)
+#pragma unroll
+        for (int col = 0; col < 2; ++col) {
+            bool ex;
+            const int gc = R.grid_cell(g, q, col, ex);
+            if (!ex) continue;
+            int c, hi;
+            R.cell(g, q, col, c, hi);
+            out[gc] = from_f32<OT>(P[c]);
+        }
+}
+
+// The whole V-cycle from level s down in one workgroup.  The two largest
+// levels (16^3 and 8^3 of a 128^3 grid) keep their cells' faces, b and
+// omega / diag in registers, loaded straight from memory once and used on the
+// way down and up; smaller ones are in LDS, decoded per visit.  The coarsest
+// level is a matrix product (any hierarchy that gets here has at most
+// kCoarseOpMax coarsest cells).
+// Latency of one CU bounds it.  From 16^3 down, in the solve's graphs of a
+// 128^3 / 32^3 grid: 21.8 / 19.8 us; with every level's faces staged in LDS
+// and its cells decoded on each visit 27.2 / 25.2.
 template <typename OT>
 __global__ __launch_bounds__(kSmallThreads) void k_small_vcycle(SmallArgs a) {
     extern __shared__ float lds[];
@@ -1431,42 +1635,45 @@ __global__ __launch_bounds__(kSmallThreads) void k_small_vcycle(SmallArgs a) {
     const int dn = a.done ? *a.done : 0;
     // segments straight from memory into LDS (lane l of a wave writes its
     // dword to the wave's LDS base + 4 l)
-    auto stage = [&](int q0, int q1) {
-        for (int q = q0; q < q1; ++q) {
-            const float* src = a.seg_src[q];
-            const int len = a.seg_len[q];
-            float* dst = lds + a.seg_dst[q];
-            for (int e0 = 0; e0 < len; e0 += nt)
-                if (e0 + tid < len)
-                    __builtin_amdgcn_global_load_lds(
-                        (const void*)(src + e0 + tid), (__attribute__((address_space(3))) void*)(dst + e0 + (tid & ~63)),
-                        4, 0, 0);
-        }
-    };
-    // the top level's faces and b first; the coarser levels' faces and the
-    // coarsest matrix are issued after that wait and land while the top
-    // level is smoothed (its barriers are LDS-only), waited for before
-    // their first use
-    stage(0, a.nseg_first);
-    __builtin_amdgcn_s_waitcnt(0);
-    if (dn) return;  // uniform: no workgroup barrier has been reached yet
-    stage(a.nseg_first, a.nseg);
-    bool staged = a.nseg_first >= a.nseg;
-    auto wait_staged = [&]() {
-        if (!staged) {
-            __builtin_amdgcn_s_waitcnt(0);
-            staged = true;
-        }
-    };
-    lds_barrier();
+    for (int q = 0; q < a.nseg; ++q) {
+        const float* src = a.seg_src[q];
+        const int len = a.seg_len[q];
+        float* dst = lds + a.seg_dst[q];
+        for (int e0 = 0; e0 < len; e0 += nt)
+            if (e0 + tid < len)
+                __builtin_amdgcn_global_load_lds(
+                    (const void*)(src + e0 + tid), (__attribute__((address_space(3))) void*)(dst + e0 + (tid & ~63)),
+                    4, 0, 0);
+    }
+    if (dn) {
+        __builtin_amdgcn_s_waitcnt(0);  // nothing may land in LDS after the workgroup has gone
+        return;                         // uniform: no workgroup barrier has been reached yet
+    }
     float* scr = lds + a.scratch;
+    const PairGeom g0 = pair_geom(a.d[a.s]), g1 = pair_geom(a.d[a.nreg > 1 ? a.s + 1 : a.s]);
+    float* P0 = lds + a.poff[0] + g0.SP;
+    float* P1 = lds + a.poff[1] + g1.SP;
+    RegPairs<kTopPairs, false> R0;
+    RegPairs<1, false> R1;
+    if (a.nreg > 0) {
+        R0.load(g0, a.rf[0][0], a.rf[0][1], a.rf[0][2], a.omega, nullptr);
+        R0.load_b(g0, a.b_top);
+        for (int e = tid; e < 2 * g0.OFF; e += nt) lds[a.poff[0] + e] = 0.0f;
+    }
+    if (a.nreg > 1) {
+        R1.load(g1, a.rf[1][0], a.rf[1][1], a.rf[1][2], a.omega, nullptr);
+        for (int e = tid; e < 2 * g1.OFF; e += nt) lds[a.poff[1] + e] = 0.0f;
+    }
+    __builtin_amdgcn_s_waitcnt(0);
+    lds_barrier();
     LevelSlots S;
     // descend: smooth from zero, restrict the residual (poisson.py:323-336)
-    for (int l = a.s; l < a.L - 1; ++l) {
-        if (l > a.s) {
-            wait_staged();
-            lds_barrier();
-        }
+    if (a.nreg > 0) reg_descend(R0, g0, P0, a.pre, scr, a.d[a.s + 1], lds + a.off[a.s + 1][4]);
+    if (a.nreg > 1) {
+        R1.load_b(g1, lds + a.off[a.s + 1][4]);
+        reg_descend(R1, g1, P1, a.pre, scr, a.d[a.s + 2], lds + a.off[a.s + 2][4]);
+    }
+    for (int l = a.s + a.nreg; l < a.L - 1; ++l) {
         const LdsLevel v = lds_level(a, lds, l);
         const LdsLevel c = lds_level(a, lds, l + 1);
         const int n = v.d.nx * v.d.ny * v.d.nz;
@@ -1475,23 +1682,12 @@ __global__ __launch_bounds__(kSmallThreads) void k_small_vcycle(SmallArgs a) {
         lds_barrier();
         small_smooth(v, S, a.pre);
         // residual of every fine cell into the scratch, then R = P^T
-#pragma unroll
-        for (int q = 0; q < kSlots; ++q) {
-            if (S.s0[q].c >= 0) {
-                const float pc = v.p[S.s0[q].c];
-                scr[S.s0[q].c] = S.s0[q].b - slot_Ap(v, S.s0[q], pc);
-            }
-            if (S.s1[q].c >= 0) {
-                const float pc = v.p[S.s1[q].c];
-                scr[S.s1[q].c] = S.s1[q].b - slot_Ap(v, S.s1[q], pc);
-            }
-        }
+        if (S.s0.c >= 0) scr[S.s0.c] = S.s0.b - slot_Ap(v, S.s0, v.p[S.s0.c]);
+        if (S.s1.c >= 0) scr[S.s1.c] = S.s1.b - slot_Ap(v, S.s1, v.p[S.s1.c]);
         lds_barrier();
         const int nc = c.d.nx * c.d.ny * c.d.nz;
-        const float inz = 1.0f / (float)c.d.nz, iny = 1.0f / (float)c.d.ny;
         for (int t = tid; t < nc; t += nt) {
-            const int row = fdiv(t, inz), K = t - row * c.d.nz;
-            const int I = fdiv(row, iny), J = row - I * c.d.ny;
+            const int K = t % c.d.nz, J = (t / c.d.nz) % c.d.ny, I = t / (c.d.nz * c.d.ny);
             float acc = 0.0f;
 #pragma unroll
             for (int x = 0; x < 2; ++x)
@@ -1503,15 +1699,13 @@ __global__ __launch_bounds__(kSmallThreads) void k_small_vcycle(SmallArgs a) {
         }
         lds_barrier();
     }
-    wait_staged();
-    lds_barrier();
-    // coarsest: sweeps, then remove the mean (poisson.py:325-328)
-    if (a.cop) {
-        // the same map, precomputed: p = M b (column j of M contiguous).
-        // Each output's sum is split over G groups of n threads (a
-        // contiguous range of j each; a wave reads 64 consecutive entries
-        // of one column), and the G partials are added in group order
-        // (the FP64 partials go through the scratch, 8-byte aligned).
+    // coarsest: sweeps, then the mean removed (poisson.py:325-328), as the
+    // precomputed matrix: p = M b (column j of M contiguous).  Each output's
+    // sum is split over G groups of n threads (a contiguous range of j each;
+    // a wave reads 64 consecutive entries of one column), and the G partials
+    // are added in group order (the FP64 partials go through the scratch,
+    // 8-byte aligned).
+    {
         const LdsLevel v = lds_level(a, lds, a.L - 1);
         const int n = v.d.nx * v.d.ny * v.d.nz;
         const int G = min(nt / n, 16), J = (n + G - 1) / G;
@@ -1540,79 +1734,51 @@ __global__ __launch_bounds__(kSmallThreads) void k_small_vcycle(SmallArgs a) {
             v.p[t] = (float)acc;
         }
         lds_barrier();
-    } else {
-        const LdsLevel v = lds_level(a, lds, a.L - 1);
-        const int n = v.d.nx * v.d.ny * v.d.nz;
-        for (int e = tid; e < n; e += nt) v.p[e] = 0.0f;
-        make_level_slots(v, 0, a.omega, nullptr, S);
-        __syncthreads();
-        small_smooth(v, S, a.coarsest);
-        __shared__ double sh[16];
-        double sm[1] = {0.0};
-        for (int e = tid; e < n; e += nt) sm[0] += (double)v.p[e];
-        block_sum<1>(sm, sh);
-        __shared__ float shift;
-        if (tid == 0) shift = (float)(-(sm[0] / (double)n));
-        __syncthreads();
-        for (int e = tid; e < n; e += nt) v.p[e] = v.p[e] + shift;
-        __syncthreads();
     }
     // ascend: prolong (poisson.py:178-182), smooth (colours (1,0))
-    for (int l = a.L - 2; l >= a.s; --l) {
+    for (int l = a.L - 2; l >= a.s + a.nreg; --l) {
         const LdsLevel v = lds_level(a, lds, l);
         const LdsLevel c = lds_level(a, lds, l + 1);
         make_level_slots(v, 1, a.omega, &c.d, S);
-#pragma unroll
-        for (int q = 0; q < kSlots; ++q) {
-            if (S.s0[q].c >= 0) v.p[S.s0[q].c] += c.p[S.s0[q].par];
-            if (S.s1[q].c >= 0) v.p[S.s1[q].c] += c.p[S.s1[q].par];
-        }
-        __syncthreads();
+        if (S.s0.c >= 0) v.p[S.s0.c] += c.p[S.s0.par];
+        if (S.s1.c >= 0) v.p[S.s1.c] += c.p[S.s1.par];
+        lds_barrier();
         small_smooth(v, S, a.post);
     }
-    {
+    OT* out = static_cast<OT*>(a.p_top);
+    if (a.nreg > 1) {
+        reg_ascend(R1, g1, P1, a.post, a.d[a.s + 2], lds + a.off[a.s + 2][3]);
+        reg_store(R1, g1, P1, lds + a.off[a.s + 1][3]);
+        lds_barrier();
+    }
+    if (a.nreg > 0) {
+        reg_ascend(R0, g0, P0, a.post, a.d[a.s + 1], lds + a.off[a.s + 1][3]);
+        reg_store(R0, g0, P0, out);
+    } else {
         const LdsLevel v = lds_level(a, lds, a.s);
         const int n = v.d.nx * v.d.ny * v.d.nz;
-        OT* out = static_cast<OT*>(a.p_top);
         for (int e = tid; e < n; e += nt) out[e] = from_f32<OT>(v.p[e]);
     }
 }
 
-// ================================================================ a coarsest level too large for the V-cycle above
+// ================================================================ a coarsest level by its sweeps
 // The coarsest level's `sweeps` red-black sweeps from zero and its mean
-// removal in one workgroup, for a level that does not fit k_small_vcycle
-// (a grid whose extents stop halving early: 104 x 76 x 52 ends at 26 x 19 x
-// 13, 200^3 at 25^3).  One launch per half-sweep costs about 3 us of launch
-// and memory latency for a few thousand cells, 120 times per V-cycle; here a
-// half-sweep is LDS reads and a barrier.  Each thread keeps the faces, b and
-// omega / diag of its cells in registers (KP pairs along k, one cell of each
-// colour per pair) and only the iterate is in LDS, since 5 n floats would
-// not fit.  The cells of even and of odd k are kept in two arrays, indexed by
-// pair: the cells of one colour in a row then lie next to each other, and a
-// wave's reads fall on all LDS banks (in cell order one colour uses every
-// other bank: 108 us instead of 69 at 26 x 19 x 13).  Faces on a wall are
-// given weight 0 in the sum (their neighbour is the cell itself, so their
-// flux is 0; they stay in the diagonal), so the neighbour addresses need no
-// clamps: zeros on either side of the arrays keep them inside.  ZL: the z
-// faces are in LDS too, which holds 8 pairs per thread without spilling in
-// the sweeps (a cell's high z face is the next cell's low one).
+// removal in one workgroup (RegPairs), for a level that is too large for the
+// precomputed matrix (a grid whose extents stop halving early: 96 x 72 x 120
+// ends at 12 x 9 x 15, 104 x 76 x 52 at 26 x 19 x 13, 200^3 at 25^3).  One
+// launch per half-sweep costs about 3 us of launch and memory latency, 120
+// times per V-cycle; here a half-sweep is LDS reads and a barrier.
 // FP32 faces and iterate in every precision, like k_small_vcycle; p is
 // rounded to ST once, when stored.
 // What is left is VALU issue and LDS bandwidth of one CU, 0.6 us per
-// half-sweep.  A V-cycle on the grid of twice the extents, launched
-// half-sweeps -> this: 26 x 19 x 13 365 -> 113 us, 33 x 25 x 11 371 -> 157,
-// 27 x 27 x 15 472 -> 188, 25^3 384 -> 297 (beyond 8 pairs per thread one CU
-// would be slower than the launches).
+// half-sweep of 26 x 19 x 13, and latency on the smallest: 12 x 9 x 15 takes
+// 24 us (40 from LDS with the cells decoded on each visit).  A V-cycle on the grid of twice the extents,
+// launched half-sweeps -> this: 26 x 19 x 13 365 -> 113 us, 33 x 25 x 11 371
+// -> 157, 27 x 27 x 15 472 -> 188, 25^3 384 -> 297 (beyond 8 pairs per thread
+// one CU would be slower than the launches).
 constexpr int kCoarsestPairs = 8;        // largest KP
 constexpr int kCoarsestPairsRegs = 5;    // largest KP with the z faces in registers
 constexpr int kCoarsestBytes = 156 * 1024;
-
-// floats from k_coarsest's even-k array to its odd-k one: the pairs, with
-// room on both sides, in whole rounds of the LDS banks
-__host__ __device__ inline int coarsest_stride(const Dims& d) {
-    const int nkp = (d.nz + 1) >> 1;
-    return (d.nx * d.ny * nkp + 2 * d.ny * nkp + 63) & ~63;
-}
 
 template <typename ST, int KP, bool ZL>
 __global__ __launch_bounds__(kSmallThreads) void k_coarsest(Dims d, const float* __restrict__ bx,
@@ -1623,91 +1789,38 @@ __global__ __launch_bounds__(kSmallThreads) void k_coarsest(Dims d, const float*
     extern __shared__ float lds[];
     __shared__ double sh[16];
     __shared__ float shift;
-    constexpr int NF = ZL ? 4 : 6;
     const int tid = threadIdx.x;
-    const int SJ = d.nz, SI = d.ny * d.nz, n = d.nx * SI;
-    const int nkp = (d.nz + 1) >> 1, npair = d.nx * d.ny * nkp, SP = d.ny * nkp;
-    const int OFF = coarsest_stride(d);  // the odd array behind the even one
-    float* P = lds + SP;                 // pair t: even k at P[t], odd k at P[OFF + t]
-    float* Z = lds + 2 * OFF;            // low z faces, the same layout
+    const PairGeom g = pair_geom(d);
+    const int n = d.nx * d.ny * d.nz;
+    float* P = lds + g.SP;         // pair t: even k at P[t], odd k at P[OFF + t]
+    float* Z = lds + 2 * g.OFF;    // low z faces, the same layout
     if (done && *done) return;  // uniform: no barrier has been reached yet
-    for (int e = tid; e < 2 * OFF; e += kSmallThreads) lds[e] = 0.0f;
-    if (ZL && tid == 0) Z[npair] = Z[OFF + npair] = 0.0f;
-    int own0[KP];  // index of the pair's colour-0 cell; -1: no pair
-    float f[2][KP][NF], rb[2][KP], w[2][KP];
-#pragma unroll
-    for (int q = 0; q < KP; ++q) {
-        const int t = tid + q * kSmallThreads, tc = min(t, npair - 1);
-        const int row = tc / nkp, kp = tc - row * nkp;
-        const int i = row / d.ny, j = row - i * d.ny;
-        const int par = (i + j) & 1;  // k = 2 kp + par has colour 0
-        own0[q] = t < npair ? t + (par ? OFF : 0) : -1;
-#pragma unroll
-        for (int col = 0; col < 2; ++col) {
-            const int kk = 2 * kp + (par ^ col), k = min(kk, d.nz - 1);
-            const int c = row * d.nz + k;
-            const int fy = c + i * d.nz, fz = c + row;
-            float v[6] = {bx[c], bx[c + SI], by[fy], by[fy + SJ], bz[fz], bz[fz + 1]};
-            const float dg = v[0] + v[1] + v[2] + v[3] + v[4] + v[5];
-            const bool own = t < npair && kk < d.nz;
-            if (i == 0) v[0] = 0.0f;
-            if (i == d.nx - 1) v[1] = 0.0f;
-            if (j == 0) v[2] = 0.0f;
-            if (j == d.ny - 1) v[3] = 0.0f;
-            if (k == 0) v[4] = 0.0f;
-            if (k == d.nz - 1) v[5] = 0.0f;
-#pragma unroll
-            for (int m = 0; m < NF; ++m) f[col][q][m] = v[m];
-            if (ZL && t < npair) Z[t + ((par ^ col) ? OFF : 0)] = own ? v[4] : 0.0f;
-            rb[col][q] = b[c];
-            // 0: a cell that is never updated (none there, or no faces)
-            w[col][q] = own && dg > 0.0f ? omega / dg : 0.0f;
-        }
-    }
+    for (int e = tid; e < 2 * g.OFF; e += kSmallThreads) lds[e] = 0.0f;
+    if (ZL && tid == 0) Z[g.npair] = Z[g.OFF + g.npair] = 0.0f;
+    RegPairs<KP, ZL> R;
+    R.load(g, bx, by, bz, omega, Z);
+    R.load_b(g, b);
     __syncthreads();
-    auto half = [&](auto colour) {
-        constexpr int col = decltype(colour)::value;
-#pragma unroll
-        for (int q = 0; q < KP; ++q) {
-#pragma clang fp contract(off)
-            // many pairs: form the addresses anew each time (kept across the
-            // loop they spill)
-            if constexpr (KP >= 5) asm volatile("" : "+v"(own0[q]));
-            if (own0[q] < 0 || w[col][q] == 0.0f) continue;
-            const int t = tid + q * kSmallThreads;
-            const int c = col == 0 ? own0[q] : 2 * t + OFF - own0[q];  // this cell
-            const int o = 2 * t + OFF - c;                            // the pair's other cell
-            const int hi = c == t ? o : o + 1;                        // the cells above and below along k
-            const float* p = P + c;
-            const float pc = p[0];
-            float s = f[col][q][0] * (pc - p[-SP]);
-            s = fmaf(f[col][q][1], pc - p[SP], s);
-            s = fmaf(f[col][q][2], pc - p[-nkp], s);
-            s = fmaf(f[col][q][3], pc - p[nkp], s);
-            s = fmaf(ZL ? Z[c] : f[col][q][NF - 2], pc - P[hi - 1], s);
-            s = fmaf(ZL ? Z[hi] : f[col][q][NF - 1], pc - P[hi], s);
-            P[c] = fmaf(rb[col][q] - s, w[col][q], pc);
-        }
-        __syncthreads();
-    };
     for (int sw = 0; sw < sweeps; ++sw) {
-        half(std::integral_constant<int, 0>{});
-        half(std::integral_constant<int, 1>{});
+        R.half(g, P, Z, 0);
+        __syncthreads();
+        R.half(g, P, Z, 1);
+        __syncthreads();
     }
     // everything outside the cells is still 0
     double sm[1] = {0.0};
-    for (int e = tid; e < 2 * OFF; e += kSmallThreads) sm[0] += (double)lds[e];
+    for (int e = tid; e < 2 * g.OFF; e += kSmallThreads) sm[0] += (double)lds[e];
     block_sum<1>(sm, sh);
     if (tid == 0) shift = (float)(-(sm[0] / (double)n));
     __syncthreads();
     for (int e = tid; e < n; e += kSmallThreads) {
         const int row = e / d.nz, k = e - row * d.nz;
-        pout[e] = from_f32<ST>(P[row * nkp + (k >> 1) + ((k & 1) ? OFF : 0)] + shift);
+        pout[e] = from_f32<ST>(P[row * g.nkp + (k >> 1) + ((k & 1) ? g.OFF : 0)] + shift);
     }
 }
 
 static int64_t coarsest_lds_bytes(const Dims& d, int kp) {
-    const int64_t npair = (int64_t)d.nx * d.ny * ((d.nz + 1) / 2), off = coarsest_stride(d);
+    const int64_t npair = (int64_t)d.nx * d.ny * ((d.nz + 1) / 2), off = pair_stride(d);
     return (2 * off + (kp > kCoarsestPairsRegs ? off + npair + 1 : 0)) * (int64_t)sizeof(float);
 }
 
@@ -1720,8 +1833,8 @@ static int coarsest_pairs(const Dims& d) {
 }
 
 template <typename ST, int KP>
-static int launch_coarsest_kp(const Dims& d, const pf_mg_level& lv, ST* p, int sweeps, float omega, const int* done,
-                              hipStream_t s) {
+static int launch_coarsest_kp(const Dims& d, const pf_mg_level& lv, const float* b, ST* p, int sweeps, float omega,
+                              const int* done, hipStream_t s) {
     constexpr bool ZL = KP > kCoarsestPairsRegs;
     static std::atomic<uint64_t> done_mask{0};  // devices whose LDS limit has been raised
     int dev = 0;
@@ -1732,23 +1845,23 @@ static int launch_coarsest_kp(const Dims& d, const pf_mg_level& lv, ST* p, int s
                                          hipFuncAttributeMaxDynamicSharedMemorySize, kCoarsestBytes));
         done_mask.fetch_or(bit);
     }
-    k_coarsest<ST, KP, ZL><<<1, kSmallThreads, (size_t)coarsest_lds_bytes(d, KP), s>>>(d, lv.bx, lv.by, lv.bz, lv.b, p, sweeps, omega, done);
+    k_coarsest<ST, KP, ZL><<<1, kSmallThreads, (size_t)coarsest_lds_bytes(d, KP), s>>>(d, lv.bx, lv.by, lv.bz, b, p, sweeps, omega, done);
     PF_CHECK_LAUNCH();
     return PF_OK;
 }
 
 template <typename ST>
-static int launch_coarsest(int kp, const Dims& d, const pf_mg_level& lv, ST* p, int sweeps, float omega,
+static int launch_coarsest(int kp, const Dims& d, const pf_mg_level& lv, const float* b, ST* p, int sweeps, float omega,
                            const int* done, hipStream_t s) {
     switch (kp) {
-    case 1:
-    case 2:  // levels this small are k_small_vcycle's
-    case 3: return launch_coarsest_kp<ST, 3>(d, lv, p, sweeps, omega, done, s);
-    case 4: return launch_coarsest_kp<ST, 4>(d, lv, p, sweeps, omega, done, s);
-    case 5: return launch_coarsest_kp<ST, 5>(d, lv, p, sweeps, omega, done, s);
-    case 6: return launch_coarsest_kp<ST, 6>(d, lv, p, sweeps, omega, done, s);
-    case 7: return launch_coarsest_kp<ST, 7>(d, lv, p, sweeps, omega, done, s);
-    case 8: return launch_coarsest_kp<ST, 8>(d, lv, p, sweeps, omega, done, s);
+    case 1: return launch_coarsest_kp<ST, 1>(d, lv, b, p, sweeps, omega, done, s);
+    case 2: return launch_coarsest_kp<ST, 2>(d, lv, b, p, sweeps, omega, done, s);
+    case 3: return launch_coarsest_kp<ST, 3>(d, lv, b, p, sweeps, omega, done, s);
+    case 4: return launch_coarsest_kp<ST, 4>(d, lv, b, p, sweeps, omega, done, s);
+    case 5: return launch_coarsest_kp<ST, 5>(d, lv, b, p, sweeps, omega, done, s);
+    case 6: return launch_coarsest_kp<ST, 6>(d, lv, b, p, sweeps, omega, done, s);
+    case 7: return launch_coarsest_kp<ST, 7>(d, lv, b, p, sweeps, omega, done, s);
+    case 8: return launch_coarsest_kp<ST, 8>(d, lv, b, p, sweeps, omega, done, s);
     }
     PF_REQUIRE(false, "launch_coarsest: at most 8 pairs per thread");
     return PF_OK;
@@ -2148,29 +2261,35 @@ __global__ __launch_bounds__(RT) void k_apply_A(Dims d, const float* __restrict_
 static Dims ldims(const pf_mg_level& l) { return Dims{l.nx, l.ny, l.nz}; }
 static int64_t ncell(const pf_mg_level& l) { return (int64_t)l.nx * l.ny * l.nz; }
 
-// LDS layout of the single-workgroup V-cycle from level s down: the face
-// arrays of every level back to back (one contiguous copy), then p and b of
-// every level, then a residual scratch of level s's size.
-static int64_t small_lds_floats(const pf_mg& mg, int s, int (*off)[5], int* scratch) {
+// LDS layout of the single-workgroup V-cycle from level s down: the register
+// levels' pair arrays; the face arrays of the LDS levels back to back (of the
+// coarsest one none: it is a matrix product); p and b of every level but a
+// register level s; the scratch.
+static int small_reg_levels(const pf_mg& mg, int s) { return std::min(2, mg.nlev - 1 - s); }
+
+static int64_t small_lds_floats(const pf_mg& mg, int s, int (*off)[5], int* poff, int* scratch) {
+    const int nreg = small_reg_levels(mg, s);
     int64_t o = 0;
-    for (int l = s; l < mg.nlev; ++l) {
-        const Dims d = ldims(mg.lev[l]);
-        if (off) off[l][0] = (int)o;
-        o += face_count(d, 0);
-        if (off) off[l][1] = (int)o;
-        o += face_count(d, 1);
-        if (off) off[l][2] = (int)o;
-        o += face_count(d, 2);
+    for (int r = 0; r < 2; ++r) {
+        if (poff) poff[r] = (int)o;
+        if (r < nreg) o += 2 * (int64_t)pair_stride(ldims(mg.lev[s + r]));
     }
-    for (int l = s; l < mg.nlev; ++l) {
+    for (int l = s + nreg; l < mg.nlev - 1; ++l) {
+        const Dims d = ldims(mg.lev[l]);
+        for (int q = 0; q < 3; ++q) {
+            if (off) off[l][q] = (int)o;
+            o += face_count(d, q);
+        }
+    }
+    for (int l = s + (nreg > 0 ? 1 : 0); l < mg.nlev; ++l) {
         const int64_t nc = ncell(mg.lev[l]);
         if (off) off[l][3] = (int)o;
         o += nc;
         if (off) off[l][4] = (int)o;
         o += nc;
     }
-    // the scratch: the top level's residual, and the FP64 partials of the
-    // coarsest level's matrix product (8-byte aligned, at most kSmallThreads)
+    // the scratch: a level's residual, and the FP64 partials of the coarsest
+    // level's matrix product (8-byte aligned, at most kSmallThreads)
     o = (o + 1) & ~(int64_t)1;
     if (scratch) *scratch = (int)o;
     return o + std::max<int64_t>(ncell(mg.lev[s]), 2 * kSmallThreads);
@@ -2460,7 +2579,8 @@ static int vcycle(const pf_mg& mg, const float* r0, ST* z0, const int* done, con
                                                               mg.lev[l + 1].b, done, l == 0 ? bscale : nullptr);
         PF_CHECK_LAUNCH();
     }
-    if (sm < L) {
+    const bool swept = sm >= L - 1 && !use_coarse_op(mg);  // the coarsest level by its sweeps
+    if (sm < L && !swept) {
         int rc0 = ensure_small_lds();
         if (rc0) return rc0;
         SmallArgs a;
@@ -2468,42 +2588,42 @@ static int vcycle(const pf_mg& mg, const float* r0, ST* z0, const int* done, con
         a.L = L;
         a.pre = mg.pre;
         a.post = mg.post;
-        a.coarsest = mg.coarsest;
+        a.nreg = small_reg_levels(mg, sm);
         a.omega = mg.omega;
         for (int l = sm; l < L; ++l) a.d[l] = ldims(mg.lev[l]);
-        const int64_t nf = small_lds_floats(mg, sm, a.off, &a.scratch);
+        const int64_t nf = small_lds_floats(mg, sm, a.off, a.poff, &a.scratch);
+        for (int r = 0; r < 2; ++r) {
+            const pf_mg_level& v = mg.lev[std::min(sm + r, L - 1)];
+            a.rf[r][0] = v.bx;
+            a.rf[r][1] = v.by;
+            a.rf[r][2] = v.bz;
+        }
+        a.b_top = B(sm);
         a.nseg = 0;
         auto seg = [&](const float* src, int dst, int64_t n) {
             a.seg_src[a.nseg] = src;
             a.seg_dst[a.nseg] = dst;
             a.seg_len[a.nseg++] = (int)n;
         };
-        // the top level's faces and b, then the coarser levels' faces
-        for (int l = sm; l < L; ++l) {
-            const Dims d = a.d[l];
-            seg(mg.lev[l].bx, a.off[l][0], face_count(d, 0));
-            seg(mg.lev[l].by, a.off[l][1], face_count(d, 1));
-            seg(mg.lev[l].bz, a.off[l][2], face_count(d, 2));
-            if (l == sm) {
-                seg(B(sm), a.off[sm][4], ncell(mg.lev[sm]));
-                a.nseg_first = a.nseg;
-            }
+        for (int l = sm + a.nreg; l < L - 1; ++l) {
+            seg(mg.lev[l].bx, a.off[l][0], face_count(a.d[l], 0));
+            seg(mg.lev[l].by, a.off[l][1], face_count(a.d[l], 1));
+            seg(mg.lev[l].bz, a.off[l][2], face_count(a.d[l], 2));
         }
+        if (a.nreg == 0) seg(B(sm), a.off[sm][4], ncell(mg.lev[sm]));
         a.done = done;
-        a.cop = use_coarse_op(mg) ? static_cast<CGState*>(mg.scalars)->coarse_op : nullptr;
+        a.cop = static_cast<CGState*>(mg.scalars)->coarse_op;
+        // stage the coarsest level's matrix too when it fits the LDS budget:
+        // its loads then overlap the others instead of costing round trips of
+        // their own in the middle of the V-cycle
         a.cop_lds = -1;
         int64_t nlds = nf;
-        if (a.cop) {
-            // stage the coarsest level's matrix too when it fits the LDS
-            // budget: its loads then overlap the faces' instead of costing
-            // round trips of their own in the middle of the V-cycle
-            const int64_t nc = ncell(mg.lev[L - 1]);
-            const int64_t off = (nf + 3) & ~(int64_t)3;  // 16-byte aligned
-            if ((off + 2 * nc * nc) * (int64_t)sizeof(float) <= kSmallMaxBytes) {
-                a.cop_lds = (int)off;
-                seg(reinterpret_cast<const float*>(a.cop), (int)off, 2 * nc * nc);
-                nlds = off + 2 * nc * nc;
-            }
+        const int64_t ncop = ncell(mg.lev[L - 1]);
+        const int64_t cop_off = (nf + 3) & ~(int64_t)3;  // 16-byte aligned
+        if ((cop_off + 2 * ncop * ncop) * (int64_t)sizeof(float) <= kSmallMaxBytes) {
+            a.cop_lds = (int)cop_off;
+            seg(reinterpret_cast<const float*>(a.cop), (int)cop_off, 2 * ncop * ncop);
+            nlds = cop_off + 2 * ncop * ncop;
         }
         const size_t lds = (size_t)nlds * sizeof(float);
         if (sm == 0) {
@@ -2515,14 +2635,21 @@ static int vcycle(const pf_mg& mg, const float* r0, ST* z0, const int* done, con
         }
         PF_CHECK_LAUNCH();
     } else {
-        // coarsest level out of HBM: sweeps, then mean removal (in one
-        // workgroup where it fits; a one-level hierarchy's level 0 has its
-        // own right-hand side scale and residual test and stays launched)
+        // the coarsest level's sweeps, then mean removal, in one workgroup
+        // where it fits (a one-level hierarchy that is too large for the
+        // single-workgroup V-cycle has its own right-hand side scale and
+        // residual test and stays launched)
         const int l = L - 1;
-        const int kp = L > 1 ? coarsest_pairs(ldims(mg.lev[l])) : 0;
+        const int kp = L > 1 || sm == 0 ? coarsest_pairs(ldims(mg.lev[l])) : 0;
         if (kp) {
-            cur[l] = P(l);
-            const int rc = launch_coarsest<ST>(kp, ldims(mg.lev[l]), mg.lev[l], cur[l], mg.coarsest, mg.omega, done, s);
+            const Dims d = ldims(mg.lev[l]);
+            int rc;
+            if (l == sm && l > 0) {  // an FP32 level in every precision, as k_small_vcycle's
+                rc = launch_coarsest<float>(kp, d, mg.lev[l], B(l), mg.lev[l].p, mg.coarsest, mg.omega, done, s);
+            } else {
+                cur[l] = P(l);
+                rc = launch_coarsest<ST>(kp, d, mg.lev[l], B(l), cur[l], mg.coarsest, mg.omega, done, s);
+            }
             if (rc) return rc;
         } else {
             int rc = smooth(l, mg.coarsest, false, true);
@@ -3084,9 +3211,9 @@ PF_API int pf_mg_setup(pf_mg* mg) {
     int sm = mg->nlev;
     for (int l = mg->nlev - 1; l >= 0; --l) {
         const int64_t nc = (int64_t)mg->lev[l].nx * mg->lev[l].ny * mg->lev[l].nz;
-        const int64_t bytes = small_lds_floats(*mg, l, nullptr, nullptr) * (int64_t)sizeof(float);
+        const int64_t bytes = small_lds_floats(*mg, l, nullptr, nullptr, nullptr) * (int64_t)sizeof(float);
         const Dims d{mg->lev[l].nx, mg->lev[l].ny, mg->lev[l].nz};
-        if (nc <= kSmallMaxCells && bytes <= kSmallMaxBytes && colour_space(d) <= kSmallThreads * kSlots)
+        if (nc <= kSmallMaxCells && bytes <= kSmallMaxBytes && colour_space(d) <= kSmallThreads * kTopPairs)
             sm = l;
         else
             break;

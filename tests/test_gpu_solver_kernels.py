@@ -23,17 +23,17 @@ def _beta(res, rng, walls):
     return out
 
 
-def _vcycle_error(pf, res, precision, walls, pre=3, post=3):
+def _vcycle_error(pf, res, precision, walls, pre=3, post=3, min_dim=4):
     rng = np.random.default_rng(17)
     beta = _beta(res, rng, walls)
     r = rng.standard_normal(res).astype(np.float32)
     r -= r.mean()
     g = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()  # noqa: E731
-    solver = pf.MGPCG(res, "cuda:0", pre=pre, post=post, precision=precision)
+    solver = pf.MGPCG(res, "cuda:0", pre=pre, post=post, precision=precision, min_dim=min_dim)
     solver.build_hierarchy(*[g(b) for b in beta])
     z = torch.zeros(res, device="cuda")
     solver.precondition(g(r), z)
-    o = O.MGPCGOracle(res, pre=pre, post=post)
+    o = O.MGPCGOracle(res, pre=pre, post=post, min_dim=min_dim)
     o.build_hierarchy(*beta)
     ref = o.precondition(r.astype(np.float64))
     return float(np.linalg.norm(z.cpu().numpy() - ref) / np.linalg.norm(ref))
@@ -59,3 +59,42 @@ def test_coarsest_level_in_one_workgroup_16_bit(pf, precision, bound):
     rounding (2^-9, 2^-12), one per smoothing pass of the level above."""
     print(f"[gpu] coarsest 16-bit {precision}", flush=True)
     assert _vcycle_error(pf, (54, 38, 26), precision, False) < bound
+
+
+# one workgroup from the largest level it takes down: register levels only,
+# LDS levels below them (min_dim 1), one register level, a coarsest level by
+# its sweeps (729 cells), by its matrix alone, and a whole grid by its sweeps
+@pytest.mark.parametrize("res,min_dim", [((16, 16, 16), 4), ((32, 32, 32), 1), ((16, 16, 16), 1), ((64, 8, 8), 2),
+                                         ((24, 12, 20), 4), ((18, 18, 18), 4), ((7, 8, 9), 4), ((11, 13, 9), 4),
+                                         ((128, 16, 8), 4)])
+@pytest.mark.parametrize("walls", [False, True])
+@pytest.mark.parametrize("pre,post", [(3, 3), (1, 2)])
+def test_small_hierarchy_in_one_workgroup(pf, res, min_dim, walls, pre, post):
+    """FP32 against FP64 over a V-cycle, the bound of the tests above."""
+    print(f"[gpu] small hierarchy {res} min_dim={min_dim} walls={walls} {pre}+{post}", flush=True)
+    assert _vcycle_error(pf, res, "fp32", walls, pre, post, min_dim) < 2e-5
+
+
+# 8 x 8 x 32 tiles: whole, cut along every axis; 1152 tiles (inner products of
+# a solve on the last sweep); 8 x 8 x 64 tiles beside them
+@pytest.mark.parametrize("res,precision", [((96, 88, 96), "fp32"), ((100, 90, 84), "fp32"), ((104, 120, 100), "bf16"),
+                                           ((192, 128, 96), "fp16"), ((128, 64, 192), "bf16")])
+def test_sweep_tiles_equal_half_sweeps(pf, res, precision):
+    """The fused sweeps of every tile shape against two half-sweep launches
+    per sweep, bit for bit, over a V-cycle and a solve of 6 iterations (the
+    inner products in a kernel of their own in both)."""
+    print(f"[gpu] sweep tiles {res} {precision}", flush=True)
+    rng = np.random.default_rng(3)
+    g = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()  # noqa: E731
+    beta = [g(b) for b in _beta(res, rng, False)]
+    r = g(rng.standard_normal(res).astype(np.float32))
+    out = []
+    for fused in (True, False):
+        s = pf.MGPCG(res, "cuda:0", pre=2, post=2, precision=precision, fused_smoother=fused, fold_dots=False)
+        s.build_hierarchy(*beta)
+        z, p = torch.zeros_like(r), torch.zeros_like(r)
+        s.precondition(r, z)
+        it, rel = s.solve(r, p, tol=1e-30, max_iter=6)
+        out.append((z.cpu().numpy(), p.cpu().numpy(), it, rel))
+    assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
+    assert out[0][2:] == out[1][2:]
