@@ -17,7 +17,7 @@ MAX_LEVELS = 16
 TILE = 8
 
 PH_VEL_FROM_MOM, PH_PHASE, PH_ZERO, PH_STAR, PH_GRAVITY, PH_RHS, PH_TAGS_IN = 1, 2, 4, 8, 16, 32, 64
-GA_G2P, GA_ADVECT, GA_REFLECT, GA_SOLIDS = 1, 2, 4, 8
+GA_G2P, GA_ADVECT, GA_REFLECT, GA_SOLIDS, GA_STATE = 1, 2, 4, 8, 16
 
 P = ctypes.c_void_p
 F3 = P * 3

@@ -856,27 +856,20 @@ __device__ inline void finish_particle(const G2PArgs& a, int64_t p, float x, flo
     a.pv[3 * p + 2] = vz;
 }
 
-// At most 5 waves per SIMD: the kernel is bound by its 60 row-pair gathers
-// per particle, and more resident waves evict each other's rows from L1/L2
-// (measured at 128^3 x 27 ppc: 7 waves/SIMD is 10 % slower than 5).
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 5))) void k_g2p_advect(G2PArgs a) {
-    const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= a.n) return;
-    bool liquid, active, dead;
-    if (a.pflag) {
-        const uint8_t fl = a.pflag[p];
-        liquid = fl & 1;
-        active = fl & 2;
-        dead = fl & 4;
-    } else {
-        const int st = a.pstate[p];
-        liquid = a.ptype[p] == 1;
-        active = st == 0;
-        dead = st == 2;
-    }
-    if (dead) return;
+// state of a particle: 0 FLIP, 1 droplet, 2 dead
+__device__ inline int particle_state(const G2PArgs& a, int64_t p) {
+    if (!a.pflag) return a.pstate[p];
+    const uint8_t fl = a.pflag[p];
+    return (fl & 2) ? 0 : ((fl & 4) ? 2 : 1);
+}
+
+// One particle through the global fields; vx, vy, vz: its velocity after.
+// Dead particles stay as they are, droplets get the walls and solids only.
+__device__ inline void g2p_advect_particle(const G2PArgs& a, int64_t p, int state, float& vx, float& vy, float& vz) {
+    if (state == 2) return;
+    const bool liquid = a.pflag ? (a.pflag[p] & 1) : a.ptype[p] == 1, active = state == 0;
     float x = a.px[3 * p], y = a.px[3 * p + 1], z = a.px[3 * p + 2];
-    float vx = a.pv[3 * p], vy = a.pv[3 * p + 1], vz = a.pv[3 * p + 2];
+    vx = a.pv[3 * p], vy = a.pv[3 * p + 1], vz = a.pv[3 * p + 2];
     const Dims d = a.d;
     const bool g2p = active && (a.flags & PF_GA_G2P);
     const bool adv = active && (a.flags & PF_GA_ADVECT);
@@ -925,6 +918,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 5))) voi
         z = fminf(fmaxf(z, a.lo[2]), a.hi[2]);
     }
     finish_particle(a, p, x, y, z, vx, vy, vz);
+}
+
+// At most 5 waves per SIMD: the kernel is bound by its 60 row-pair gathers
+// per particle, and more resident waves evict each other's rows from L1/L2
+// (measured at 128^3 x 27 ppc: 7 waves/SIMD is 10 % slower than 5).
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 5))) void k_g2p_advect(G2PArgs a) {
+    const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (p >= a.n) return;
+    float vx, vy, vz;
+    g2p_advect_particle(a, p, particle_state(a, p), vx, vy, vz);
 }
 
 // Per-particle terms of the CFL speed and the P2G fixed-point bounds: |v|,
@@ -1091,6 +1094,11 @@ __device__ inline void stage_fields(float* box, const G2PArgs& a, bool g2p, bool
 
 // bounds (optional, with pmass): the CFL speed and P2G bounds of the
 // particles after the step, as pf_max_speed would compute them next step.
+// STATE (PF_GA_STATE): states may have changed since the binning (the droplet
+// stage between G2P and advection), so each particle's is read: the advection
+// of 22.4M particles takes 480 us from the tiles, 600 through the global
+// fields, and leaves the bounds.
+template <bool STATE>
 __global__ __launch_bounds__(kG2PThreads) void k_g2p_tiled(G2PArgs a, const int* __restrict__ perm,
                                                            const int* __restrict__ start, int ntx, int nty,
                                                            int ntz, const float* __restrict__ pmass,
@@ -1113,23 +1121,31 @@ __global__ __launch_bounds__(kG2PThreads) void k_g2p_tiled(G2PArgs a, const int*
     int s = s0 + (int)threadIdx.x;
     int64_t pn = 0;
     bool liq_n = false;
+    int st_n = 0;
     float xn = 0.f, yn = 0.f, zn = 0.f, vxn = 0.f, vyn = 0.f, vzn = 0.f;
     if (s < s1) {
         pn = perm[s];
         liq_n = a.pflag ? (a.pflag[pn] & 1) : (a.ptype[pn] == 1);
+        if (STATE) st_n = particle_state(a, pn);
         xn = a.px[3 * pn], yn = a.px[3 * pn + 1], zn = a.px[3 * pn + 2];
         vxn = a.pv[3 * pn], vyn = a.pv[3 * pn + 1], vzn = a.pv[3 * pn + 2];
     }
     for (; s < s1; s += kG2PThreads) {
         const int64_t p = pn;
         const bool liquid = liq_n;
+        const int st = st_n;
         float x = xn, y = yn, z = zn;
         float vx = vxn, vy = vyn, vz = vzn;
         if (s + kG2PThreads < s1) {
             pn = perm[s + kG2PThreads];
             liq_n = a.pflag ? (a.pflag[pn] & 1) : (a.ptype[pn] == 1);
+            if (STATE) st_n = particle_state(a, pn);
             xn = a.px[3 * pn], yn = a.px[3 * pn + 1], zn = a.px[3 * pn + 2];
             vxn = a.pv[3 * pn], vyn = a.pv[3 * pn + 1], vzn = a.pv[3 * pn + 2];
+        }
+        if (STATE && st != 0) {
+            if (st == 1) finish_particle(a, p, x, y, z, vx, vy, vz);
+            continue;
         }
         const float* fk = liquid ? box + 6 * GB3 : box;                 // RK3 field in LDS
         const float* const* gk = liquid ? a.vel_liq : a.vel;            // and in HBM
@@ -1217,26 +1233,29 @@ __global__ __launch_bounds__(kG2PThreads) void k_g2p_tiled(G2PArgs a, const int*
     }
 }
 
-// Particles outside the bins (pstate != 0 and not dead, i.e. droplets) after
-// the tiled pass: wall reflection and solids only, as in the per-particle
-// kernel.  Exits at once when the bins held every particle.
-__global__ __launch_bounds__(256) void k_g2p_unbinned(G2PArgs a, const int* __restrict__ n_binned) {
-    if (*n_binned == a.n) return;
-    for (int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; p < a.n;
-         p += (int64_t)gridDim.x * blockDim.x) {
-        bool active, dead;
-        if (a.pflag) {
-            const uint8_t fl = a.pflag[p];
-            active = fl & 2;
-            dead = fl & 4;
-        } else {
-            const int st = a.pstate[p];
-            active = st == 0;
-            dead = st == 2;
-        }
-        if (active || dead) continue;
-        float vx = a.pv[3 * p], vy = a.pv[3 * p + 1], vz = a.pv[3 * p + 2];
-        finish_particle(a, p, a.px[3 * p], a.px[3 * p + 1], a.px[3 * p + 2], vx, vy, vz);
+// The particles outside the bins (the last of the permutation) after the tiled
+// pass, as the per-particle kernel treats them: droplets get wall reflection
+// and solids only, and (PF_GA_STATE) one that has become a FLIP particle since
+// the binning is advected through the global fields and counts for the bounds.
+__global__ __launch_bounds__(256) void k_g2p_unbinned(G2PArgs a, const int* __restrict__ perm,
+                                                      const int* __restrict__ n_binned,
+                                                      const float* __restrict__ pmass, float* __restrict__ bounds) {
+    const int64_t nb = *n_binned;
+    if (nb == a.n) return;
+    const bool later = a.flags & PF_GA_STATE;
+    SpeedBounds sb;
+    for (int64_t q = nb + (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < a.n;
+         q += (int64_t)gridDim.x * blockDim.x) {
+        const int64_t p = perm[q];
+        const int st = particle_state(a, p);
+        if (st == 0 && !later) continue;
+        float vx, vy, vz;
+        g2p_advect_particle(a, p, st, vx, vy, vz);
+        if (st == 0 && bounds) sb.add(vx, vy, vz, pmass[p]);
+    }
+    if (later && bounds) {
+        __shared__ float sh[4];
+        sb.flush(bounds, sh);
     }
 }
 
@@ -1563,13 +1582,18 @@ PF_API int pf_g2p_advect_binned(const pf_g2p_args* args, const int32_t* perm, co
         const int rc = fill_u32(bounds_out, 3, 0u, S(stream));
         if (rc) return rc;
     }
-    k_g2p_tiled<<<(unsigned)nt, kG2PThreads, 0, S(stream)>>>(a, perm, cell_start, g.ntx, g.nty, g.ntz, pmass,
-                                                             bounds_out);
+    if (in.flags & PF_GA_STATE)
+        k_g2p_tiled<true><<<(unsigned)nt, kG2PThreads, 0, S(stream)>>>(a, perm, cell_start, g.ntx, g.nty, g.ntz,
+                                                                       pmass, bounds_out);
+    else
+        k_g2p_tiled<false><<<(unsigned)nt, kG2PThreads, 0, S(stream)>>>(a, perm, cell_start, g.ntx, g.nty, g.ntz,
+                                                                        pmass, bounds_out);
     PF_CHECK_LAUNCH();
-    // particles outside the bins (droplets): reflection and solids only
-    if (in.flags & (PF_GA_REFLECT | PF_GA_SOLIDS)) {
+    // particles outside the bins
+    if (in.flags & (PF_GA_REFLECT | PF_GA_SOLIDS | PF_GA_STATE)) {
         const int64_t nb = cdiv(in.n, 256);
-        k_g2p_unbinned<<<(unsigned)(nb < 2048 ? nb : 2048), 256, 0, S(stream)>>>(a, n_active);
+        k_g2p_unbinned<<<(unsigned)(nb < 2048 ? nb : 2048), 256, 0, S(stream)>>>(a, perm, n_active, pmass,
+                                                                                 bounds_out);
         PF_CHECK_LAUNCH();
     }
     return PF_OK;

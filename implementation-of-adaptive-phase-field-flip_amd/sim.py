@@ -357,8 +357,12 @@ class Simulator:
             a = self._g2p_args(_lib.GA_G2P, dt)
             _lib.call("pf_g2p_advect_binned", ctypes.byref(a), *bins, None, None, _lib.stream())
             self._launch_droplets(dt)
-            a = self._g2p_args(_lib.GA_ADVECT | _lib.GA_REFLECT, dt)
-            _lib.call("pf_g2p_advect", ctypes.byref(a), _lib.stream())
+            # the FLIP particles are still where they were binned, but the
+            # stage has changed states
+            a = self._g2p_args(_lib.GA_ADVECT | _lib.GA_REFLECT | _lib.GA_STATE, dt)
+            _lib.call("pf_g2p_advect_binned", ctypes.byref(a), *bins, _lib.ptr(self.pmass),
+                      _lib.ptr(self._bounds), _lib.stream())
+            self._bounds_token = self._bounds_key()
         else:
             # the same pass leaves the next step's CFL / P2G bounds
             a = self._g2p_args(_lib.GA_G2P | _lib.GA_ADVECT | _lib.GA_REFLECT, dt)

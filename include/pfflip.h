@@ -316,6 +316,7 @@ int pf_extrapolate(float* const vel[3], const int32_t* is_liquid, float* const v
 #define PF_GA_ADVECT 2
 #define PF_GA_REFLECT 4
 #define PF_GA_SOLIDS 8
+#define PF_GA_STATE 16 /* pf_g2p_advect_binned only, see there */
 
 typedef struct pf_g2p_args {
     float* px;
@@ -337,9 +338,11 @@ int pf_g2p_advect(const pf_g2p_args* args, pf_stream_t stream);
 
 /* The same stages for particles binned by pf_bin_sort at their current
  * positions (perm, cell_start, n_active from that call; pstate unchanged
- * since): one workgroup per 8^3 tile samples LDS copies of the tile's face
- * fields, then particles outside the bins (pstate 1) get the reflection /
- * solids part.  Results equal pf_g2p_advect's.  If bounds_out is non-NULL
+ * since, or with PF_GA_STATE read anew per particle: the droplet stage may
+ * come between): one workgroup per 8^3 tile samples LDS copies of the tile's
+ * face fields, then particles outside the bins (pstate 1) get the reflection /
+ * solids part (with PF_GA_STATE all of it if they have become FLIP particles).
+ * Results equal pf_g2p_advect's.  If bounds_out is non-NULL
  * (then pmass is required) it receives what pf_max_speed(pv, pmass, pstate)
  * returns after the call, computed from the updated particles in the same
  * pass.  Replaces the same reference kernels (kernels.py:468-549,552-564,
