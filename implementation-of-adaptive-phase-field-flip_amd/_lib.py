@@ -176,6 +176,10 @@ SIGNATURES = {
     "pf_msbg_coarse_op": (ctypes.c_int, [ctypes.POINTER(MsbgGrid), P, P, I32, F32, P, P]),
     "pf_msbg_coarse_apply": (ctypes.c_int, [P, P, P, I32, P]),
     "pf_msbg_coarsest_smooth": (ctypes.c_int, [ctypes.POINTER(MsbgGrid), P, P, P, P, I32, F32, P]),
+    "pf_msbg_rows_bytes": (ctypes.c_size_t, [I32]),
+    "pf_msbg_rows_build": (ctypes.c_int, [ctypes.POINTER(MsbgGrid), P, P, P, P]),
+    "pf_msbg_rows_smooth": (ctypes.c_int, [ctypes.POINTER(MsbgGrid), P, P, P, P, I32, I32, I32, F32, P]),
+    "pf_msbg_rows_apply": (ctypes.c_int, [ctypes.POINTER(MsbgGrid), P, P, P, P, P]),
     "pf_msbg_coarsen_beta": (ctypes.c_int, [ctypes.POINTER(MsbgGrid), ctypes.POINTER(MsbgGrid), P, P, P]),
     "pf_msbg_restrict": (ctypes.c_int, [ctypes.POINTER(MsbgGrid), ctypes.POINTER(MsbgGrid), P, P, P]),
     "pf_msbg_prolong_add": (ctypes.c_int, [ctypes.POINTER(MsbgGrid), ctypes.POINTER(MsbgGrid), P, P, P]),

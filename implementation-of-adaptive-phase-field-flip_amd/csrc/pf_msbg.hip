@@ -766,6 +766,280 @@ __global__ __launch_bounds__(256) void k_vec_jacobi(const float* __restrict__ r,
     }
 }
 
+// ------------------------------------------------------------------ stored rows
+// The couplings of every cell as a table, built once per set of face
+// coefficients.  Walking the block structure is a chain of five dependent
+// loads (cell -> block -> neighbour block -> its offset -> value) and some 300
+// instructions per cell, and a solve does it 24 times per level and V-cycle
+// with the same result; from the table it is one load and one gather.
+// Per half-sweep: 1.4M cells 19.0 -> 12.1 us (bound by reading 48 bytes of rows
+// per cell, 5 TB/s in all), 205k 8.4 -> 4.1, 32k 6.6 -> 3.1, 25k 8.1 -> 3.5
+// (bound by the launch); A p at 1.4M cells 28 -> 17.6 us; the table takes 48 us
+// there and 8 at 32k cells.
+//
+// Cells 2t and 2t + 1 form pair t.  A pair with one cell of each colour keeps
+// its colour-c row at position c H + t (H pairs), so that a half-sweep reads
+// its colour's half of the table only, without gaps; any other pair keeps cell
+// 2t + s at s H + t.  A row's first kRowIn couplings stand in `in` (entry k of
+// all positions is contiguous); rows with more (a cell facing finer ones) are
+// marked by bit 31 of the last and keep the rest in `more`, in order of arrival
+// (which changes no result).  A coarse cell has 3 couplings more than faces for
+// each finer block it faces, and a block of (2 m)^3 cells is faced by at most
+// 6 m^2 coarser cells, so 18 m^2 <= 9/4 (2 m)^3 bounds `more`.  Same couplings,
+// same order and same arithmetic as the kernels without the table.
+constexpr int kRowIn = 6;
+
+struct MRows {
+    int2* in;    // [kRowIn][2 H] (coefficient bits, neighbour)
+    int2* more;  // [cap], cap = 9/4 of the cells
+    int2* ext;   // [2 H] (first of `more`, count); set for marked rows
+    float* d;    // [2 H] sum of the couplings
+    unsigned* used;  // of `more`
+    uint8_t* code;  // [H] colours of cells 2t (bit 0) and 2t + 1 (bit 1)
+    int H;
+    unsigned cap;
+};
+
+inline size_t mrows_layout(int ncells, char* base, MRows* r) {
+    const size_t H = ((size_t)ncells + 1) / 2, cap = (size_t)ncells * 9 / 4;
+    size_t o = 0;
+    const auto take = [&](size_t bytes) {
+        char* q = base ? base + o : nullptr;
+        o += (bytes + 15) & ~(size_t)15;
+        return q;
+    };
+    MRows m;
+    m.in = reinterpret_cast<int2*>(take(kRowIn * 2 * H * sizeof(int2)));
+    m.more = reinterpret_cast<int2*>(take(cap * sizeof(int2)));
+    m.ext = reinterpret_cast<int2*>(take(2 * H * sizeof(int2)));
+    m.d = reinterpret_cast<float*>(take(2 * H * sizeof(float)));
+    m.used = reinterpret_cast<unsigned*>(take(sizeof(unsigned)));
+    m.code = reinterpret_cast<uint8_t*>(take(H));
+    m.H = (int)H;
+    m.cap = (unsigned)cap;
+    if (r) *r = m;
+    return o;
+}
+
+__device__ inline int cell_colour(const int4 o) { return ((o.x >> o.w) + (o.y >> o.w) + (o.z >> o.w)) & 1; }
+
+// position of cell 2t + s
+__device__ inline int row_pos(int code, int s, int t, int H) {
+    const int half = (code == 1 || code == 2) ? ((code >> s) & 1) : s;
+    return half * H + t;
+}
+
+__global__ __launch_bounds__(256) void k_msbg_rows(MGrid g, const float* __restrict__ bface, MRows r,
+                                                   float* __restrict__ diag) {
+    const int a = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+    if (a >= g.ncells) return;
+    BlockRef br;
+    const int4 o = origin_ref(g, a, br);
+    const int t = a >> 1, s = a & 1, c = cell_colour(o);
+    // (the missing partner of an odd last cell counts as the other colour)
+    const int cp = (a ^ 1) < g.ncells ? cell_colour(origin(g, a ^ 1)) : 1 - c;
+    const int code = s ? (cp | (c << 1)) : (c | (cp << 1));
+    const int pos = row_pos(code, s, t, r.H);
+    if (s == 0) r.code[t] = (uint8_t)code;
+    const size_t W = 2 * (size_t)r.H;
+    int k = 0;
+    int2 last = make_int2(0, a);
+    float sum = 0.0f;
+    for_each_coupling_from(g, bface, a, o, br, [&](int nb, float w) {
+        sum += w;
+        if (k < kRowIn) {
+            last = make_int2(__float_as_int(w), nb);
+            if (k < kRowIn - 1) r.in[k * W + pos] = last;
+        }
+        ++k;
+    });
+    diag[a] = sum;
+    r.d[pos] = sum;
+    for (int q = k; q < kRowIn - 1; ++q) r.in[q * W + pos] = make_int2(0, a);
+    if (k < kRowIn) last = make_int2(0, a);
+    if (k > kRowIn) {
+        const unsigned cnt = k - kRowIn, at = atomicAdd(r.used, cnt);
+        if (at + cnt <= r.cap) {
+            r.ext[pos] = make_int2((int)at, (int)cnt);
+            last.y |= (int)0x80000000;
+            k = 0;
+            for_each_coupling_from(g, bface, a, o, br, [&](int nb, float w) {
+                if (k >= kRowIn) r.more[at + k - kRowIn] = make_int2(__float_as_int(w), nb);
+                ++k;
+            });
+        }
+    }
+    r.in[(kRowIn - 1) * W + pos] = last;
+}
+
+// the couplings past the first kRowIn added to acc
+template <class V>
+__device__ inline float row_rest(const MRows& r, int pos, float pa, const V* p, float acc) {
+    const int2 e = r.ext[pos];
+    for (int q = 0; q < e.y; ++q) {
+        const int2 m = r.more[e.x + q];
+        acc += __int_as_float(m.x) * (pa - p[m.y]);
+    }
+    return acc;
+}
+
+// sum_f T_f (p_A - p_B) of cell a at position pos
+__device__ inline float row_acc(const MRows& r, int pos, float pa, const float* __restrict__ p) {
+    const size_t W = 2 * (size_t)r.H;
+    int2 e[kRowIn];
+#pragma unroll
+    for (int k = 0; k < kRowIn; ++k) e[k] = r.in[k * W + pos];
+    const bool rest = e[kRowIn - 1].y < 0;
+    e[kRowIn - 1].y &= 0x7fffffff;
+    float q[kRowIn];
+#pragma unroll
+    for (int k = 0; k < kRowIn; ++k) q[k] = p[e[k].y];
+    float acc = 0.0f;
+#pragma unroll
+    for (int k = 0; k < kRowIn; ++k) acc += __int_as_float(e[k].x) * (pa - q[k]);
+    if (rest) acc = row_rest(r, pos, pa, p, acc);
+    return acc;
+}
+
+// One half-sweep, a pair per thread; ZERO: pin is all zeros and not read (the
+// first half-sweep of a V-cycle level).
+template <bool ZERO>
+__global__ __launch_bounds__(256) void k_msbg_rows_sweep(MRows r, int n, const float* __restrict__ pin,
+                                                         float* __restrict__ pout, const float* __restrict__ b,
+                                                         int colour, float omega) {
+    const int t = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+    if (t >= r.H) return;
+    const int code = r.code[t];
+    const bool two = 2 * t + 1 < n;
+    float v[2] = {0.0f, 0.0f};
+    if (!ZERO) {
+        if (two) {
+            const float2 w = reinterpret_cast<const float2*>(pin)[t];
+            v[0] = w.x;
+            v[1] = w.y;
+        } else {
+            v[0] = pin[2 * t];
+        }
+    }
+    const auto update = [&](int s, int pos, float x) {
+        const int a = 2 * t + s;
+        const float d = r.d[pos];
+        if (d > 0.0f) x = x + omega * (b[a] - (ZERO ? 0.0f : row_acc(r, pos, x, pin))) / d;
+        return x;
+    };
+    if (code == 1 || code == 2) {  // one of each colour
+        const int s = (code & 1) == colour ? 0 : 1;
+        if (s == 0 || two) {
+            const float x = update(s, colour * r.H + t, s ? v[1] : v[0]);
+            v[0] = s ? v[0] : x;
+            v[1] = s ? x : v[1];
+        }
+    } else if ((code & 1) == colour) {
+        v[0] = update(0, t, v[0]);
+        v[1] = update(1, r.H + t, v[1]);  // (the missing partner makes a pair of two colours)
+    }
+    if (two)
+        reinterpret_cast<float2*>(pout)[t] = make_float2(v[0], v[1]);
+    else
+        pout[2 * t] = v[0];
+}
+
+// All half-sweeps of a smoothing phase in one workgroup, for a level of up to
+// 2048 PP cells: rows in registers, the iterate and b in LDS.  New values are
+// held until every thread has read the old ones.  Three sweeps: 11.7 us at
+// 4096 cells (15.5 with rows past six couplings, whose rest is read from
+// memory each time), of which the loads take half; six launches take 19.  Four
+// pairs per thread do not fit the registers, hence the limit.
+constexpr int kRowsSmallThreads = 1024;
+constexpr int kRowsSmallMax = 4096;
+
+template <int PP>
+__global__ __launch_bounds__(kRowsSmallThreads) void k_msbg_rows_small(MRows r, int n, float* __restrict__ p,
+                                                                       const float* __restrict__ b, int sweeps,
+                                                                       int first, int zero, float omega) {
+    __shared__ float x[2048 * PP], bb[2048 * PP];
+    const size_t W = 2 * (size_t)r.H;
+    float w[PP][2][kRowIn], dd[PP][2];
+    unsigned nb[PP][2][kRowIn / 2];
+    int code[PP];
+    unsigned rest = 0;
+#pragma unroll
+    for (int m = 0; m < PP; ++m) {
+        const int t = (int)threadIdx.x + m * kRowsSmallThreads;
+        code[m] = 4;  // no pair here
+        if (t < r.H) {
+            code[m] = r.code[t];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const int a = 2 * t + h, pos = h * r.H + t;
+                // (an odd last cell's partner has no row)
+                const bool has = 2 * t + 1 < n || h == (code[m] & 1);
+                dd[m][h] = has ? r.d[pos] : 0.0f;
+                int2 e[kRowIn];
+#pragma unroll
+                for (int k = 0; k < kRowIn; ++k) e[k] = has ? r.in[k * W + pos] : make_int2(0, 0);
+                if (e[kRowIn - 1].y < 0) rest |= 1u << (2 * m + h);
+#pragma unroll
+                for (int k = 0; k < kRowIn; ++k) w[m][h][k] = __int_as_float(e[k].x);
+#pragma unroll
+                for (int k = 0; k < kRowIn; k += 2)
+                    nb[m][h][k / 2] = (unsigned)(e[k].y & 0x7fff) | ((unsigned)(e[k + 1].y & 0x7fff) << 16);
+                x[a] = zero || a >= n ? 0.0f : p[a];
+                bb[a] = a < n ? b[a] : 0.0f;
+            }
+        }
+    }
+    __syncthreads();
+    for (int hs = 0; hs < 2 * sweeps; ++hs) {
+        const int colour = (hs & 1) ^ first;
+        float nv[PP][2];
+        int at[PP][2];
+#pragma unroll
+        for (int m = 0; m < PP; ++m) {
+            const int t = (int)threadIdx.x + m * kRowsSmallThreads;
+            const bool mixed = code[m] == 1 || code[m] == 2;
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                // row h: the cell of colour h, or cell 2t + h
+                at[m][h] = -1;
+                const bool on = mixed ? h == colour : (code[m] != 4 && (code[m] & 1) == colour);
+                if (on && dd[m][h] > 0.0f) {
+                    const int s = mixed ? ((code[m] & 1) == h ? 0 : 1) : h;
+                    const int a = 2 * t + s;
+                    const float pa = x[a];
+                    float acc = 0.0f;
+#pragma unroll
+                    for (int k = 0; k < kRowIn; ++k) {
+                        const unsigned q = nb[m][h][k / 2];
+                        acc += w[m][h][k] * (pa - x[k & 1 ? q >> 16 : q & 0xffffu]);
+                    }
+                    if (rest >> (2 * m + h) & 1) acc = row_rest(r, h * r.H + t, pa, x, acc);
+                    nv[m][h] = pa + omega * (bb[a] - acc) / dd[m][h];
+                    at[m][h] = a;
+                }
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int m = 0; m < PP; ++m)
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+                if (at[m][h] >= 0) x[at[m][h]] = nv[m][h];
+        __syncthreads();
+    }
+    for (int a = threadIdx.x; a < n; a += kRowsSmallThreads) p[a] = x[a];
+}
+
+// out = A p, or b - A p
+__global__ __launch_bounds__(256) void k_msbg_rows_apply(MRows r, int n, const float* __restrict__ p,
+                                                         const float* __restrict__ b, float* __restrict__ out) {
+    const int a = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
+    if (a >= n) return;
+    const int pos = row_pos(r.code[a >> 1], a & 1, a >> 1, r.H);
+    const float acc = row_acc(r, pos, p[a], p);
+    out[a] = b ? b[a] - acc : acc;
+}
+
 constexpr int kVecBlocks = 1024;
 
 }  // namespace pf
@@ -906,6 +1180,75 @@ PF_API int pf_msbg_coarse_op(const pf_msbg_grid* g, const float* bface, const fl
 PF_API int pf_msbg_coarse_apply(const double* op, const float* b, float* p, int32_t n, pf_stream_t stream) {
     PF_REQUIRE(op && b && p && n > 0 && n <= kMsbgCoarseOpMax, "pf_msbg_coarse_apply: bad arguments");
     k_msbg_coarse_apply<<<cdiv(n, kApplyRows), 1024, 0, S(stream)>>>(op, b, p, n);
+    PF_CHECK_LAUNCH();
+    return PF_OK;
+}
+
+PF_API size_t pf_msbg_rows_bytes(int32_t ncells) {
+    return ncells > 0 && ncells <= kMsbgMaxCells ? mrows_layout(ncells, nullptr, nullptr) : 0;
+}
+
+static int check_rows(const pf_msbg_grid* g, const void* rows, const char* who, MRows* r) {
+    int rc = check_grid(g, who);
+    if (rc) return rc;
+    PF_REQUIRE(rows && (reinterpret_cast<uintptr_t>(rows) & 15) == 0, "%s: rows must be 16-byte aligned", who);
+    mrows_layout(g->ncells, static_cast<char*>(const_cast<void*>(rows)), r);
+    return PF_OK;
+}
+
+PF_API int pf_msbg_rows_build(const pf_msbg_grid* g, const float* bface, float* diag, void* rows,
+                              pf_stream_t stream) {
+    MRows r;
+    int rc = check_rows(g, rows, "pf_msbg_rows_build", &r);
+    if (rc) return rc;
+    PF_REQUIRE(bface && diag, "pf_msbg_rows_build: null vector");
+    rc = fill_u32(r.used, 1, 0u, S(stream));
+    if (rc) return rc;
+    k_msbg_rows<<<cdiv(g->ncells, 256), 256, 0, S(stream)>>>(mgrid(*g), bface, r, diag);
+    PF_CHECK_LAUNCH();
+    return PF_OK;
+}
+
+PF_API int pf_msbg_rows_smooth(const pf_msbg_grid* g, const void* rows, float* p, float* p2, const float* b,
+                               int32_t sweeps, int32_t first_colour, int32_t from_zero, float omega,
+                               pf_stream_t stream) {
+    MRows r;
+    int rc = check_rows(g, rows, "pf_msbg_rows_smooth", &r);
+    if (rc) return rc;
+    PF_REQUIRE(p && p2 && p != p2 && b, "pf_msbg_rows_smooth: null or equal vectors");
+    PF_REQUIRE(((reinterpret_cast<uintptr_t>(p) | reinterpret_cast<uintptr_t>(p2)) & 7) == 0,
+               "pf_msbg_rows_smooth: p and p2 must be 8-byte aligned");
+    PF_REQUIRE(sweeps >= 0 && (first_colour == 0 || first_colour == 1), "pf_msbg_rows_smooth: bad sweeps or colour");
+    if (sweeps == 0) return from_zero ? fill_u32(p, g->ncells, 0u, S(stream)) : PF_OK;
+    if (g->ncells <= kRowsSmallMax) {
+        const auto k = g->ncells <= 2048 ? k_msbg_rows_small<1> : k_msbg_rows_small<2>;
+        k<<<1, kRowsSmallThreads, 0, S(stream)>>>(r, g->ncells, p, b, sweeps, first_colour, from_zero, omega);
+        PF_CHECK_LAUNCH();
+        return PF_OK;
+    }
+    const int nb = cdiv(r.H, 256);
+    float *in = p, *out = p2;
+    for (int h = 0; h < 2 * sweeps; ++h) {  // an even number: the result is in p
+        const int c = (h & 1) ^ first_colour;
+        if (h == 0 && from_zero)
+            k_msbg_rows_sweep<true><<<nb, 256, 0, S(stream)>>>(r, g->ncells, in, out, b, c, omega);
+        else
+            k_msbg_rows_sweep<false><<<nb, 256, 0, S(stream)>>>(r, g->ncells, in, out, b, c, omega);
+        PF_CHECK_LAUNCH();
+        float* t = in;
+        in = out;
+        out = t;
+    }
+    return PF_OK;
+}
+
+PF_API int pf_msbg_rows_apply(const pf_msbg_grid* g, const void* rows, const float* p, const float* b, float* out,
+                              pf_stream_t stream) {
+    MRows r;
+    int rc = check_rows(g, rows, "pf_msbg_rows_apply", &r);
+    if (rc) return rc;
+    PF_REQUIRE(p && out && out != p, "pf_msbg_rows_apply: null vector, or p == out");
+    k_msbg_rows_apply<<<cdiv(g->ncells, 256), 256, 0, S(stream)>>>(r, g->ncells, p, b, out);
     PF_CHECK_LAUNCH();
     return PF_OK;
 }

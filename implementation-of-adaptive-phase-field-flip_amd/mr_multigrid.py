@@ -16,7 +16,6 @@ import numpy as np
 import torch
 
 from . import _lib
-from . import mr_operator as mro
 from .msbg import MSBG
 
 
@@ -28,6 +27,17 @@ class _MGLevel:
         self.bface = torch.zeros(n * 3, dtype=torch.float32, device=grid.dev)
         self.diag, self.p, self.p2, self.b, self.r = z(), z(), z(), z(), z()
         self.n = n
+        # the operator's rows, rebuilt with every set of face coefficients
+        self.rows = torch.empty(int(_lib.load().pf_msbg_rows_bytes(n)), dtype=torch.uint8, device=grid.dev)
+
+    def build_rows(self):
+        _lib.call("pf_msbg_rows_build", self.grid.ref(), _lib.ptr(self.bface), _lib.ptr(self.diag),
+                  _lib.ptr(self.rows), _lib.stream())
+
+    def apply(self, p, out, b=None):
+        """out = A p, or b - A p."""
+        _lib.call("pf_msbg_rows_apply", self.grid.ref(), _lib.ptr(self.rows), _lib.ptr(p), _lib.ptr(b),
+                  _lib.ptr(out), _lib.stream())
 
 
 def reduce(op, x, y, work):
@@ -107,42 +117,42 @@ class MRMultigrid:
                 f = self.levels[i - 1]
                 _lib.call("pf_msbg_coarsen_beta", lv.grid.ref(), f.grid.ref(), _lib.ptr(f.bface),
                           _lib.ptr(lv.bface), _lib.stream())
-            mro._diag(lv.grid, lv.bface, lv.diag)
+            lv.build_rows()
         if self._coarse_op is not None:
             c = self.levels[-1]
             _lib.call("pf_msbg_coarse_op", c.grid.ref(), _lib.ptr(c.bface), _lib.ptr(c.diag), self.coarsest_sweeps,
                       self.omega, _lib.ptr(self._coarse_op), _lib.stream())
 
-    def _smooth(self, lv: _MGLevel, n_sweeps, reverse=False, index=None):
+    def _smooth(self, lv: _MGLevel, n_sweeps, reverse=False, index=None, from_zero=False):
         """n_sweeps red-black sweeps, or the adaptive relaxation loop on a
-        non-coarsest level when the smoother is adaptive (mr_multigrid.py:200-211)."""
+        non-coarsest level when the smoother is adaptive (mr_multigrid.py:200-211);
+        from_zero: of p = 0, whatever lv.p holds."""
         if self.adaptive is not None and index is not None and index < self.nlev - 1:
+            if from_zero:
+                lv.p.zero_()
             self.adaptive[index].smooth(lv, record=self._record)
             return
-        colours = (1, 0) if reverse else (0, 1)
-        for _ in range(n_sweeps):
-            for c in colours:
-                mro._rbgs(lv.grid, lv.p, lv.p2, lv.b, lv.bface, lv.diag, c, self.omega)
-                lv.p, lv.p2 = lv.p2, lv.p
+        _lib.call("pf_msbg_rows_smooth", lv.grid.ref(), _lib.ptr(lv.rows), _lib.ptr(lv.p), _lib.ptr(lv.p2),
+                  _lib.ptr(lv.b), int(n_sweeps), int(reverse), int(from_zero), self.omega, _lib.stream())
 
     def _vcycle(self, i=0):
-        """mr_multigrid.py:213-235."""
+        """mr_multigrid.py:213-235, from p = 0."""
         lv = self.levels[i]
         if i == self.nlev - 1:
             if self.coarsest_mode == "matrix" and self._coarse_op is not None:
                 _lib.call("pf_msbg_coarse_apply", _lib.ptr(self._coarse_op), _lib.ptr(lv.b), _lib.ptr(lv.p), lv.n,
                           _lib.stream())
             elif self.coarsest_mode in ("matrix", "lds"):
+                lv.p.zero_()
                 _lib.call("pf_msbg_coarsest_smooth", lv.grid.ref(), _lib.ptr(lv.p), _lib.ptr(lv.b),
                           _lib.ptr(lv.bface), _lib.ptr(lv.diag), self.coarsest_sweeps, self.omega, _lib.stream())
             else:
-                self._smooth(lv, self.coarsest_sweeps)
+                self._smooth(lv, self.coarsest_sweeps, from_zero=True)
             remove_mean(lv.p, self._work)
             return
-        self._smooth(lv, self.pre, index=i)
-        mro._residual(lv.grid, lv.p, lv.b, lv.bface, lv.r)
+        self._smooth(lv, self.pre, index=i, from_zero=True)
+        lv.apply(lv.p, lv.r, lv.b)
         c = self.levels[i + 1]
-        c.p.zero_()
         _lib.call("pf_msbg_restrict", lv.grid.ref(), c.grid.ref(), _lib.ptr(lv.r), _lib.ptr(c.b), _lib.stream())
         self._vcycle(i + 1)
         _lib.call("pf_msbg_prolong_add", lv.grid.ref(), c.grid.ref(), _lib.ptr(c.p), _lib.ptr(lv.p),
@@ -153,7 +163,6 @@ class MRMultigrid:
         """z = V-cycle(r), mean removed (mr_multigrid.py:237-243)."""
         L0 = self.levels[0]
         L0.b.copy_(r_in)
-        L0.p.zero_()
         self._vcycle(0)
         z_out.copy_(L0.p)
         remove_mean(z_out, self._work)

@@ -470,6 +470,21 @@ int32_t pf_msbg_coarse_op_max_cells(void);
 int pf_msbg_coarse_op(const pf_msbg_grid* g, const float* bface, const float* diag, int32_t sweeps, float omega,
                       double* op, pf_stream_t stream);
 int pf_msbg_coarse_apply(const double* op, const float* b, float* p, int32_t n, pf_stream_t stream);
+/* The operator's rows as a table (no counterpart: the reference walks the
+ * blocks in every sweep).  pf_msbg_rows_build writes the couplings of all
+ * cells for these face coefficients into rows (pf_msbg_rows_bytes(ncells)
+ * bytes, 16-byte aligned) and their sums into diag; the others take that table
+ * with the grid it was built from, and give bit for bit what
+ * pf_msbg_apply, pf_msbg_residual and pf_msbg_rbgs give.
+ * pf_msbg_rows_smooth: `sweeps` red-black sweeps of p in place (p2: scratch of
+ * the same size; both 8-byte aligned), first_colour first; from_zero: p counts
+ * as zero and is not read.  pf_msbg_rows_apply: out = A p, or b - A p if b. */
+size_t pf_msbg_rows_bytes(int32_t ncells);
+int pf_msbg_rows_build(const pf_msbg_grid* g, const float* bface, float* diag, void* rows, pf_stream_t stream);
+int pf_msbg_rows_smooth(const pf_msbg_grid* g, const void* rows, float* p, float* p2, const float* b, int32_t sweeps,
+                        int32_t first_colour, int32_t from_zero, float omega, pf_stream_t stream);
+int pf_msbg_rows_apply(const pf_msbg_grid* g, const void* rows, const float* p, const float* b, float* out,
+                       pf_stream_t stream);
 /* coarsen_beta (mr_multigrid.py:52-89): coarse face = mean of the 2x2 fine
  * faces it covers. */
 int pf_msbg_coarsen_beta(const pf_msbg_grid* coarse, const pf_msbg_grid* fine, const float* bfine, float* bcoarse,
