@@ -180,6 +180,9 @@ SIGNATURES = {
     "pf_msbg_rows_build": (ctypes.c_int, [ctypes.POINTER(MsbgGrid), P, P, P, P]),
     "pf_msbg_rows_smooth": (ctypes.c_int, [ctypes.POINTER(MsbgGrid), P, P, P, P, I32, I32, I32, F32, P]),
     "pf_msbg_rows_apply": (ctypes.c_int, [ctypes.POINTER(MsbgGrid), P, P, P, P, P]),
+    "pf_msbg_rows_apply_dot": (ctypes.c_int, [ctypes.POINTER(MsbgGrid), P, P, P, P, P]),
+    "pf_mrcg_update": (ctypes.c_int, [P, P, I32, P, P, P, P, P, P, I64, P, P]),
+    "pf_mrcg_direction": (ctypes.c_int, [P, P, I32, P, P, P, P, P, I64, P, P, P, P]),
     "pf_msbg_coarsen_beta": (ctypes.c_int, [ctypes.POINTER(MsbgGrid), ctypes.POINTER(MsbgGrid), P, P, P]),
     "pf_msbg_restrict": (ctypes.c_int, [ctypes.POINTER(MsbgGrid), ctypes.POINTER(MsbgGrid), P, P, P]),
     "pf_msbg_prolong_add": (ctypes.c_int, [ctypes.POINTER(MsbgGrid), ctypes.POINTER(MsbgGrid), P, P, P]),

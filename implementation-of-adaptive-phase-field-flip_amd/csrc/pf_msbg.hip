@@ -644,6 +644,8 @@ __global__ __launch_bounds__(256) void k_msbg_cover(MGrid g, int* __restrict__ h
     if (c.addr >= 0) atomicAdd(hits + c.addr, 1);
 }
 
+constexpr int kVecBlocks = 1024;
+
 // FP64 partial sums over blocks, combined in block order by one block
 __global__ __launch_bounds__(256) void k_vec_part(int op, const float* __restrict__ x, const float* __restrict__ y,
                                                   int64_t n, double* __restrict__ part) {
@@ -725,8 +727,7 @@ __global__ __launch_bounds__(256) void k_vec_sub_mean(float* __restrict__ y, int
 // rz == 0 or rz_new <= 0.
 enum MrcgOp { MRCG_INIT = 0, MRCG_RZ, MRCG_ALPHA, MRCG_REL, MRCG_BETA };
 
-__global__ void k_mrcg_scalar(int op, double* st, int* flag, const double* a, const double* b, double tol) {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
+__device__ inline void mrcg_scalar(int op, double* st, int* flag, const double* a, const double* b, double tol) {
     if (op == MRCG_INIT) {  // a = max|b|
         st[4] = *a;
         st[5] = tol;
@@ -755,6 +756,152 @@ __global__ void k_mrcg_scalar(int op, double* st, int* flag, const double* a, co
         }
     }
     st[7] = (double)flag[0];  // the host reads st[0..7] in one copy
+}
+
+__global__ void k_mrcg_scalar(int op, double* st, int* flag, const double* a, const double* b, double tol) {
+    if (threadIdx.x == 0 && blockIdx.x == 0) mrcg_scalar(op, st, flag, a, b, tol);
+}
+
+// One PCG iteration's vector work in five launches (twenty when every vector
+// operation, reduction and scalar step had its own; at 32k cells each costs its
+// launch, at 1.4M a pass over memory: adaptive 32^3 step 2.26 -> 1.95 ms, 128^3
+// 7.83 -> 7.60).  A reduction's partials stay in
+// its work buffer (work + 1, kVecBlocks entries, those past the launch's blocks
+// zero) and every block of the next kernel combines them anew, in the order of
+// k_vec_comb; block 0 leaves the scalars in st.  A block reads no entry of st
+// that block 0 of the same launch writes, but the flag: both of its values
+// lead a block to the same decision.
+__device__ inline double comb_parts(int op, const double* __restrict__ part) {
+    __shared__ double total;
+    __syncthreads();
+    if (threadIdx.x < 64) {
+        double x[kVecBlocks / 64], r = 0.0;
+#pragma unroll
+        for (int q = 0; q < kVecBlocks / 64; ++q) x[q] = part[q * 64 + threadIdx.x];
+#pragma unroll
+        for (int q = 0; q < kVecBlocks / 64; ++q) r = op == 2 ? fmax(r, x[q]) : r + x[q];
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) {
+            const double t = __shfl_xor(r, o, 64);
+            r = op == 2 ? fmax(r, t) : r + t;
+        }
+        if (threadIdx.x == 0) total = r;
+    }
+    __syncthreads();
+    return total;
+}
+
+// alpha = rz / <q, Ap>; x += alpha q, r_prev = r, r -= alpha Ap, and the
+// partials of max |r|.  rz: slot of st that holds it.
+__global__ __launch_bounds__(256) void k_mrcg_update(double* st, int* flag, int rz, const double* __restrict__ qap,
+                                                     const float* __restrict__ q, const float* __restrict__ ap,
+                                                     float* __restrict__ x, float* __restrict__ r,
+                                                     float* __restrict__ r_prev, int64_t n,
+                                                     double* __restrict__ rmax) {
+    __shared__ float sh[4];
+    const double d = comb_parts(1, qap);
+    const bool go = flag[0] == 0 && !(d <= 0.0);
+    const double al = go ? st[rz] / d : 0.0;
+    const float a = (float)al, am = (float)-al;
+    float m = 0.0f;
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
+        float ri = r[i];
+        r_prev[i] = ri;
+        if (go) {
+            x[i] = __fmaf_rn(a, q[i], x[i]);
+            ri = __fmaf_rn(am, ap[i], ri);
+            r[i] = ri;
+        }
+        m = fmaxf(m, fabsf(ri));
+    }
+    m = block_max(m, sh);
+    if (threadIdx.x == 0) rmax[blockIdx.x] = (double)m;
+    if (blockIdx.x == 0 && threadIdx.x == 0 && flag[0] == 0) {
+        st[6] = d;
+        if (go)
+            st[1] = al;
+        else
+            flag[0] = 1;
+    }
+}
+
+// rel = max |r| / |b|, convergence, and the flag where the host reads it
+__global__ __launch_bounds__(64) void k_mrcg_rel(double* st, int* flag, const double* __restrict__ rmax) {
+    const double m = comb_parts(2, rmax);
+    if (threadIdx.x == 0) mrcg_scalar(MRCG_REL, st, flag, &m, nullptr, 0.0);
+}
+
+// z = y - mean(y) from the partials of its sum, and the partials of <r, z>
+// and <r_prev, z>
+__global__ __launch_bounds__(256) void k_mrcg_z(const float* y, float* z, int64_t n,
+                                                const double* __restrict__ sum, const float* __restrict__ r,
+                                                const float* __restrict__ r_prev, double* __restrict__ rz,
+                                                double* __restrict__ rpz) {
+    __shared__ double sh[2 * 16];
+    const float a = (float)(-comb_parts(0, sum) / (double)n);
+    double v[2] = {0.0, 0.0};
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
+        const float zi = 1.0f * y[i] + a;
+        z[i] = zi;
+        v[0] += (double)r[i] * (double)zi;
+        v[1] += (double)r_prev[i] * (double)zi;
+    }
+    block_sum<2>(v, sh);
+    if (threadIdx.x == 0) {
+        rz[blockIdx.x] = v[0];
+        rpz[blockIdx.x] = v[1];
+    }
+}
+
+// beta = max((<r, z> - <r_prev, z>) / rz, 0), q = z + beta q; the new rz goes
+// to the other slot, since every block reads the old one
+__global__ __launch_bounds__(256) void k_mrcg_q(double* st, int* flag, int rz, int rz_next,
+                                                const double* __restrict__ rzp, const double* __restrict__ rpzp,
+                                                const float* __restrict__ z, float* __restrict__ q, int64_t n) {
+    const double rz_new = comb_parts(1, rzp), rpz = comb_parts(1, rpzp), old = st[rz];
+    const bool go = flag[0] == 0 && !(old == 0.0 || rz_new <= 0.0);
+    const double beta = go ? fmax((rz_new - rpz) / old, 0.0) : 0.0;
+    if (go) {
+        const float b = (float)beta;
+        for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
+#pragma clang fp contract(off)
+            const float t = b * q[i];  // rounded, as in k_vec_axpby_dev
+            q[i] = z[i] + t;
+        }
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        if (go) {
+            st[2] = beta;
+            st[rz_next] = rz_new;
+        } else if (flag[0] == 0) {
+            flag[0] = 3;
+        }
+        st[7] = (double)flag[0];
+    }
+}
+
+// x -= mean(x) in one workgroup, for a coarsest level
+constexpr int kMeanSmallMax = 4096;
+
+__global__ __launch_bounds__(1024) void k_vec_remove_mean_small(float* __restrict__ x, int n) {
+    __shared__ double sh[16];
+    __shared__ float shift;
+    float v[kMeanSmallMax / 1024];
+    double s[1] = {0.0};
+#pragma unroll
+    for (int q = 0; q < kMeanSmallMax / 1024; ++q) {
+        const int i = q * 1024 + (int)threadIdx.x;
+        v[q] = i < n ? x[i] : 0.0f;
+        s[0] += (double)v[q];
+    }
+    block_sum<1>(s, sh);
+    if (threadIdx.x == 0) shift = (float)(-s[0] / (double)n);
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < kMeanSmallMax / 1024; ++q) {
+        const int i = q * 1024 + (int)threadIdx.x;
+        if (i < n) x[i] = 1.0f * v[q] + shift;
+    }
 }
 
 // z = r / diag where diag > 0, else 0 (mr_solver.py:64-69)
@@ -1030,17 +1177,37 @@ __global__ __launch_bounds__(kRowsSmallThreads) void k_msbg_rows_small(MRows r, 
     for (int a = threadIdx.x; a < n; a += kRowsSmallThreads) p[a] = x[a];
 }
 
-// out = A p, or b - A p
+// out = A p, or b - A p, a pair per thread (twelve row loads in flight); DOT:
+// part[block] = the block's share of <p, out> too.  At 1.4M cells 18.4 us, 22.6
+// with the product (28 + 9 from the blocks and in three launches): 84 MB.
+template <bool DOT>
 __global__ __launch_bounds__(256) void k_msbg_rows_apply(MRows r, int n, const float* __restrict__ p,
-                                                         const float* __restrict__ b, float* __restrict__ out) {
-    const int a = xcd_block(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
-    if (a >= n) return;
-    const int pos = row_pos(r.code[a >> 1], a & 1, a >> 1, r.H);
-    const float acc = row_acc(r, pos, p[a], p);
-    out[a] = b ? b[a] - acc : acc;
+                                                         const float* __restrict__ b, float* __restrict__ out,
+                                                         double* __restrict__ part) {
+    __shared__ double sh[16];
+    double v[1] = {0.0};
+    const int nb = (r.H + 255) / 256;
+    for (int q = xcd_block(blockIdx.x, gridDim.x); q < nb; q += gridDim.x) {
+        const int t = q * 256 + (int)threadIdx.x;
+        if (t >= r.H) continue;
+        const int code = r.code[t], a = 2 * t;
+        const bool two = a + 1 < n, swap = code == 1;  // (the row at t is cell a + 1's)
+        const float p0 = p[a], p1 = two ? p[a + 1] : 0.0f;
+        const float lo = two || !swap ? row_acc(r, t, swap ? p1 : p0, p) : 0.0f;
+        const float hi = two || swap ? row_acc(r, r.H + t, swap ? p0 : p1, p) : 0.0f;
+        const float y0 = swap ? hi : lo, y1 = swap ? lo : hi;
+        out[a] = b ? b[a] - y0 : y0;
+        if (two) out[a + 1] = b ? b[a + 1] - y1 : y1;
+        if (DOT) {
+            v[0] += (double)p0 * (double)y0;
+            if (two) v[0] += (double)p1 * (double)y1;
+        }
+    }
+    if (DOT) {
+        block_sum<1>(v, sh);
+        if (threadIdx.x == 0) part[blockIdx.x] = v[0];
+    }
 }
-
-constexpr int kVecBlocks = 1024;
 
 }  // namespace pf
 
@@ -1248,7 +1415,20 @@ PF_API int pf_msbg_rows_apply(const pf_msbg_grid* g, const void* rows, const flo
     int rc = check_rows(g, rows, "pf_msbg_rows_apply", &r);
     if (rc) return rc;
     PF_REQUIRE(p && out && out != p, "pf_msbg_rows_apply: null vector, or p == out");
-    k_msbg_rows_apply<<<cdiv(g->ncells, 256), 256, 0, S(stream)>>>(r, g->ncells, p, b, out);
+    k_msbg_rows_apply<false><<<cdiv(r.H, 256), 256, 0, S(stream)>>>(r, g->ncells, p, b, out, nullptr);
+    PF_CHECK_LAUNCH();
+    return PF_OK;
+}
+
+PF_API int pf_msbg_rows_apply_dot(const pf_msbg_grid* g, const void* rows, const float* p, float* out, double* work,
+                                  pf_stream_t stream) {
+    MRows r;
+    int rc = check_rows(g, rows, "pf_msbg_rows_apply_dot", &r);
+    if (rc) return rc;
+    PF_REQUIRE(p && out && out != p && work, "pf_msbg_rows_apply_dot: null vector, or p == out");
+    const int nb = cdiv(r.H, 256);
+    k_msbg_rows_apply<true><<<nb < kVecBlocks ? nb : kVecBlocks, 256, 0, S(stream)>>>(r, g->ncells, p, nullptr, out,
+                                                                                   work + 1);
     PF_CHECK_LAUNCH();
     return PF_OK;
 }
@@ -1347,6 +1527,12 @@ PF_API int pf_vec_axpby_dev(const double* st, int32_t ia, float a_sign, const fl
 }
 
 PF_API int pf_vec_remove_mean(float* x, int64_t n, double* work, pf_stream_t stream) {
+    PF_REQUIRE(x && work && n > 0, "pf_vec_remove_mean: null or empty vector");
+    if (n <= kMeanSmallMax) {
+        k_vec_remove_mean_small<<<1, 1024, 0, S(stream)>>>(x, (int)n);
+        PF_CHECK_LAUNCH();
+        return PF_OK;
+    }
     int rc = pf_vec_reduce(0, x, nullptr, n, work, stream);
     if (rc) return rc;
     const int64_t nb64 = cdiv(n, 256 * 4);
@@ -1371,6 +1557,38 @@ PF_API int pf_vec_jacobi(const float* r, const float* diag, float* z, int64_t n,
     const int64_t nb64 = cdiv(n, 256 * 4);
     const int nb = (int)(nb64 < kVecBlocks ? nb64 : kVecBlocks);
     k_vec_jacobi<<<nb, 256, 0, S(stream)>>>(r, diag, z, n);
+    PF_CHECK_LAUNCH();
+    return PF_OK;
+}
+
+static int vec_blocks(int64_t n) {
+    const int64_t nb = cdiv(n, 256 * 4);
+    return (int)(nb < kVecBlocks ? nb : kVecBlocks);
+}
+
+PF_API int pf_mrcg_update(double* st, int32_t* flag, int32_t rz, const double* qap, const float* q, const float* ap,
+                          float* x, float* r, float* r_prev, int64_t n, double* rmax, pf_stream_t stream) {
+    PF_REQUIRE(st && flag && qap && q && ap && x && r && r_prev && rmax && n > 0, "pf_mrcg_update: null or empty");
+    PF_REQUIRE(rz == 0 || rz == 8, "pf_mrcg_update: rz is st[0] or st[8]");
+    k_mrcg_update<<<vec_blocks(n), 256, 0, S(stream)>>>(st, flag, rz, qap + 1, q, ap, x, r, r_prev, n, rmax + 1);
+    PF_CHECK_LAUNCH();
+    k_mrcg_rel<<<1, 64, 0, S(stream)>>>(st, flag, rmax + 1);
+    PF_CHECK_LAUNCH();
+    return PF_OK;
+}
+
+PF_API int pf_mrcg_direction(double* st, int32_t* flag, int32_t rz, const float* y, float* z, const float* r,
+                             const float* r_prev, float* q, int64_t n, double* sum, double* rzw, double* rpzw,
+                             pf_stream_t stream) {
+    PF_REQUIRE(st && flag && y && z && r && r_prev && q && sum && rzw && rpzw && n > 0,
+               "pf_mrcg_direction: null or empty");
+    PF_REQUIRE(rz == 0 || rz == 8, "pf_mrcg_direction: rz is st[0] or st[8]");
+    const int nb = vec_blocks(n);
+    k_vec_part<<<nb, 256, 0, S(stream)>>>(0, y, nullptr, n, sum + 1);
+    PF_CHECK_LAUNCH();
+    k_mrcg_z<<<nb, 256, 0, S(stream)>>>(y, z, n, sum + 1, r, r_prev, rzw + 1, rpzw + 1);
+    PF_CHECK_LAUNCH();
+    k_mrcg_q<<<nb, 256, 0, S(stream)>>>(st, flag, rz, 8 - rz, rzw + 1, rpzw + 1, z, q, n);
     PF_CHECK_LAUNCH();
     return PF_OK;
 }

@@ -39,6 +39,11 @@ class _MGLevel:
         _lib.call("pf_msbg_rows_apply", self.grid.ref(), _lib.ptr(self.rows), _lib.ptr(p), _lib.ptr(b),
                   _lib.ptr(out), _lib.stream())
 
+    def apply_dot(self, p, out, work):
+        """out = A p, with the partials of <p, out> left in work."""
+        _lib.call("pf_msbg_rows_apply_dot", self.grid.ref(), _lib.ptr(self.rows), _lib.ptr(p), _lib.ptr(out),
+                  _lib.ptr(work), _lib.stream())
+
 
 def reduce(op, x, y, work):
     """FP64 sum (op 0), dot (1) or max |x| (2) of float32 device vectors."""
@@ -159,12 +164,16 @@ class MRMultigrid:
                   _lib.stream())
         self._smooth(lv, self.post, reverse=True, index=i)
 
-    def precondition(self, r_in, z_out):
-        """z = V-cycle(r), mean removed (mr_multigrid.py:237-243)."""
+    def vcycle(self, r_in):
+        """The V-cycle of r; returns level 0's iterate, valid until the next one."""
         L0 = self.levels[0]
         L0.b.copy_(r_in)
         self._vcycle(0)
-        z_out.copy_(L0.p)
+        return L0.p
+
+    def precondition(self, r_in, z_out):
+        """z = V-cycle(r), mean removed (mr_multigrid.py:237-243)."""
+        z_out.copy_(self.vcycle(r_in))
         remove_mean(z_out, self._work)
 
     def describe(self):

@@ -33,8 +33,8 @@ class MRSolver:
         nw = int(_lib.load().pf_vec_reduce_bytes()) // 8
         self._work = torch.zeros(nw, dtype=torch.float64, device=grid.dev)
         # one reduction buffer per scalar of an iteration; the state and flag
-        self._works = [torch.zeros(nw, dtype=torch.float64, device=grid.dev) for _ in range(6)]
-        self._st = torch.zeros(8, dtype=torch.float64, device=grid.dev)
+        self._works = [torch.zeros(nw, dtype=torch.float64, device=grid.dev) for _ in range(7)]
+        self._st = torch.zeros(16, dtype=torch.float64, device=grid.dev)
         self._flag = torch.zeros(2, dtype=torch.int32, device=grid.dev)
         self._host = torch.empty(8, dtype=torch.float64, pin_memory=True)  # the per-iteration state read
 
@@ -78,20 +78,16 @@ class MRSolver:
         it, rel = 0, 1.0
         host = self._host
         for it in range(1, max_iter + 1):
+            rz = 8 * ((it - 1) % 2)
             if self.mg is not None:
-                self.mg.levels[0].apply(self.q, self.Ap)
+                self.mg.levels[0].apply_dot(self.q, self.Ap, W[2])
             else:
                 mro._apply(self.grid, self.q, bface, self.Ap)
-            _lib.call("pf_vec_reduce", 1, _lib.ptr(self.q), _lib.ptr(self.Ap), self.n, _lib.ptr(W[2]), s)
-            _lib.call("pf_mrcg_scalar", 2, _lib.ptr(st), _lib.ptr(flag), _lib.ptr(W[2]), None, 0.0, s)
-            _lib.call("pf_vec_axpby_dev", _lib.ptr(st), 1, 1.0, _lib.ptr(self.q), -1, _lib.ptr(p_out), self.n,
-                      _lib.ptr(flag), s)
-            self.r_prev.copy_(self.r)
-            _lib.call("pf_vec_axpby_dev", _lib.ptr(st), 1, -1.0, _lib.ptr(self.Ap), -1, _lib.ptr(self.r), self.n,
-                      _lib.ptr(flag), s)
-            _lib.call("pf_vec_reduce", 2, _lib.ptr(self.r), None, self.n, _lib.ptr(W[3]), s)
-            _lib.call("pf_mrcg_scalar", 3, _lib.ptr(st), _lib.ptr(flag), _lib.ptr(W[3]), None, 0.0, s)
-            host.copy_(st)  # one read per iteration: the scalars and the stop flag (st[7])
+                _lib.call("pf_vec_reduce", 1, _lib.ptr(self.q), _lib.ptr(self.Ap), self.n, _lib.ptr(W[2]), s)
+            _lib.call("pf_mrcg_update", _lib.ptr(st), _lib.ptr(flag), rz, _lib.ptr(W[2]), _lib.ptr(self.q),
+                      _lib.ptr(self.Ap), _lib.ptr(p_out), _lib.ptr(self.r), _lib.ptr(self.r_prev), self.n,
+                      _lib.ptr(W[3]), s)
+            host.copy_(st[:8])  # one read per iteration: the scalars and the stop flag (st[7])
             rel = float(host[3])
             stop = int(host[7])
             if stop == 3:  # stopped at the previous iteration's beta
@@ -100,11 +96,13 @@ class MRSolver:
                 break
             if verbose and it % 50 == 0:
                 print(f"    cg {it:5d}  {rel:.3e}")
-            self._apply_preconditioner(self.r, self.zv)
-            _lib.call("pf_vec_reduce", 1, _lib.ptr(self.r), _lib.ptr(self.zv), self.n, _lib.ptr(W[4]), s)
-            _lib.call("pf_vec_reduce", 1, _lib.ptr(self.r_prev), _lib.ptr(self.zv), self.n, _lib.ptr(W[5]), s)
-            _lib.call("pf_mrcg_scalar", 4, _lib.ptr(st), _lib.ptr(flag), _lib.ptr(W[4]), _lib.ptr(W[5]), 0.0, s)
-            _lib.call("pf_vec_axpby_dev", _lib.ptr(st), -1, 1.0, _lib.ptr(self.zv), 2, _lib.ptr(self.q), self.n,
-                      _lib.ptr(flag), s)
+            if self.mg is not None:
+                y = self.mg.vcycle(self.r)
+            else:
+                y = self.zv
+                _lib.call("pf_vec_jacobi", _lib.ptr(self.r), _lib.ptr(self.diag), _lib.ptr(y), self.n, s)
+            _lib.call("pf_mrcg_direction", _lib.ptr(st), _lib.ptr(flag), rz, _lib.ptr(y), _lib.ptr(self.zv),
+                      _lib.ptr(self.r), _lib.ptr(self.r_prev), _lib.ptr(self.q), self.n, _lib.ptr(W[6]),
+                      _lib.ptr(W[4]), _lib.ptr(W[5]), s)
         remove_mean(p_out, self._work)
         return it, rel

@@ -485,6 +485,10 @@ int pf_msbg_rows_smooth(const pf_msbg_grid* g, const void* rows, float* p, float
                         int32_t first_colour, int32_t from_zero, float omega, pf_stream_t stream);
 int pf_msbg_rows_apply(const pf_msbg_grid* g, const void* rows, const float* p, const float* b, float* out,
                        pf_stream_t stream);
+/* out = A p, and <p, out> left in work as pf_vec_reduce's partials (work + 1;
+ * pf_vec_reduce_bytes() bytes, zero before the first call). */
+int pf_msbg_rows_apply_dot(const pf_msbg_grid* g, const void* rows, const float* p, float* out, double* work,
+                           pf_stream_t stream);
 /* coarsen_beta (mr_multigrid.py:52-89): coarse face = mean of the 2x2 fine
  * faces it covers. */
 int pf_msbg_coarsen_beta(const pf_msbg_grid* coarse, const pf_msbg_grid* fine, const float* bfine, float* bcoarse,
@@ -528,6 +532,19 @@ int pf_vec_axpby_dev(const double* st, int32_t ia, float a_sign, const float* x,
 int pf_vec_remove_mean(float* x, int64_t n, double* work, pf_stream_t stream);
 int pf_mrcg_scalar(int32_t op, double* st, int32_t* flag, const double* a, const double* b, double tol,
                    pf_stream_t stream);
+/* The two halves of a PCG iteration around the preconditioner, equal to the
+ * calls above one by one.  st holds 16 doubles here, rz in st[0] or st[8]
+ * (`rz`: which); qap, rmax, sum, rzw and rpzw are separate work buffers as for
+ * pf_vec_reduce, zero before their first use, qap with the partials of
+ * <q, ap> from pf_msbg_rows_apply_dot or pf_vec_reduce.
+ * pf_mrcg_update: alpha, x += alpha q, r_prev = r, r -= alpha ap, rel and flag.
+ * pf_mrcg_direction: z = y - mean(y) (z may be y), beta, q = z + beta q, the
+ * new rz in the other slot (st[8 - rz]). */
+int pf_mrcg_update(double* st, int32_t* flag, int32_t rz, const double* qap, const float* q, const float* ap,
+                   float* x, float* r, float* r_prev, int64_t n, double* rmax, pf_stream_t stream);
+int pf_mrcg_direction(double* st, int32_t* flag, int32_t rz, const float* y, float* z, const float* r,
+                      const float* r_prev, float* q, int64_t n, double* sum, double* rzw, double* rpzw,
+                      pf_stream_t stream);
 /* _jacobi (mr_solver.py:64-69): z = r / diag where diag > 0, else 0. */
 int pf_vec_jacobi(const float* r, const float* diag, float* z, int64_t n, pf_stream_t stream);
 

@@ -51,6 +51,12 @@ def test_rows_are_the_walk(mods, nb, n0, levels):
         row.apply(p, out, rhs)
         mro.apply_A(g, p, row.bface, ref) if rhs is None else mro.residual(g, p, b, row.bface, ref)
         assert torch.equal(out, ref)
+    work = torch.zeros(int(lib.load().pf_vec_reduce_bytes()) // 8, dtype=torch.float64, device="cuda")
+    mro.apply_A(g, p, row.bface, ref)
+    row.apply_dot(p, out, work)
+    assert torch.equal(out, ref)
+    terms = p.double() * ref.double()   # products exact, n FP64 additions in some order
+    assert float((work.sum() - terms.sum()).abs()) <= 2 * n * 2.0 ** -53 * float(terms.abs().sum())
     for sweeps, first, zero in ((1, 0, 0), (3, 1, 0), (3, 0, 1), (2, 1, 1), (0, 0, 0), (0, 0, 1)):
         got, tmp = p.clone(), torch.full_like(p, float("nan"))
         a, c = (torch.zeros_like(p) if zero else p.clone()), tmp.clone()
@@ -61,3 +67,70 @@ def test_rows_are_the_walk(mods, nb, n0, levels):
                  first, zero, 6.0 / 7.0, lib.stream())
         torch.cuda.synchronize()
         assert torch.equal(got, a), (sweeps, first, zero)
+
+
+# whole and partial workgroups, more elements than one pass of 1024 blocks
+@pytest.mark.parametrize("n", [1, 255, 4096, 4097, 70001, 1 << 21])
+@pytest.mark.parametrize("case", ["go", "qap <= 0", "rz <= 0", "stopped"])
+def test_cg_halves_are_the_single_steps(mods, n, case):
+    """pf_mrcg_update and pf_mrcg_direction against the vector operations,
+    reductions and scalar steps one by one: the same bits, also where an
+    iteration stops."""
+    print("mrcg", n, case, flush=True)
+    lib = mods["_lib"]
+    rng = np.random.default_rng(n)
+    v = lambda: torch.from_numpy(rng.standard_normal(n).astype(np.float32)).cuda()  # noqa: E731
+    nw = int(lib.load().pf_vec_reduce_bytes()) // 8
+    w = lambda: torch.zeros(nw, dtype=torch.float64, device="cuda")  # noqa: E731
+    s, P = lib.stream(), lib.ptr
+    q, ap, x, r, z = v(), v(), v(), v(), v()
+    if case != "qap <= 0":
+        ap.copy_(q)
+    else:
+        ap.copy_(-q)
+    z.copy_(-r if case == "rz <= 0" else r)
+    runs = []
+    for fused in (0, 1):
+        st = torch.zeros(16, dtype=torch.float64, device="cuda")
+        st[:6] = torch.tensor([0.7, 0.2, 0.3, 0.4, 2.0, 1e-6])
+        if fused:
+            st[8], st[0] = st[0].item(), 0.0
+        flag = torch.zeros(2, dtype=torch.int32, device="cuda")
+        flag[0] = 2 if case == "stopped" else 0
+        X, R, Q, Z, RP = x.clone(), r.clone(), q.clone(), torch.zeros_like(r), torch.zeros_like(r)
+        W = [w() for _ in range(5)]
+        lib.call("pf_vec_reduce", 1, P(Q), P(ap), n, P(W[0]), s)
+        if fused:
+            lib.call("pf_mrcg_update", P(st), P(flag), 8, P(W[0]), P(Q), P(ap), P(X), P(R), P(RP), n, P(W[1]), s)
+            lib.call("pf_mrcg_direction", P(st), P(flag), 8, P(z), P(Z), P(R), P(RP), P(Q), n, P(W[2]), P(W[3]),
+                     P(W[4]), s)
+        else:
+            lib.call("pf_mrcg_scalar", 2, P(st), P(flag), P(W[0]), None, 0.0, s)
+            lib.call("pf_vec_axpby_dev", P(st), 1, 1.0, P(Q), -1, P(X), n, P(flag), s)
+            RP.copy_(R)
+            lib.call("pf_vec_axpby_dev", P(st), 1, -1.0, P(ap), -1, P(R), n, P(flag), s)
+            lib.call("pf_vec_reduce", 2, P(R), None, n, P(W[1]), s)
+            lib.call("pf_mrcg_scalar", 3, P(st), P(flag), P(W[1]), None, 0.0, s)
+            Z.copy_(z)
+            lib.call("pf_vec_reduce", 0, P(Z), None, n, P(W[2]), s)
+            Z.copy_(1.0 * Z + np.float32(-float(W[2][0]) / n).item())
+            lib.call("pf_vec_reduce", 1, P(R), P(Z), n, P(W[3]), s)
+            lib.call("pf_vec_reduce", 1, P(RP), P(Z), n, P(W[4]), s)
+            lib.call("pf_mrcg_scalar", 4, P(st), P(flag), P(W[3]), P(W[4]), 0.0, s)
+            lib.call("pf_vec_axpby_dev", P(st), -1, 1.0, P(Z), 2, P(Q), n, P(flag), s)
+        torch.cuda.synchronize()
+        runs.append((X, R, RP, Z, Q, st[1:8], flag))
+    for a, b in zip(*runs):
+        assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("n", [1, 63, 1024, 4095, 4096])
+def test_mean_of_a_small_level(mods, n):
+    """One workgroup: FP64 sum, the shift rounded to FP32 (half a unit of the
+    mean) and one FP32 subtraction (half a unit of the largest value)."""
+    lib = mods["_lib"]
+    x = torch.from_numpy((3.0 + np.random.default_rng(n).standard_normal(n)).astype(np.float32)).cuda()
+    y, work = x.clone(), torch.zeros(int(lib.load().pf_vec_reduce_bytes()) // 8, dtype=torch.float64, device="cuda")
+    lib.call("pf_vec_remove_mean", lib.ptr(y), n, lib.ptr(work), lib.stream())
+    ref = x.double() - x.double().mean()
+    assert float((y.double() - ref).abs().max()) <= 2.0 ** -23 * float(x.double().abs().max())
