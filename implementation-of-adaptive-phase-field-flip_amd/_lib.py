@@ -213,6 +213,11 @@ SIGNATURES = {
                                  ctypes.POINTER(MrFields), P]),
     "pf_mr_advect": (ctypes.c_int, [ctypes.POINTER(MsbgGrid), ctypes.POINTER(MrParticles), ctypes.POINTER(MrParams),
                                     P, P]),
+    "pf_mr_neighbours": (ctypes.c_int, [ctypes.POINTER(MsbgGrid), P, P]),
+    "pf_mr_g2p_near": (ctypes.c_int, [ctypes.POINTER(MsbgGrid), P, ctypes.POINTER(MrParticles),
+                                      ctypes.POINTER(MrParams), ctypes.POINTER(MrFields), P]),
+    "pf_mr_advect_near": (ctypes.c_int, [ctypes.POINTER(MsbgGrid), P, ctypes.POINTER(MrParticles),
+                                         ctypes.POINTER(MrParams), P, P]),
     "pf_mr_block_distance": (ctypes.c_int, [ctypes.POINTER(MsbgGrid), P, P, P, P, F32, P]),
     "pf_mr_scan_tmp_ints": (I64, [I64]),
     "pf_mr_classify": (ctypes.c_int, [ctypes.POINTER(MrParticles), P, I32, I32, I32, F32, F32, I32, I32, I32, P, P,

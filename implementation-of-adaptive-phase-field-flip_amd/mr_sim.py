@@ -264,8 +264,8 @@ class AdaptiveSimulator:
     def stage_g2p(self, prm):
         """mr_sim.py:262-273: per-particle alpha_FLIP and G2P."""
         src = self.particles.struct()
-        _lib.call("pf_mr_g2p", self.grid.ref(), ctypes.byref(src), ctypes.byref(prm), ctypes.byref(self._fields),
-                  _lib.stream())
+        _lib.call("pf_mr_g2p_near", self.grid.ref(), _lib.ptr(self.grid.neighbours()), ctypes.byref(src),
+                  ctypes.byref(prm), ctypes.byref(self._fields), _lib.stream())
 
     def stage_resample(self):
         """Step 6 (mr_sim.py:280-289) -> (n_before, n_after)."""
@@ -279,8 +279,8 @@ class AdaptiveSimulator:
     def stage_advect(self, prm):
         """Step 7 (mr_sim.py:291-298)."""
         src = self.particles.struct()
-        _lib.call("pf_mr_advect", self.grid.ref(), ctypes.byref(src), ctypes.byref(prm), _lib.ptr(self._fvel),
-                  _lib.stream())
+        _lib.call("pf_mr_advect_near", self.grid.ref(), _lib.ptr(self.grid.neighbours()), ctypes.byref(src),
+                  ctypes.byref(prm), _lib.ptr(self._fvel), _lib.stream())
 
     # ------------------------------------------------------------------ main
     def step(self, dt: float | None = None, verbose=False) -> dict:

@@ -634,6 +634,14 @@ int pf_mr_g2p(const pf_msbg_grid* g, const pf_mr_particles* ps, const pf_mr_para
 /* Step 7, advect_rk3 + reflect_at_walls (mr_kernels.py:421-461): x, v. */
 int pf_mr_advect(const pf_msbg_grid* g, const pf_mr_particles* ps, const pf_mr_params* prm, const float* fvel,
                  pf_stream_t stream);
+/* The same two with the table that pf_mr_neighbours writes for this grid (27
+ * ints per slot): taps in blocks of the sample's level are addressed from it
+ * instead of through the block map.  Same results; nbr NULL: without it. */
+int pf_mr_neighbours(const pf_msbg_grid* g, int32_t* nbr, pf_stream_t stream);
+int pf_mr_g2p_near(const pf_msbg_grid* g, const int32_t* nbr, const pf_mr_particles* ps, const pf_mr_params* prm,
+                   const pf_mr_fields* f, pf_stream_t stream);
+int pf_mr_advect_near(const pf_msbg_grid* g, const int32_t* nbr, const pf_mr_particles* ps, const pf_mr_params* prm,
+                      const float* fvel, pf_stream_t stream);
 /* Step 6a, interface_flag_per_block + block_distance_field
  * (mr_kernels.py:464-477, particles.py:387-419, mr_sim.py:163-182):
  * mixed[blk] = 1 where a block holds both phases, dist (nbx nby nbz) =
