@@ -172,10 +172,12 @@ __device__ inline int2 touched_blocks(float x, float r, float bext, int nb) {
     return make_int2(max((int)floorf((x - r) / bext), 0), min((int)floorf((x + r) / bext), nb - 1));
 }
 
-template <class Add>
+// PARTS threads share a particle: thread `part` takes every PARTS-th row of
+// cells its support touches.
+template <int PARTS = 1, class Add>
 __device__ inline void splat_particle(const MGrid& g, const float* __restrict__ x, const float* __restrict__ v,
                                       const int* __restrict__ type, const int* __restrict__ lev, int64_t p,
-                                      const MRConst& c, Add&& add) {
+                                      const MRConst& c, Add&& add, int part = 0) {
     const float px = x[3 * p], py = x[3 * p + 1], pz = x[3 * p + 2];
     const float vel[3] = {v[3 * p], v[3 * p + 1], v[3 * p + 2]};
     const int lp = lev[p];
@@ -183,6 +185,7 @@ __device__ inline void splat_particle(const MGrid& g, const float* __restrict__ 
     const float rp = c.r0 * (float)(1 << lp);
     const float r2 = rp * rp, inv_r2 = 1.0f / r2;
     const float bext = (float)g.n0 * g.h0;
+    int row = 0;
     const int2 bi_ = touched_blocks(px, rp, bext, g.nbx), bj_ = touched_blocks(py, rp, bext, g.nby),
                bk_ = touched_blocks(pz, rp, bext, g.nbz);
     for (int bi = bi_.x; bi <= bi_.y; ++bi)
@@ -215,6 +218,7 @@ __device__ inline void splat_particle(const MGrid& g, const float* __restrict__ 
                         const float dyc = centre_dist(oy, j, h, py), dyf = dyc - half;
                         const float yc2 = square(dyc), yf2 = square(dyf);
                         if (fminf(xc2, xf2) + fminf(yc2, yf2) >= r2) continue;
+                        if (PARTS > 1 && row++ % PARTS != part) continue;
                         for (int k = k0; k <= k1; ++k) {
                             const float dzc = centre_dist(oz, k, h, pz), dzf = dzc - half;
                             const float zc2 = square(dzc), zf2 = square(dzf);
@@ -298,7 +302,7 @@ __global__ __launch_bounds__(256) void k_mr_cell_scatter(const int* __restrict__
 // A hash of cells in LDS for every particle (what k_mr_p2g_list does) was
 // bound by its lookups, one per touched cell.
 // 128^3 grid, 9.2M particles (6 % one level coarser than their block):
-// 4.95 -> 1.15 ms (0.47 own level, 0.33 one coarser, 0.35 the walk).
+// 4.95 -> 1.06 ms (0.47 own level, 0.33 one coarser, 0.26 the walk).
 template <int R>
 struct P2GTile {
     static constexpr int E = 8 + 2 * R, E3 = E * E * E;
@@ -542,9 +546,13 @@ __global__ __launch_bounds__(P2GTile<R>::NT) void k_mr_p2g_tile(MGrid g, int sub
 // atomics, and flushes every cached cell with one global atomic per non-zero
 // channel.  A contribution whose slot holds another cell goes to global
 // memory directly.  Integer sums, so the result equals the uncached kernel's
-// bit for bit.
+// bit for bit.  kP2GParts threads share a particle: one particle's walk is a
+// serial chain over up to a few hundred cells, and 46k particles (0.5 % of a
+// 9.2M dam break) at one per thread were 180 workgroups waiting for it.
+// 350 -> 256 us.
 constexpr int kP2GSlots = 512;
-constexpr int kP2GPerBlock = 256;  // particles per chunk (1 per thread)
+constexpr int kP2GParts = 8;
+constexpr int kP2GPerBlock = 256 / kP2GParts;  // particles per chunk
 constexpr unsigned kP2GListBlocks = 1024;
 static_assert(kP2GSlots == 1 << 9, "the slot hash keeps 9 bits");
 
@@ -562,10 +570,10 @@ __global__ __launch_bounds__(256) void k_mr_p2g_list(MGrid g, const float* __res
         for (int s = threadIdx.x; s < kP2GSlots; s += blockDim.x) tag[s] = -1;
         for (int s = threadIdx.x; s < kP2GSlots * kAcc; s += blockDim.x) lacc[s] = 0ull;
         __syncthreads();
-        if (p0 + (int)threadIdx.x < n) {
-            const int q = p0 + (int)threadIdx.x;
+        const int q = p0 + (int)threadIdx.x / kP2GParts;
+        if (q < n) {
             const int64_t p = q < nl ? list[q] : perm[out0 + q - nl];
-            splat_particle(g, x, v, type, lev, p, c, [&](int addr, const long long* val, unsigned mask) {
+            splat_particle<kP2GParts>(g, x, v, type, lev, p, c, [&](int addr, const long long* val, unsigned mask) {
                 const int s = (int)(((unsigned)addr * 2654435761u) >> 23);  // 9-bit multiplicative hash
                 int t = tag[s];
                 if (t != addr && t == -1) {
@@ -581,7 +589,7 @@ __global__ __launch_bounds__(256) void k_mr_p2g_list(MGrid g, const float* __res
                     for (int ch = 0; ch < kAcc; ++ch)
                         if (mask & (1u << ch)) atomicAdd(acc + ch * nc + addr, (unsigned long long)val[ch]);
                 }
-            });
+            }, (int)threadIdx.x % kP2GParts);
         }
         __syncthreads();
         for (int s = threadIdx.x; s < kP2GSlots; s += blockDim.x) {
