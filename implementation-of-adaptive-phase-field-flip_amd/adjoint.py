@@ -61,8 +61,8 @@ class StepAdjoint:
     def rebuild(self, x: torch.Tensor, v: torch.Tensor, dt: float, pressure: torch.Tensor | None = None) -> None:
         """Grid fields of the step that starts at (x, v); particles stay put.
         ``pressure`` is that step's pressure where the caller has kept it: the
-        solve, most of a rebuild (3.4 of 3.9 ms at 64^3 to 1e-8), is then a
-        copy of one cell field."""
+        solve, most of a rebuild, is then a copy of one cell field (a forward
+        and backward step at 64^3, solved to 1e-8: 11.2 -> 8.0 ms)."""
         sim = self.sim
         cfg = sim.cfg
         sim.px.copy_(x)

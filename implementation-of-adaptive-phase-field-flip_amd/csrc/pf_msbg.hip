@@ -883,7 +883,8 @@ __global__ __launch_bounds__(256) void k_mrcg_q(double* st, int* flag, int rz, i
 // x -= mean(x) in one workgroup, for a coarsest level
 constexpr int kMeanSmallMax = 4096;
 
-__global__ __launch_bounds__(1024) void k_vec_remove_mean_small(float* __restrict__ x, int n) {
+__global__ __launch_bounds__(1024) void k_vec_remove_mean_small(float* __restrict__ x, int n,
+                                                               double* __restrict__ sum) {
     __shared__ double sh[16];
     __shared__ float shift;
     float v[kMeanSmallMax / 1024];
@@ -895,7 +896,10 @@ __global__ __launch_bounds__(1024) void k_vec_remove_mean_small(float* __restric
         s[0] += (double)v[q];
     }
     block_sum<1>(s, sh);
-    if (threadIdx.x == 0) shift = (float)(-s[0] / (double)n);
+    if (threadIdx.x == 0) {
+        *sum = s[0];
+        shift = (float)(-s[0] / (double)n);
+    }
     __syncthreads();
 #pragma unroll
     for (int q = 0; q < kMeanSmallMax / 1024; ++q) {
@@ -1529,7 +1533,7 @@ PF_API int pf_vec_axpby_dev(const double* st, int32_t ia, float a_sign, const fl
 PF_API int pf_vec_remove_mean(float* x, int64_t n, double* work, pf_stream_t stream) {
     PF_REQUIRE(x && work && n > 0, "pf_vec_remove_mean: null or empty vector");
     if (n <= kMeanSmallMax) {
-        k_vec_remove_mean_small<<<1, 1024, 0, S(stream)>>>(x, (int)n);
+        k_vec_remove_mean_small<<<1, 1024, 0, S(stream)>>>(x, (int)n, work);
         PF_CHECK_LAUNCH();
         return PF_OK;
     }

@@ -133,4 +133,5 @@ def test_mean_of_a_small_level(mods, n):
     y, work = x.clone(), torch.zeros(int(lib.load().pf_vec_reduce_bytes()) // 8, dtype=torch.float64, device="cuda")
     lib.call("pf_vec_remove_mean", lib.ptr(y), n, lib.ptr(work), lib.stream())
     ref = x.double() - x.double().mean()
+    assert abs(float(work[0]) - float(x.double().sum())) <= 2.0 ** -40 * n
     assert float((y.double() - ref).abs().max()) <= 2.0 ** -23 * float(x.double().abs().max())

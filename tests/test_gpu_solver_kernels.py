@@ -55,8 +55,8 @@ def test_coarsest_level_in_one_workgroup(pf, coarsest, walls):
 
 @pytest.mark.parametrize("precision,bound", [("bf16", 2e-2), ("fp16", 3e-3)])
 def test_coarsest_level_in_one_workgroup_16_bit(pf, precision, bound):
-    """16-bit V-cycles: the bound is 8 units of the storage format's relative
-    rounding (2^-9, 2^-12), one per smoothing pass of the level above."""
+    """16-bit V-cycles: the level above stores its iterate once per colour of
+    its 3 + 3 sweeps, 12 relative roundings of 2^-9 or 2^-12 (2.3e-2, 2.9e-3)."""
     print(f"[gpu] coarsest 16-bit {precision}", flush=True)
     assert _vcycle_error(pf, (54, 38, 26), precision, False) < bound
 
