@@ -629,7 +629,9 @@ def run_surge256(pf, torch, args):
 def msbg_sweep_bytes(n_cells):
     """Algorithmic bytes of one MSBG red-black half-sweep: p read and written,
     b, the diagonal, the three owned face coefficients and the cell's block
-    slot read once per cell (32 B/cell); block tables are a few KB."""
+    slot read once per cell (32 B/cell); block tables are a few KB.  The
+    V-cycle's sweeps read the rows from a table instead of the last two: 48
+    bytes for each cell of the active colour."""
     return 32 * n_cells
 
 
@@ -664,27 +666,26 @@ def run_adaptive128(pf, torch, args):
     n_in = [sim.stats[-args.steps - 1]["particles"] if len(sim.stats) > args.steps else n0] + \
         [r["particles"] for r in recs[:-1]]
     # dominant kernel: the level-0 half-sweep of the MSBG V-cycle, timed with
-    # HIP events on the stream the kernels run on
+    # HIP events on the stream the kernels run on (ten sweeps per call)
     lib = pf._lib
     lv = sim.solver.mg.levels[0]
     g = lv.grid
     e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
     reps = 20
     e0.record()
-    for i in range(reps):
-        lib.call("pf_msbg_rbgs", g.ref(), lib.ptr(lv.p), lib.ptr(lv.p2), lib.ptr(lv.b), lib.ptr(lv.bface),
-                 lib.ptr(lv.diag), i & 1, 6.0 / 7.0, lib.stream())
+    lib.call("pf_msbg_rows_smooth", g.ref(), lib.ptr(lv.rows), lib.ptr(lv.p), lib.ptr(lv.p2), lib.ptr(lv.b),
+             reps // 2, 0, 0, 6.0 / 7.0, lib.stream())
     e1.record()
     torch.cuda.synchronize()
     sweep_ms = e0.elapsed_time(e1) / reps
-    rl = roofline(f"k_msbg_rbgs_pairs level-0 half-sweep ({g.ncells} cells)", msbg_sweep_bytes(g.ncells), sweep_ms)
+    rl = roofline(f"k_msbg_rows_sweep level-0 half-sweep ({g.ncells} cells)", msbg_sweep_bytes(g.ncells), sweep_ms)
     workload = "adaptive dam break y-up 128^3 MSBG n0=16 levels 0-2, 8 ppc, 1000:1, MG-PCG tol 1e-4"
     tr = measured_traffic(workload, "fp32")
-    if tr is not None:
+    m = tr["kernels"].get("k_msbg_rows_sweep level-0 half-sweep") if tr is not None else None
+    if m is not None:
         # HBM bytes per cell of the level-0 half-sweep, measured on this
         # workload's grid; the sweep streams its arrays once, so the figure
         # scales with the cell count
-        m = tr["kernels"]["k_msbg_rbgs_pairs level-0 half-sweep"]
         rl["traffic"] = m["bytes_per_cell"] * g.ncells
         rl["traffic_source"] = tr["source"]
     return {
