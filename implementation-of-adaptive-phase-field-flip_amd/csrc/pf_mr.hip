@@ -302,7 +302,7 @@ __global__ __launch_bounds__(256) void k_mr_cell_scatter(const int* __restrict__
 // A hash of cells in LDS for every particle (what k_mr_p2g_list does) was
 // bound by its lookups, one per touched cell.
 // 128^3 grid, 9.2M particles (6 % one level coarser than their block):
-// 4.95 -> 1.06 ms (0.47 own level, 0.33 one coarser, 0.26 the walk).
+// 4.95 -> 1.02 ms (0.47 own level, 0.33 one coarser, 0.22 the walk).
 template <int R>
 struct P2GTile {
     static constexpr int E = 8 + 2 * R, E3 = E * E * E;
@@ -549,9 +549,11 @@ __global__ __launch_bounds__(P2GTile<R>::NT) void k_mr_p2g_tile(MGrid g, int sub
 // bit for bit.  kP2GParts threads share a particle: one particle's walk is a
 // serial chain over up to a few hundred cells, and 46k particles (0.5 % of a
 // 9.2M dam break) at one per thread were 180 workgroups waiting for it.
-// 350 -> 256 us.
+// 1, 2, 4, 8 threads:
+// 350, 300, 221, 253 us; in a flow that lists far more of them 795, 725, 705,
+// 730, and 16 or 32 threads 855 and 1030.
 constexpr int kP2GSlots = 512;
-constexpr int kP2GParts = 8;
+constexpr int kP2GParts = 4;
 constexpr int kP2GPerBlock = 256 / kP2GParts;  // particles per chunk
 constexpr unsigned kP2GListBlocks = 1024;
 static_assert(kP2GSlots == 1 << 9, "the slot hash keeps 9 bits");
