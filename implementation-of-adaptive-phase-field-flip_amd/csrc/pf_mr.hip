@@ -150,20 +150,23 @@ __device__ inline long long fixed(float v, float scale) {
 }
 
 // Distance of a cell centre (axis index i of a block with low corner o) from
-// a particle, squared distances and eq. (6) weights, written without
-// contraction: the compiler would otherwise fuse different products in
-// different kernels, and the P2G kernels are to agree bit for bit.
+// a particle, squared distances and eq. (6) weights.  Which products are fused
+// is spelled out: left to the compiler it differs from kernel to kernel, and
+// the P2G kernels are to agree bit for bit.
 __device__ inline float centre_dist(float o, int i, float h, float x) {
 #pragma clang fp contract(off)
-    return o + ((float)i + 0.5f) * h - x;
+    return fmaf(h, (float)i + 0.5f, o) - x;
 }
 __device__ inline float square(float d) {
 #pragma clang fp contract(off)
     return d * d;
 }
-__device__ inline float eq6_weight(float x2, float y2, float z2, float inv_r2) {
+// q = 0: the centre, 1-3: the low face of axis q - 1; x2, y2: squared
+// distances, z: the distance
+__device__ inline float eq6_weight(int q, float x2, float y2, float z, float inv_r2) {
 #pragma clang fp contract(off)
-    const float t = fmaxf(1.0f - (x2 + y2 + z2) * inv_r2, 0.0f);
+    const float xy = x2 + y2, d2 = q == 0 || q == 3 ? fmaf(z, z, xy) : xy + z * z;
+    const float t = fmaxf(fmaf(-d2, inv_r2, 1.0f), 0.0f);
     return t * t * t;
 }
 
@@ -221,10 +224,10 @@ __device__ inline void splat_particle(const MGrid& g, const float* __restrict__ 
                         if (PARTS > 1 && row++ % PARTS != part) continue;
                         for (int k = k0; k <= k1; ++k) {
                             const float dzc = centre_dist(oz, k, h, pz), dzf = dzc - half;
-                            const float zc2 = square(dzc), zf2 = square(dzf);
                             const int addr = base + (i * nn + j) * nn + k;
-                            const float wt[4] = {eq6_weight(xc2, yc2, zc2, inv_r2), eq6_weight(xf2, yc2, zc2, inv_r2),
-                                                 eq6_weight(xc2, yf2, zc2, inv_r2), eq6_weight(xc2, yc2, zf2, inv_r2)};
+                            const float wt[4] = {
+                                eq6_weight(0, xc2, yc2, dzc, inv_r2), eq6_weight(1, xf2, yc2, dzc, inv_r2),
+                                eq6_weight(2, xc2, yf2, dzc, inv_r2), eq6_weight(3, xc2, yc2, dzf, inv_r2)};
                             long long val[kAcc];
                             unsigned mask = 0u;
 #pragma unroll
@@ -338,15 +341,15 @@ __device__ inline int p2g_class(const MGrid& g, const TileRef& t, unsigned ok, c
     return d;
 }
 
-// squared distances of cell i's centre and low face along axis a, from the
-// block that holds it; a cell of a block the support does not touch gets a
-// distance that makes its weight zero
-__device__ inline void cell_dist2(const TileRef& t, int a, int i, const int2& blk, float x, float& c2, float& f2) {
+// distances of cell i's centre and low face along axis a, from the block that
+// holds it; a cell of a block the support does not touch gets a distance that
+// makes its weight zero
+__device__ inline void cell_dist(const TileRef& t, int a, int i, const int2& blk, float x, float& c, float& f) {
     const int side = i < 0 ? -1 : (i >= t.nn ? 1 : 0), b = t.b[a] + side;
     const float d = centre_dist((float)b * t.bext, i - side * t.nn, t.h, x);
     const bool touched = b >= blk.x && b <= blk.y;
-    c2 = touched ? square(d) : 1e30f;
-    f2 = touched ? square(d - 0.5f * t.h) : 1e30f;
+    c = touched ? d : 1e15f;
+    f = touched ? d - 0.5f * t.h : 1e15f;
 }
 
 template <int R>
@@ -436,18 +439,24 @@ __global__ __launch_bounds__(P2GTile<R>::NT) void k_mr_p2g_tile(MGrid g, int sub
             };
             if constexpr (R == 1) {
                 // per axis: the two centres (first index it) and the two low
-                // faces (first index ic) within the radius
-                float c2[3][2], f2[3][2];
+                // faces (first index ic) within the radius: squared distances
+                // along x and y, distances along z
+                float dc[3][2], df[3][2];
                 int lc[3], lf[3];
 #pragma unroll
                 for (int a = 0; a < 3; ++a) {
                     const float gx = (px[a] - (float)t.b[a] * t.bext) / t.h;
                     const int it = gx - (float)ic[a] < 0.5f ? ic[a] - 1 : ic[a];
                     float unused;
-                    cell_dist2(t, a, it, tb[a], px[a], c2[a][0], unused);
-                    cell_dist2(t, a, it + 1, tb[a], px[a], c2[a][1], unused);
-                    cell_dist2(t, a, ic[a], tb[a], px[a], unused, f2[a][0]);
-                    cell_dist2(t, a, ic[a] + 1, tb[a], px[a], unused, f2[a][1]);
+                    cell_dist(t, a, it, tb[a], px[a], dc[a][0], unused);
+                    cell_dist(t, a, it + 1, tb[a], px[a], dc[a][1], unused);
+                    cell_dist(t, a, ic[a], tb[a], px[a], unused, df[a][0]);
+                    cell_dist(t, a, ic[a] + 1, tb[a], px[a], unused, df[a][1]);
+#pragma unroll
+                    for (int e = 0; e < 2 && a < 2; ++e) {
+                        dc[a][e] = square(dc[a][e]);
+                        df[a][e] = square(df[a][e]);
+                    }
                     lc[a] = it - t.t0[a] + R;
                     lf[a] = ic[a] - t.t0[a] + R;
                 }
@@ -459,8 +468,8 @@ __global__ __launch_bounds__(P2GTile<R>::NT) void k_mr_p2g_tile(MGrid g, int sub
 #pragma unroll
                     for (int m = 0; m < 8; ++m) {
                         const int i = m >> 2, j = (m >> 1) & 1, k = m & 1;
-                        const float w = eq6_weight(q4 == 1 ? f2[0][i] : c2[0][i], q4 == 2 ? f2[1][j] : c2[1][j],
-                                                   q4 == 3 ? f2[2][k] : c2[2][k], inv_r2);
+                        const float w = eq6_weight(q4, q4 == 1 ? df[0][i] : dc[0][i], q4 == 2 ? df[1][j] : dc[1][j],
+                                                   q4 == 3 ? df[2][k] : dc[2][k], inv_r2);
                         if (!(w > 0.0f)) continue;
                         const int at = at0 + (i * E + j) * E + k;
                         const float wm = w * mp;
@@ -476,22 +485,27 @@ __global__ __launch_bounds__(P2GTile<R>::NT) void k_mr_p2g_tile(MGrid g, int sub
             } else {
                 float zc[5], zf[5];
 #pragma unroll
-                for (int k = 0; k < 5; ++k) cell_dist2(t, 2, ic[2] - 2 + k, tb[2], px[2], zc[k], zf[k]);
+                for (int k = 0; k < 5; ++k) cell_dist(t, 2, ic[2] - 2 + k, tb[2], px[2], zc[k], zf[k]);
                 const float r2 = rp * rp;
                 for (int i = 0; i < 5; ++i) {
                     float xc, xf;
-                    cell_dist2(t, 0, ic[0] - 2 + i, tb[0], px[0], xc, xf);
+                    cell_dist(t, 0, ic[0] - 2 + i, tb[0], px[0], xc, xf);
+                    xc = square(xc);
+                    xf = square(xf);
                     if (fminf(xc, xf) >= r2) continue;
                     for (int j = 0; j < 5; ++j) {
                         float yc, yf;
-                        cell_dist2(t, 1, ic[1] - 2 + j, tb[1], px[1], yc, yf);
+                        cell_dist(t, 1, ic[1] - 2 + j, tb[1], px[1], yc, yf);
+                        yc = square(yc);
+                        yf = square(yf);
                         if (fminf(xc, xf) + fminf(yc, yf) >= r2) continue;
                         const int row = ((ic[0] - 2 + i - t.t0[0] + R) * E + ic[1] - 2 + j - t.t0[1] + R) * E +
                                         ic[2] - 2 - t.t0[2] + R;
 #pragma unroll
                         for (int k = 0; k < 5; ++k) {
-                            const float wt[4] = {eq6_weight(xc, yc, zc[k], inv_r2), eq6_weight(xf, yc, zc[k], inv_r2),
-                                                 eq6_weight(xc, yf, zc[k], inv_r2), eq6_weight(xc, yc, zf[k], inv_r2)};
+                            const float wt[4] = {
+                                eq6_weight(0, xc, yc, zc[k], inv_r2), eq6_weight(1, xf, yc, zc[k], inv_r2),
+                                eq6_weight(2, xc, yf, zc[k], inv_r2), eq6_weight(3, xc, yc, zf[k], inv_r2)};
 #pragma unroll
                             for (int q4 = 0; q4 < 4; ++q4) {
                                 if (!(wt[q4] > 0.0f)) continue;
@@ -991,6 +1005,12 @@ __global__ __launch_bounds__(256) void k_mr_g2p(MGrid g, const int* __restrict__
     for (int ax = 0; ax < 3; ++ax) v[3 * p + ax] = alpha * (vp[ax] + delta[ax]) + (1.0f - alpha) * pic[ax];
 }
 
+// x + dt (2 k1 + 3 k2 + 4 k3) / 9, with the roundings spelled out
+__device__ inline float rk3_end(float x, float dt, float k1, float k2, float k3) {
+#pragma clang fp contract(off)
+    return fmaf(dt, fmaf(2.0f / 9.0f, k1, (3.0f / 9.0f) * k2) + (4.0f / 9.0f) * k3, x);
+}
+
 // Ralston RK3 through the MSBG velocity, clamped to [lo, hi]
 // (mr_kernels.py:421-438), then the wall reflection of the velocity
 // (mr_kernels.py:441-461).  nbr as above.  9.2M particles: 1150 -> 669 us.
@@ -1024,7 +1044,7 @@ __global__ __launch_bounds__(256) void k_mr_advect(MGrid g, const int* __restric
     }
 #pragma unroll
     for (int ax = 0; ax < 3; ++ax) {
-        float xa = q[ax] + c.dt * ((2.0f / 9.0f) * k1[ax] + (3.0f / 9.0f) * k2[ax] + (4.0f / 9.0f) * k[ax]);
+        float xa = rk3_end(q[ax], c.dt, k1[ax], k2[ax], k[ax]);
         xa = fminf(fmaxf(xa, c.lo[ax]), c.hi[ax]);
         float va = v[3 * p + ax];
         if (xa <= c.lo[ax])
