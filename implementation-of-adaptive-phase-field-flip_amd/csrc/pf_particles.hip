@@ -1097,7 +1097,7 @@ __device__ inline void stage_fields(float* box, const G2PArgs& a, bool g2p, bool
 // STATE (PF_GA_STATE): states may have changed since the binning (the droplet
 // stage between G2P and advection), so each particle's is read: the advection
 // of 22.4M particles takes 480 us from the tiles, 600 through the global
-// fields, and leaves the bounds.
+// fields.
 template <bool STATE>
 __global__ __launch_bounds__(kG2PThreads) void k_g2p_tiled(G2PArgs a, const int* __restrict__ perm,
                                                            const int* __restrict__ start, int ntx, int nty,

@@ -56,6 +56,24 @@ def _rho_tilde_0(cfg: Config) -> float:
     return acc
 
 
+class _AsIs:
+    """A tensor as it is now: equal as long as it is the same tensor at the
+    same memory with no write through torch since.  The reference and the
+    alias are kept, so that neither an id nor an address comes back for
+    another tensor."""
+
+    __slots__ = ("tensor", "memory", "version")
+
+    def __init__(self, tensor):
+        self.tensor, self.memory, self.version = tensor, tensor.detach(), tensor._version
+
+    def __eq__(self, other):
+        return (self.tensor is other.tensor and self.memory.data_ptr() == other.memory.data_ptr()
+                and self.version == other.version)
+
+    __hash__ = None
+
+
 class Simulator:
     def __init__(self, cfg: Config):
         self.cfg = cfg
@@ -274,9 +292,9 @@ class Simulator:
                   _lib.ptr(self._p2g_stage), 8 * self._p2g_stage.numel(), _lib.stream())
 
     def _bounds_key(self):
-        # torch bumps _version on every in-place write through torch; the
+        # a replaced tensor and a write through torch both change the key; the
         # kernels here write through raw pointers and reset the token instead
-        return (self._particles_epoch, self.pv._version, self.pstate._version, self.pmass._version)
+        return (self._particles_epoch, _AsIs(self.pv), _AsIs(self.pstate), _AsIs(self.pmass))
 
     def _particle_bounds(self):
         """max |v| (CFL) and the P2G fixed-point bounds, on the device (kept
@@ -358,11 +376,11 @@ class Simulator:
             _lib.call("pf_g2p_advect_binned", ctypes.byref(a), *bins, None, None, _lib.stream())
             self._launch_droplets(dt)
             # the FLIP particles are still where they were binned, but the
-            # stage has changed states
+            # stage has changed states.  (Its bounds are not asked for: a
+            # program that steers droplets writes particles between steps by
+            # any means, so the next step looks at them anew.)
             a = self._g2p_args(_lib.GA_ADVECT | _lib.GA_REFLECT | _lib.GA_STATE, dt)
-            _lib.call("pf_g2p_advect_binned", ctypes.byref(a), *bins, _lib.ptr(self.pmass),
-                      _lib.ptr(self._bounds), _lib.stream())
-            self._bounds_token = self._bounds_key()
+            _lib.call("pf_g2p_advect_binned", ctypes.byref(a), *bins, None, None, _lib.stream())
         else:
             # the same pass leaves the next step's CFL / P2G bounds
             a = self._g2p_args(_lib.GA_G2P | _lib.GA_ADVECT | _lib.GA_REFLECT, dt)

@@ -880,6 +880,42 @@ def test_step_bounds_from_g2p_equal_max_speed(pf):
     assert sim._bounds_key() != key
 
 
+@pytest.mark.parametrize("droplets", [False, True])
+@pytest.mark.parametrize("how", ["pv", "pv.data", "pstate", "pmass", "pv in place", "nothing"])
+def test_step_bounds_follow_replaced_particles(pf, droplets, how):
+    """A step after its particle tensors were replaced (new ones start at
+    version 0, where the old ones stand too) takes its CFL step and P2G bounds
+    from the new ones."""
+    say(f"bounds after replacing {how}, droplets={droplets}")
+    cfg, sim = make(pf, 16, 8, vel_noise=0.3)
+    cfg.droplets = droplets
+    # the fastest particles are dead, so reviving them raises the bounds
+    st = torch.zeros_like(sim.pstate)
+    st[::3] = 2
+    v = sim.pv.clone()
+    v[::3] *= 5.0
+    sim.pstate, sim.pv = st.clone(), v.clone()
+    sim.step()
+    if how == "pv":
+        sim.pv = sim.pv * 4.0
+    elif how == "pv.data":
+        sim.pv.data = sim.pv * 4.0
+    elif how == "pstate":
+        sim.pstate = torch.zeros_like(sim.pstate)
+    elif how == "pmass":
+        sim.pmass = sim.pmass * 3.0
+    elif how == "pv in place":
+        sim.pv.mul_(4.0)
+    sim._particle_bounds()
+    got = np_(sim._bounds)[:3].copy()
+    sim._bounds_token = None
+    sim._particle_bounds()
+    assert np.array_equal(np_(sim._bounds)[:3], got)
+    if how == "pv" or how == "pv.data":
+        v = np_(sim.pv)[np_(sim.pstate) == 0]
+        assert abs(got[0] / np.sqrt((v ** 2).sum(1)).max() - 1) < 1e-6
+
+
 # ------------------------------------------------------------------ whole step
 @pytest.mark.parametrize("n,ppc", [(16, 8), (16, 27)])
 def test_step_matches_oracle(pf, n, ppc):
