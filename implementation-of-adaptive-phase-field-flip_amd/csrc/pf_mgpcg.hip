@@ -2768,14 +2768,15 @@ static bool fold_residual_test(const pf_mg& mg) {
 
 // The inner products after the V-cycle ride on its last level-0 kernel when
 // that is the post phase or a plain fused sweep (at least two post-sweeps on
-// an HBM level 0) whose workgroups fit the partials array.
+// an HBM level 0) whose workgroups fit the partials array.  A grid that cannot
+// be halved has no post-smoothing: its only level ends with the mean removal.
 static int64_t dot_blocks(const pf_mg& mg) {
     const Dims d = ldims(mg.lev[0]);
     return level_fused(mg, 0) ? (int64_t)phase_tiles(d, phase_tile(d)) : sweep_tiles(d, sweep_shape(d, mg.precision != 0));
 }
 static bool fold_dots(const pf_mg& mg) {
-    return !(mg.options & PF_MG_SEPARATE_DOTS) && mg.small_from > 0 && (mg.post >= 2 || level_fused(mg, 0)) &&
-           fused_smoother(mg, 0) && dot_blocks(mg) <= PS;
+    return !(mg.options & PF_MG_SEPARATE_DOTS) && mg.nlev > 1 && mg.small_from > 0 &&
+           (mg.post >= 2 || level_fused(mg, 0)) && fused_smoother(mg, 0) && dot_blocks(mg) <= PS;
 }
 
 template <typename ST>

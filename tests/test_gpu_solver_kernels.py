@@ -98,3 +98,39 @@ def test_sweep_tiles_equal_half_sweeps(pf, res, precision):
         out.append((z.cpu().numpy(), p.cpu().numpy(), it, rel))
     assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
     assert out[0][2:] == out[1][2:]
+
+
+def _residual(beta, b, p):
+    """max |b - mean b - A p| / max |b - mean b| in FP64."""
+    b, p = b.double(), p.double()
+    b = b - b.mean()
+    r = b.clone()
+    for a, f in enumerate(beta):
+        n = p.shape[a]
+        flux = f.double().narrow(a, 1, n - 1) * (p.narrow(a, 1, n - 1) - p.narrow(a, 0, n - 1))
+        r.narrow(a, 0, n - 1).add_(flux)
+        r.narrow(a, 1, n - 1).sub_(flux)
+    return float(r.abs().max() / b.abs().max())
+
+
+# nx odd, one axis too short, more than 1024 sweep tiles; nz even throughout,
+# so that level 0 has fused sweeps
+@pytest.mark.parametrize("res", [(25, 24, 32), (6, 64, 64), (161, 160, 160)])
+@pytest.mark.parametrize("precision", ["fp32", "bf16", "fp16"])
+def test_solve_on_a_grid_that_cannot_be_halved(pf, res, precision):
+    """A hierarchy of one level above the sizes that one workgroup takes.  The
+    FP32 recursive residual follows b - A p to within the rounding of its
+    updates, some 1e-6 of max |b| here."""
+    print(f"[gpu] one level {res} {precision}", flush=True)
+    rng = np.random.default_rng(8)
+    g = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()  # noqa: E731
+    beta = [g(b) for b in _beta(res, rng, False)]
+    b = g(rng.standard_normal(res).astype(np.float32))
+    s = pf.MGPCG(res, "cuda:0", pre=3, post=3, precision=precision)
+    assert s.nlev == 1 and s.small_from == 1
+    s.build_hierarchy(*beta)
+    p = torch.zeros_like(b)
+    for _ in range(2):  # the second from the captured graphs
+        it, rel = s.solve(b, p, tol=1e-4, max_iter=400)
+        assert 0 < it < 400 and rel < 1e-4
+        assert _residual(beta, b, p) < 1.2e-4
