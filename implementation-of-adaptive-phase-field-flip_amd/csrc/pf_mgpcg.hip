@@ -2661,8 +2661,10 @@ static int vcycle(const pf_mg& mg, const float* r0, ST* z0, const int* done, con
             PF_CHECK_LAUNCH();
             k_comb<<<1, RT, 0, s>>>(st, C_MEAN, (int)red_blocks(n), n, &st->mu_x, 0.0);
             PF_CHECK_LAUNCH();
-            k_shift<ST, ST><<<red_blocks(n), RT, 0, s>>>(cur[l], cur[l], n, &st->mu_x);
+            // (an odd number of sweeps ends in the second buffer)
+            k_shift<ST, ST><<<red_blocks(n), RT, 0, s>>>(cur[l], P(l), n, &st->mu_x);
             PF_CHECK_LAUNCH();
+            cur[l] = P(l);
         }
     }
     for (int l = G - 1; l >= 0; --l) {

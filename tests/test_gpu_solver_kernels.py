@@ -23,17 +23,17 @@ def _beta(res, rng, walls):
     return out
 
 
-def _vcycle_error(pf, res, precision, walls, pre=3, post=3, min_dim=4):
+def _vcycle_error(pf, res, precision, walls, pre=3, post=3, min_dim=4, coarsest=60):
     rng = np.random.default_rng(17)
     beta = _beta(res, rng, walls)
     r = rng.standard_normal(res).astype(np.float32)
     r -= r.mean()
     g = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()  # noqa: E731
-    solver = pf.MGPCG(res, "cuda:0", pre=pre, post=post, precision=precision, min_dim=min_dim)
+    solver = pf.MGPCG(res, "cuda:0", pre=pre, post=post, precision=precision, min_dim=min_dim, coarsest=coarsest)
     solver.build_hierarchy(*[g(b) for b in beta])
     z = torch.zeros(res, device="cuda")
     solver.precondition(g(r), z)
-    o = O.MGPCGOracle(res, pre=pre, post=post, min_dim=min_dim)
+    o = O.MGPCGOracle(res, pre=pre, post=post, min_dim=min_dim, coarsest=coarsest)
     o.build_hierarchy(*beta)
     ref = o.precondition(r.astype(np.float64))
     return float(np.linalg.norm(z.cpu().numpy() - ref) / np.linalg.norm(ref))
@@ -134,3 +134,13 @@ def test_solve_on_a_grid_that_cannot_be_halved(pf, res, precision):
         it, rel = s.solve(b, p, tol=1e-4, max_iter=400)
         assert 0 < it < 400 and rel < 1e-4
         assert _residual(beta, b, p) < 1.2e-4
+
+
+@pytest.mark.parametrize("res", [(25, 24, 32), (25, 24, 31), (50, 48, 62)])
+@pytest.mark.parametrize("coarsest", [1, 7, 8])
+def test_odd_number_of_coarsest_sweeps(pf, res, coarsest):
+    """An odd number of fused sweeps ends in the level's second buffer: the
+    result of a one-level hierarchy is moved from there (nz even; in place for
+    an odd nz; and on a level below another)."""
+    print(f"[gpu] coarsest sweeps {res} {coarsest}", flush=True)
+    assert _vcycle_error(pf, res, "fp32", False, coarsest=coarsest) < 2e-5
