@@ -319,9 +319,18 @@ struct TileRef {
     float h, bext;
 };
 
+// position along axis a in cells of the block.  Without contraction: both tile
+// kernels and p2g_class place a particle by it, and a particle that they
+// placed in different cells would be splatted twice or not at all.
+__device__ inline float block_coord(const TileRef& t, int a, float x) {
+#pragma clang fp contract(off)
+    return (x - (float)t.b[a] * t.bext) / t.h;
+}
+
 // How a particle whose centre lies in the tile is splatted: 0, 1: by the
 // R = 1, 2 tile kernel, 2: by the walk.  ok: which of the 27 blocks around
-// exist at the tile's level.
+// exist at the tile's level.  (The other float operation that decides,
+// touched_blocks, has no product to fuse: r is r0 times a power of two.)
 __device__ inline int p2g_class(const MGrid& g, const TileRef& t, unsigned ok, const float (&x)[3], float r0,
                                 float rp, int lp, int2 (&blk)[3], int (&ic)[3]) {
     const int nb[3] = {g.nbx, g.nby, g.nbz};
@@ -329,7 +338,7 @@ __device__ inline int p2g_class(const MGrid& g, const TileRef& t, unsigned ok, c
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
         blk[a] = touched_blocks(x[a], rp, t.bext, nb[a]);
-        ic[a] = (int)floorf((x[a] - (float)t.b[a] * t.bext) / t.h);
+        ic[a] = (int)floorf(block_coord(t, a, x[a]));
         in = in && (unsigned)(ic[a] - t.t0[a]) < (unsigned)t.tn && blk[a].x >= t.b[a] - 1 && blk[a].y <= t.b[a] + 1;
     }
     const int d = lp - t.level;
@@ -445,8 +454,7 @@ __global__ __launch_bounds__(P2GTile<R>::NT) void k_mr_p2g_tile(MGrid g, int sub
                 int lc[3], lf[3];
 #pragma unroll
                 for (int a = 0; a < 3; ++a) {
-                    const float gx = (px[a] - (float)t.b[a] * t.bext) / t.h;
-                    const int it = gx - (float)ic[a] < 0.5f ? ic[a] - 1 : ic[a];
+                    const int it = block_coord(t, a, px[a]) - (float)ic[a] < 0.5f ? ic[a] - 1 : ic[a];
                     float unused;
                     cell_dist(t, a, it, tb[a], px[a], dc[a][0], unused);
                     cell_dist(t, a, it + 1, tb[a], px[a], dc[a][1], unused);

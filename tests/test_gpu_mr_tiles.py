@@ -50,6 +50,40 @@ def test_tiled_p2g_equals_per_particle_atomics(nb, n0, max_level, seed):
     assert np.abs(out[0]["fmass"]).max() > 0
 
 
+@pytest.mark.parametrize("n0,level", [(16, 0), (32, 1), (8, 0)])
+@pytest.mark.parametrize("coarser", [0, 1])
+def test_particles_at_tile_edges_are_splatted_once(n0, level, coarser):
+    """Particles of the tiles' level and one level coarser, on tile and block
+    edges and a few units in the last place beside them, with a spacing that
+    is no power of two: the two tile kernels and the walk share them out
+    without losing one or taking one twice."""
+    from importlib import import_module
+    pf = load_pkg()
+    cfgm, mrs = (import_module(pf.__name__ + "." + m) for m in ("config", "mr_sim"))
+    print(f"[gpu] tile edges n0={n0} level={level} coarser={coarser}", flush=True)
+    rng = np.random.default_rng(6)
+    nb, dx = (5, 4, 3), 0.37 / 11
+    cfg = cfgm.Config(res=tuple(n * n0 for n in nb), dx=dx, ppc=27, droplets=False)
+    sim = mrs.AdaptiveSimulator(cfg, nb, n0=n0, max_level=2, frozen_levels=np.full(int(np.prod(nb)), level))
+    n, edge = 30000, (8 << level) * np.float32(dx)
+    cells = np.array(nb) * n0 // (8 << level)
+    x = (rng.random((n, 3)) * np.array(nb) * n0 * dx).astype(np.float32)
+    on = rng.integers(0, 3, n)  # the axis along which it sits at an edge
+    at = (rng.integers(1, np.maximum(cells, 2)[on], n).astype(np.float32) * edge).view(np.int32)
+    x[np.arange(n), on] = (at + rng.integers(-3, 4, n).astype(np.int32)).view(np.float32)
+    lev = np.full(n, level + coarser, np.int32)
+    sim.set_particles(x, rng.standard_normal((n, 3)).astype(np.float32), np.ones(n, np.int32), lev)
+    sim._rebuild_grid(1e-3)
+    prm = sim._params(1e-3, sim._max_speed())
+    out = []
+    for sorted_ in (True, False):
+        sim.p2g_sorted = sorted_
+        sim.stage_p2g(prm)
+        out.append({k: getattr(sim, k).cpu().numpy().copy() for k in ("cwsum", "phi", "fmass", "fvel", "is_liquid")})
+    for k in out[0]:
+        assert np.array_equal(out[0][k], out[1][k]), k
+
+
 @pytest.mark.parametrize("nb,n0,levels", [((8, 8, 8), 2, "one"), ((3, 3, 3), 4, "jump"), ((1, 2, 1), 4, "one"),
                                           ((7, 7, 9), 2, "one")])
 def test_coarse_level_matrix_matches_the_sweeps(nb, n0, levels):
