@@ -836,12 +836,73 @@ __device__ inline float sample_face(const MGrid& g, const float* __restrict__ f,
                 if (w <= 0.0f) continue;
                 const MCell nc = locate_near(g, br, (i0 + di) * ext, (j0 + dj) * ext, (k0 + dk) * ext);
                 if (nc.addr < 0) continue;
-                acc += w * f[nc.addr * 3 + ax];
+                acc = fmaf(w, f[nc.addr * 3 + ax], acc);
                 wsum += w;
             }
         }
     }
     return wsum > 0.0f ? acc / wsum : 0.0f;
+}
+
+// Without a table (see below), G2P samples two fields at one point through the
+// same taps: the taps of the three staggered components (weight and cell
+// address; -1: not summed, a zero weight or no cell) are resolved once and the
+// 48 values loaded together: 9.2M particles 672 us, 1210 with a walk per
+// component and field.  The advection's three samples at three points are
+// walked per component: with the taps batched per point it took 1.38 ms instead
+// of 1.20 (more registers, the out-of-block lookups still serial), and with
+// one body for the three stages 1.65 instead of 1.05.
+struct WalkTaps {
+    float w[3][8];
+    int addr[3][8];
+};
+
+__device__ inline void walk_taps(const MGrid& g, float x, float y, float z, const SamplePoint& sp, WalkTaps& t) {
+    const MCell& c = sp.c;
+    const BlockRef& br = sp.br;
+    const int ext = 1 << c.level;
+    const float h = cell_size(g, c.level);
+#pragma unroll
+    for (int ax = 0; ax < 3; ++ax) {
+        const float sx = x / h - (ax == 0 ? 0.0f : 0.5f);
+        const float sy = y / h - (ax == 1 ? 0.0f : 0.5f);
+        const float sz = z / h - (ax == 2 ? 0.0f : 0.5f);
+        const float fi = floorf(sx), fj = floorf(sy), fk = floorf(sz);
+        const int i0 = (int)fi, j0 = (int)fj, k0 = (int)fk;
+        const float tx = sx - fi, ty = sy - fj, tz = sz - fk;
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            const int di = q >> 2, dj = (q >> 1) & 1, dk = q & 1;
+            const float w = tap_weight(di ? tx : 1.0f - tx, dj ? ty : 1.0f - ty, dk ? tz : 1.0f - tz);
+            t.w[ax][q] = w;
+            t.addr[ax][q] =
+                w > 0.0f ? locate_near(g, br, (i0 + di) * ext, (j0 + dj) * ext, (k0 + dk) * ext).addr : -1;
+        }
+    }
+}
+
+// The tap values of field f (address -1 reads entry 0, masked in the sum):
+// all 24 loads are issued before the first is used.
+__device__ inline void walk_values(const float* __restrict__ f, const WalkTaps& t, float (&v)[3][8]) {
+#pragma unroll
+    for (int ax = 0; ax < 3; ++ax)
+#pragma unroll
+        for (int q = 0; q < 8; ++q) v[ax][q] = f[max(t.addr[ax][q], 0) * 3 + ax];
+}
+
+// sample_face's sums for the three components
+__device__ inline void walk_sum(const WalkTaps& t, const float (&v)[3][8], float (&out)[3]) {
+#pragma unroll
+    for (int ax = 0; ax < 3; ++ax) {
+        float acc = 0.0f, wsum = 0.0f;
+#pragma unroll
+        for (int q = 0; q < 8; ++q)
+            if (t.addr[ax][q] >= 0) {
+                acc = fmaf(t.w[ax][q], v[ax][q], acc);
+                wsum += t.w[ax][q];
+            }
+        out[ax] = wsum > 0.0f ? acc / wsum : 0.0f;
+    }
 }
 
 // Where a sample's 24 taps are: per axis the two lattice points of a face
@@ -948,7 +1009,7 @@ __device__ inline void tap_sum(const SampleTaps& t, const int (&addr)[3][8], con
 #pragma unroll
         for (int q = 0; q < 8; ++q) {
             const float w = tap_weight(t.w[0][ax != 0][q >> 2], t.w[1][ax != 1][q >> 1 & 1], t.w[2][ax != 2][q & 1]);
-            acc += w * v[ax][q];
+            acc = fmaf(w, v[ax][q], acc);
             wsum += w;
         }
         out[ax] = wsum > 0.0f ? acc / wsum : 0.0f;
@@ -983,8 +1044,10 @@ __global__ __launch_bounds__(256) void k_mr_neighbours(MGrid g, int* __restrict_
 
 // alpha_FLIP from the local grid spacing (particles.py:251-276), then
 // u_p = alpha (u_p + I(du)) + (1 - alpha) I(u), eq. (12) (mr_kernels.py:413-430).
-// nbr: see sample_taps; NULL, or a tap in a block of another level: the walk.
-// 9.2M particles, 6 % of them along 2:1 jumps: 630 -> 274 us.
+// NEAR: with the table of sample_taps, the walk only for a particle that has a
+// tap in a block of another level.  9.2M particles, 6 % of them along 2:1
+// jumps: 672 us without the table, 371 with it.
+template <bool NEAR>
 __global__ __launch_bounds__(256) void k_mr_g2p(MGrid g, const int* __restrict__ nbr, const float* __restrict__ x,
                                                 float* __restrict__ v, const int* __restrict__ type, int64_t n,
                                                 MRConst c, const float* __restrict__ fvel,
@@ -992,25 +1055,40 @@ __global__ __launch_bounds__(256) void k_mr_g2p(MGrid g, const int* __restrict__
     const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= n) return;
     const float q[3] = {x[3 * p], x[3 * p + 1], x[3 * p + 2]};
-    float vp[3] = {v[3 * p], v[3 * p + 1], v[3 * p + 2]};
+    const float vp[3] = {v[3 * p], v[3 * p + 1], v[3 * p + 2]};
     const float nu = type[p] == 1 ? c.nu_l : c.nu_g;
     float delta[3] = {0.0f, 0.0f, 0.0f}, pic[3] = {0.0f, 0.0f, 0.0f};
-    SampleTaps t;
-    const bool in = sample_taps(g, q, t);
-    if (in) {
-        int addr[3][8];
-        if (nbr && tap_addresses(t, nbr, addr)) {
-            tap_sum(t, addr, fdvel, delta);
-            tap_sum(t, addr, fvel, pic);
-        } else {
-            sample_walk(g, fdvel, q, delta);
-            sample_walk(g, fvel, q, pic);
+    int level = 0;
+    if constexpr (NEAR) {
+        SampleTaps t;
+        if (sample_taps(g, q, t)) {
+            level = t.level;
+            int addr[3][8];
+            if (tap_addresses(t, nbr, addr)) {
+                tap_sum(t, addr, fdvel, delta);
+                tap_sum(t, addr, fvel, pic);
+            } else {
+                sample_walk(g, fdvel, q, delta);
+                sample_walk(g, fvel, q, pic);
+            }
+        }
+    } else {
+        const SamplePoint sp = sample_point(g, q[0], q[1], q[2]);
+        if (sp.c.addr >= 0) {
+            level = sp.c.level;
+            WalkTaps t;
+            walk_taps(g, q[0], q[1], q[2], sp, t);
+            float vd[3][8], vu[3][8];
+            walk_values(fdvel, t, vd);
+            walk_values(fvel, t, vu);
+            walk_sum(t, vd, delta);
+            walk_sum(t, vu, pic);
         }
     }
-    const float dx = cell_size(g, in ? t.level : 0);
+    const float dx = cell_size(g, level);
     const float alpha = fminf(fmaxf(1.0f - 6.0f * nu * c.dt / (dx * dx), 0.0f), c.alpha_cap);
 #pragma unroll
-    for (int ax = 0; ax < 3; ++ax) v[3 * p + ax] = alpha * (vp[ax] + delta[ax]) + (1.0f - alpha) * pic[ax];
+    for (int ax = 0; ax < 3; ++ax) v[3 * p + ax] = fmaf(1.0f - alpha, pic[ax], alpha * (vp[ax] + delta[ax]));
 }
 
 // x + dt (2 k1 + 3 k2 + 4 k3) / 9, with the roundings spelled out
@@ -1021,8 +1099,9 @@ __device__ inline float rk3_end(float x, float dt, float k1, float k2, float k3)
 
 // Ralston RK3 through the MSBG velocity, clamped to [lo, hi]
 // (mr_kernels.py:421-438), then the wall reflection of the velocity
-// (mr_kernels.py:441-461).  nbr as above.  9.2M particles: 1150 -> 669 us.
-// One body for the three stages keeps it at 123 registers.
+// (mr_kernels.py:441-461).  NEAR as above; one body for the three stages keeps
+// it at 123 registers.  9.2M particles: 1048 us without the table, 682 with it.
+template <bool NEAR>
 __global__ __launch_bounds__(256) void k_mr_advect(MGrid g, const int* __restrict__ nbr, float* __restrict__ x,
                                                    float* __restrict__ v, int64_t n, MRConst c,
                                                    const float* __restrict__ fvel) {
@@ -1030,25 +1109,42 @@ __global__ __launch_bounds__(256) void k_mr_advect(MGrid g, const int* __restric
     if (p >= n) return;
     const float q[3] = {x[3 * p], x[3 * p + 1], x[3 * p + 2]};
     float k[3] = {0.0f, 0.0f, 0.0f}, k1[3], k2[3];
+    if constexpr (NEAR) {
 #pragma unroll 1
-    for (int s = 0; s < 3; ++s) {
-        const float a = s == 0 ? 0.0f : (s == 1 ? 0.5f * c.dt : 0.75f * c.dt);
-        float y[3];
+        for (int s = 0; s < 3; ++s) {
+            const float a = s == 0 ? 0.0f : (s == 1 ? 0.5f * c.dt : 0.75f * c.dt);
+            float y[3];
 #pragma unroll
-        for (int ax = 0; ax < 3; ++ax) {
-            k1[ax] = s == 1 ? k[ax] : k1[ax];
-            k2[ax] = s == 2 ? k[ax] : k2[ax];
-            y[ax] = s == 0 ? q[ax] : q[ax] + a * k[ax];
-            k[ax] = 0.0f;
+            for (int ax = 0; ax < 3; ++ax) {
+                k1[ax] = s == 1 ? k[ax] : k1[ax];
+                k2[ax] = s == 2 ? k[ax] : k2[ax];
+                y[ax] = s == 0 ? q[ax] : fmaf(a, k[ax], q[ax]);
+                k[ax] = 0.0f;
+            }
+            SampleTaps t;
+            if (sample_taps(g, y, t)) {
+                int addr[3][8];
+                if (tap_addresses(t, nbr, addr))
+                    tap_sum(t, addr, fvel, k);
+                else
+                    sample_walk(g, fvel, y, k);
+            }
         }
-        SampleTaps t;
-        if (sample_taps(g, y, t)) {
-            int addr[3][8];
-            if (nbr && tap_addresses(t, nbr, addr))
-                tap_sum(t, addr, fvel, k);
-            else
-                sample_walk(g, fvel, y, k);
-        }
+    } else {
+        float y[3];
+        SamplePoint sp = sample_point(g, q[0], q[1], q[2]);
+#pragma unroll
+        for (int ax = 0; ax < 3; ++ax) k1[ax] = sample_face(g, fvel, q[0], q[1], q[2], ax, sp);
+#pragma unroll
+        for (int ax = 0; ax < 3; ++ax) y[ax] = fmaf(0.5f * c.dt, k1[ax], q[ax]);
+        sp = sample_point(g, y[0], y[1], y[2]);
+#pragma unroll
+        for (int ax = 0; ax < 3; ++ax) k2[ax] = sample_face(g, fvel, y[0], y[1], y[2], ax, sp);
+#pragma unroll
+        for (int ax = 0; ax < 3; ++ax) y[ax] = fmaf(0.75f * c.dt, k2[ax], q[ax]);
+        sp = sample_point(g, y[0], y[1], y[2]);
+#pragma unroll
+        for (int ax = 0; ax < 3; ++ax) k[ax] = sample_face(g, fvel, y[0], y[1], y[2], ax, sp);
     }
 #pragma unroll
     for (int ax = 0; ax < 3; ++ax) {
@@ -1424,8 +1520,9 @@ PF_API int pf_mr_g2p_near(const pf_msbg_grid* g, const int32_t* nbr, const pf_mr
     if (rc) return rc;
     PF_REQUIRE(prm && f && f->fvel && f->fdvel, "pf_mr_g2p: null field");
     if (ps->n == 0) return PF_OK;
-    k_mr_g2p<<<pgrid(ps->n), 256, 0, S(stream)>>>(mgrid(*g), nbr, ps->x, ps->v, ps->type, ps->n, mrconst(*prm), f->fvel,
-                                                  f->fdvel);
+    const auto k = nbr ? k_mr_g2p<true> : k_mr_g2p<false>;
+    k<<<pgrid(ps->n), 256, 0, S(stream)>>>(mgrid(*g), nbr, ps->x, ps->v, ps->type, ps->n, mrconst(*prm), f->fvel,
+                                           f->fdvel);
     PF_CHECK_LAUNCH();
     return PF_OK;
 }
@@ -1443,7 +1540,8 @@ PF_API int pf_mr_advect_near(const pf_msbg_grid* g, const int32_t* nbr, const pf
     if (rc) return rc;
     PF_REQUIRE(prm && fvel, "pf_mr_advect: null pointer");
     if (ps->n == 0) return PF_OK;
-    k_mr_advect<<<pgrid(ps->n), 256, 0, S(stream)>>>(mgrid(*g), nbr, ps->x, ps->v, ps->n, mrconst(*prm), fvel);
+    const auto k = nbr ? k_mr_advect<true> : k_mr_advect<false>;
+    k<<<pgrid(ps->n), 256, 0, S(stream)>>>(mgrid(*g), nbr, ps->x, ps->v, ps->n, mrconst(*prm), fvel);
     PF_CHECK_LAUNCH();
     return PF_OK;
 }
