@@ -851,7 +851,7 @@ __device__ inline float sample_face(const MGrid& g, const float* __restrict__ f,
 // component and field.  The advection's three samples at three points are
 // walked per component: with the taps batched per point it took 1.38 ms instead
 // of 1.20 (more registers, the out-of-block lookups still serial), and with
-// one body for the three stages 1.65 instead of 1.05.
+// one body for the three stages 1.65 instead of 1.04.
 struct WalkTaps {
     float w[3][8];
     int addr[3][8];
@@ -1009,7 +1009,7 @@ __device__ inline void tap_sum(const SampleTaps& t, const int (&addr)[3][8], con
 #pragma unroll
         for (int q = 0; q < 8; ++q) {
             const float w = tap_weight(t.w[0][ax != 0][q >> 2], t.w[1][ax != 1][q >> 1 & 1], t.w[2][ax != 2][q & 1]);
-            acc = fmaf(w, v[ax][q], acc);
+            acc = w > 0.0f ? fmaf(w, v[ax][q], acc) : acc;  // (a tap of weight 0 may be no number)
             wsum += w;
         }
         out[ax] = wsum > 0.0f ? acc / wsum : 0.0f;
@@ -1046,7 +1046,7 @@ __global__ __launch_bounds__(256) void k_mr_neighbours(MGrid g, int* __restrict_
 // u_p = alpha (u_p + I(du)) + (1 - alpha) I(u), eq. (12) (mr_kernels.py:413-430).
 // NEAR: with the table of sample_taps, the walk only for a particle that has a
 // tap in a block of another level.  9.2M particles, 6 % of them along 2:1
-// jumps: 672 us without the table, 371 with it.
+// jumps: 672 us without the table, 378 with it.
 template <bool NEAR>
 __global__ __launch_bounds__(256) void k_mr_g2p(MGrid g, const int* __restrict__ nbr, const float* __restrict__ x,
                                                 float* __restrict__ v, const int* __restrict__ type, int64_t n,
@@ -1100,7 +1100,7 @@ __device__ inline float rk3_end(float x, float dt, float k1, float k2, float k3)
 // Ralston RK3 through the MSBG velocity, clamped to [lo, hi]
 // (mr_kernels.py:421-438), then the wall reflection of the velocity
 // (mr_kernels.py:441-461).  NEAR as above; one body for the three stages keeps
-// it at 123 registers.  9.2M particles: 1048 us without the table, 682 with it.
+// it at 123 registers.  9.2M particles: 1036 us without the table, 690 with it.
 template <bool NEAR>
 __global__ __launch_bounds__(256) void k_mr_advect(MGrid g, const int* __restrict__ nbr, float* __restrict__ x,
                                                    float* __restrict__ v, int64_t n, MRConst c,

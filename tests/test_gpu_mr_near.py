@@ -67,3 +67,59 @@ def test_near_is_the_walk(mods, nb, n0, levels, speed):
     for a, b in zip(*runs):
         assert torch.isfinite(a).all() and torch.equal(a, b)
     assert not torch.equal(runs[0][1], x)
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+@pytest.mark.parametrize("axis", [0, 1, 2])
+def test_taps_of_weight_zero_are_not_read_into_the_sum(mods, axis, bad):
+    """Points on lattice planes: the tap beyond has weight exactly 0, and what
+    stands there (here no number, on the planes beside them) does not count,
+    with the table as without it."""
+    print("mr near zero weights", axis, bad, flush=True)
+    lib = mods["_lib"]
+    rng = np.random.default_rng(12)
+    h0, nb, n0 = 1.0 / 16, (2, 2, 2), 8
+    g = mods["msbg"].MSBG(nb, n0=n0, h0=h0, device="cuda:0", max_level=0)
+    g.build(np.zeros(8, np.int32))
+    cell = (g.geometry()[0] / h0).floor().int()[:, axis]
+    n = 4000
+    x = rng.uniform(1.0, 15.0, (n, 3))
+    x[:, axis] = 2 * rng.integers(1, 7, n) + 0.5 * rng.integers(0, 2, n)  # faces 2m, centres 2m (+ 1/2)
+    t = lambda a, d=np.float32: torch.from_numpy(a.astype(d)).cuda()  # noqa: E731
+    fvel, fdvel = (t(rng.standard_normal((g.ncells, 3))) for _ in range(2))
+    half = t(x)[:, axis].frac() == 0.5
+    X = t(x * h0)
+    prm = lib.MrParams()
+    prm.dt, prm.nu_l, prm.nu_g, prm.alpha_cap = 0.0, 1e-4, 2e-4, 0.999
+    prm.lo[:], prm.hi[:] = [-10.0] * 3, [10.0] * 3
+    ones = torch.ones(n, dtype=torch.int32, device="cuda")
+    out = {}
+    for kind in ("own", "others"):
+        # along the axis the component of that axis lies on 2m (weight 0 at
+        # 2m + 1) and the others on 2m + 1/2 (weight 0 at the next centre)
+        comps = [axis] if kind == "own" else [a for a in range(3) if a != axis]
+        pick = ~half if kind == "own" else half
+        for poison in (False, True):
+            fv, fd = fvel.clone(), fdvel.clone()
+            if poison:
+                for f in (fv, fd):
+                    for a in comps:
+                        f[cell % 2 == 1, a] = bad
+            f = lib.MrFields()
+            f.fvel, f.fdvel = fv.data_ptr(), fd.data_ptr()
+            for nbr in (None, g.neighbours()):
+                p, v = X.clone(), torch.zeros_like(X)
+                ps = lib.MrParticles()
+                ps.n, ps.x, ps.v = n, p.data_ptr(), v.data_ptr()
+                ps.type = ps.level = ps.defer = ones.data_ptr()
+                B = ctypes.byref
+                lib.call("pf_mr_g2p_near", g.ref(), lib.ptr(nbr), B(ps), B(prm), B(f), lib.stream())
+                # (no time passes, but 0 times no number is none)
+                lib.call("pf_mr_advect_near", g.ref(), lib.ptr(nbr), B(ps), B(prm), lib.ptr(fv), lib.stream())
+                torch.cuda.synchronize()
+                out[kind, poison, nbr is None] = torch.stack([p[pick][:, comps], v[pick][:, comps]])
+        want = out[kind, False, True]
+        assert want.numel() > 2000 and torch.isfinite(want).all() and torch.equal(want[0], X[pick][:, comps])
+        for poison in (False, True):
+            for table in (False, True):
+                assert torch.equal(out[kind, poison, table], want), (kind, poison, table)
