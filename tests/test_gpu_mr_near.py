@@ -123,3 +123,32 @@ def test_taps_of_weight_zero_are_not_read_into_the_sum(mods, axis, bad):
         for poison in (False, True):
             for table in (False, True):
                 assert torch.equal(out[kind, poison, table], want), (kind, poison, table)
+
+
+def test_table_on_other_streams_and_under_capture(mods):
+    """The table is written by a kernel on the stream that first asks for it:
+    another stream waits for that kernel, and a capture goes without a table
+    that its stream has not written."""
+    print("mr near streams", flush=True)
+    rng = np.random.default_rng(5)
+    g = mods["msbg"].MSBG((6, 5, 4), n0=8, h0=1.0 / 16, device="cuda:0", max_level=2)
+    g.build(rng.integers(0, 3, 120).astype(np.int32))
+    want = g.neighbours().cpu()
+    side = torch.cuda.Stream()
+    for first in (side, torch.cuda.current_stream()):
+        other = torch.cuda.current_stream() if first is side else side
+        g.build(g.level_h)
+        with torch.cuda.stream(first):
+            torch.cuda._sleep(20_000_000)  # some milliseconds
+            nbr = g.neighbours()
+        with torch.cuda.stream(other):
+            got = g.neighbours().clone()
+        torch.cuda.synchronize()
+        assert g.neighbours() is nbr and torch.equal(got.cpu(), want) and torch.equal(nbr.cpu(), want)
+    x = torch.zeros(1, device="cuda")
+    g.build(g.level_h)
+    for _ in range(2):  # before and after the table is there
+        with torch.cuda.graph(torch.cuda.CUDAGraph()):
+            x += 1
+            assert g.neighbours() is None
+        assert torch.equal(g.neighbours().cpu(), want)
