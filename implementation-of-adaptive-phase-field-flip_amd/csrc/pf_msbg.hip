@@ -935,9 +935,11 @@ __global__ __launch_bounds__(256) void k_vec_jacobi(const float* __restrict__ r,
 // all positions is contiguous); rows with more (a cell facing finer ones) are
 // marked by bit 31 of the last and keep the rest in `more`, in order of arrival
 // (which changes no result).  A coarse cell has 3 couplings more than faces for
-// each finer block it faces, and a block of (2 m)^3 cells is faced by at most
-// 6 m^2 coarser cells, so 18 m^2 <= 9/4 (2 m)^3 bounds `more`.  Same couplings,
-// same order and same arithmetic as the kernels without the table.
+// each finer block it faces, however much finer (always a 2x2 patch), and a
+// block of (2 m)^3 cells is faced by at most 6 m^2 coarser cells, so 18 m^2 <=
+// 9/4 (2 m)^3 bounds `more` for any map of levels, graded 2:1 or not (the
+// largest share, on blocks of 2^3 cells between blocks of one).  Same
+// couplings, same order and same arithmetic as the kernels without the table.
 constexpr int kRowIn = 6;
 
 struct MRows {

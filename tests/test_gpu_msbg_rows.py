@@ -25,6 +25,9 @@ def mods():
     ((1, 1, 2), 2, "coarse"), ((3, 3, 3), 2, "coarse"), ((3, 3, 3), 2, "checker"), ((3, 5, 3), 2, "random"),
     ((5, 5, 5), 4, "random"), ((2, 4, 4), 4, "fine"), ((8, 8, 8), 2, "fine"), ((8, 8, 9), 2, "fine"),
     ((17, 9, 13), 2, "checker"), ((6, 5, 7), 8, "random"), ((4, 4, 8), 16, "random"), ((5, 6, 7), 16, "random"),
+    # jumps of several levels, and the map with the most couplings past six per cell
+    ((6, 5, 7), 8, "ungraded"), ((5, 6, 7), 16, "ungraded"), ((9, 11, 7), 4, "ungraded checker"),
+    ((17, 18, 19), 2, "ungraded checker"),
 ])
 def test_rows_are_the_walk(mods, nb, n0, levels):
     print("msbg rows", nb, n0, levels, flush=True)
@@ -34,9 +37,10 @@ def test_rows_are_the_walk(mods, nb, n0, levels):
     nblk = int(np.prod(nb))
     lv = {"coarse": np.full(nblk, top), "fine": np.zeros(nblk),
           "checker": np.indices(nb).sum(0).reshape(-1) % 2,
-          "random": rng.integers(0, top + 1, nblk)}[levels].astype(np.int32)
+          "ungraded checker": np.indices(nb).sum(0).reshape(-1) % 2 * top,
+          "random": (lv := rng.integers(0, top + 1, nblk)), "ungraded": lv}[levels].astype(np.int32)
     g = mods["msbg"].MSBG(nb, n0=n0, h0=1.0 / 24, device="cuda:0", max_level=top)
-    g.build(lv)
+    g.build(lv, grade=not levels.startswith("ungraded"))
     n = g.ncells
     t32 = lambda a: torch.from_numpy(a.astype(np.float32)).cuda()  # noqa: E731
     row = mods["mr_multigrid"]._MGLevel(g)
