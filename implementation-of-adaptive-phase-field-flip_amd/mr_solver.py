@@ -29,7 +29,8 @@ class MRSolver:
         n = grid.ncells
         self.n = n
         z = lambda: torch.zeros(n, dtype=torch.float32, device=grid.dev)  # noqa: E731
-        self.diag, self.r, self.zv, self.q, self.Ap, self.b, self.r_prev = (z() for _ in range(7))
+        self.diag = self.mg.levels[0].diag if self.mg is not None else z()
+        self.r, self.zv, self.q, self.Ap, self.b, self.r_prev = (z() for _ in range(6))
         nw = int(_lib.load().pf_vec_reduce_bytes()) // 8
         self._work = torch.zeros(nw, dtype=torch.float64, device=grid.dev)
         # one reduction buffer per scalar of an iteration; the state and flag
@@ -40,8 +41,7 @@ class MRSolver:
 
     def prepare(self, bface):
         if self.mg is not None:
-            self.mg.build_hierarchy(bface)
-            self.diag.copy_(self.mg.levels[0].diag)
+            self.mg.build_hierarchy(bface)  # with the diagonal
         else:
             mro._diag(self.grid, bface, self.diag)
 
