@@ -522,13 +522,13 @@ def test_fused_smoother_is_bitwise_split(pf, res, pre, post, precision):
     """The fused full-sweep smoother (LDS tile, halo recomputation, ping-pong
     buffers) and the one-launch phases of the small levels give exactly the
     bits of two in-place half-sweeps per sweep, including partial tiles and
-    odd sweep counts; 68 x 136 x 120 takes the large-level kernel (from 2^20
-    cells) with partial tiles along i and k, and 104 x 118 x 190 (585 tiles)
-    with partial tiles along j and k.  One-launch phases: level 1 of 64^3
-    (32^3, pre 2 / post 1) and of 128 x 64 x 32 (pre 1 / post 2), level 2 of
-    128^3, level 1 of 68 x 60 x 44 (34 x 30 x 22: partial tiles on every
-    axis), and level 1 of 112 x 112 x 20 (56 x 56 x 10, whose coarse level
-    28 x 28 x 5 is the coarsest and runs out of HBM)."""
+    odd sweep counts; level 0 of 128^3 takes 8x8x64 tiles, 68 x 136 x 120
+    8x8x32 ones with partial tiles along i and k, and 104 x 118 x 190 (1170
+    tiles) with partial tiles along j and k.  One-launch phases: levels 0 and 1
+    of 64^3 (pre 2 / post 1) and of 128 x 64 x 32 (pre 1 / post 2), levels 1
+    and 2 of 128^3, levels 0 and 1 of 68 x 60 x 44 (34 x 30 x 22: partial tiles
+    on every axis), and level 1 of 112 x 112 x 20 (56 x 56 x 10, whose coarse
+    level 28 x 28 x 5 is the coarsest and runs in one workgroup)."""
     say(f"fused smoother {res} pre={pre} post={post} {precision}")
     rng = np.random.default_rng(11)
     bx, by, bz = random_beta(res, rng, 1000.0)
@@ -570,9 +570,9 @@ def test_fused_smoother_solve_is_bitwise_split(pf):
 
 @pytest.mark.parametrize("precision", ["fp32", "bf16", "fp16"])
 def test_fused_levels_solve_is_bitwise_split(pf, precision):
-    """Whole FPCG solves at 128^3 with the 32^3 level's smoothing phases as
-    one launch each and as one launch per sweep: same iterations, residual
-    and pressure bit for bit."""
+    """Whole FPCG solves at 128^3 with the smoothing phases of the 64^3 and
+    32^3 levels as one launch each and as one launch per sweep: same
+    iterations, residual and pressure bit for bit."""
     say(f"fused levels solve 128^3 {precision}")
     res = (128, 128, 128)
     rng = np.random.default_rng(15)
@@ -601,8 +601,10 @@ def test_inner_products_on_the_last_sweep_match_their_own_kernel(pf, res, precis
     own: the two FPCG runs differ only by the order of FP64 additions (which
     can also move a 16-bit V-cycle's power-of-two input scale), so they take
     the same iterations to within two and reach pressures equal to 1e-5 of
-    their size, the bound the solver tests hold every precision to.  128^3 takes the 8x8x64 tiles, 64^3 the 8x8x16 ones, 40 x
-    48 x 56 the small ones with partial tiles along i and k."""
+    their size, the bound the solver tests hold every precision to.  128^3
+    takes the 8x8x64 sweep tiles, 64^3 and 40 x 48 x 56 the post phase in one
+    launch (the latter with partial tiles along k); the other sweep tiles are
+    in test_gpu_solver_kernels.py."""
     say(f"inner products on the last sweep {res} {precision}")
     rng = np.random.default_rng(14)
     bx, by, bz = random_beta(res, rng, 1000.0)

@@ -75,8 +75,8 @@ def test_small_hierarchy_in_one_workgroup(pf, res, min_dim, walls, pre, post):
     assert _vcycle_error(pf, res, "fp32", walls, pre, post, min_dim) < 2e-5
 
 
-# 8 x 8 x 32 tiles: whole, cut along every axis; 1152 tiles (inner products of
-# a solve on the last sweep); 8 x 8 x 64 tiles beside them
+# 8 x 8 x 32 tiles: whole, cut along every axis, 1152 of them; 8 x 8 x 64 tiles
+# beside them
 @pytest.mark.parametrize("res,precision", [((96, 88, 96), "fp32"), ((100, 90, 84), "fp32"), ((104, 120, 100), "bf16"),
                                            ((192, 128, 96), "fp16"), ((128, 64, 192), "bf16")])
 def test_sweep_tiles_equal_half_sweeps(pf, res, precision):
@@ -98,6 +98,57 @@ def test_sweep_tiles_equal_half_sweeps(pf, res, precision):
         out.append((z.cpu().numpy(), p.cpu().numpy(), it, rel))
     assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
     assert out[0][2:] == out[1][2:]
+
+
+def _solve_both(pf, res, precision, tell, pre=3, post=3, **kw):
+    """Six FPCG iterations and a V-cycle with two settings of a solver."""
+    rng = np.random.default_rng(21)
+    g = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()  # noqa: E731
+    beta = [g(b) for b in _beta(res, rng, False)]
+    r = g(rng.standard_normal(res).astype(np.float32))
+    out = []
+    for v in (True, False):
+        s = pf.MGPCG(res, "cuda:0", pre=pre, post=post, precision=precision, **{tell: v}, **kw)
+        s.build_hierarchy(*beta)
+        z, p = torch.zeros_like(r), torch.zeros_like(r)
+        s.precondition(r, z)
+        it, rel = s.solve(r, p, tol=1e-30, max_iter=6)
+        out.append((z.cpu().numpy(), p.cpu().numpy().astype(np.float64), it, rel))
+    return out
+
+
+# one partial per tile: 1152 and cut 8 x 8 x 32 tiles, 8 x 8 x 16 and 4 x 8 x 16
+# (whole and cut), cut 8 x 8 x 64 ones, and the post phase of a level 0 with cut
+# tiles
+@pytest.mark.parametrize("res,split", [((192, 128, 96), False), ((100, 90, 84), False), ((80, 80, 80), False),
+                                       ((64, 64, 64), True), ((52, 60, 44), True), ((32, 32, 32), True),
+                                       ((40, 48, 56), True),
+                                       ((124, 100, 128), False), ((40, 48, 56), False), ((22, 30, 26), False)])
+@pytest.mark.parametrize("precision", ["fp32", "bf16", "fp16"])
+def test_inner_products_of_every_tile_shape(pf, res, split, precision):
+    """The CG's inner products from the last level-0 kernel of a V-cycle
+    against a kernel of their own.  The two differ by the order of FP64
+    additions, so a scalar that scales a vector differs by one unit in the
+    last place of FP32 at most, and rarely; six iterations carry 1e-5 of the
+    result, as in the solver tests."""
+    print(f"[gpu] inner products {res} split={split} {precision}", flush=True)
+    a, b = _solve_both(pf, res, precision, "fold_dots", split_levels=split)
+    assert np.array_equal(a[0], b[0]) and a[2] == b[2] == 6
+    assert np.abs(a[1] - b[1]).max() < 1e-5 * np.abs(b[1]).max()
+
+
+# tiles of 8 x 8 x 16 cells cut along k and along every axis, of 4 x 4 x 8 cut
+# along every axis and along k, on level 0 and on the levels below
+@pytest.mark.parametrize("res", [(40, 48, 56), (36, 28, 44), (22, 30, 26), (20, 28, 12), (60, 68, 76)])
+@pytest.mark.parametrize("pre,post", [(3, 3), (1, 2), (2, 1)])
+@pytest.mark.parametrize("precision", ["fp32", "bf16", "fp16"])
+def test_phases_with_cut_tiles_equal_sweeps(pf, res, pre, post, precision):
+    """Smoothing phases in one launch each against one launch per sweep, bit
+    for bit, over a V-cycle and a solve (which takes its residual test from
+    level 0's first kernel)."""
+    print(f"[gpu] phases {res} {pre}+{post} {precision}", flush=True)
+    a, b = _solve_both(pf, res, precision, "split_levels", pre, post, fold_dots=False)
+    assert np.array_equal(a[0], b[0]) and np.array_equal(a[1], b[1]) and a[2:] == b[2:]
 
 
 def _residual(beta, b, p):
