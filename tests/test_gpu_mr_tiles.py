@@ -17,6 +17,8 @@ pytestmark = pytest.mark.gpu
     ((4, 3, 5), 8, 3, 3),    # down to one cell per block
     ((5, 4, 3), 2, 1, 4),    # blocks of 2 and of 1 cells: every support crosses blocks
     ((1, 1, 1), 8, 0, 5),    # one block: every neighbour is missing
+    ((2, 2, 1), 64, 6, 6),   # 512 tiles down to one cell per block
+    ((3, 2, 2), 64, 1, 7),
 ])
 def test_tiled_p2g_equals_per_particle_atomics(nb, n0, max_level, seed):
     from importlib import import_module
@@ -47,6 +49,33 @@ def test_tiled_p2g_equals_per_particle_atomics(nb, n0, max_level, seed):
     for k in out[0]:
         assert np.array_equal(out[0][k], out[1][k]), k
         assert np.array_equal(out[2][k], out[1][k]), k
+    assert np.abs(out[0]["fmass"]).max() > 0
+
+
+def test_tiled_p2g_on_coarse_levels_of_large_blocks():
+    """8192 blocks of 512^3 finest cells, all at one cell per block: as many
+    tiles as blocks, where 2^31 would be one for every 8^3 finest cells."""
+    from importlib import import_module
+    pf = load_pkg()
+    cfgm, mrs = (import_module(pf.__name__ + "." + m) for m in ("config", "mr_sim"))
+    print("[gpu] tiled adaptive P2G, one cell per 512^3 block", flush=True)
+    rng = np.random.default_rng(8)
+    nb, n0, dx = (32, 16, 16), 512, 0.37 / 512
+    cfg = cfgm.Config(res=tuple(n * n0 for n in nb), dx=dx, ppc=27, droplets=False)
+    sim = mrs.AdaptiveSimulator(cfg, nb, n0=n0, max_level=9, frozen_levels=np.full(int(np.prod(nb)), 9))
+    n = 30000
+    x = (rng.random((n, 3)) * np.array(nb) * n0 * dx).astype(np.float32)
+    sim.set_particles(x, rng.standard_normal((n, 3)).astype(np.float32), np.ones(n, np.int32),
+                      rng.choice([8, 9], n).astype(np.int32))
+    sim._rebuild_grid(1e-3)
+    prm = sim._params(1e-3, sim._max_speed())
+    out = []
+    for sorted_ in (True, False):
+        sim.p2g_sorted = sorted_
+        sim.stage_p2g(prm)
+        out.append({k: getattr(sim, k).cpu().numpy().copy() for k in ("cwsum", "phi", "fmass", "fvel", "is_liquid")})
+    for k in out[0]:
+        assert np.array_equal(out[0][k], out[1][k]), k
     assert np.abs(out[0]["fmass"]).max() > 0
 
 
