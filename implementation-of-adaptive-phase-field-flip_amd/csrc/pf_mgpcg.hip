@@ -2343,8 +2343,18 @@ static int ensure_small_lds() {
 //   192x128x96     17.3 / 18.2   14.8 / 14.1   17.5 / 15.3
 //   160^3          26.6 / 28.1   24.0 / 21.6   29.4 / 25.3
 //   256^3           112 / 82.4    123 / 73.0    164 / 89.8
+//   320x320x8        --           17.6 / 16.6   11.4 / 10.8
+//   512x512x16      66.2 / 73.1   34.0 / 35.4   21.3 / 21.0
+//   300x300x18      27.2 / 26.5   15.0 / 15.0   16.8 / 16.5
+//   160x160x40       --           11.2 / 11.2    9.4 /  9.1
+//   192x192x40      16.0 / 16.4   13.3 / 13.1   12.6 / 11.4
+//   256x256x48      20.5 / 21.0   19.7 / 20.1   20.8 / 17.9
+//   200x200x80      25.6 / 27.7   20.5 / 20.7   23.5 / 20.6
 // So 8x8x64 where its tiles are whole along k, in 16 bits only while they are
-// all resident at once (two per CU); otherwise 8x8x32 from 5 x 2^17 cells.
+// all resident at once (two per CU); otherwise 8x8x32 from 5 x 2^17 cells,
+// unless it is padded by another 8x8x16 tile of one or of three: that is its
+// whole gain and more up to 16 cells along k, and from 33 to 48 in 16 bits or
+// below 2^21 cells.
 enum SweepShape { SWEEP_64, SWEEP_32, SWEEP_16, SWEEP_SMALL };
 
 static int64_t sweep_tiles(const Dims& d, SweepShape s) {
@@ -2355,7 +2365,8 @@ static int64_t sweep_tiles(const Dims& d, SweepShape s) {
 static SweepShape sweep_shape(const Dims& d, bool half) {
     const int64_t n = (int64_t)d.nx * d.ny * d.nz;
     if (n >= (int64_t)1 << 20 && d.nz % 64 == 0 && (!half || sweep_tiles(d, SWEEP_64) <= 512)) return SWEEP_64;
-    if (n >= (int64_t)5 << 17) return SWEEP_32;
+    const bool padded = d.nz <= 16 || (d.nz > 32 && d.nz <= 48 && (half || n < (int64_t)1 << 21));
+    if (n >= (int64_t)5 << 17 && !padded) return SWEEP_32;
     return n >= (int64_t)1 << 17 ? SWEEP_16 : SWEEP_SMALL;
 }
 

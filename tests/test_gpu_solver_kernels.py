@@ -76,9 +76,11 @@ def test_small_hierarchy_in_one_workgroup(pf, res, min_dim, walls, pre, post):
 
 
 # 8 x 8 x 32 tiles: whole, cut along every axis, 1152 of them; 8 x 8 x 64 tiles
-# beside them
+# beside them; 8 x 8 x 16 where the longer ones would be padded most
 @pytest.mark.parametrize("res,precision", [((96, 88, 96), "fp32"), ((100, 90, 84), "fp32"), ((104, 120, 100), "bf16"),
-                                           ((192, 128, 96), "fp16"), ((128, 64, 192), "bf16")])
+                                           ((192, 128, 96), "fp16"), ((128, 64, 192), "bf16"),
+                                           ((260, 256, 12), "fp32"), ((260, 256, 16), "bf16"),
+                                           ((148, 140, 36), "bf16"), ((212, 208, 48), "fp32")])
 def test_sweep_tiles_equal_half_sweeps(pf, res, precision):
     """The fused sweeps of every tile shape against two half-sweep launches
     per sweep, bit for bit, over a V-cycle and a solve of 6 iterations (the
