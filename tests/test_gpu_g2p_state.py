@@ -71,3 +71,27 @@ def test_advection_after_state_changes(pf, res, speed, solids, change):
     assert torch.equal(sim.px, x1) and torch.equal(sim.pv, v1)
     assert torch.equal(b2[:3], b1) and float(b2[3]) == 7.0
     assert change == "all dead" or not torch.equal(v1, v0) or not torch.equal(x1, x0)
+
+
+@pytest.mark.parametrize("res,ppc,live,tiles", [((64, 64, 64), 8, 0, True), ((64, 64, 64), 8, 200000, False),
+                                                ((64, 64, 56), 8, 0, False), ((64, 64, 64), 1, 0, False)])
+def test_both_advections_give_the_same_step(pf, res, ppc, live, tiles):
+    """Steps with the droplet stage on both sides of the rule that chooses the
+    advection (tiles, particles per tile, live droplets), bit for bit."""
+    print("state step", res, ppc, live, flush=True)
+    out = []
+    for forced in (None, True, False):
+        cfg = pf.Config(res=res, dx=1.0 / 64, ppc=ppc, droplets=True, delta_phi=0.05)
+        sim = pf.Simulator(cfg)
+        sim.set_particles(*pf.scenes.dam_break(cfg, frac=(0.4, 1.0, 0.6)))
+        rng = np.random.default_rng(5)
+        sim.pv.copy_(torch.from_numpy(rng.standard_normal((sim.n_particles, 3)).astype(np.float32)))
+        sim._live_droplets = live
+        assert sim._advect_from_tiles() == tiles
+        if forced is not None:
+            sim._advect_from_tiles = lambda: forced
+        recs = [sim.step(2e-3) for _ in range(2)]
+        out.append((sim.px.clone(), sim.pv.clone(), sim.pstate.clone(), recs[-1]["droplets"], recs[-1]["pcg_iter"]))
+        print("  droplets", [r["droplets"] for r in recs], flush=True)
+    for o in out[1:]:
+        assert all(torch.equal(a, b) for a, b in zip(o[:3], out[0][:3])) and o[3:] == out[0][3:]
