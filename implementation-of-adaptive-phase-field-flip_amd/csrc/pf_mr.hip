@@ -14,6 +14,8 @@
 // P2G adds into 64-bit fixed-point accumulators (one power-of-two scale per
 // quantity, chosen on the host from the largest single contribution), so
 // the sums do not depend on the order of the atomics.
+#include <algorithm>
+
 #include "pf_msbg.hpp"
 
 namespace pf {
@@ -285,7 +287,7 @@ __global__ __launch_bounds__(256) void k_mr_cell_scatter(const int* __restrict__
                                                          const int* __restrict__ start, int64_t n,
                                                          int* __restrict__ perm, int* __restrict__ nlist) {
     const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (p == 0) *nlist = 0;  // the particles k_mr_p2g_tile leaves to the cached walk
+    if (p < 2) nlist[p] = 0;  // what k_mr_p2g_tile leaves to the walk: particles, whole tiles
     if (p >= n) return;
     perm[start[key[p]] + rank[p]] = (int)p;
 }
@@ -299,13 +301,15 @@ __global__ __launch_bounds__(256) void k_mr_cell_scatter(const int* __restrict__
 // per axis), which fill a ring of blocks that a neighbouring finer level has
 // refined; in both every block the support touches must have this block's
 // level.  What remains (about 0.5 % of the particles of a settled dam break,
-// along the 2:1 jumps, and those outside the grid) is left to k_mr_p2g_list.  The sums are those of
-// the per-particle walk bit for bit: the same cells, weights and fixed-point
-// roundings, and integer adds.
-// A hash of cells in LDS for every particle (what k_mr_p2g_list does) was
+// along the 2:1 jumps, and those outside the grid) is left to k_mr_p2g_walk: up
+// to kP2GLight of a tile by a list, more by naming the tile (they are marked in
+// the order, ~p).  The sums are those of the per-particle walk bit for bit: the
+// same cells, weights and fixed-point roundings, and integer adds.
+// A hash of cells in LDS for every particle (what k_mr_p2g_walk does) was
 // bound by its lookups, one per touched cell.
 // 128^3 grid, 9.2M particles (6 % one level coarser than their block):
-// 4.95 -> 1.02 ms (0.47 own level, 0.33 one coarser, 0.22 the walk).
+// 4.95 -> 0.95 ms (0.41 own level, 0.32 one coarser, 0.22 the walk).
+constexpr int kP2GLight = 512;
 template <int R>
 struct P2GTile {
     static constexpr int E = 8 + 2 * R, E3 = E * E * E;
@@ -361,179 +365,211 @@ __device__ inline void cell_dist(const TileRef& t, int a, int i, const int2& blk
     f = touched ? d - 0.5f * t.h : 1e15f;
 }
 
-// Workgroups: one per 512 cells of the grid, then one per block.  The multiples
-// of 512 among a block's cell addresses are as many as its tiles if it has at
-// least 8 cells per axis, so the workgroup of such an address takes one of
-// them; a smaller block is its own workgroup's tile.  (One workgroup for every
-// tile of a block at level 0 left nearly all idle on coarse levels of large
-// blocks: 512 blocks of 64^3 finest cells at level 3, 262144 workgroups for 512
-// tiles, P2G 1.28 ms instead of 0.17.)
+// Workgroups: one per 512 cells of the grid.  The multiples of 512 among a
+// block's cell addresses are as many as its tiles if it has at least 8 cells
+// per axis, so the workgroup of such an address takes one of them.  (One
+// workgroup for every tile of a block at level 0 left nearly all idle on coarse
+// levels of large blocks: 512 blocks of 64^3 finest cells at level 3, 262144
+// workgroups for 512 tiles, P2G 1.28 ms instead of 0.17.)  Then up to
+// kP2GWhole that look for the blocks of 4 cells per axis, a tile each.  Smaller
+// blocks are left to the walk: at 8 particles per cell, P2G of 13824 of 2^3
+// cells took 0.38 ms with tiles and takes 0.33, of 32768 of one cell 0.87 and
+// 0.16.
+constexpr int kP2GWhole = 1024;
+
 template <int R>
 __global__ __launch_bounds__(P2GTile<R>::NT) void k_mr_p2g_tile(MGrid g, int chunks, const float* __restrict__ x,
                                                                 const float* __restrict__ v,
                                                                 const int* __restrict__ type,
                                                                 const int* __restrict__ lev,
-                                                                const int* __restrict__ perm,
+                                                                int* __restrict__ perm,
                                                                 const int* __restrict__ start, MRConst c,
                                                                 int* __restrict__ coarse_tile, int* __restrict__ list,
-                                                                int* __restrict__ nlist,
+                                                                int2* __restrict__ heavy, int* __restrict__ nlist,
                                                                 unsigned long long* __restrict__ acc) {
     using PT = P2GTile<R>;
     constexpr int E = PT::E, E3 = PT::E3, NT = PT::NT;
     __shared__ unsigned long long L[kAcc * E3];
-    __shared__ int s_ok;
+    __shared__ int s_ok, s_n, s_at;
+    __shared__ int s_walk[R == 1 ? kP2GLight : 1];
     const bool whole = (int)blockIdx.x >= chunks;
-    const int wg = whole ? 0 : xcd_block(blockIdx.x, chunks);
-    const int slot = whole ? blockIdx.x - chunks : g.cslot[512 * wg];
-    TileRef t;
-    t.level = g.blev[slot];
-    t.nn = g.n0 >> t.level;
-    t.base = g.coff[slot];
-    if (whole != (t.nn < 8)) return;
-    t.tn = min(t.nn, 8);
-    const int ns = t.nn / t.tn;  // tiles per axis
-    const int sub = whole ? 0 : wg - (t.base + 511) / 512;
-    int* flag = coarse_tile + t.base + sub;  // (a block has at least as many cells as tiles)
-    if (R == 2 && *flag == 0) return;
-    const int blk = g.blk[slot];
-    t.b[2] = blk % g.nbz;
-    t.b[1] = (blk / g.nbz) % g.nby;
-    t.b[0] = blk / (g.nbz * g.nby);
-    t.t0[0] = sub / (ns * ns) * t.tn;
-    t.t0[1] = sub / ns % ns * t.tn;
-    t.t0[2] = sub % ns * t.tn;
-    t.h = cell_size(g, t.level);
-    t.bext = (float)g.n0 * g.h0;
-    const int tid = threadIdx.x;
-    for (int e = tid; e < kAcc * E3; e += NT) L[e] = 0ull;
-    if (tid < 64) {
-        bool same = false;
-        if (tid < 27) {
-            const int i = t.b[0] + tid / 9 - 1, j = t.b[1] + tid / 3 % 3 - 1, k = t.b[2] + tid % 3 - 1;
-            if (i >= 0 && j >= 0 && k >= 0 && i < g.nbx && j < g.nby && k < g.nbz) {
-                const int s = g.slot[(i * g.nby + j) * g.nbz + k];
-                same = s >= 0 && g.blev[s] == t.level;
+    // (the R = 2 tiles lie together in the order: dealt out over the XCDs)
+    const int wg = whole ? 0 : (R == 1 ? xcd_block(blockIdx.x, chunks) : blockIdx.x);
+    if (R == 2 && !whole && coarse_tile[wg] == 0) return;
+    const int step = whole ? gridDim.x - chunks : g.nslots;
+    for (int slot = whole ? blockIdx.x - chunks : g.cslot[512 * wg]; slot < g.nslots; slot += step) {
+        TileRef t;
+        t.level = g.blev[slot];
+        t.nn = g.n0 >> t.level;
+        if (whole ? t.nn != 4 : t.nn < 8) continue;
+        t.base = g.coff[slot];
+        t.tn = min(t.nn, 8);
+        const int ns = t.nn / t.tn;  // tiles per axis
+        const int sub = whole ? 0 : wg - (t.base + 511) / 512;
+        int* flag = coarse_tile + (whole ? chunks + t.base : wg);
+        if (R == 2 && *flag == 0) continue;
+        const int blk = g.blk[slot];
+        t.b[2] = blk % g.nbz;
+        t.b[1] = (blk / g.nbz) % g.nby;
+        t.b[0] = blk / (g.nbz * g.nby);
+        t.t0[0] = sub / (ns * ns) * t.tn;
+        t.t0[1] = sub / ns % ns * t.tn;
+        t.t0[2] = sub % ns * t.tn;
+        t.h = cell_size(g, t.level);
+        t.bext = (float)g.n0 * g.h0;
+        const int tid = threadIdx.x;
+        // entries of the tile and its ring: all E3 of a tile of 8^3 cells
+        const int ext = t.tn + 2 * R, ext3 = ext * ext * ext;
+        const auto entry = [&](int e, int& i, int& j, int& k) {
+            if (ext == E) {  // (divisions by constants)
+                k = e % E;
+                j = e / E % E;
+                i = e / (E * E);
+                return e;
+            }
+            k = e % ext;
+            j = e / ext % ext;
+            i = e / (ext * ext);
+            return (i * E + j) * E + k;
+        };
+        if (t.tn == 8) {
+            for (int e = tid; e < kAcc * E3; e += NT) L[e] = 0ull;
+        } else {
+            for (int e = tid; e < ext3; e += NT) {
+                int i, j, k;
+                const int at = entry(e, i, j, k);
+#pragma unroll
+                for (int ch = 0; ch < kAcc; ++ch) L[ch * E3 + at] = 0ull;
             }
         }
-        const unsigned long long m = __ballot(same);
-        if (tid == 0) s_ok = (int)(unsigned)m;
-    }
-    __syncthreads();
-    const unsigned ok = (unsigned)s_ok;
-    const int tn3 = t.tn * t.tn * t.tn;
-    bool coarse = false;
-    // lanes of a wave take different cells; the threads beyond one per cell
-    // share its particles
-    const int parts = tn3 <= NT ? NT / tn3 : 1;
-    const int cell0 = tid % tn3, part = min(tid / tn3, parts);
-    if (part < parts) {
-        const int li = cell0 / (t.tn * t.tn), lj = cell0 / t.tn % t.tn, lk = cell0 % t.tn;
-        const int addr = t.base + ((t.t0[0] + li) * t.nn + t.t0[1] + lj) * t.nn + t.t0[2] + lk;
-        const unsigned e0 = start[addr + 1];
-        for (unsigned q = start[addr] + part; q < e0; q += parts) {
-            const int p = perm[q];
-            const float px[3] = {x[3 * (int64_t)p], x[3 * (int64_t)p + 1], x[3 * (int64_t)p + 2]};
-            const float vel[3] = {v[3 * (int64_t)p], v[3 * (int64_t)p + 1], v[3 * (int64_t)p + 2]};
-            const int lp = lev[p];
-            const float mp = (type[p] == 1 ? c.rho_l : c.rho_g) * (float)(1 << (3 * lp));
-            const float rp = c.r0 * (float)(1 << lp);
-            const float inv_r2 = 1.0f / (rp * rp);
-            int2 tb[3];
-            int ic[3];
-            const int cls = p2g_class(g, t, ok, px, c.r0, rp, lp, tb, ic);
-            if (R == 1) {
-                if (cls == 1) coarse = true;
-                if (cls == 2) {  // one atomic for the lanes that are here
-                    const unsigned long long m = __ballot(1);
-                    const int lane = tid & 63, first = __ffsll((long long)m) - 1;
-                    int at = 0;
-                    if (lane == first) at = atomicAdd(nlist, __popcll(m));
-                    at = __shfl(at, first, 64);
-                    list[at + __popcll(m & ((1ull << lane) - 1))] = p;
+        if (tid == 0) s_n = 0;
+        if (tid < 64) {
+            bool same = false;
+            if (tid < 27) {
+                const int i = t.b[0] + tid / 9 - 1, j = t.b[1] + tid / 3 % 3 - 1, k = t.b[2] + tid % 3 - 1;
+                if (i >= 0 && j >= 0 && k >= 0 && i < g.nbx && j < g.nby && k < g.nbz) {
+                    const int s = g.slot[(i * g.nby + j) * g.nbz + k];
+                    same = s >= 0 && g.blev[s] == t.level;
                 }
             }
-            if (cls != R - 1) continue;
-            auto add = [&](int ch, int at, float value, float scale) {
-                atomicAdd(L + ch * E3 + at, (unsigned long long)fixed(value, scale));
-            };
-            if constexpr (R == 1) {
-                // per axis: the two centres (first index it) and the two low
-                // faces (first index ic) within the radius: squared distances
-                // along x and y, distances along z
-                float dc[3][2], df[3][2];
-                int lc[3], lf[3];
-#pragma unroll
-                for (int a = 0; a < 3; ++a) {
-                    const int it = block_coord(t, a, px[a]) - (float)ic[a] < 0.5f ? ic[a] - 1 : ic[a];
-                    float unused;
-                    cell_dist(t, a, it, tb[a], px[a], dc[a][0], unused);
-                    cell_dist(t, a, it + 1, tb[a], px[a], dc[a][1], unused);
-                    cell_dist(t, a, ic[a], tb[a], px[a], unused, df[a][0]);
-                    cell_dist(t, a, ic[a] + 1, tb[a], px[a], unused, df[a][1]);
-#pragma unroll
-                    for (int e = 0; e < 2 && a < 2; ++e) {
-                        dc[a][e] = square(dc[a][e]);
-                        df[a][e] = square(df[a][e]);
+            const unsigned long long m = __ballot(same);
+            if (tid == 0) s_ok = (int)(unsigned)m;
+        }
+        __syncthreads();
+        const unsigned ok = (unsigned)s_ok;
+        const int tn3 = t.tn * t.tn * t.tn;
+        bool coarse = false;
+        // lanes of a wave take different cells; the threads beyond one per cell
+        // share its particles
+        const int parts = tn3 <= NT ? NT / tn3 : 1;
+        const int cell0 = tid % tn3, part = min(tid / tn3, parts);
+        if (part < parts) {
+            const int li = cell0 / (t.tn * t.tn), lj = cell0 / t.tn % t.tn, lk = cell0 % t.tn;
+            const int addr = t.base + ((t.t0[0] + li) * t.nn + t.t0[1] + lj) * t.nn + t.t0[2] + lk;
+            const unsigned e0 = start[addr + 1];
+            for (unsigned q = start[addr] + part; q < e0; q += parts) {
+                const int p = perm[q];
+                if (R == 2 && p < 0) continue;  // left to the walk
+                const float px[3] = {x[3 * (int64_t)p], x[3 * (int64_t)p + 1], x[3 * (int64_t)p + 2]};
+                const float vel[3] = {v[3 * (int64_t)p], v[3 * (int64_t)p + 1], v[3 * (int64_t)p + 2]};
+                const int lp = lev[p];
+                const float mp = (type[p] == 1 ? c.rho_l : c.rho_g) * (float)(1 << (3 * lp));
+                const float rp = c.r0 * (float)(1 << lp);
+                const float inv_r2 = 1.0f / (rp * rp);
+                int2 tb[3];
+                int ic[3];
+                const int cls = p2g_class(g, t, ok, px, c.r0, rp, lp, tb, ic);
+                if (R == 1) {
+                    if (cls == 1) coarse = true;
+                    if (cls == 2) {
+                        const int at = atomicAdd(&s_n, 1);
+                        if (at < kP2GLight) s_walk[at] = p;
+                        perm[q] = ~p;
                     }
-                    lc[a] = it - t.t0[a] + R;
-                    lf[a] = ic[a] - t.t0[a] + R;
                 }
+                if (cls != R - 1) continue;
+                auto add = [&](int ch, int at, float value, float scale) {
+                    atomicAdd(L + ch * E3 + at, (unsigned long long)fixed(value, scale));
+                };
+                if constexpr (R == 1) {
+                    // per axis: the two centres (first index it) and the two low
+                    // faces (first index ic) within the radius: squared distances
+                    // along x and y, distances along z
+                    float dc[3][2], df[3][2];
+                    int lc[3], lf[3];
 #pragma unroll
-                for (int q4 = 0; q4 < 4; ++q4) {
-                    // q4 = 0: centres, 1-3: low faces of axis q4 - 1
-                    const int at0 = ((q4 == 1 ? lf[0] : lc[0]) * E + (q4 == 2 ? lf[1] : lc[1])) * E +
-                                    (q4 == 3 ? lf[2] : lc[2]);
+                    for (int a = 0; a < 3; ++a) {
+                        const int it = block_coord(t, a, px[a]) - (float)ic[a] < 0.5f ? ic[a] - 1 : ic[a];
+                        float unused;
+                        cell_dist(t, a, it, tb[a], px[a], dc[a][0], unused);
+                        cell_dist(t, a, it + 1, tb[a], px[a], dc[a][1], unused);
+                        cell_dist(t, a, ic[a], tb[a], px[a], unused, df[a][0]);
+                        cell_dist(t, a, ic[a] + 1, tb[a], px[a], unused, df[a][1]);
 #pragma unroll
-                    for (int m = 0; m < 8; ++m) {
-                        const int i = m >> 2, j = (m >> 1) & 1, k = m & 1;
-                        const float w = eq6_weight(q4, q4 == 1 ? df[0][i] : dc[0][i], q4 == 2 ? df[1][j] : dc[1][j],
-                                                   q4 == 3 ? df[2][k] : dc[2][k], inv_r2);
-                        if (!(w > 0.0f)) continue;
-                        const int at = at0 + (i * E + j) * E + k;
-                        const float wm = w * mp;
-                        if (q4 == 0) {
-                            add(0, at, wm, c.mass_scale);
-                            add(1, at, w, c.w_scale);
-                        } else {
-                            add(1 + q4, at, wm, c.mass_scale);
-                            add(4 + q4, at, wm * vel[q4 - 1], c.mom_scale);
+                        for (int e = 0; e < 2 && a < 2; ++e) {
+                            dc[a][e] = square(dc[a][e]);
+                            df[a][e] = square(df[a][e]);
+                        }
+                        lc[a] = it - t.t0[a] + R;
+                        lf[a] = ic[a] - t.t0[a] + R;
+                    }
+#pragma unroll
+                    for (int q4 = 0; q4 < 4; ++q4) {
+                        // q4 = 0: centres, 1-3: low faces of axis q4 - 1
+                        const int at0 = ((q4 == 1 ? lf[0] : lc[0]) * E + (q4 == 2 ? lf[1] : lc[1])) * E +
+                                        (q4 == 3 ? lf[2] : lc[2]);
+#pragma unroll
+                        for (int m = 0; m < 8; ++m) {
+                            const int i = m >> 2, j = (m >> 1) & 1, k = m & 1;
+                            const float w = eq6_weight(q4, q4 == 1 ? df[0][i] : dc[0][i], q4 == 2 ? df[1][j] : dc[1][j],
+                                                       q4 == 3 ? df[2][k] : dc[2][k], inv_r2);
+                            if (!(w > 0.0f)) continue;
+                            const int at = at0 + (i * E + j) * E + k;
+                            const float wm = w * mp;
+                            if (q4 == 0) {
+                                add(0, at, wm, c.mass_scale);
+                                add(1, at, w, c.w_scale);
+                            } else {
+                                add(1 + q4, at, wm, c.mass_scale);
+                                add(4 + q4, at, wm * vel[q4 - 1], c.mom_scale);
+                            }
                         }
                     }
-                }
-            } else {
-                float zc[5], zf[5];
+                } else {
+                    float zc[5], zf[5];
 #pragma unroll
-                for (int k = 0; k < 5; ++k) cell_dist(t, 2, ic[2] - 2 + k, tb[2], px[2], zc[k], zf[k]);
-                const float r2 = rp * rp;
-                for (int i = 0; i < 5; ++i) {
-                    float xc, xf;
-                    cell_dist(t, 0, ic[0] - 2 + i, tb[0], px[0], xc, xf);
-                    xc = square(xc);
-                    xf = square(xf);
-                    if (fminf(xc, xf) >= r2) continue;
-                    for (int j = 0; j < 5; ++j) {
-                        float yc, yf;
-                        cell_dist(t, 1, ic[1] - 2 + j, tb[1], px[1], yc, yf);
-                        yc = square(yc);
-                        yf = square(yf);
-                        if (fminf(xc, xf) + fminf(yc, yf) >= r2) continue;
-                        const int row = ((ic[0] - 2 + i - t.t0[0] + R) * E + ic[1] - 2 + j - t.t0[1] + R) * E +
-                                        ic[2] - 2 - t.t0[2] + R;
+                    for (int k = 0; k < 5; ++k) cell_dist(t, 2, ic[2] - 2 + k, tb[2], px[2], zc[k], zf[k]);
+                    const float r2 = rp * rp;
+                    for (int i = 0; i < 5; ++i) {
+                        float xc, xf;
+                        cell_dist(t, 0, ic[0] - 2 + i, tb[0], px[0], xc, xf);
+                        xc = square(xc);
+                        xf = square(xf);
+                        if (fminf(xc, xf) >= r2) continue;
+                        for (int j = 0; j < 5; ++j) {
+                            float yc, yf;
+                            cell_dist(t, 1, ic[1] - 2 + j, tb[1], px[1], yc, yf);
+                            yc = square(yc);
+                            yf = square(yf);
+                            if (fminf(xc, xf) + fminf(yc, yf) >= r2) continue;
+                            const int row = ((ic[0] - 2 + i - t.t0[0] + R) * E + ic[1] - 2 + j - t.t0[1] + R) * E +
+                                            ic[2] - 2 - t.t0[2] + R;
 #pragma unroll
-                        for (int k = 0; k < 5; ++k) {
-                            const float wt[4] = {
-                                eq6_weight(0, xc, yc, zc[k], inv_r2), eq6_weight(1, xf, yc, zc[k], inv_r2),
-                                eq6_weight(2, xc, yf, zc[k], inv_r2), eq6_weight(3, xc, yc, zf[k], inv_r2)};
+                            for (int k = 0; k < 5; ++k) {
+                                const float wt[4] = {
+                                    eq6_weight(0, xc, yc, zc[k], inv_r2), eq6_weight(1, xf, yc, zc[k], inv_r2),
+                                    eq6_weight(2, xc, yf, zc[k], inv_r2), eq6_weight(3, xc, yc, zf[k], inv_r2)};
 #pragma unroll
-                            for (int q4 = 0; q4 < 4; ++q4) {
-                                if (!(wt[q4] > 0.0f)) continue;
-                                const float wm = wt[q4] * mp;
-                                if (q4 == 0) {
-                                    add(0, row + k, wm, c.mass_scale);
-                                    add(1, row + k, wt[0], c.w_scale);
-                                } else {
-                                    add(1 + q4, row + k, wm, c.mass_scale);
-                                    add(4 + q4, row + k, wm * vel[q4 - 1], c.mom_scale);
+                                for (int q4 = 0; q4 < 4; ++q4) {
+                                    if (!(wt[q4] > 0.0f)) continue;
+                                    const float wm = wt[q4] * mp;
+                                    if (q4 == 0) {
+                                        add(0, row + k, wm, c.mass_scale);
+                                        add(1, row + k, wt[0], c.w_scale);
+                                    } else {
+                                        add(1 + q4, row + k, wm, c.mass_scale);
+                                        add(4 + q4, row + k, wm * vel[q4 - 1], c.mom_scale);
+                                    }
                                 }
                             }
                         }
@@ -541,101 +577,209 @@ __global__ __launch_bounds__(P2GTile<R>::NT) void k_mr_p2g_tile(MGrid g, int chu
                 }
             }
         }
-    }
-    if (R == 1) {
-        const bool any = __syncthreads_or(coarse);
-        if (tid == 0) *flag = any ? 1 : 0;
-    } else {
-        __syncthreads();
-    }
-    // flush: an entry beyond the block belongs to the neighbouring block
-    const int64_t nc = g.ncells;
-    const int ext = t.tn + 2 * R;
-    for (int e = tid; e < E3; e += NT) {
-        const int ek = e % E, ej = e / E % E, ei = e / (E * E);
-        if (ei >= ext || ej >= ext || ek >= ext) continue;
-        bool any = false;
-#pragma unroll
-        for (int ch = 0; ch < kAcc; ++ch) any = any || L[ch * E3 + e] != 0ull;
-        if (!any) continue;
-        const int i = t.t0[0] + ei - R, j = t.t0[1] + ej - R, k = t.t0[2] + ek - R;
-        const int di = i < 0 ? -1 : (i >= t.nn ? 1 : 0), dj = j < 0 ? -1 : (j >= t.nn ? 1 : 0),
-                  dk = k < 0 ? -1 : (k >= t.nn ? 1 : 0);
-        int base = t.base;
-        if (di | dj | dk)  // (non-zero entries only lie in blocks of this level)
-            base = g.coff[g.slot[((t.b[0] + di) * g.nby + t.b[1] + dj) * g.nbz + t.b[2] + dk]];
-        const int64_t a = base + ((i - di * t.nn) * t.nn + j - dj * t.nn) * t.nn + k - dk * t.nn;
-#pragma unroll
-        for (int ch = 0; ch < kAcc; ++ch) {
-            const unsigned long long val = L[ch * E3 + e];
-            if (val != 0ull) atomicAdd(acc + ch * nc + a, val);
+        if (R == 1) {
+            const bool any = __syncthreads_or(coarse);
+            if (tid == 0) *flag = any ? 1 : 0;
+            const int walk = s_n;
+            if (walk > kP2GLight) {
+                if (tid == 0) heavy[atomicAdd(nlist + 1, 1)] = make_int2(slot, sub);
+            } else if (walk > 0) {
+                if (tid == 0) s_at = atomicAdd(nlist, walk);
+                __syncthreads();
+                for (int e = tid; e < walk; e += NT) list[s_at + e] = s_walk[e];
+            }
+        } else {
+            __syncthreads();
         }
-    }
-}
-
-// The listed particles, by the walk: a workgroup keeps a hash of kP2GSlots
-// cells in LDS (tag + the 8 fixed-point channels), adds there with LDS
-// atomics, and flushes every cached cell with one global atomic per non-zero
-// channel.  A contribution whose slot holds another cell goes to global
-// memory directly.  Integer sums, so the result equals the uncached kernel's
-// bit for bit.  kP2GParts threads share a particle: one particle's walk is a
-// serial chain over up to a few hundred cells, and 46k particles (0.5 % of a
-// 9.2M dam break) at one per thread were 180 workgroups waiting for it.
-// 1, 2, 4, 8 threads:
-// 350, 300, 221, 253 us; in a flow that lists far more of them 795, 725, 705,
-// 730, and 16 or 32 threads 855 and 1030.
-constexpr int kP2GSlots = 512;
-constexpr int kP2GParts = 4;
-constexpr int kP2GPerBlock = 256 / kP2GParts;  // particles per chunk
-constexpr unsigned kP2GListBlocks = 1024;
-static_assert(kP2GSlots == 1 << 9, "the slot hash keeps 9 bits");
-
-__global__ __launch_bounds__(256) void k_mr_p2g_list(MGrid g, const float* __restrict__ x, const float* __restrict__ v,
-                                                     const int* __restrict__ type, const int* __restrict__ lev,
-                                                     const int* __restrict__ list, const int* __restrict__ nlist,
-                                                     const int* __restrict__ perm, const int* __restrict__ outside,
-                                                     int np, MRConst c, unsigned long long* __restrict__ acc) {
-    __shared__ int tag[kP2GSlots];
-    __shared__ unsigned long long lacc[kP2GSlots * kAcc];
-    const int64_t nc = g.ncells;
-    // the listed ones, then those outside every block (the last of the order)
-    const int nl = *nlist, out0 = *outside, n = nl + (np - out0);
-    for (int64_t p0 = blockIdx.x * kP2GPerBlock; p0 < n; p0 += gridDim.x * kP2GPerBlock) {
-        for (int s = threadIdx.x; s < kP2GSlots; s += blockDim.x) tag[s] = -1;
-        for (int s = threadIdx.x; s < kP2GSlots * kAcc; s += blockDim.x) lacc[s] = 0ull;
-        __syncthreads();
-        const int64_t q = p0 + (int)threadIdx.x / kP2GParts;
-        if (q < n) {
-            const int64_t p = q < nl ? list[q] : perm[out0 + q - nl];
-            splat_particle<kP2GParts>(g, x, v, type, lev, p, c, [&](int addr, const long long* val, unsigned mask) {
-                const int s = (int)(((unsigned)addr * 2654435761u) >> 23);  // 9-bit multiplicative hash
-                int t = tag[s];
-                if (t != addr && t == -1) {
-                    t = atomicCAS(tag + s, -1, addr);
-                    if (t == -1) t = addr;
-                }
-                if (t == addr) {
+        // flush: an entry beyond the block belongs to the neighbouring block
+        const int64_t nc = g.ncells;
+        for (int e0 = tid; e0 < ext3; e0 += NT) {
+            int ei, ej, ek;
+            const int e = entry(e0, ei, ej, ek);
+            bool any = false;
 #pragma unroll
-                    for (int ch = 0; ch < kAcc; ++ch)
-                        if (mask & (1u << ch)) atomicAdd(lacc + s * kAcc + ch, (unsigned long long)val[ch]);
-                } else {
-#pragma unroll
-                    for (int ch = 0; ch < kAcc; ++ch)
-                        if (mask & (1u << ch)) atomicAdd(acc + ch * nc + addr, (unsigned long long)val[ch]);
-                }
-            }, (int)threadIdx.x % kP2GParts);
-        }
-        __syncthreads();
-        for (int s = threadIdx.x; s < kP2GSlots; s += blockDim.x) {
-            const int a = tag[s];
-            if (a < 0) continue;
+            for (int ch = 0; ch < kAcc; ++ch) any = any || L[ch * E3 + e] != 0ull;
+            if (!any) continue;
+            const int i = t.t0[0] + ei - R, j = t.t0[1] + ej - R, k = t.t0[2] + ek - R;
+            const int di = i < 0 ? -1 : (i >= t.nn ? 1 : 0), dj = j < 0 ? -1 : (j >= t.nn ? 1 : 0),
+                      dk = k < 0 ? -1 : (k >= t.nn ? 1 : 0);
+            int base = t.base;
+            if (di | dj | dk)  // (non-zero entries only lie in blocks of this level)
+                base = g.coff[g.slot[((t.b[0] + di) * g.nby + t.b[1] + dj) * g.nbz + t.b[2] + dk]];
+            const int64_t a = base + ((i - di * t.nn) * t.nn + j - dj * t.nn) * t.nn + k - dk * t.nn;
 #pragma unroll
             for (int ch = 0; ch < kAcc; ++ch) {
-                const unsigned long long val = lacc[s * kAcc + ch];
+                const unsigned long long val = L[ch * E3 + e];
                 if (val != 0ull) atomicAdd(acc + ch * nc + a, val);
             }
         }
         __syncthreads();
+    }
+}
+
+// The particles left to the walk: a workgroup keeps a hash of kP2GSlots
+// cells in LDS (tag + the 8 fixed-point channels), adds there with LDS
+// atomics, and flushes every cached cell with one global atomic per non-zero
+// channel.  A contribution whose slot holds another cell goes to global
+// memory directly.  Integer sums, so the result equals the uncached kernel's
+// bit for bit.
+constexpr int kP2GSlots = 512;
+constexpr unsigned kP2GWalkBlocks = 1024;
+static_assert(kP2GSlots == 1 << 9, "the slot hash keeps 9 bits");
+
+// 256 / PARTS particles, or none (p < 0), one per PARTS threads
+template <int PARTS>
+__device__ inline void p2g_walk(const MGrid& g, const float* __restrict__ x, const float* __restrict__ v,
+                                const int* __restrict__ type, const int* __restrict__ lev, int64_t p, const MRConst& c,
+                                int* tag, unsigned long long* lacc, unsigned long long* __restrict__ acc) {
+    const int64_t nc = g.ncells;
+    for (int s = threadIdx.x; s < kP2GSlots; s += 256) tag[s] = -1;
+    for (int s = threadIdx.x; s < kP2GSlots * kAcc; s += 256) lacc[s] = 0ull;
+    __syncthreads();
+    if (p >= 0)
+        splat_particle<PARTS>(g, x, v, type, lev, p, c, [&](int addr, const long long* val, unsigned mask) {
+            const int s = (int)(((unsigned)addr * 2654435761u) >> 23);  // 9-bit multiplicative hash
+            int t = tag[s];
+            if (t != addr && t == -1) {
+                t = atomicCAS(tag + s, -1, addr);
+                if (t == -1) t = addr;
+            }
+            if (t == addr) {
+#pragma unroll
+                for (int ch = 0; ch < kAcc; ++ch)
+                    if (mask & (1u << ch)) atomicAdd(lacc + s * kAcc + ch, (unsigned long long)val[ch]);
+            } else {
+#pragma unroll
+                for (int ch = 0; ch < kAcc; ++ch)
+                    if (mask & (1u << ch)) atomicAdd(acc + ch * nc + addr, (unsigned long long)val[ch]);
+            }
+        }, (int)threadIdx.x % PARTS);
+    __syncthreads();
+    for (int s = threadIdx.x; s < kP2GSlots; s += 256) {
+        const int a = tag[s];
+        if (a < 0) continue;
+#pragma unroll
+        for (int ch = 0; ch < kAcc; ++ch) {
+            const unsigned long long val = lacc[s * kAcc + ch];
+            if (val != 0ull) atomicAdd(acc + ch * nc + a, val);
+        }
+    }
+    __syncthreads();
+}
+
+// The listed particles and those outside the grid, kP2GParts threads each:
+// one particle's walk is a serial chain over up to a few hundred cells, and 46k
+// particles (0.5 % of a 9.2M dam break) at one per thread were 180 workgroups
+// waiting for it: 1, 2, 4, 8 threads: 350, 300, 221, 253 us; in a flow that
+// lists far more of them 795, 725, 705, 730, and 16 or 32 threads 855 and 1030.
+// Then the blocks of fewer than 4 cells per axis, and the tiles that leave many,
+// an eighth (8 rows of 8 cells) per workgroup, in the cells' order, in which the
+// particles of a workgroup share cells: with jumps between all blocks of 16^3
+// cells, alternately of levels 0 and 1, P2G of 16.8M particles took 8.8 ms from
+// the list, 4.1 so (3.1 where all are walked: those that a tile has taken leave
+// gaps).  nlist NULL: every particle, in that order.
+constexpr int kP2GParts = 4;
+
+__global__ __launch_bounds__(256) void k_mr_p2g_walk(MGrid g, const float* __restrict__ x, const float* __restrict__ v,
+                                                     const int* __restrict__ type, const int* __restrict__ lev,
+                                                     const int* __restrict__ list, const int2* __restrict__ heavy,
+                                                     const int* __restrict__ nlist, const int* __restrict__ perm,
+                                                     const int* __restrict__ start, int np, MRConst c,
+                                                     unsigned long long* __restrict__ acc) {
+    __shared__ int tag[kP2GSlots];
+    __shared__ unsigned long long lacc[kP2GSlots * kAcc];
+    if (!nlist) {
+        for (int64_t p0 = blockIdx.x * 256; p0 < np; p0 += gridDim.x * 256) {
+            const int64_t q = p0 + threadIdx.x;
+            p2g_walk<1>(g, x, v, type, lev, q < np ? perm[q] : -1, c, tag, lacc, acc);
+        }
+        return;
+    }
+    const int nl = nlist[0], out0 = start[g.ncells], n = nl + (np - out0);
+    constexpr int B = 256 / kP2GParts;
+    for (int64_t p0 = blockIdx.x * B; p0 < n; p0 += gridDim.x * B) {
+        const int64_t q = p0 + (int)threadIdx.x / kP2GParts;
+        const int p = q < n ? (q < nl ? list[q] : perm[out0 + q - nl]) : -1;
+        p2g_walk<kP2GParts>(g, x, v, type, lev, p, c, tag, lacc, acc);
+    }
+    // the blocks of fewer than 4 cells per axis, 32 neighbours in the order at a
+    // time and of their particles every fourth 256
+    const int groups = (g.nslots + 31) / 32;
+    __shared__ int first[32], before[33], some[512], nsome;
+    const int lane = threadIdx.x & 63;
+    for (int w = blockIdx.x; w < 4 * groups; w += gridDim.x) {
+        const int slot = 32 * (w % groups) + (int)threadIdx.x;
+        if (threadIdx.x < 64) {
+            int f = 0, len = 0;
+            if (threadIdx.x < 32 && slot < g.nslots) {
+                const int nn = g.n0 >> g.blev[slot], a = g.coff[slot];
+                if (nn < 4) {
+                    f = start[a];
+                    len = start[a + nn * nn * nn] - f;
+                }
+            }
+            int sum = len;
+#pragma unroll
+            for (int o = 1; o < 32; o <<= 1) {
+                const int t = __shfl_up(sum, o, 64);
+                sum += lane >= o ? t : 0;
+            }
+            if (threadIdx.x < 32) {
+                first[lane] = f;
+                before[lane + 1] = sum;
+            }
+            if (threadIdx.x == 0) before[0] = 0;
+        }
+        __syncthreads();
+        const int m = before[32];
+        for (int q0 = 256 * (w / groups); q0 < m; q0 += 1024) {
+            const int q = q0 + (int)threadIdx.x;
+            int r = 0;
+#pragma unroll
+            for (int o = 16; o > 0; o >>= 1) r += q >= before[r + o] ? o : 0;
+            p2g_walk<1>(g, x, v, type, lev, q < m ? perm[first[r] + q - before[r]] : -1, c, tag, lacc, acc);
+        }
+        __syncthreads();
+    }
+    const int nw = 8 * nlist[1];
+    for (int w = blockIdx.x; w < nw; w += gridDim.x) {
+        const int2 h = heavy[w >> 3];
+        const int nn = g.n0 >> g.blev[h.x], tn = min(nn, 8), ns = nn / tn, li = w & 7;
+        if (li >= tn) continue;
+        if ((int)threadIdx.x < tn) {
+            const int i = h.y / (ns * ns) * tn + li, j = h.y / ns % ns * tn + (int)threadIdx.x, k = h.y % ns * tn;
+            const int a = g.coff[h.x] + (i * nn + j) * nn + k;
+            first[threadIdx.x] = start[a];
+            before[threadIdx.x + 1] = start[a + tn] - start[a];
+        }
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            before[0] = 0;
+            for (int r = 0; r < tn; ++r) before[r + 1] += before[r];
+        }
+        __syncthreads();
+        const int m = before[tn];
+        if (threadIdx.x == 0) nsome = 0;
+        __syncthreads();
+        for (int q0 = 0; q0 < m; q0 += 256) {
+            // the marked ones, walked 256 at a time
+            const int q = q0 + (int)threadIdx.x;
+            int r = 0;
+            while (r + 1 < tn && q >= before[r + 1]) ++r;
+            const int e = q < m ? perm[first[r] + q - before[r]] : 0;
+            if (e < 0) some[atomicAdd(&nsome, 1)] = ~e;
+            __syncthreads();
+            const int have = nsome;
+            __syncthreads();
+            if (have < 256 && q0 + 256 < m) continue;
+            p2g_walk<1>(g, x, v, type, lev, (int)threadIdx.x < have ? some[threadIdx.x] : -1, c, tag, lacc, acc);
+            const int rest = max(have - 256, 0), later = (int)threadIdx.x < rest ? some[256 + threadIdx.x] : 0;
+            if (q0 + 256 >= m && rest > 0)
+                p2g_walk<1>(g, x, v, type, lev, (int)threadIdx.x < rest ? later : -1, c, tag, lacc, acc);
+            some[threadIdx.x] = later;
+            if (threadIdx.x == 0) nsome = rest;
+            __syncthreads();
+        }
     }
 }
 
@@ -1402,8 +1546,9 @@ PF_API int pf_mr_p2g(const pf_msbg_grid* g, const pf_mr_particles* ps, const pf_
 }
 
 PF_API int64_t pf_mr_p2g_scratch_ints(int64_t n, int32_t ncells) {
-    // key, rank, perm (n each); count (ncells + 1); start (ncells + 2); scan
-    return 3 * (n > 0 ? n : 1) + 2 * ((int64_t)ncells + 2) + scan_tmp_ints((int64_t)ncells + 1);
+    // key, rank, perm (n each); count (ncells + 1, then flags of as many blocks
+    // and of ncells / 512 tiles); start (ncells + 2); scan
+    return 3 * (n > 0 ? n : 1) + 2 * ((int64_t)ncells + 2) + cdiv(ncells, 512) + scan_tmp_ints((int64_t)ncells + 1);
 }
 
 PF_API int pf_mr_p2g_sorted(const pf_msbg_grid* g, const pf_mr_particles* ps, const pf_mr_params* prm,
@@ -1421,7 +1566,7 @@ PF_API int pf_mr_p2g_sorted(const pf_msbg_grid* g, const pf_mr_particles* ps, co
     int* rank = key + n;
     int* perm = rank + n;
     int* count = perm + n;
-    int* start = count + (nk + 1);
+    int* start = count + (nk + 1) + cdiv(g->ncells, 512);
     int* tmp = start + (nk + 1);
     hipStream_t s = S(stream);
     rc = fill_u32(count, nk, 0u, s);
@@ -1431,24 +1576,33 @@ PF_API int pf_mr_p2g_sorted(const pf_msbg_grid* g, const pf_mr_particles* ps, co
     PF_CHECK_LAUNCH();
     rc = exclusive_scan(count, nk, start, tmp, s);
     if (rc) return rc;
-    // the scan's scratch and the counts are free now: the walk list's length,
-    // and a flag per tile (at the block's first cell + tile); the list takes
-    // the keys' place once the scatter has read them
+    // the scan's scratch and the counts are free now: the lengths of the walk's
+    // lists, and a flag per workgroup of the tiles (then at the first cell of a
+    // block of 4 cells per axis); the lists take the places of the keys and
+    // ranks once the scatter has read them
     int* nlist = tmp;
     k_mr_cell_scatter<<<pgrid(n), 256, 0, s>>>(key, rank, start, n, perm, nlist);
     PF_CHECK_LAUNCH();
     const MRConst c = mrconst(*prm);
     unsigned long long* acc = reinterpret_cast<unsigned long long*>(f->acc);
-    const int chunks = (int)cdiv(m.ncells, 512);
-    const unsigned tiles = (unsigned)chunks + (unsigned)m.nslots;
-    k_mr_p2g_tile<1><<<tiles, P2GTile<1>::NT, 0, s>>>(m, chunks, ps->x, ps->v, ps->type, ps->level, perm, start, c,
-                                                      count, key, nlist, acc);
-    PF_CHECK_LAUNCH();
-    k_mr_p2g_tile<2><<<tiles, P2GTile<2>::NT, 0, s>>>(m, chunks, ps->x, ps->v, ps->type, ps->level, perm, start, c,
-                                                      count, key, nlist, acc);
-    PF_CHECK_LAUNCH();
-    k_mr_p2g_list<<<kP2GListBlocks, 256, 0, s>>>(m, ps->x, ps->v, ps->type, ps->level, key, nlist, perm, start + g->ncells,
-                                                (int)n, c, acc);
+    // (a heavy tile has more than kP2GLight particles: the ranks' place holds
+    // their names)
+    int2* heavy = reinterpret_cast<int2*>(rank + (reinterpret_cast<uintptr_t>(rank) / 4 & 1));
+    // few particles leave most of the chip idle between the tile launches: 33k
+    // and 111k in tiles 77 and 80 us, all by the walk 65 and 75; 262k 86 and 109
+    const bool tiled = n >= (int64_t)1 << 17;
+    if (tiled) {
+        const int chunks = (int)cdiv(m.ncells, 512);
+        const unsigned tiles = (unsigned)chunks + (unsigned)std::min(m.nslots, kP2GWhole);
+        k_mr_p2g_tile<1><<<tiles, P2GTile<1>::NT, 0, s>>>(m, chunks, ps->x, ps->v, ps->type, ps->level, perm, start, c,
+                                                          count, key, heavy, nlist, acc);
+        PF_CHECK_LAUNCH();
+        k_mr_p2g_tile<2><<<tiles, P2GTile<2>::NT, 0, s>>>(m, chunks, ps->x, ps->v, ps->type, ps->level, perm, start, c,
+                                                          count, key, heavy, nlist, acc);
+        PF_CHECK_LAUNCH();
+    }
+    k_mr_p2g_walk<<<tiled ? kP2GWalkBlocks : std::min(kP2GWalkBlocks, cdiv(n, 256)), 256, 0, s>>>(m, ps->x, ps->v, ps->type, ps->level, key, heavy,
+                                                tiled ? nlist : nullptr, perm, start, (int)n, c, acc);
     PF_CHECK_LAUNCH();
     return PF_OK;
 }

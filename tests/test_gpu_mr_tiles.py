@@ -31,7 +31,7 @@ def test_tiled_p2g_equals_per_particle_atomics(nb, n0, max_level, seed):
     levels = rng.integers(0, max_level + 1, size=int(np.prod(nb)))
     sim = mrs.AdaptiveSimulator(cfg, nb, n0=n0, max_level=max_level, frozen_levels=levels)
     L = np.array(nb) * n0 * dx
-    n = 40000
+    n = 150000  # (fewer than 2^17 are all walked)
     x = rng.random((n, 3)) * L
     x[: n // 50] = rng.random((n // 50, 3)) * (1.2 * L) - 0.1 * L       # some outside the box
     on = rng.integers(0, n, size=n // 20)
@@ -52,6 +52,38 @@ def test_tiled_p2g_equals_per_particle_atomics(nb, n0, max_level, seed):
     assert np.abs(out[0]["fmass"]).max() > 0
 
 
+@pytest.mark.parametrize("n", [1, 1000, 131071, 131072, 400000])
+@pytest.mark.parametrize("levels,plev", [("checker", 0), ("checker", 1), ("small", 2), ("one", 0)])
+def test_tiled_p2g_leaves_particles_to_the_walk(n, levels, plev):
+    """Few particles (all walked), tiles that leave more than 512 particles to
+    the walk (all blocks facing others of another level, and particles finer
+    than their block), blocks of 4, 2 and 1 cells per axis among larger ones."""
+    from importlib import import_module
+    pf = load_pkg()
+    cfgm, mrs = (import_module(pf.__name__ + "." + m) for m in ("config", "mr_sim"))
+    print(f"[gpu] tiled adaptive P2G, walk {n} {levels} {plev}", flush=True)
+    rng = np.random.default_rng(n)
+    nb, n0, dx = (5, 4, 7), 8, 0.37 / 8
+    if levels == "checker":
+        n0 = 16
+    lv = {"checker": np.indices(nb).sum(0).ravel() % 2, "small": rng.integers(1, 4, 140), "one": np.zeros(140)}[levels]
+    cfg = cfgm.Config(res=tuple(k * n0 for k in nb), dx=dx, ppc=27, droplets=False)
+    sim = mrs.AdaptiveSimulator(cfg, nb, n0=n0, max_level=3, frozen_levels=lv.astype(int))
+    x = (rng.random((n, 3)) * np.array(nb) * n0 * dx).astype(np.float32)
+    x[::101] *= 1.3  # some outside
+    sim.set_particles(x, rng.standard_normal((n, 3)).astype(np.float32), rng.integers(0, 2, n).astype(np.int32),
+                      np.full(n, plev, np.int32))
+    sim._rebuild_grid(1e-3)
+    prm = sim._params(1e-3, sim._max_speed())
+    out = []
+    for sorted_ in (True, False, True):
+        sim.p2g_sorted = sorted_
+        sim.stage_p2g(prm)
+        out.append({k: getattr(sim, k).cpu().numpy().copy() for k in ("cwsum", "phi", "fmass", "fvel", "is_liquid")})
+    for k in out[0]:
+        assert np.array_equal(out[0][k], out[1][k]) and np.array_equal(out[2][k], out[1][k]), k
+
+
 def test_tiled_p2g_on_coarse_levels_of_large_blocks():
     """8192 blocks of 512^3 finest cells, all at one cell per block: as many
     tiles as blocks, where 2^31 would be one for every 8^3 finest cells."""
@@ -63,7 +95,7 @@ def test_tiled_p2g_on_coarse_levels_of_large_blocks():
     nb, n0, dx = (32, 16, 16), 512, 0.37 / 512
     cfg = cfgm.Config(res=tuple(n * n0 for n in nb), dx=dx, ppc=27, droplets=False)
     sim = mrs.AdaptiveSimulator(cfg, nb, n0=n0, max_level=9, frozen_levels=np.full(int(np.prod(nb)), 9))
-    n = 30000
+    n = 150000
     x = (rng.random((n, 3)) * np.array(nb) * n0 * dx).astype(np.float32)
     sim.set_particles(x, rng.standard_normal((n, 3)).astype(np.float32), np.ones(n, np.int32),
                       rng.choice([8, 9], n).astype(np.int32))
@@ -94,7 +126,7 @@ def test_particles_at_tile_edges_are_splatted_once(n0, level, coarser):
     nb, dx = (5, 4, 3), 0.37 / 11
     cfg = cfgm.Config(res=tuple(n * n0 for n in nb), dx=dx, ppc=27, droplets=False)
     sim = mrs.AdaptiveSimulator(cfg, nb, n0=n0, max_level=2, frozen_levels=np.full(int(np.prod(nb)), level))
-    n, edge = 30000, (8 << level) * np.float32(dx)
+    n, edge = 150000, (8 << level) * np.float32(dx)
     cells = np.array(nb) * n0 // (8 << level)
     x = (rng.random((n, 3)) * np.array(nb) * n0 * dx).astype(np.float32)
     on = rng.integers(0, 3, n)  # the axis along which it sits at an edge
