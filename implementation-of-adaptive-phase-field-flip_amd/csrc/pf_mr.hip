@@ -1070,12 +1070,15 @@ struct SampleTaps {
     float w[3][2][2];
     int at[3][2][2];   // local cell times the axis' stride
     int blk[3][2][2];  // 0, 1, 2 times 9, 3, 1
+    int cell[3];       // the sample's cell, in the grid at its level
+    bool below[3];     // ... and the one below it (else above) for the others
     int slot, base, level;
     bool cross;        // some tap is in another block
 };
 
-// false: no cell here.  A tap outside the grid takes the other one's place
-// with weight zero: it adds nothing to either sum.
+// false: no cell here.  A tap outside the grid, or of weight 0 (it may hold no
+// number), takes the other one's place with weight 0: it adds nothing to either
+// sum.  The sample's own cell has some weight in each component.
 __device__ inline bool sample_taps(const MGrid& g, const float (&x)[3], SampleTaps& t) {
     const int nb[3] = {g.nbx, g.nby, g.nbz};
     float u[3];
@@ -1102,13 +1105,17 @@ __device__ inline bool sample_taps(const MGrid& g, const float (&x)[3], SampleTa
         const int at0 = lc << shift, atm = ((lc - 1) & (n - 1)) << shift, atp = ((lc + 1) & (n - 1)) << shift;
         const int bm = lc == 0 ? 0 : bs, bp = lc == n - 1 ? 2 * bs : bs;
         const float tf = sf - floorf(sf), fc = floorf(sc), tc = sc - fc;
+        const bool next = hi && tf != 0.0f;
         t.w[a][0][0] = 1.0f - tf;
-        t.w[a][0][1] = hi ? tf : 0.0f;
+        t.w[a][0][1] = next ? tf : 0.0f;
         t.at[a][0][0] = at0;
         t.blk[a][0][0] = bs;
-        t.at[a][0][1] = hi ? atp : at0;
-        t.blk[a][0][1] = hi ? bp : bs;
-        const bool below = (int)fc < c, other = below ? lo : hi;  // the cell and the one below it, or above
+        t.at[a][0][1] = next ? atp : at0;
+        t.blk[a][0][1] = next ? bp : bs;
+        const bool below = (int)fc < c;  // the cell and the one below it, or above (tc >= 1/2 below)
+        const bool other = below ? lo : hi && tc != 0.0f;
+        t.cell[a] = c;
+        t.below[a] = below;
         const int ao = other ? (below ? atm : atp) : at0, bo = other ? (below ? bm : bp) : bs;
         t.w[a][1][0] = below && !lo ? 0.0f : 1.0f - tc;
         t.w[a][1][1] = !below && !hi ? 0.0f : tc;
@@ -1121,31 +1128,52 @@ __device__ inline bool sample_taps(const MGrid& g, const float (&x)[3], SampleTa
     return true;
 }
 
-// the 24 addresses; false: some tap's block has another level or is absent
-__device__ inline bool tap_addresses(const SampleTaps& t, const int* __restrict__ nbr, int (&addr)[3][8]) {
-    int ok = 0;
+// The 24 addresses; a tap whose block has another level is looked up by itself.
+// (With the whole sample by the walk instead, jumps between levels everywhere
+// cost more than no table at all: 2.1M particles over random levels, G2P 132 us
+// without it, 292 and now 124 with it; the advection 225, 400 and 284.)  false:
+// a tap with weight has no cell.
+__device__ inline bool tap_addresses(const MGrid& g, const SampleTaps& t, const int* __restrict__ nbr,
+                                     int (&addr)[3][8]) {
 #pragma unroll
     for (int ax = 0; ax < 3; ++ax)
 #pragma unroll
         for (int q = 0; q < 8; ++q)
             addr[ax][q] = t.at[0][ax != 0][q >> 2] + t.at[1][ax != 1][q >> 1 & 1] + t.at[2][ax != 2][q & 1];
-    if (t.cross) {
-        const int* nb = nbr + 27 * (int64_t)t.slot;
-#pragma unroll
-        for (int ax = 0; ax < 3; ++ax)
-#pragma unroll
-            for (int q = 0; q < 8; ++q) {
-                const int b = nb[t.blk[0][ax != 0][q >> 2] + t.blk[1][ax != 1][q >> 1 & 1] + t.blk[2][ax != 2][q & 1]];
-                ok |= b;
-                addr[ax][q] += b;
-            }
-    } else {
+    if (!t.cross) {
 #pragma unroll
         for (int ax = 0; ax < 3; ++ax)
 #pragma unroll
             for (int q = 0; q < 8; ++q) addr[ax][q] += t.base;
+        return true;
     }
-    return ok >= 0;
+    int all = 0;
+    const int* nb = nbr + 27 * (int64_t)t.slot;
+#pragma unroll
+    for (int ax = 0; ax < 3; ++ax)
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            const int b = nb[t.blk[0][ax != 0][q >> 2] + t.blk[1][ax != 1][q >> 1 & 1] + t.blk[2][ax != 2][q & 1]];
+            all |= b;
+            addr[ax][q] = b < 0 ? -1 : addr[ax][q] + b;
+        }
+    if (all >= 0) return true;
+    bool found = true;
+#pragma unroll
+    for (int ax = 0; ax < 3; ++ax)
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            if (addr[ax][q] >= 0) continue;
+            const int e[3] = {q >> 2, q >> 1 & 1, q & 1};
+            int x[3];
+#pragma unroll
+            for (int a = 0; a < 3; ++a) x[a] = (t.cell[a] + e[a] - (ax != a && t.below[a] ? 1 : 0)) << t.level;
+            const int at = locate(g, x[0], x[1], x[2]).addr;
+            found = found && (at >= 0 || !(tap_weight(t.w[0][ax != 0][e[0]], t.w[1][ax != 1][e[1]],
+                                                      t.w[2][ax != 2][e[2]]) > 0.0f));
+            addr[ax][q] = max(at, 0);
+        }
+    return found;
 }
 
 // the samples of sample_face for all three components: the same values,
@@ -1163,7 +1191,7 @@ __device__ inline void tap_sum(const SampleTaps& t, const int (&addr)[3][8], con
 #pragma unroll
         for (int q = 0; q < 8; ++q) {
             const float w = tap_weight(t.w[0][ax != 0][q >> 2], t.w[1][ax != 1][q >> 1 & 1], t.w[2][ax != 2][q & 1]);
-            acc = w > 0.0f ? fmaf(w, v[ax][q], acc) : acc;  // (a tap of weight 0 may be no number)
+            acc = fmaf(w, v[ax][q], acc);
             wsum += w;
         }
         out[ax] = wsum > 0.0f ? acc / wsum : 0.0f;
@@ -1198,9 +1226,9 @@ __global__ __launch_bounds__(256) void k_mr_neighbours(MGrid g, int* __restrict_
 
 // alpha_FLIP from the local grid spacing (particles.py:251-276), then
 // u_p = alpha (u_p + I(du)) + (1 - alpha) I(u), eq. (12) (mr_kernels.py:413-430).
-// NEAR: with the table of sample_taps, the walk only for a particle that has a
-// tap in a block of another level.  9.2M particles, 6 % of them along 2:1
-// jumps: 672 us without the table, 378 with it.
+// NEAR: with the table of sample_taps, the walk only for a sample with a tap
+// that has no cell.  9.2M particles, 6 % of them along 2:1 jumps: 672 us
+// without the table, 365 with it.
 template <bool NEAR>
 __global__ __launch_bounds__(256) void k_mr_g2p(MGrid g, const int* __restrict__ nbr, const float* __restrict__ x,
                                                 float* __restrict__ v, const int* __restrict__ type, int64_t n,
@@ -1218,7 +1246,7 @@ __global__ __launch_bounds__(256) void k_mr_g2p(MGrid g, const int* __restrict__
         if (sample_taps(g, q, t)) {
             level = t.level;
             int addr[3][8];
-            if (tap_addresses(t, nbr, addr)) {
+            if (tap_addresses(g, t, nbr, addr)) {
                 tap_sum(t, addr, fdvel, delta);
                 tap_sum(t, addr, fvel, pic);
             } else {
@@ -1254,7 +1282,7 @@ __device__ inline float rk3_end(float x, float dt, float k1, float k2, float k3)
 // Ralston RK3 through the MSBG velocity, clamped to [lo, hi]
 // (mr_kernels.py:421-438), then the wall reflection of the velocity
 // (mr_kernels.py:441-461).  NEAR as above; one body for the three stages keeps
-// it at 123 registers.  9.2M particles: 1036 us without the table, 690 with it.
+// it at 128 registers.  9.2M particles: 1036 us without the table, 660 with it.
 template <bool NEAR>
 __global__ __launch_bounds__(256) void k_mr_advect(MGrid g, const int* __restrict__ nbr, float* __restrict__ x,
                                                    float* __restrict__ v, int64_t n, MRConst c,
@@ -1278,7 +1306,7 @@ __global__ __launch_bounds__(256) void k_mr_advect(MGrid g, const int* __restric
             SampleTaps t;
             if (sample_taps(g, y, t)) {
                 int addr[3][8];
-                if (tap_addresses(t, nbr, addr))
+                if (tap_addresses(g, t, nbr, addr))
                     tap_sum(t, addr, fvel, k);
                 else
                     sample_walk(g, fvel, y, k);

@@ -19,11 +19,12 @@ def mods():
     return {m: import_module(f"{PKG}.{m}") for m in ("_lib", "msbg")}
 
 
-# one block, single-cell blocks, every level, holes; a step of a fraction of a
-# cell and one of many blocks
+# one block, single-cell blocks, every level (graded 2:1 and not), holes; a step of
+# a fraction of a cell and one of many blocks
 @pytest.mark.parametrize("nb,n0,levels", [((1, 1, 1), 4, "fine"), ((3, 2, 4), 2, "random"), ((3, 2, 3), 1, "fine"),
                                           ((4, 3, 5), 8, "random"), ((4, 3, 5), 8, "holes"), ((3, 3, 3), 16, "random"),
-                                          ((4, 4, 4), 8, "fine")])
+                                          ((4, 4, 4), 8, "fine"), ((4, 3, 5), 8, "ungraded"),
+                                          ((3, 4, 3), 16, "ungraded holes")])
 @pytest.mark.parametrize("speed", [0.3, 30.0])
 def test_near_is_the_walk(mods, nb, n0, levels, speed):
     print("mr near", nb, n0, levels, speed, flush=True)
@@ -32,11 +33,11 @@ def test_near_is_the_walk(mods, nb, n0, levels, speed):
     top = n0.bit_length() - 1
     nblk = int(np.prod(nb))
     lv = np.zeros(nblk) if levels == "fine" else rng.integers(0, top + 1, nblk)
-    if levels == "holes":
+    if levels.endswith("holes"):
         lv[::7] = -1
     h0 = 1.0 / 24
     g = mods["msbg"].MSBG(nb, n0=n0, h0=h0, device="cuda:0", max_level=top)
-    g.build(lv.astype(np.int32))
+    g.build(lv.astype(np.int32), grade=not levels.startswith("ungraded"))
     dom = np.array(nb) * n0 * h0
     n = 6000
     x = rng.uniform(-0.02, 1.02, (n, 3)) * dom
