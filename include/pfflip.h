@@ -526,7 +526,9 @@ int pf_vec_axpby(float a, const float* x, float b, float* y, int64_t n, pf_strea
  * beta, rel, bnorm, tol, qAq, flag[0] as a double}; op 0 (init: bnorm = *a, tol), 1 (rz = *a),
  * 2 (alpha = rz / *a, or flag 1 when *a <= 0), 3 (rel = *a / bnorm, flag 2
  * below tol), 4 (beta = max((*a - *b) / rz, 0), rz = *a, or flag 3 when
- * rz == 0 or *a <= 0); ops 2-4 do nothing once flag[0] != 0. */
+ * rz == 0 or *a <= 0); ops 2-4 do nothing once flag[0] != 0.  MRSolver uses
+ * ops 0 and 1; pf_vec_axpby_dev and ops 2-4 are the single steps of the two
+ * calls below, for other solvers. */
 int pf_vec_axpby_dev(const double* st, int32_t ia, float a_sign, const float* x, int32_t ib, float* y, int64_t n,
                      const int32_t* flag, pf_stream_t stream);
 int pf_vec_remove_mean(float* x, int64_t n, double* work, pf_stream_t stream);
@@ -609,10 +611,10 @@ int pf_mr_max_speed(const float* v, int64_t n, float* out, pf_stream_t stream);
  * (particles.py:234-248) folded in: adds into acc. */
 int pf_mr_p2g(const pf_msbg_grid* g, const pf_mr_particles* ps, const pf_mr_params* prm, pf_mr_fields* f,
               pf_stream_t stream);
-/* pf_mr_p2g over a cell-sorted visit order with a per-workgroup LDS cache
- * of cells (a counting sort by cell address, then the splat); the same
- * sums as pf_mr_p2g bit for bit.  scratch holds
- * pf_mr_p2g_scratch_ints(n, ncells) int32. */
+/* pf_mr_p2g over a cell-sorted visit order (a counting sort by cell address,
+ * then the splat into LDS tiles of a block, what they cannot take by the walk
+ * with an LDS cache of cells); the same sums as pf_mr_p2g bit for bit.
+ * scratch holds pf_mr_p2g_scratch_ints(n, ncells) int32. */
 int64_t pf_mr_p2g_scratch_ints(int64_t n, int32_t ncells);
 int pf_mr_p2g_sorted(const pf_msbg_grid* g, const pf_mr_particles* ps, const pf_mr_params* prm, pf_mr_fields* f,
                      int32_t* scratch, pf_stream_t stream);
