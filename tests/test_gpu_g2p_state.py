@@ -86,12 +86,15 @@ def test_both_advections_give_the_same_step(pf, res, ppc, live, tiles):
         sim.set_particles(*pf.scenes.dam_break(cfg, frac=(0.4, 1.0, 0.6)))
         rng = np.random.default_rng(5)
         sim.pv.copy_(torch.from_numpy(rng.standard_normal((sim.n_particles, 3)).astype(np.float32)))
+        st = np.zeros(sim.n_particles, np.int32)
+        st[::40], st[7::90] = 1, 2
+        sim.pstate.copy_(torch.from_numpy(st))
         sim._live_droplets = live
         assert sim._advect_from_tiles() == tiles
         if forced is not None:
             sim._advect_from_tiles = lambda: forced
         recs = [sim.step(2e-3) for _ in range(2)]
         out.append((sim.px.clone(), sim.pv.clone(), sim.pstate.clone(), recs[-1]["droplets"], recs[-1]["pcg_iter"]))
-        print("  droplets", [r["droplets"] for r in recs], flush=True)
+        assert recs[0]["droplets"] > 0
     for o in out[1:]:
         assert all(torch.equal(a, b) for a, b in zip(o[:3], out[0][:3])) and o[3:] == out[0][3:]
